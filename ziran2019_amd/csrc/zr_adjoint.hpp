@@ -122,18 +122,18 @@ __device__ bool collide_jacobian(const ColliderSet& cs, double dt, const double 
   return true;
 }
 
-// reverse of tau = 2 mu (F - R) F^T + lam (J - 1) J I from the SVD of F:
-// adds (dtau/dF)^T taubar to Fb, returns mubar and lambar
+// reverse of tau = 2 mu (F - R) F^T + lam (J - 1) J I: adds (dtau/dF)^T
+// taubar to Fb, returns mubar and lambar.  The rotation's part is 2 mu R W
+// with the skew W that solves S W + W S = R^T A - A^T R, A = taubar F:
+// where Newton's iteration gives R (polar_newton), (tr S I - S) w = axial of
+// the right-hand side with S = R^T F; elsewhere in the SVD's frame, where W_ij
+// is divided by s_i + s_j.
 __device__ __forceinline__ void fcr_kirchhoff_adjoint(double mu, double lam, const M3<double>& f,
-                                                      const M3<double>& u, const double s[3], const M3<double>& v,
                                                       const double tb[3][3], double Fb[3][3], double& mub,
                                                       double& lab)
 {
-  double r[3][3], A[3][3], Ah[3][3], Mb[3][3], c[3][3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) r[i][j] = u.a[i][0] * v.a[j][0] + u.a[i][1] * v.a[j][1] + u.a[i][2] * v.a[j][2];
+  double A[3][3], W[3][3], c[3][3];
+  M3<double> r;
   const double J = det3(f);
   c[0][0] = f.a[1][1] * f.a[2][2] - f.a[1][2] * f.a[2][1];
   c[0][1] = f.a[1][2] * f.a[2][0] - f.a[1][0] * f.a[2][2];
@@ -149,43 +149,82 @@ __device__ __forceinline__ void fcr_kirchhoff_adjoint(double mu, double lam, con
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j) A[i][j] = tb[i][0] * f.a[0][j] + tb[i][1] * f.a[1][j] + tb[i][2] * f.a[2][j];
+  if (polar_newton(f, J, r)) {
+    double B[3][3], S[3][3];
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      double acc = 0.0;
+      for (int j = 0; j < 3; ++j) {
+        B[i][j] = r.a[0][i] * A[0][j] + r.a[1][i] * A[1][j] + r.a[2][i] * A[2][j];
+        S[i][j] = r.a[0][i] * f.a[0][j] + r.a[1][i] * f.a[1][j] + r.a[2][i] * f.a[2][j];
+      }
+    // G = tr S I - S, symmetric positive definite
+    const double g00 = S[1][1] + S[2][2], g11 = S[0][0] + S[2][2], g22 = S[0][0] + S[1][1];
+    const double g01 = -0.5 * (S[0][1] + S[1][0]), g02 = -0.5 * (S[0][2] + S[2][0]), g12 = -0.5 * (S[1][2] + S[2][1]);
+    const double h00 = g11 * g22 - g12 * g12, h11 = g00 * g22 - g02 * g02, h22 = g00 * g11 - g01 * g01;
+    const double h01 = g02 * g12 - g01 * g22, h02 = g01 * g12 - g02 * g11, h12 = g01 * g02 - g00 * g12;
+    const double inv = 1.0 / (g00 * h00 + g01 * h01 + g02 * h02);
+    const double a0 = B[2][1] - B[1][2], a1 = B[0][2] - B[2][0], a2 = B[1][0] - B[0][1];
+    const double w0 = inv * (h00 * a0 + h01 * a1 + h02 * a2), w1 = inv * (h01 * a0 + h11 * a1 + h12 * a2),
+                 w2 = inv * (h02 * a0 + h12 * a1 + h22 * a2);
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int l = 0; l < 3; ++l) acc += u.a[k][i] * A[k][l] * v.a[l][j];
-      Ah[i][j] = acc;
+    for (int i = 0; i < 3; ++i) {  // R [w]x
+      W[i][0] = r.a[i][1] * w2 - r.a[i][2] * w1;
+      W[i][1] = r.a[i][2] * w0 - r.a[i][0] * w2;
+      W[i][2] = r.a[i][0] * w1 - r.a[i][1] * w0;
     }
+  } else {
+    M3<double> u, v;
+    double s[3], Ah[3][3], Mb[3][3];
+    svd3(f, u, s, v);
 #pragma unroll
-  for (int i = 0; i < 3; ++i) Mb[i][i] = 0.0;
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
+      for (int j = 0; j < 3; ++j) {
+        r.a[i][j] = u.a[i][0] * v.a[j][0] + u.a[i][1] * v.a[j][1] + u.a[i][2] * v.a[j][2];
+        double acc = 0.0;
 #pragma unroll
-    for (int j = i + 1; j < 3; ++j) {
-      double den = s[i] + s[j];
-      if (fabs(den) < 1e-12) den = den < 0.0 ? -1e-12 : 1e-12;
-      const double x = (Ah[i][j] - Ah[j][i]) / den;
-      Mb[i][j] = x;
-      Mb[j][i] = -x;
-    }
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+          for (int l = 0; l < 3; ++l) acc += u.a[k][i] * A[k][l] * v.a[l][j];
+        Ah[i][j] = acc;
+      }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) Mb[i][i] = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = i + 1; j < 3; ++j) {
+        double den = s[i] + s[j];
+        if (fabs(den) < 1e-12) den = den < 0.0 ? -1e-12 : 1e-12;
+        const double x = (Ah[i][j] - Ah[j][i]) / den;
+        Mb[i][j] = x;
+        Mb[j][i] = -x;
+      }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          acc += u.a[i][k] * (Mb[k][0] * v.a[j][0] + Mb[k][1] * v.a[j][1] + Mb[k][2] * v.a[j][2]);
+        W[i][j] = acc;
+      }
+  }
   double mb = 0.0;
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      double t1 = 0.0, t2 = 0.0, t3 = 0.0, fr = 0.0;
+      double t1 = 0.0, t2 = 0.0, fr = 0.0;
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         t1 += (tb[i][k] + tb[k][i]) * f.a[k][j];
-        t2 += tb[k][i] * r[k][j];
-        t3 += u.a[i][k] * (Mb[k][0] * v.a[j][0] + Mb[k][1] * v.a[j][1] + Mb[k][2] * v.a[j][2]);
-        fr += (f.a[i][k] - r[i][k]) * f.a[j][k];
+        t2 += tb[k][i] * r.a[k][j];
+        fr += (f.a[i][k] - r.a[i][k]) * f.a[j][k];
       }
-      Fb[i][j] += 2.0 * mu * (t1 - t2 - t3) + lam * (2.0 * J - 1.0) * trtb * c[i][j];
+      Fb[i][j] += 2.0 * mu * (t1 - t2 - W[i][j]) + lam * (2.0 * J - 1.0) * trtb * c[i][j];
       mb += tb[i][j] * 2.0 * fr;
     }
   mub = mb;
@@ -372,7 +411,7 @@ __global__ __launch_bounds__(256) void k_adj_grid(uint32_t nn, const uint32_t* _
 // tile holds no SVD (one kernel of 256 VGPRs + 134 AGPRs ran at one wave
 // per SIMD): k_adj_stress writes V0 tau per particle, k_adj_p2g reverses
 // the momentum and stress transfer over the tile, k_adj_stress_rev reverses
-// the stress (the SVD again) into the F, mu and lambda adjoints.
+// the stress into the F, mu and lambda adjoints.
 
 // forward V0 tau = V0 (2 mu (F - R) F^T + lam (J - 1) J I), per particle
 __global__ __launch_bounds__(256) void k_adj_stress(ParticlesView P, AdjointView A, uint32_t n)
@@ -380,27 +419,17 @@ __global__ __launch_bounds__(256) void k_adj_stress(ParticlesView P, AdjointView
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i >= n) return;
   const int64_t S = P.stride;
-  M3<double> f, u, v;
-  double s[3];
+  M3<double> f, tau;
 #pragma unroll
   for (int c = 0; c < 3; ++c)
 #pragma unroll
     for (int r = 0; r < 3; ++r) f.a[r][c] = P.F[(c * 3 + r) * S + i];
-  svd3(f, u, s, v);
-  const double mu = P.mu[i], lam = P.lam[i], vol = P.vol[i];
-  const double J = det3(f);
+  const double vol = P.vol[i];
+  fcr_kirchhoff(P.mu[i], P.lam[i], f, tau);
 #pragma unroll
   for (int r = 0; r < 3; ++r)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      double acc = 0.0;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const double rk = u.a[r][0] * v.a[k][0] + u.a[r][1] * v.a[k][1] + u.a[r][2] * v.a[k][2];
-        acc += (f.a[r][k] - rk) * f.a[c][k];
-      }
-      A.vt[(c * 3 + r) * S + i] = vol * (2.0 * mu * acc + (r == c ? lam * (J - 1.0) * J : 0.0));
-    }
+    for (int c = 0; c < 3; ++c) A.vt[(c * 3 + r) * S + i] = vol * tau.a[r][c];
 }
 
 // the transfer's reverse over the group's node tile (per group): x, v and C
@@ -511,19 +540,20 @@ __global__ __launch_bounds__(256) void k_adj_p2g(ParticlesView P, AdjointView A,
 }
 
 // the stress's reverse per particle: F adjoint = that of the F update plus
-// (d V0 tau / dF)^T tb, and the mu and lambda adjoints accumulated
+// (d V0 tau / dF)^T tb, and the mu and lambda adjoints accumulated.  198 VGPRs
+// with both of the rotation's paths (two waves per SIMD), 16.9 us on 262,144
+// particles against 26.7 with the SVD alone at three; held to three waves it
+// spills 30 registers and takes 30.1
 __global__ __launch_bounds__(256) void k_adj_stress_rev(ParticlesView P, AdjointView A, uint32_t n)
 {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i >= n) return;
   const int64_t S = P.stride;
-  M3<double> f, u, v;
-  double s[3];
+  M3<double> f;
 #pragma unroll
   for (int c = 0; c < 3; ++c)
 #pragma unroll
     for (int r = 0; r < 3; ++r) f.a[r][c] = P.F[(c * 3 + r) * S + i];
-  svd3(f, u, s, v);
   const double mu = P.mu[i], lam = P.lam[i], vol = P.vol[i];
   double Fb[3][3], tb[3][3];
 #pragma unroll
@@ -534,7 +564,7 @@ __global__ __launch_bounds__(256) void k_adj_stress_rev(ParticlesView P, Adjoint
       tb[r][c] = A.tb[(c * 3 + r) * S + i] * vol;
     }
   double mub, lab;
-  fcr_kirchhoff_adjoint(mu, lam, f, u, s, v, tb, Fb, mub, lab);
+  fcr_kirchhoff_adjoint(mu, lam, f, tb, Fb, mub, lab);
 #pragma unroll
   for (int c = 0; c < 3; ++c)
 #pragma unroll
