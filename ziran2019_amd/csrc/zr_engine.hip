@@ -370,9 +370,12 @@ __global__ void k_scatter(uint32_t n, const uint32_t* p_page, const uint32_t* p_
 // sorts each group's keys (cell << 32 | particle index) ascending: the
 // particles are bucketed by cell (LDS counters), and each particle's place in
 // its cell's bucket is the number of the bucket's indices below its own
+// and records where each cell's run begins within the group (cell_off,
+// 32 entries per group), for the transfers that work cell by cell
 __global__ __launch_bounds__(256) void k_sort_groups(const uint64_t* __restrict__ keys,
                                                      const uint32_t* __restrict__ group_start,
-                                                     uint32_t* __restrict__ order, GroupBound gb)
+                                                     uint32_t* __restrict__ order, uint32_t* __restrict__ cell_off,
+                                                     GroupBound gb)
 {
   __shared__ uint32_t bucket[kSortLds];  // particle indices by cell, unordered within a cell
   __shared__ uint32_t pidx[kSortLds];    // particle index of each key position
@@ -384,25 +387,17 @@ __global__ __launch_bounds__(256) void k_sort_groups(const uint64_t* __restrict_
   if (g >= gb.get()) return;
   const uint32_t start = group_start[g];
   const uint32_t n = group_start[g + 1] - start;
-  if (n > (uint32_t)kSortLds) {
-    // a page holding more than kSortLds particles: rank sort over its keys
-    // in memory (the keys are unique)
-    for (uint32_t k = tid; k < n; k += 256) {
-      const uint64_t key = keys[start + k];
-      uint32_t rank = 0;
-      for (uint32_t j = 0; j < n; ++j) rank += keys[start + j] < key ? 1u : 0u;
-      order[start + rank] = (uint32_t)(key & 0xffffffffull);
-    }
-    return;
-  }
   if (tid < 32) cnt[tid] = 0u;
   __syncthreads();
+  const bool in_lds = n <= (uint32_t)kSortLds;
   for (uint32_t k = tid; k < n; k += 256) {
     const uint64_t key = keys[start + k];
     const uint32_t c = (uint32_t)(key >> 32) & 31u;
     const uint32_t slot = atomicAdd(&cnt[c], 1u);
-    code[k] = (uint16_t)(c | (slot << 5));
-    pidx[k] = (uint32_t)key;
+    if (in_lds) {
+      code[k] = (uint16_t)(c | (slot << 5));
+      pidx[k] = (uint32_t)key;
+    }
   }
   __syncthreads();
   if (tid < 64) {  // exclusive scan of the 32 cell counts
@@ -413,9 +408,23 @@ __global__ __launch_bounds__(256) void k_sort_groups(const uint64_t* __restrict_
       const uint32_t y = __shfl_up(incl, o, 64);
       if (tid >= o) incl += y;
     }
-    if (tid < 32) off[tid] = incl - v;
+    if (tid < 32) {
+      off[tid] = incl - v;
+      cell_off[32 * (size_t)g + tid] = incl - v;
+    }
   }
   __syncthreads();
+  if (!in_lds) {
+    // a page holding more than kSortLds particles: rank sort over its keys
+    // in memory (the keys are unique)
+    for (uint32_t k = tid; k < n; k += 256) {
+      const uint64_t key = keys[start + k];
+      uint32_t rank = 0;
+      for (uint32_t j = 0; j < n; ++j) rank += keys[start + j] < key ? 1u : 0u;
+      order[start + rank] = (uint32_t)(key & 0xffffffffull);
+    }
+    return;
+  }
   for (uint32_t k = tid; k < n; k += 256) {
     const uint32_t cs = code[k];
     bucket[off[cs & 31u] + (cs >> 5)] = pidx[k];
@@ -548,124 +557,228 @@ __device__ __forceinline__ void particle_kirchhoff_t(const ParticlesView& P, uin
 
 // FORCE = true: MLS with force (explicit).  FORCE = false: APIC mass and
 // momentum only, particlesToGridHelper<APIC> (MpmSimulationBase.cpp:563-608).
-// T: the precision of the per-particle terms (stress, weights, products);
-// the node sums are FP64 either way.  FUSED (with FORCE, inside a whole
-// explicit step of size fdt): the force term goes into the momentum sum as
-// mv + fdt f, so that the grid update's v + dt (f / m + g) becomes
-// (mv + dt f) / m + dt g, with three fields fewer to add per node
-// waves per SIMD the register budget is held to: three for the FP64 fused
-// NeoHookeanBorden instance, which would otherwise miss that occupancy by
-// one register
-template <int MODEL, class T, bool FUSED>
-constexpr int p2g_min_waves()
+// T: the precision of the per-particle terms (stress, products with the
+// mass); weights, moments and node sums are FP64 either way.  FUSED (with
+// FORCE, inside a whole explicit step of size fdt): the force term goes into
+// the momentum sum as mv + fdt f, so that the grid update's v + dt (f / m + g)
+// becomes (mv + dt f) / m + dt g, with three fields fewer to add per node.
+//
+// What a particle adds to a node is its weight times an affine function of
+// the node: w (q + L0 o0 + L1 o1 + L2 o2) with o = the node's offset from the
+// middle node of the stencil, in {-1, 0, 1}^3.  Over the particles of one
+// cell, which share their 27 nodes, the sums of w q and w L are a matrix
+// product, [16 moments x particles] [particles x 27 weights], and the node's
+// value follows from its four moments per direction.  So:
+//   phase 1  thread per particle of a chunk of 256: stress, then its 13
+//            moments (mass; q and L of three directions) and its three
+//            fractions as one row of 16 in LDS (columns exchanged by the
+//            particle's index, so that neither this phase's column stores
+//            nor the next one's row loads collide on banks)
+//   phase 2  wave per cell: v_mfma_f64_16x16x4 over the cell's particles,
+//            four at a time, with two accumulators (nodes 0-15 and 16-26);
+//            each lane forms its nodes' weights from the fractions.  Row
+//            4 t + d of the moments puts the four moments of direction d at
+//            one node into one lane's four accumulator registers (row 4 r +
+//            lane / 16 in register r), so the node's value takes three
+//            multiply-adds and no exchange, and goes into the wave's tile
+// 108 LDS adds per cell rather than per particle, all lanes on different
+// nodes.  The FP64 matrix pipe shares its issue with FP64 vector instructions
+// here (measured: they add up), so the gain is the LDS adds and the lanes'
+// order: neighbouring lanes now load neighbouring particles.
+typedef double v4d __attribute__((ext_vector_type(4)));
+constexpr int kMoments = 16;
+// waves per SIMD the register budget is held to: what the LDS allows (51 KB
+// with four fields, 64 KB with seven), and two for particles of mixed models,
+// whose instance spills 50 registers at three
+template <bool FORCE, bool FUSED, int MODEL>
+constexpr int p2g_waves()
 {
-  return MODEL == ZR_MODEL_NEO_HOOKEAN_BORDEN && sizeof(T) == sizeof(double) && FUSED ? 3 : 1;
+  return FORCE && (!FUSED || MODEL == kAnyModel) ? 2 : 3;
 }
+
+// the 1-D quadratic weight of stencil offset a (0, 1, 2) at fraction f =
+// x/dx - base, k (f - s) (f - s) + e as bspline_w forms it
+struct LaneWeight {
+  double s, k, e;
+  __device__ __forceinline__ void set(int a)
+  {
+    s = 1.5 - 0.5 * a;
+    k = a == 1 ? -1.0 : 0.5;
+    e = a == 1 ? 0.75 : 0.0;
+  }
+  __device__ __forceinline__ double operator()(double f) const
+  {
+    const double t = f - s;
+    return fma(k * t, t, e);
+  }
+};
+
+// one row of the staged moments: element j of row p
+__device__ __forceinline__ int moment_at(uint32_t p, uint32_t j) { return (int)(p * kMoments + (j ^ (p & 15u))); }
+
+// row 4 t + d: t = 0 the constant q_d, t = 1..3 L_d along axis t - 1
+// (multiplied by the spacing); e_d = the middle node minus the particle
+template <class T>
+__device__ __forceinline__ void store_moments(double* row, uint32_t p, double m, const T q[3], const T A[3][3],
+                                              const double e[3], double dx)
+{
+  row[moment_at(p, 3)] = m;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    double c = (double)q[d];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      c = fma((double)A[d][t], e[t], c);
+      row[moment_at(p, 4 * (t + 1) + d)] = (double)A[d][t] * dx;
+    }
+    row[moment_at(p, d)] = c;
+  }
+}
+
+// phase 2: the staged rows [0, count) of the chunk at c0 into the wave's tile
+// (fields f0, f0 + 1, f0 + 2 for the three directions, and the mass field
+// when `mass`)
+__device__ __forceinline__ void cells_to_tile(const double* row, const uint32_t* coff, uint32_t c0, uint32_t count,
+                                              double* wt, int f0, bool mass)
+{
+  // opaque, so that the lane's constants are formed here and not held in
+  // registers across phase 1
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));
+  const int wv = threadIdx.x >> 6;
+  const uint32_t col = (uint32_t)lane & 15u, kk = (uint32_t)lane >> 4;
+  LaneWeight W[2][3];
+  double o[2][3];
+  int toff[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int nd = h == 0 ? (int)col : (col < 11u ? 16 + (int)col : 26);
+    const int a = nd / 9, b = (nd / 3) % 3, c = nd % 3;
+    W[h][0].set(a);
+    W[h][1].set(b);
+    W[h][2].set(c);
+    // lanes 48..63 hold the mass (moment t = 0 only)
+    o[h][0] = kk == 3u ? 0.0 : (double)(a - 1);
+    o[h][1] = kk == 3u ? 0.0 : (double)(b - 1);
+    o[h][2] = kk == 3u ? 0.0 : (double)(c - 1);
+    toff[h] = (a * kTileY + b) * kTileZ + c + (kk == 3u ? 0 : (f0 + (int)kk) * kTileNodes);
+  }
+  const bool adds = kk != 3u || mass;
+#pragma unroll 1
+  for (int i = 0; i < 8; ++i) {
+    // eight cells per wave, spread over the page so that a page cut by the
+    // body's surface still gives every wave some
+    const int cx = i >> 2, cy = i & 3, cz = (wv + cy + 2 * cx) & 3;
+    const int e = (cx << 4) | (cy << 2) | cz;
+    const uint32_t b0 = coff[e], b1 = coff[e + 1];
+    const uint32_t kb = b0 > c0 ? b0 - c0 : 0u;
+    const uint32_t ke = b1 > c0 ? (b1 - c0 < count ? b1 - c0 : count) : 0u;
+    if (kb >= ke) continue;
+    v4d D[2] = { { 0.0, 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0, 0.0 } };
+    for (uint32_t k = kb; k < ke; k += 4u) {
+      const bool live = k + kk < ke;
+      const uint32_t p = live ? k + kk : ke - 1u;
+      const double m = row[moment_at(p, col)];
+      const double f[3] = { row[moment_at(p, 7)], row[moment_at(p, 11)], row[moment_at(p, 15)] };
+      const double a = live ? m : 0.0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const double w = W[h][0](f[0]) * W[h][1](f[1]) * W[h][2](f[2]);
+        D[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, w, D[h], 0, 0, 0);
+      }
+    }
+    const int t0 = (cx * kTileY + cy) * kTileZ + cz;
+    if (adds) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const double v = fma(o[h][2], D[h][3], fma(o[h][1], D[h][2], fma(o[h][0], D[h][1], D[h][0])));
+        if (h == 0 || col < 11u) atomicAdd(&wt[t0 + toff[h]], v);
+      }
+    }
+  }
+}
+
 template <bool FORCE, int MODEL = kAnyModel, class T = double, bool FUSED = false>
-__global__ __launch_bounds__(kTransferThreads, (p2g_min_waves<MODEL, T, FUSED>())) void k_p2g(ParticlesView P, const uint32_t* __restrict__ order,
-                                             const uint32_t* __restrict__ group_start,
-                                             const uint32_t* __restrict__ group_page, double* __restrict__ stage,
-                                             double dx, double inv_dx, double Dinv, double fdt)
+__global__ __launch_bounds__(kTransferThreads, (p2g_waves<FORCE, FUSED, MODEL>())) void k_p2g(
+    ParticlesView P, const uint32_t* __restrict__ order, const uint32_t* __restrict__ group_start,
+    const uint32_t* __restrict__ group_page, const uint32_t* __restrict__ cell_off, double* __restrict__ stage,
+    double dx, double inv_dx, double Dinv, double fdt)
 {
   static_assert(!FUSED || FORCE, "the fused form needs the force");
   constexpr int NF = FORCE && !FUSED ? kP2GFields : 4;
   constexpr int SS = NF * kTileNodes;
   constexpr int NT = kTransferThreads, NW = NT / 64;
+  static_assert(NW == 4, "eight of the 32 cells per wave");
   __shared__ double tile[NW * SS];
+  __shared__ double row[NT * kMoments];
+  __shared__ uint32_t coff[33];
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;
   for (int k = tid; k < NW * SS; k += NT) tile[k] = 0.0;
   const uint32_t start = group_start[g];
   const uint32_t n = group_start[g + 1] - start;
-  uint32_t px, py, pz;
-  page_decode(group_page[g], px, py, pz);
-  const int ox = 2 * (int)px, oy = 4 * (int)py, oz = 4 * (int)pz;
-  __syncthreads();
+  if (tid < 33) coff[tid] = tid < 32 ? cell_off[32 * (size_t)g + tid] : n;
   double* wt = tile + (tid >> 6) * SS;
-  // lanes of a wave take particles NT/32 apart so that they mostly sit in
-  // different cells and their LDS adds rarely collide
-  const uint32_t perm = (uint32_t)((tid & 31) * (NT / 32) + (tid >> 5));
   const int64_t S = P.stride;
-  for (uint32_t j0 = 0; j0 < n; j0 += NT) {
-    const uint32_t j = j0 + perm;
-    if (j >= n) continue;
-    const uint32_t i = order[start + j];
-    double xp[3] = { P.x[i], P.x[S + i], P.x[2 * S + i] };
-    const T mass = (T)P.m[i];
-    T mom[3] = { mass * (T)P.v[i], mass * (T)P.v[S + i], mass * (T)P.v[2 * S + i] };
-    T mC[3][3], st[3][3];
-    if constexpr (FORCE) {
-      M3<T> tau;
-      particle_kirchhoff_t<MODEL, T>(P, i, tau);
-      const T vol = (T)P.vol[i];
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int r = 0; r < 3; ++r) st[r][c] = vol * tau.a[r][c];
-      if (P.vtau_add)
+  for (uint32_t c0 = 0; c0 < n; c0 += NT) {
+    const uint32_t count = n - c0 < (uint32_t)NT ? n - c0 : (uint32_t)NT;
+    T st[3][3];
+    double e[3];
+    if ((uint32_t)tid < count) {
+      const uint32_t i = order[start + c0 + tid];
+      const double xp[3] = { P.x[i], P.x[S + i], P.x[2 * S + i] };
+      const T mass = (T)P.m[i];
+      T mom[3] = { mass * (T)P.v[i], mass * (T)P.v[S + i], mass * (T)P.v[2 * S + i] };
+      T A[3][3];
+      if constexpr (FORCE) {
+        M3<T> tau;
+        particle_kirchhoff_t<MODEL, T>(P, i, tau);
+        const T vol = (T)P.vol[i];
 #pragma unroll
         for (int c = 0; c < 3; ++c)
 #pragma unroll
-          for (int r = 0; r < 3; ++r) st[r][c] += (T)P.vtau_add[(c * 3 + r) * S + i];
-    }
+          for (int r = 0; r < 3; ++r) st[r][c] = vol * tau.a[r][c];
+        if (P.vtau_add)
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
+          for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int r = 0; r < 3; ++r) mC[r][c] = mass * (T)P.C[(c * 3 + r) * S + i];
-    // base node and the offsets x_i - x_p in FP64, the weights and the
-    // products in T
-    T w[3][3];
-    int b[3];
+            for (int r = 0; r < 3; ++r) st[r][c] += (T)P.vtau_add[(c * 3 + r) * S + i];
+        const T sc = (T)((FUSED ? fdt : 1.0) * Dinv);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      double w64[3];
-      b[d] = bspline_w(xp[d] * inv_dx, w64);
+        for (int r = 0; r < 3; ++r)
 #pragma unroll
-      for (int a = 0; a < 3; ++a) w[d][a] = (T)w64[a];
-    }
-    const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
-    if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
-    const T Dinv_t = (T)Dinv;
-    if constexpr (FUSED) {  // dt D^-1 V0 tau, so that a node takes (vd - st dx) w
-      const T sc = (T)(fdt * Dinv);
-#pragma unroll
-      for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) st[r][c] *= sc;
-    }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const T dx0 = (T)((double)(b[0] + a) * dx - xp[0]);
-#pragma unroll
-      for (int bb = 0; bb < 3; ++bb) {
-        const T wab = w[0][a] * w[1][bb];
-        const T dx1 = (T)((double)(b[1] + bb) * dx - xp[1]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const T wt_ = wab * w[2][c];
-          const T dx2 = (T)((double)(b[2] + c) * dx - xp[2]);
-          const int t = ((lx + a) * kTileY + (ly + bb)) * kTileZ + (lz + c);
-          const T fw = wt_ * Dinv_t;
-          atomicAdd(&wt[t], (double)(mass * wt_));
-#pragma unroll
-          for (int r = 0; r < 3; ++r) {
-            T vd = mC[r][0] * dx0 + mC[r][1] * dx1 + mC[r][2] * dx2 + mom[r];
-            if constexpr (FUSED) {
-              T fd = st[r][0] * dx0 + st[r][1] * dx1 + st[r][2] * dx2;
-              atomicAdd(&wt[(1 + r) * kTileNodes + t], (double)((vd - fd) * wt_));
-            } else {
-              atomicAdd(&wt[(1 + r) * kTileNodes + t], (double)(vd * wt_));
-              if constexpr (FORCE) {
-                T fd = st[r][0] * dx0 + st[r][1] * dx1 + st[r][2] * dx2;
-                atomicAdd(&wt[(4 + r) * kTileNodes + t], (double)(-(fd * fw)));
-              }
-            }
-          }
-        }
+          for (int c = 0; c < 3; ++c) st[r][c] *= -sc;  // -[dt] D^-1 V0 tau
       }
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+          A[r][c] = mass * (T)P.C[(c * 3 + r) * S + i];
+          if constexpr (FUSED) A[r][c] += st[r][c];
+        }
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double xi = xp[d] * inv_dx;
+        const int b = int_floor(xi - 0.5);
+        row[moment_at(tid, 4 * (d + 1) + 3)] = xi - (double)b;
+        e[d] = (double)(b + 1) * dx - xp[d];
+      }
+      store_moments(row, tid, (double)mass, mom, A, e, dx);
     }
+    __syncthreads();
+    cells_to_tile(row, coff, c0, count, wt, 1, true);
+    if constexpr (FORCE && !FUSED) {
+      // the force's moments in a second pass over the same rows
+      __syncthreads();
+      if ((uint32_t)tid < count) {
+        const T zero[3] = { (T)0, (T)0, (T)0 };
+        store_moments(row, tid, 0.0, zero, st, e, dx);
+      }
+      __syncthreads();
+      cells_to_tile(row, coff, c0, count, wt, 4, false);
+    }
+    __syncthreads();
   }
-  __syncthreads();
   double* out = stage + (size_t)g * SS;
   for (int k = tid; k < SS; k += NT) {
     double acc = tile[k];
@@ -1249,6 +1362,8 @@ struct zr_engine {
   // launch size of the sort's group kernels: the last sort's group count
   // with headroom (0: read the count first)
   uint32_t a_hint = 0;
+  uint32_t* cell_off = nullptr;  // [32 * groups] start of each cell's run in its group
+  size_t cell_cap = 0;           // groups
   // the CFL flag counter is zero (the sort clears every counter; only G2P sets it)
   bool cfl_clear = false;
   // inside a rollout: a step does not wait for its CFL flags; the next
@@ -1519,7 +1634,14 @@ int sort_groups(zr_engine* e, uint32_t hint)
   if (rc) return rc;
   k_scatter<<<blocks_for(n, 256), 256, 0, s>>>(n, e->p_page, e->p_re, e->page_group, e->group_start, e->keys, gb,
                                                e->dcount + CNT_TOTAL);
-  k_sort_groups<<<hint, 256, 0, s>>>(e->keys, e->group_start, e->order, gb);
+  if (e->cell_cap < hint) {
+    dfree(e->cell_off);
+    e->cell_cap = 0;
+    const size_t cap = (size_t)hint + hint / 4 + 64;
+    ZR_HIP(e, hipMalloc(&e->cell_off, 32 * cap * sizeof(uint32_t)));
+    e->cell_cap = cap;
+  }
+  k_sort_groups<<<hint, 256, 0, s>>>(e->keys, e->group_start, e->order, e->cell_off, gb);
   k_touch<<<blocks_for(8ull * hint, 256), 256, 0, s>>>(gb, e->group_page, e->touch_page, e->page_touch);
   ZR_LAUNCH_CHECK(e);
   rc = run_scan(e, LdFirstTouch{ e->touch_page, e->page_touch, gb }, 8u * hint, e->touch_slot,
@@ -1637,7 +1759,7 @@ int do_p2g(zr_engine* e, bool mls, double fuse_dt = 0.0)
     const bool fp32 = e->cfg.precision == ZR_FP32_REFINED, fused = fuse_dt > 0.0;
 #define ZR_P2G_LAUNCH_T(M, T, F)                                                                        \
   k_p2g<true, M, T, F><<<e->A, kTransferThreads, 0, e->stream>>>(pv, e->order, e->group_start, e->group_page, \
-                                                                 e->stage, dx, 1.0 / dx, Dinv, fuse_dt)
+                                                                 e->cell_off, e->stage, dx, 1.0 / dx, Dinv, fuse_dt)
 #define ZR_P2G_LAUNCH(M)                       \
   do {                                         \
     if (fp32 && fused)                         \
@@ -1663,8 +1785,8 @@ int do_p2g(zr_engine* e, bool mls, double fuse_dt = 0.0)
   }
   else
   {
-    k_p2g<false><<<e->A, kTransferThreads, 0, e->stream>>>(pview(e), e->order, e->group_start, e->group_page, e->stage, dx,
-                                              1.0 / dx, 4.0 / (dx * dx), 0.0);
+    k_p2g<false><<<e->A, kTransferThreads, 0, e->stream>>>(pview(e), e->order, e->group_start, e->group_page, e->cell_off,
+                                              e->stage, dx, 1.0 / dx, 4.0 / (dx * dx), 0.0);
     e->grid_nf = 4;
   }
   ZR_LAUNCH_CHECK(e);
@@ -2843,7 +2965,7 @@ void zr_destroy(zr_engine* e)
   free_particles(e);
   dfree(e->page_count); dfree(e->page_group); dfree(e->page_touch); dfree(e->page_slot); dfree(e->page_bits);
   dfree(e->page_sum); dfree(e->page_sumcnt); dfree(e->sum_base); dfree(e->stage); dfree(e->gm); dfree(e->gv); dfree(e->gf); dfree(e->gvs);
-  dfree(e->scan_tmp); dfree(e->speed); dfree(e->dcount); dfree(e->ticket); dfree(e->slot_src);
+  dfree(e->scan_tmp); dfree(e->cell_off); dfree(e->speed); dfree(e->dcount); dfree(e->ticket); dfree(e->slot_src);
   dfree(e->ivn); dfree(e->idv); dfree(e->ir); dfree(e->ix); dfree(e->irc); dfree(e->iq); dfree(e->ip); dfree(e->iap);
   dfree(e->partial); dfree(e->partial2); dfree(e->sc); dfree(e->ci); dfree(e->hvp_ctr); dfree(e->hvp_bounds); dfree(e->hvp_order); dfree(e->cell_order); dfree(e->jstage); dfree(e->pinv); dfree(e->collided); dfree(e->c64); dfree(e->c32); dfree(e->ccell);
   dfree(e->pf_node); dfree(e->pf_partial); dfree(e->adj_grid); dfree(e->admm_node); dfree(e->admm_coll); dfree(e->act); dfree(e->act_scan); dfree(e->be_fb); dfree(e->admm_c32); dfree(e->admm_cell32); dfree(e->admm_node32);
