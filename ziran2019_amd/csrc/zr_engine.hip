@@ -571,12 +571,13 @@ __device__ __forceinline__ void particle_kirchhoff_t(const ParticlesView& P, uin
 // value follows from its four moments per direction.  So:
 //   phase 1  thread per particle of a chunk of 256: stress, then its 13
 //            moments (mass; q and L of three directions) and its three
-//            fractions as one row of 16 in LDS (columns exchanged by the
-//            particle's index, so that neither this phase's column stores
-//            nor the next one's row loads collide on banks)
+//            fractions as one row in LDS (17 doubles apart, so that neither
+//            this phase's column stores nor the next one's row loads collide
+//            on banks)
 //   phase 2  wave per cell: v_mfma_f64_16x16x4 over the cell's particles,
-//            four at a time, with two accumulators (nodes 0-15 and 16-26);
-//            each lane forms its nodes' weights from the fractions.  Row
+//            four at a time, with two accumulators of 16 nodes each; a lane
+//            forms its two nodes' weights from the fractions, and the nodes
+//            are dealt so that the two share two of three 1-D weights.  Row
 //            4 t + d of the moments puts the four moments of direction d at
 //            one node into one lane's four accumulator registers (row 4 r +
 //            lane / 16 in register r), so the node's value takes three
@@ -584,11 +585,15 @@ __device__ __forceinline__ void particle_kirchhoff_t(const ParticlesView& P, uin
 // 108 LDS adds per cell rather than per particle, all lanes on different
 // nodes.  The FP64 matrix pipe shares its issue with FP64 vector instructions
 // here (measured: they add up), so the gain is the LDS adds and the lanes'
-// order: neighbouring lanes now load neighbouring particles.
+// order: neighbouring lanes now load neighbouring particles.  Against a tile
+// add per particle and node: 1,728 particles 25.1 -> 9.8 us, 140,608 47.4 ->
+// 25.8, 2.1M 296 -> 238 (with the stress alike), 3M FP32 terms 338 -> 285.
+// At 2.1M the vector instructions take about half of the time and the
+// particles' loads (0.65 GB fetched for 0.47 read) most of the rest.
 typedef double v4d __attribute__((ext_vector_type(4)));
 constexpr int kMoments = 16;
-// waves per SIMD the register budget is held to: what the LDS allows (51 KB
-// with four fields, 64 KB with seven), and two for particles of mixed models,
+// waves per SIMD the register budget is held to: what the LDS allows (53 KB
+// with four fields, 67 KB with seven), and two for particles of mixed models,
 // whose instance spills 50 registers at three
 template <bool FORCE, bool FUSED, int MODEL>
 constexpr int p2g_waves()
@@ -613,8 +618,25 @@ struct LaneWeight {
   }
 };
 
-// one row of the staged moments: element j of row p
-__device__ __forceinline__ int moment_at(uint32_t p, uint32_t j) { return (int)(p * kMoments + (j ^ (p & 15u))); }
+// element j of the staged row p
+constexpr uint32_t kRow = kMoments + 1;
+__device__ __forceinline__ uint32_t moment_at(uint32_t p, uint32_t j) { return p * kRow + j; }
+
+// The stencil nodes (9 a + 3 b + c) of column `col` of the two accumulators,
+// as (axis, first, second): the nodes differ along `axis` only, with offsets
+// `first` and `second` there, and share the offsets (o1, o2) of the next two
+// axes.  Columns 0-8: a = 0 and 1 of each (b, c); 9-10: b = 1 and 2 of
+// (a = 2, c = 1, 2); 11-15: the rest of a = 2, one node each.
+struct NodePair {
+  int axis, o1, o2, first, second;
+};
+__device__ __forceinline__ NodePair node_pair(int col)
+{
+  if (col < 9) return { 0, col / 3, col % 3, 0, 1 };
+  if (col < 11) return { 1, col - 8, 2, 1, 2 };  // axis b; next axes: c, a
+  const int bc = col == 15 ? 6 : col - 11;       // (b, c) = 0, 1, 2, 3, 6
+  return { 0, bc / 3, bc % 3, 2, 2 };
+}
 
 // row 4 t + d: t = 0 the constant q_d, t = 1..3 L_d along axis t - 1
 // (multiplied by the spacing); e_d = the middle node minus the particle
@@ -645,18 +667,23 @@ __device__ __forceinline__ void cells_to_tile(const double* row, const uint32_t*
   // registers across phase 1
   int lane = threadIdx.x & 63;
   asm volatile("" : "+v"(lane));
-  const int wv = threadIdx.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t col = (uint32_t)lane & 15u, kk = (uint32_t)lane >> 4;
-  LaneWeight W[2][3];
+  const NodePair np = node_pair((int)col);
+  const int ax1 = np.axis == 2 ? 0 : np.axis + 1, ax2 = ax1 == 2 ? 0 : ax1 + 1;
+  LaneWeight W0[2], W1, W2;
+  W0[0].set(np.first);
+  W0[1].set(np.second);
+  W1.set(np.o1);
+  W2.set(np.o2);
+  // fractions at columns 7, 11, 15 of the row
+  const uint32_t j0 = 4u * (uint32_t)np.axis + 7u, j1 = 4u * (uint32_t)ax1 + 7u, j2 = 4u * (uint32_t)ax2 + 7u;
   double o[2][3];
   int toff[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int nd = h == 0 ? (int)col : (col < 11u ? 16 + (int)col : 26);
-    const int a = nd / 9, b = (nd / 3) % 3, c = nd % 3;
-    W[h][0].set(a);
-    W[h][1].set(b);
-    W[h][2].set(c);
+    const int q = h == 0 ? np.first : np.second;
+    const int a = np.axis == 0 ? q : np.o2, b = np.axis == 0 ? np.o1 : q, c = np.axis == 0 ? np.o2 : np.o1;
     // lanes 48..63 hold the mass (moment t = 0 only)
     o[h][0] = kk == 3u ? 0.0 : (double)(a - 1);
     o[h][1] = kk == 3u ? 0.0 : (double)(b - 1);
@@ -670,22 +697,21 @@ __device__ __forceinline__ void cells_to_tile(const double* row, const uint32_t*
     // body's surface still gives every wave some
     const int cx = i >> 2, cy = i & 3, cz = (wv + cy + 2 * cx) & 3;
     const int e = (cx << 4) | (cy << 2) | cz;
-    const uint32_t b0 = coff[e], b1 = coff[e + 1];
+    const uint32_t b0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)coff[e]);
+    const uint32_t b1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)coff[e + 1]);
     const uint32_t kb = b0 > c0 ? b0 - c0 : 0u;
     const uint32_t ke = b1 > c0 ? (b1 - c0 < count ? b1 - c0 : count) : 0u;
     if (kb >= ke) continue;
     v4d D[2] = { { 0.0, 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0, 0.0 } };
     for (uint32_t k = kb; k < ke; k += 4u) {
       const bool live = k + kk < ke;
-      const uint32_t p = live ? k + kk : ke - 1u;
-      const double m = row[moment_at(p, col)];
-      const double f[3] = { row[moment_at(p, 7)], row[moment_at(p, 11)], row[moment_at(p, 15)] };
+      const double* r = row + (live ? k + kk : ke - 1u) * kRow;
+      const double m = r[col];
+      const double f0_ = r[j0], f1_ = r[j1], f2_ = r[j2];
       const double a = live ? m : 0.0;
+      const double w12 = W1(f1_) * W2(f2_);
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const double w = W[h][0](f[0]) * W[h][1](f[1]) * W[h][2](f[2]);
-        D[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, w, D[h], 0, 0, 0);
-      }
+      for (int h = 0; h < 2; ++h) D[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, W0[h](f0_) * w12, D[h], 0, 0, 0);
     }
     const int t0 = (cx * kTileY + cy) * kTileZ + cz;
     if (adds) {
@@ -710,7 +736,7 @@ __global__ __launch_bounds__(kTransferThreads, (p2g_waves<FORCE, FUSED, MODEL>()
   constexpr int NT = kTransferThreads, NW = NT / 64;
   static_assert(NW == 4, "eight of the 32 cells per wave");
   __shared__ double tile[NW * SS];
-  __shared__ double row[NT * kMoments];
+  __shared__ double row[NT * kRow];
   __shared__ uint32_t coff[33];
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;

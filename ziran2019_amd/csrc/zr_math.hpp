@@ -447,14 +447,31 @@ ZR_HD int svd3(const M3<T>& a, M3<T>& u, T s[3], M3<T>& v)
 // ---------------------------------------------------------------------------
 // R of the polar decomposition F = R S by Newton's iteration
 // X <- (X + X^-T) / 2 (Higham 1986), X^-T = cof(X) / det(X).  It converges
-// quadratically to U V^T for J > 0; once a step changes no entry by more
-// than 1e-8 the next would change it below rounding.  Taken for J >= 1/4 and
-// |F|^2 <= 9 (singular values within [0.05, 3], where at most 9 steps are
-// needed and cofactors lose no more than the SVD's rounding); returns false
-// outside, for the caller's SVD.  About 70 operations a step and 3 to 4 steps
+// quadratically to U V^T for J > 0.  After the first step every singular
+// value is 1 + d_i with d_i >= 0, and a step takes d_i to d_i^2 / 2, so the
+// step from det X - 1 ~ sum d_i <= 4e-9 is the last that changes anything.
+// Taken for J >= 1/4 and |F|^2 <= 9 (singular values within [0.05, 3], where
+// at most 9 steps are needed and cofactors lose no more than the SVD's
+// rounding); returns false outside, for the caller's SVD.  About 70 operations a step and 3 to 4 steps
 // at a few percent of strain, against the SVD's square roots, divisions and
 // rotations: k_adj_stress, which does little else, 22.8 -> 9.7 us on 262,144
 // particles.
+template <class T>
+ZR_HD T half_reciprocal(T d)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (sizeof(T) == sizeof(double)) {
+    // the hardware's estimate and two Newton steps: half the instructions
+    // of the IEEE quotient, to the last place or two, which the iteration
+    // it scales corrects until its last step
+    double y = __builtin_amdgcn_rcp(d);
+    y = fma(fma(-d, y, 1.0), y, y);
+    y = fma(fma(-d, y, 1.0), y, y);
+    return (T)(0.5 * y);
+  }
+#endif
+  return (T)0.5 / d;
+}
 template <class T>
 ZR_HD bool polar_newton(const M3<T>& f, T J, M3<T>& r)
 {
@@ -467,7 +484,7 @@ ZR_HD bool polar_newton(const M3<T>& f, T J, M3<T>& r)
   r = f;
   T d = J;
   for (int it = 0; it < 12; ++it) {
-    const T h = (T)0.5 / d;
+    const T h = half_reciprocal(d);
     M3<T> x;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -476,16 +493,8 @@ ZR_HD bool polar_newton(const M3<T>& f, T J, M3<T>& r)
         const int i1 = (i + 1) % 3, i2 = (i + 2) % 3, j1 = (j + 1) % 3, j2 = (j + 2) % 3;
         x.a[i][j] = (T)0.5 * r.a[i][j] + h * (r.a[i1][j1] * r.a[i2][j2] - r.a[i1][j2] * r.a[i2][j1]);
       }
-    T change = (T)0;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const T c = fabs(x.a[i][j] - r.a[i][j]);
-        change = c > change ? c : change;
-      }
     r = x;
-    if (change <= (T)1e-8) return true;
+    if (it > 0 && d - (T)1 <= (T)4e-9) return true;
     d = det3(r);
   }
   return false;
