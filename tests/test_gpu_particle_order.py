@@ -1,0 +1,141 @@
+"""The engine keeps large particle sets in the sort's order in memory.  The
+caller sees none of it: every array goes in and comes out in the caller's
+order, and a particle's results are the same bits whether its set was moved or
+not.  Sets of 65,536 particles are the smallest that move, once the steps since
+the last move have lost a step's worth of traffic; shuffled ones move at the
+second step."""
+import numpy as np
+import pytest
+
+from ziran2019_amd import scenes
+from ziran2019_amd.engine import (ZR_MODEL_NEO_HOOKEAN_BORDEN, ZR_MODEL_STVK_HENCKY, MpmEngine, admm_opts,
+                                  drucker_prager_alpha, implicit_opts, phase_field_opts)
+from _helpers import make_pair, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(n, seed=3):
+    """n particles of a moving, strained cube in random storage order."""
+    s = scenes.cube_scene(dx=1.0 / 64, lo_cell=20, ncells=21, ppc=8, seed=seed)
+    rng = np.random.default_rng(seed)
+    keep = rng.permutation(len(s["mass"]))[:n]
+    for k in ("X", "V", "C", "F", "mass", "vol", "mu", "lam"):
+        s[k] = np.ascontiguousarray(np.asarray(s[k])[keep])
+    s["V"] = 0.3 * rng.normal(size=3) + (s["X"] - 0.5) @ rng.normal(size=(3, 3))
+    s["F"] = s["F"] + 0.02 * rng.normal(size=(n, 9))
+    s["mu"] *= np.exp(0.2 * rng.normal(size=n))
+    return s
+
+
+def _same(a, b):
+    for k in a:
+        assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("n", [65535, 65536, 70001])
+def test_steps_against_the_oracle(n):
+    s = _scene(n)
+    eng, ora = make_pair(s, colliders=s["colliders"])
+    for _ in range(4):
+        eng.advanceOneTimeStep(1e-4)
+        ora.step(1e-4)
+    X, V, C, F = ora.get_particles()
+    out = eng.download()
+    for k, r in (("X", X), ("V", V), ("C", C), ("F", F)):
+        assert rel_err(out[k], r) < 1e-10, k  # the explicit parity tests' bound
+    eng.sortParticlesAndPolluteGrid()
+    ora.sort_and_pollute()
+    r = ora.sort_result()
+    assert np.array_equal(eng.dump("order"), r["order"])
+    assert np.array_equal(eng.dump("sorter"), r["sorter"])
+    assert np.array_equal(eng.dump("base_offset"), r["base_offset"])
+    eng.close()
+
+
+def _explicit(e, s):
+    return lambda: e.advanceOneTimeStep(1e-4), lambda: e.download()
+
+
+def _plastic(e, s):
+    n = e.n
+    rng = np.random.default_rng(1)
+    pl = rng.integers(0, 3, size=n).astype(np.int32)
+    pp = np.zeros((n, 4))
+    pp[pl == 1] = (1e3, 1e30, 0, 0)
+    pp[pl == 2] = (drucker_prager_alpha(30.0), 1.0, 0.0, 1.0)
+    e.set_materials(model=ZR_MODEL_STVK_HENCKY, plasticity=pl, plastic_param=pp,
+                    plastic_state=np.where(pl == 1, 100.0, 0.0))
+    return lambda: e.advanceOneTimeStep(1e-4), lambda: dict(e.download(), **e.get_materials())
+
+
+def _fracture(e, s):
+    n = e.n
+    rng = np.random.default_rng(2)
+    e.set_phase_field(phase_field_opts(naive=2, sigma_F=50.0), l0=0.5 / 64, one_over_sigma_c=0.01 * (1 + rng.random(n)),
+                      allow_damage=rng.integers(0, 2, size=n).astype(np.int32))
+    return lambda: e.advanceOneTimeStep(1e-4), lambda: dict(e.download(), **e.get_phase_field())
+
+
+def _visco(e, s):
+    e.set_materials(model=ZR_MODEL_NEO_HOOKEAN_BORDEN)
+    e.set_viscoelastic(None, s["mu"], s["lam"], 50.0, 70.0)
+    return lambda: e.advanceOneTimeStep(1e-4), lambda: dict(e.download(), Fneq=e.get_viscoelastic())
+
+
+def _implicit(e, s):
+    o = implicit_opts(cg_max_iterations=30, cg_tolerance=1.0, cg_relative_tolerance=1e-6)
+    return lambda: e.advanceOneTimeStepImplicit(1e-3, o), lambda: e.download()
+
+
+def _admm(e, s):
+    e.set_materials(model=ZR_MODEL_STVK_HENCKY)
+    return (lambda: e.advanceOneTimeStepAdmm(1e-3, admm_opts(admm_iterations=4)),
+            lambda: dict(e.download(), **e.get_admm_state()))
+
+
+@pytest.mark.parametrize("setup", [_explicit, _plastic, _fracture, _visco, _implicit, _admm])
+def test_moved_and_unmoved_sets_agree_bit_for_bit(setup):
+    """One engine steps undisturbed; the other's particles go back to the
+    caller's order before every step (a dump of the sort's order asks for it),
+    so that it never reads a moved set twice."""
+    s = _scene(66001)
+    outs = []
+    for disturb in (False, True):
+        e = MpmEngine(dx=s["dx"])
+        e.upload(s)
+        e.set_colliders(s["colliders"])
+        step, read = setup(e, s)
+        for _ in range(5):
+            if disturb:
+                e.sortParticlesAndPolluteGrid()
+                e.dump("order")
+            step()
+        outs.append(read())
+        e.close()
+    _same(*outs)
+
+
+def test_checkpoint_of_a_moved_set():
+    s = _scene(66001)
+    e = MpmEngine(dx=s["dx"])
+    e.upload(s)
+    e.set_colliders(s["colliders"])
+    e.checkpoint_save(0)
+    first = e.download()
+    for _ in range(3):
+        e.advanceOneTimeStep(1e-4)
+    e.checkpoint_save(1)
+    moved = e.download()
+    e.advanceOneTimeStep(1e-4)
+    after = e.download()
+    e.checkpoint_restore(1)  # saved and restored while moved
+    _same(e.download(), moved)
+    e.advanceOneTimeStep(1e-4)
+    _same(e.download(), after)
+    e.checkpoint_restore(0)  # saved before the set was moved
+    _same(e.download(), first)
+    for _ in range(3):
+        e.advanceOneTimeStep(1e-4)
+    _same(e.download(), moved)
+    e.close()

@@ -52,6 +52,9 @@ constexpr int kP2GFields = 7;                          // m, mv[3], f[3]
 constexpr int kStageStride = kP2GFields * kTileNodes;  // doubles per group
 constexpr int kMaxColliders = 8;
 constexpr int kSortLds = 2048;  // particles per page sorted in LDS
+constexpr uint32_t kMoveMin = 65536;  // fewer particles are not moved
+constexpr double kDisorder = 1.0;
+constexpr uint32_t kBreakSample = 64;  // every 64th group reports how scattered its particles are
 constexpr uint32_t kNone = 0xffffffffu;
 
 // a collider as the kernels read it: its rates and its frame x = R s X + b
@@ -80,10 +83,12 @@ enum {
   CNT_DOMAIN = 2,
   CNT_CFL = 3,
   CNT_TOTAL = 4,
-  CNT_SORT = 5,
-  CNT_ADJ_BAD = 5,
-  CNT_CFL_RUN = 6,
-  CNT_N = 8
+  CNT_BREAKS = 5,   // sampled groups' places where the order is not consecutive
+  CNT_SAMPLED = 6,  // their particles
+  CNT_SORT = 7,
+  CNT_ADJ_BAD = 7,
+  CNT_CFL_RUN = 8,
+  CNT_N = 10
 };
 
 // ---------------------------------------------------------------------------
@@ -352,9 +357,12 @@ struct LdFirstTouch {
   }
 };
 
+// a particle's sort key: cell within the page (5 bits) | the caller's index
+// (27 bits) | its place in the engine's arrays (32 bits)
 // (thread 0 also closes group_start with the particle total)
 __global__ void k_scatter(uint32_t n, const uint32_t* p_page, const uint32_t* p_re, const int32_t* page_group,
-                          uint32_t* group_start, uint64_t* keys, GroupBound gb, const uint32_t* total)
+                          uint32_t* group_start, uint64_t* keys, GroupBound gb, const uint32_t* total,
+                          const uint32_t* uid)
 {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t ng = gb.get();
@@ -364,21 +372,24 @@ __global__ void k_scatter(uint32_t n, const uint32_t* p_page, const uint32_t* p_
   int32_t g = page_group[p_page[i]];
   if ((uint32_t)g >= ng) return;
   uint32_t dst = group_start[g] + (re >> 5);
-  keys[dst] = ((uint64_t)(re & 31u) << 32) | (uint64_t)i;
+  const uint32_t u = uid ? uid[i] : i;
+  keys[dst] = ((uint64_t)(((re & 31u) << 27) | u) << 32) | (uint64_t)i;
 }
 
-// sorts each group's keys (cell << 32 | particle index) ascending: the
-// particles are bucketed by cell (LDS counters), and each particle's place in
-// its cell's bucket is the number of the bucket's indices below its own
+// sorts each group's keys ascending: the particles are bucketed by cell (LDS
+// counters), and each particle's place in its cell's bucket is the number of
+// the bucket's caller's indices below its own;
 // and records where each cell's run begins within the group (cell_off,
 // 32 entries per group), for the transfers that work cell by cell
 __global__ __launch_bounds__(256) void k_sort_groups(const uint64_t* __restrict__ keys,
                                                      const uint32_t* __restrict__ group_start,
-                                                     uint32_t* __restrict__ order, uint32_t* __restrict__ cell_off,
-                                                     GroupBound gb)
+                                                     uint32_t* order,
+                                                     uint32_t* __restrict__ cell_off, GroupBound gb,
+                                                     uint32_t* counters)
 {
-  __shared__ uint32_t bucket[kSortLds];  // particle indices by cell, unordered within a cell
-  __shared__ uint32_t pidx[kSortLds];    // particle index of each key position
+  __shared__ uint32_t bucket[kSortLds];  // caller's indices by cell, unordered within a cell
+  __shared__ uint32_t pidx[kSortLds];    // caller's index of each key position
+  __shared__ uint32_t place[kSortLds];   // place in the engine's arrays of each key position
   __shared__ uint16_t code[kSortLds];    // cell | slot << 5 of each key position
   __shared__ uint32_t cnt[32], off[32];
   static_assert(kSortLds <= 2048, "slot << 5 fits 16 bits");
@@ -392,11 +403,12 @@ __global__ __launch_bounds__(256) void k_sort_groups(const uint64_t* __restrict_
   const bool in_lds = n <= (uint32_t)kSortLds;
   for (uint32_t k = tid; k < n; k += 256) {
     const uint64_t key = keys[start + k];
-    const uint32_t c = (uint32_t)(key >> 32) & 31u;
+    const uint32_t hi = (uint32_t)(key >> 32), c = hi >> 27;
     const uint32_t slot = atomicAdd(&cnt[c], 1u);
     if (in_lds) {
       code[k] = (uint16_t)(c | (slot << 5));
-      pidx[k] = (uint32_t)key;
+      pidx[k] = hi & 0x7ffffffu;
+      place[k] = (uint32_t)key;
     }
   }
   __syncthreads();
@@ -435,7 +447,20 @@ __global__ __launch_bounds__(256) void k_sort_groups(const uint64_t* __restrict_
     const uint32_t b0 = off[c], b1 = b0 + cnt[c];
     uint32_t rank = 0;
     for (uint32_t j = b0; j < b1; ++j) rank += bucket[j] < i ? 1u : 0u;
-    order[start + b0 + rank] = i;
+    order[start + b0 + rank] = place[k];
+  }
+  if ((g & (kBreakSample - 1u)) != 0u) return;
+  // how far the particles' places in memory are from this order
+  __syncthreads();
+  uint32_t breaks = 0;
+  for (uint32_t k = tid + 1u; k < n; k += 256) breaks += order[start + k] != order[start + k - 1u] + 1u ? 1u : 0u;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) breaks += __shfl_xor(breaks, o, 64);
+  if ((tid & 63) == 0) cnt[tid >> 6] = breaks;
+  __syncthreads();
+  if (tid == 0) {
+    atomicAdd(&counters[CNT_BREAKS], cnt[0] + cnt[1] + cnt[2] + cnt[3]);
+    atomicAdd(&counters[CNT_SAMPLED], n);
   }
 }
 
@@ -1211,13 +1236,56 @@ __global__ void k_aos_to_soa(const double* __restrict__ aos, double* __restrict_
   int c = (int)(t % ncomp);
   soa[c * stride + i] = aos[t];
 }
-__global__ void k_soa_to_aos(const double* __restrict__ soa, double* __restrict__ aos, uint32_t n, int ncomp, int64_t stride)
+// uid: the caller's index of each place (null: the same)
+__global__ void k_soa_to_aos(const double* __restrict__ soa, double* __restrict__ aos, uint32_t n, int ncomp,
+                             int64_t stride, const uint32_t* __restrict__ uid)
 {
   uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (uint64_t)n * ncomp) return;
   uint32_t i = (uint32_t)(t / ncomp);
   int c = (int)(t % ncomp);
-  aos[t] = soa[c * stride + i];
+  aos[uid ? (uint64_t)uid[i] * ncomp + c : t] = soa[c * stride + i];
+}
+
+// Moves every per-particle array to another order in one launch: thread k
+// copies each row's element from[k] -> k (gather), or k -> to[k] (scatter)
+constexpr int kMoveArrays = 32;
+struct MoveList {
+  const void* src[kMoveArrays];
+  void* dst[kMoveArrays];
+  int rows[kMoveArrays];  // rows of n elements; negative: 4-byte elements
+  int count;
+};
+__global__ __launch_bounds__(256) void k_move(MoveList L, uint32_t n, const uint32_t* __restrict__ from,
+                                              const uint32_t* __restrict__ to)
+{
+  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+  if (k >= n) return;
+  const uint32_t a = from ? from[k] : k, b = to ? to[k] : k;
+  for (int q = 0; q < L.count; ++q) {
+    if (L.rows[q] > 0) {
+      const double* __restrict__ s = static_cast<const double*>(L.src[q]);
+      double* __restrict__ d = static_cast<double*>(L.dst[q]);
+#pragma unroll 3
+      for (int r = 0; r < L.rows[q]; ++r) d[(size_t)r * n + b] = s[(size_t)r * n + a];
+    } else {
+      static_cast<uint32_t*>(L.dst[q])[b] = static_cast<const uint32_t*>(L.src[q])[a];
+    }
+  }
+}
+// gather: order[k] = k and, the first time, uid[k] = the old order[k];
+// scatter: order[k] = the caller's index of the particle at order[k]
+__global__ __launch_bounds__(256) void k_iota_order(uint32_t n, uint32_t* order, uint32_t* uid, int first)
+{
+  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+  if (k >= n) return;
+  if (first) uid[k] = order[k];
+  order[k] = k;
+}
+__global__ __launch_bounds__(256) void k_user_order(uint32_t n, uint32_t* order, const uint32_t* __restrict__ uid)
+{
+  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+  if (k < n) order[k] = uid[order[k]];
 }
 __global__ void k_dump_sorter(uint32_t n, const uint32_t* order, const uint32_t* p_page, const uint32_t* p_re, uint64_t* out)
 {
@@ -1389,6 +1457,19 @@ struct zr_engine {
   // with headroom (0: read the count first)
   uint32_t a_hint = 0;
   uint32_t* cell_off = nullptr;  // [32 * groups] start of each cell's run in its group
+  // The particles' order in memory.  permuted: place k holds the caller's
+  // particle uid[k]; otherwise places are the caller's indices.  alt: the
+  // second copy of each per-particle array that a move writes to (the two
+  // swap); disorder: sum over the steps since the last move of the share of
+  // particles not next to their predecessor in the sort's order.
+  bool permuted = false;
+  uint32_t* uid = nullptr;
+  struct Spare {
+    void* p = nullptr;
+    size_t bytes = 0;
+  };
+  std::vector<Spare> alt;
+  double disorder = 0.0;
   size_t cell_cap = 0;           // groups
   // the CFL flag counter is zero (the sort clears every counter; only G2P sets it)
   bool cfl_clear = false;
@@ -1533,6 +1614,11 @@ void free_particles(zr_engine* e)
   dfree(e->pf_c); dfree(e->pf_H); dfree(e->pf_l0); dfree(e->pf_osc); dfree(e->pf_Fp); dfree(e->pf_Hmax);
   dfree(e->pf_k); dfree(e->pf_vol); dfree(e->pf_allow);
   e->pf_on = false;
+  for (auto& a : e->alt) dfree(a.p);
+  e->alt.clear();
+  dfree(e->uid);
+  e->permuted = false;
+  e->disorder = 0.0;
   dfree(e->adj);
   e->adj_n = 0;
   dfree(e->admm_p);
@@ -1659,7 +1745,7 @@ int sort_groups(zr_engine* e, uint32_t hint)
   int rc = run_scan(e, LdGroupCount{ e->group_count, gb }, hint, e->group_start, e->dcount + CNT_TOTAL);
   if (rc) return rc;
   k_scatter<<<blocks_for(n, 256), 256, 0, s>>>(n, e->p_page, e->p_re, e->page_group, e->group_start, e->keys, gb,
-                                               e->dcount + CNT_TOTAL);
+                                               e->dcount + CNT_TOTAL, e->permuted ? e->uid : nullptr);
   if (e->cell_cap < hint) {
     dfree(e->cell_off);
     e->cell_cap = 0;
@@ -1667,7 +1753,7 @@ int sort_groups(zr_engine* e, uint32_t hint)
     ZR_HIP(e, hipMalloc(&e->cell_off, 32 * cap * sizeof(uint32_t)));
     e->cell_cap = cap;
   }
-  k_sort_groups<<<hint, 256, 0, s>>>(e->keys, e->group_start, e->order, e->cell_off, gb);
+  k_sort_groups<<<hint, 256, 0, s>>>(e->keys, e->group_start, e->order, e->cell_off, gb, e->dcount);
   k_touch<<<blocks_for(8ull * hint, 256), 256, 0, s>>>(gb, e->group_page, e->touch_page, e->page_touch);
   ZR_LAUNCH_CHECK(e);
   rc = run_scan(e, LdFirstTouch{ e->touch_page, e->page_touch, gb }, 8u * hint, e->touch_slot,
@@ -1677,6 +1763,107 @@ int sort_groups(zr_engine* e, uint32_t hint)
                                                              e->slot_page, e->page_slot);
   k_group_slots<<<blocks_for(8ull * hint, 256), 256, 0, s>>>(gb, e->touch_page, e->page_slot, e->group_nslot);
   ZR_LAUNCH_CHECK(e);
+  return ZR_OK;
+}
+
+// every array that holds a value per particle across steps (scratch arrays
+// that a step fills before it reads them are not moved)
+struct ParticleArray {
+  void** p;
+  int rows;  // negative: one row of 4-byte elements
+};
+std::vector<ParticleArray> particle_arrays(zr_engine* e)
+{
+  auto v = [](auto*& p) { return reinterpret_cast<void**>(&p); };
+  return { { v(e->x), 3 },       { v(e->v), 3 },       { v(e->C), 9 },       { v(e->F), 9 },
+           { v(e->m), 1 },       { v(e->vol), 1 },     { v(e->mu), 1 },      { v(e->lam), 1 },
+           { v(e->mat), -1 },    { v(e->pparam), 4 },  { v(e->pstate), 1 },  { v(e->gdeg), 1 },
+           { v(e->broken), -1 }, { v(e->fneq), 9 },    { v(e->mu_neq), 1 },  { v(e->lam_neq), 1 },
+           { v(e->pf_c), 1 },    { v(e->pf_H), 1 },    { v(e->pf_l0), 1 },   { v(e->pf_osc), 1 },
+           { v(e->pf_Fp), 1 },   { v(e->pf_Hmax), 1 }, { v(e->pf_k), 1 },    { v(e->pf_allow), -1 },
+           { v(e->admm_p), e->admm_visco ? 41 : 22 },  { v(e->p_page), -1 }, { v(e->p_re), -1 },
+           { v(e->uid), -1 } };
+}
+
+int move_particles(zr_engine* e, const uint32_t* from, const uint32_t* to)
+{
+  const std::vector<ParticleArray> arrays = particle_arrays(e);
+  if (e->alt.size() != arrays.size()) e->alt.resize(arrays.size());
+  MoveList L{};
+  static_assert(kMoveArrays >= 28, "one entry per array");
+  size_t bytes[kMoveArrays];
+  for (size_t q = 0; q < arrays.size(); ++q) {
+    const ParticleArray& a = arrays[q];
+    if (!*a.p) continue;
+    bytes[q] = (size_t)e->n * (a.rows > 0 ? 8 * (size_t)a.rows : 4);
+    if (e->alt[q].bytes != bytes[q]) {  // an array whose size changed (the ADMM state) needs a spare of its own size
+      dfree(e->alt[q].p);
+      e->alt[q].bytes = 0;
+      ZR_HIP(e, hipMalloc(&e->alt[q].p, bytes[q]));
+      e->alt[q].bytes = bytes[q];
+    }
+    L.src[L.count] = *a.p;
+    L.dst[L.count] = e->alt[q].p;
+    L.rows[L.count++] = a.rows;
+  }
+  k_move<<<blocks_for((uint64_t)e->n, 256), 256, 0, e->stream>>>(L, (uint32_t)e->n, from, to);
+  ZR_LAUNCH_CHECK(e);
+  for (size_t q = 0; q < arrays.size(); ++q)
+    if (*arrays[q].p) std::swap(*arrays[q].p, e->alt[q].p);
+  return ZR_OK;
+}
+
+// The particles into the order of the sort that has just run: the transfers
+// of this step and the next then read and write neighbouring places.  A
+// particle's results do not depend on it (the sort's ties go by the caller's
+// index).
+int order_particles(zr_engine* e)
+{
+  const uint32_t n = (uint32_t)e->n, nb = blocks_for(n, 256);
+  if (!e->uid) ZR_HIP(e, hipMalloc(&e->uid, (size_t)n * sizeof(uint32_t)));
+  int rc = move_particles(e, e->order, nullptr);
+  if (rc) return rc;
+  k_iota_order<<<nb, 256, 0, e->stream>>>(n, e->order, e->uid, e->permuted ? 0 : 1);
+  ZR_LAUNCH_CHECK(e);
+  e->permuted = true;
+  e->disorder = 0.0;
+  return ZR_OK;
+}
+
+// one row of n values (rows as in ParticleArray) to the caller's array in the
+// caller's order, through the sort's key array as scratch (8 bytes per
+// particle, written again before every use)
+int download_row(zr_engine* e, void* host, const void* dev, int rows)
+{
+  const uint32_t n = (uint32_t)e->n;
+  if (e->permuted) {
+    MoveList L{};
+    L.src[0] = dev;
+    L.dst[0] = e->keys;
+    L.rows[0] = rows;
+    L.count = 1;
+    k_move<<<blocks_for(n, 256), 256, 0, e->stream>>>(L, n, nullptr, e->uid);
+    ZR_LAUNCH_CHECK(e);
+    dev = e->keys;
+  }
+  ZR_HIP(e, hipMemcpyAsync(host, dev, (size_t)n * (rows > 0 ? 8 : 4), hipMemcpyDeviceToHost, e->stream));
+  ZR_HIP(e, hipStreamSynchronize(e->stream));
+  return ZR_OK;
+}
+
+// back to the caller's order, for the calls that take or give arrays in it;
+// the sort's tables, the grid and the step's state stay valid
+int user_order(zr_engine* e)
+{
+  if (!e->permuted) return ZR_OK;
+  const uint32_t n = (uint32_t)e->n;
+  k_user_order<<<blocks_for(n, 256), 256, 0, e->stream>>>(n, e->order, e->uid);
+  int rc = move_particles(e, nullptr, e->uid);
+  if (rc) return rc;
+  e->permuted = false;
+  e->disorder = 0.0;
+  // the callers copy from and to these arrays outside the stream
+  ZR_HIP(e, hipStreamSynchronize(e->stream));
   return ZR_OK;
 }
 
@@ -1750,6 +1937,21 @@ int do_sort(zr_engine* e, zr_step_stats* st)
   // a rollout's earlier step asked for a restart: the particles are those
   // after that step (a sort moves none)
   if (e->defer_cfl && (e->hcount[CNT_CFL_RUN] & 1u)) return ZR_CFL_RESTART;
+  // Moving the particles costs about what a step loses to an order in which
+  // no particle follows its predecessor (2.1M particles in raster order:
+  // k_move 225 us; k_g2p 282 -> 164 us and k_p2g 238 -> 195, the G2P's writes
+  // of 24 rows reaching memory 2.2 times in partial lines before), so they
+  // are moved once the steps since the last move have lost that much
+  // (kDisorder); a rollout keeps the caller's order, which its records and
+  // adjoints are in.  Below kMoveMin the arrays stay in the caches and a
+  // move's launches cost more than they give.
+  if (n >= kMoveMin && !e->defer_cfl && e->hcount[CNT_SAMPLED]) {
+    e->disorder += (double)e->hcount[CNT_BREAKS] / (double)e->hcount[CNT_SAMPLED];
+    if (e->disorder >= kDisorder) {
+      rc = order_particles(e);
+      if (rc) return rc;
+    }
+  }
   rc = ensure_grid(e);
   if (rc) return rc;
   if (e->S) {
@@ -3232,7 +3434,8 @@ int zr_download_particles(zr_engine* e, zr_particles* p)
                 { p->mass, e->m, 1 }, { p->vol, e->vol, 1 }, { p->mu, e->mu, 1 }, { p->lambda, e->lam, 1 } };
   for (auto& it : items) {
     if (!it.dst) continue;
-    k_soa_to_aos<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(it.src, tmp, (uint32_t)N, it.nc, e->n);
+    k_soa_to_aos<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(it.src, tmp, (uint32_t)N, it.nc, e->n,
+                                                                              e->permuted ? e->uid : nullptr);
     hipError_t st = hipGetLastError();
     if (st == hipSuccess) st = hipMemcpyAsync(it.dst, tmp, it.nc * N * sizeof(double), hipMemcpyDeviceToHost, e->stream);
     if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
@@ -3251,6 +3454,7 @@ int zr_set_materials(zr_engine* e, const zr_materials* mt)
   if (mt->n != e->n) return fail(e, ZR_ERR_ARG, "material count differs from the particle count");
   const int64_t n = e->n;
   if (n == 0) return ZR_OK;
+  if (int rc_order = user_order(e)) return rc_order;
   const size_t N = (size_t)n;
   std::vector<int32_t> code(N, 0);
   bool models = false, plastic = false;
@@ -3310,6 +3514,7 @@ int zr_set_viscoelastic(zr_engine* e, const double* F_neq, const double* mu, con
   if (!(viscosity_d > 0.0) || !(viscosity_v > 0.0)) return fail(e, ZR_ERR_ARG, "viscosities must be positive");
   const size_t N = (size_t)e->n;
   if (N == 0) return fail(e, ZR_ERR_STATE, "upload the particles before the viscoelastic branch");
+  if (int rc_order = user_order(e)) return rc_order;
   if (!e->fneq) {
     ZR_HIP(e, hipMalloc(&e->fneq, 9 * N * sizeof(double)));
     ZR_HIP(e, hipMalloc(&e->vtau_neq, 9 * N * sizeof(double)));
@@ -3333,6 +3538,7 @@ int zr_get_viscoelastic(zr_engine* e, double* F_neq)
 {
   if (!e || !F_neq) return ZR_ERR_ARG;
   if (!e->visco) return fail(e, ZR_ERR_STATE, "no viscoelastic branch");
+  if (int rc_order = user_order(e)) return rc_order;
   const size_t N = (size_t)e->n;
   std::vector<double> f(9 * N);
   ZR_HIP(e, hipStreamSynchronize(e->stream));
@@ -3356,14 +3562,11 @@ int zr_get_materials(zr_engine* e, zr_materials* mt)
     }
     return ZR_OK;
   }
-  if (mt->plastic_state)
-    ZR_HIP(e, hipMemcpyAsync(mt->plastic_state, e->pstate, N * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-  if (mt->degradation)
-    ZR_HIP(e, hipMemcpyAsync(mt->degradation, e->gdeg, N * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-  if (mt->broken)
-    ZR_HIP(e, hipMemcpyAsync(mt->broken, e->broken, N * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
-  ZR_HIP(e, hipStreamSynchronize(e->stream));
-  return ZR_OK;
+  int rc = ZR_OK;
+  if (mt->plastic_state) rc = download_row(e, mt->plastic_state, e->pstate, 1);
+  if (!rc && mt->degradation) rc = download_row(e, mt->degradation, e->gdeg, 1);
+  if (!rc && mt->broken) rc = download_row(e, mt->broken, e->broken, -1);
+  return rc;
 }
 
 int zr_set_phase_field(zr_engine* e, const zr_phase_field* pf, const zr_phase_field_opts* o)
@@ -3378,6 +3581,7 @@ int zr_set_phase_field(zr_engine* e, const zr_phase_field* pf, const zr_phase_fi
     return fail(e, ZR_ERR_ARG, "the phase field needs l0 and one_over_sigma_c");
   const size_t N = (size_t)e->n;
   if (N == 0) return ZR_OK;
+  if (int rc_order = user_order(e)) return rc_order;
   // every particle becomes NeoHookeanBorden (keeping its plasticity code)
   std::vector<int32_t> code(N, ZR_MODEL_NEO_HOOKEAN_BORDEN);
   if (e->mat) {
@@ -3420,11 +3624,11 @@ int zr_get_phase_field(zr_engine* e, zr_phase_field* pf)
   if (!e->pf_on) return fail(e, ZR_ERR_STATE, "no phase field was set");
   const size_t N = (size_t)e->n;
   if (N == 0) return ZR_OK;
-  if (pf->c) ZR_HIP(e, hipMemcpyAsync(pf->c, e->pf_c, N * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-  if (pf->H) ZR_HIP(e, hipMemcpyAsync(pf->H, e->pf_H, N * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-  if (pf->pf_Fp) ZR_HIP(e, hipMemcpyAsync(pf->pf_Fp, e->pf_Fp, N * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-  ZR_HIP(e, hipStreamSynchronize(e->stream));
-  return ZR_OK;
+  int rc = ZR_OK;
+  if (pf->c) rc = download_row(e, pf->c, e->pf_c, 1);
+  if (!rc && pf->H) rc = download_row(e, pf->H, e->pf_H, 1);
+  if (!rc && pf->pf_Fp) rc = download_row(e, pf->pf_Fp, e->pf_Fp, 1);
+  return rc;
 }
 
 int zr_phase_field_solve(zr_engine* e, double dt, zr_phase_field_stats* st)
@@ -3504,7 +3708,7 @@ int zr_adjoint_get(zr_engine* e, zr_particles_adjoint* a)
                 { a->lambda, A.lam, 1 } };
   for (auto& it : items) {
     if (!it.dst) continue;
-    k_soa_to_aos<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(it.src, tmp, (uint32_t)N, it.nc, e->n);
+    k_soa_to_aos<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(it.src, tmp, (uint32_t)N, it.nc, e->n, nullptr);
     hipError_t st = hipGetLastError();
     if (st == hipSuccess) st = hipMemcpyAsync(it.dst, tmp, it.nc * N * sizeof(double), hipMemcpyDeviceToHost, e->stream);
     if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
@@ -3523,38 +3727,35 @@ int zr_adjoint_step(zr_engine* e, double dt)
   if (!(dt > 0.0)) return fail(e, ZR_ERR_ARG, "dt must be positive");
   if (!adjoint_supported(e)) return ZR_ERR_ARG;
   if (!e->adj || e->adj_n != e->n) return fail(e, ZR_ERR_STATE, "zr_adjoint_set was not called");
+  if (int rc_order = user_order(e)) return rc_order;
   ZR_HIP(e, hipMemsetAsync(e->dcount + CNT_ADJ_BAD, 0, sizeof(uint32_t), e->stream));
   return do_adjoint_step(e, dt, true);
 }
 
 namespace {
 // the checkpoint arrays X, V, C, F and a 24n-double checkpoint, copied in
-// one pass (to: state -> checkpoint, else back)
-__global__ __launch_bounds__(256) void k_ckpt_copy(double* x, double* v, double* C, double* F, double* c, uint64_t N,
-                                                   int to)
+// one pass (to: state -> checkpoint, else back), the checkpoint in the
+// caller's order (uid as in k_soa_to_aos)
+__global__ __launch_bounds__(256) void k_ckpt_copy(double* x, double* v, double* C, double* F, double* c, uint32_t n,
+                                                   int to, const uint32_t* __restrict__ uid)
 {
-  const uint64_t total = 24 * N, stride = (uint64_t)gridDim.x * 256u;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < total; i += stride) {
-    double* a;
-    uint64_t j;
-    if (i < 3 * N) {
-      a = x;
-      j = i;
-    } else if (i < 6 * N) {
-      a = v;
-      j = i - 3 * N;
-    } else if (i < 15 * N) {
-      a = C;
-      j = i - 6 * N;
-    } else {
-      a = F;
-      j = i - 15 * N;
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t u = uid ? uid[i] : i;
+  const size_t N = n;
+  auto rows = [&](double* a, double* k, int m) {
+#pragma unroll 9
+    for (int r = 0; r < m; ++r) {
+      if (to)
+        k[r * N + u] = a[r * N + i];
+      else
+        a[r * N + i] = k[r * N + u];
     }
-    if (to)
-      c[i] = a[j];
-    else
-      a[j] = c[i];
-  }
+  };
+  rows(x, c, 3);
+  rows(v, c + 3 * N, 3);
+  rows(C, c + 6 * N, 9);
+  rows(F, c + 15 * N, 9);
 }
 
 // checkpoint save / restore, enqueued on the engine's stream
@@ -3568,8 +3769,8 @@ int ckpt_save(zr_engine* e, int32_t slot)
   }
   if (!e->ckpt[slot]) ZR_HIP(e, hipMalloc(&e->ckpt[slot], 24 * (N ? N : 1) * sizeof(double)));
   if (N) {
-    const uint64_t b = blocks_for(24 * (uint64_t)N, 256);
-    k_ckpt_copy<<<b < 2048 ? (uint32_t)b : 2048u, 256, 0, e->stream>>>(e->x, e->v, e->C, e->F, e->ckpt[slot], N, 1);
+    k_ckpt_copy<<<blocks_for(N, 256), 256, 0, e->stream>>>(e->x, e->v, e->C, e->F, e->ckpt[slot], (uint32_t)N, 1,
+                                                           e->permuted ? e->uid : nullptr);
     ZR_LAUNCH_CHECK(e);
   }
   e->ckpt_time[slot] = e->time;
@@ -3582,8 +3783,8 @@ int ckpt_restore(zr_engine* e, int32_t slot)
     return fail(e, ZR_ERR_ARG, "no such checkpoint");
   const size_t N = (size_t)e->n;
   if (N) {
-    const uint64_t b = blocks_for(24 * (uint64_t)N, 256);
-    k_ckpt_copy<<<b < 2048 ? (uint32_t)b : 2048u, 256, 0, e->stream>>>(e->x, e->v, e->C, e->F, e->ckpt[slot], N, 0);
+    k_ckpt_copy<<<blocks_for(N, 256), 256, 0, e->stream>>>(e->x, e->v, e->C, e->F, e->ckpt[slot], (uint32_t)N, 0,
+                                                           e->permuted ? e->uid : nullptr);
     ZR_LAUNCH_CHECK(e);
   }
   e->time = e->ckpt_time[slot];
@@ -3633,6 +3834,7 @@ int zr_rollout_forward(zr_engine* e, int32_t steps, double dt, int32_t every, in
 {
   if (!e) return ZR_ERR_ARG;
   if (steps < 0 || every < 1 || slot0 < 0 || !(dt > 0.0)) return fail(e, ZR_ERR_ARG, "bad rollout arguments");
+  if (int rc_order = user_order(e)) return rc_order;
   ZR_HIP(e, hipMemsetAsync(e->dcount + CNT_CFL_RUN, 0, sizeof(uint32_t), e->stream));
   DeferCfl defer(e);
   for (int32_t k = 0; k < steps; ++k) {
@@ -3655,6 +3857,7 @@ int zr_rollout_backward(zr_engine* e, int32_t steps, double dt, int32_t every, i
     return fail(e, ZR_ERR_ARG, "bad rollout arguments");
   if (!adjoint_supported(e)) return ZR_ERR_ARG;
   if (!e->adj || e->adj_n != e->n) return fail(e, ZR_ERR_STATE, "zr_adjoint_set was not called");
+  if (int rc_order = user_order(e)) return rc_order;
   static_assert(CNT_CFL_RUN == CNT_ADJ_BAD + 1, "cleared together");
   ZR_HIP(e, hipMemsetAsync(e->dcount + CNT_ADJ_BAD, 0, 2 * sizeof(uint32_t), e->stream));
   DeferCfl defer(e);
@@ -3732,6 +3935,7 @@ int zr_get_admm_state(zr_engine* e, double* F, double* y, double* omega)
 {
   if (!e) return ZR_ERR_ARG;
   if (!e->admm_p || e->admm_n != e->n) return fail(e, ZR_ERR_STATE, "no ADMM step has run");
+  if (int rc_order = user_order(e)) return rc_order;
   const size_t N = (size_t)e->n;
   double* tmp = nullptr;
   ZR_HIP(e, hipMalloc(&tmp, 9 * N * sizeof(double)));
@@ -3742,7 +3946,7 @@ int zr_get_admm_state(zr_engine* e, double* F, double* y, double* omega)
   } items[] = { { F, e->admm_p, 9 }, { y, e->admm_p + 9 * N, 9 }, { omega, e->admm_p + 18 * N, 1 } };
   for (auto& it : items) {
     if (!it.dst) continue;
-    k_soa_to_aos<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(it.src, tmp, (uint32_t)N, it.nc, e->n);
+    k_soa_to_aos<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(it.src, tmp, (uint32_t)N, it.nc, e->n, nullptr);
     hipError_t stt = hipGetLastError();
     if (stt == hipSuccess)
       stt = hipMemcpyAsync(it.dst, tmp, it.nc * N * sizeof(double), hipMemcpyDeviceToHost, e->stream);
@@ -3983,6 +4187,8 @@ int zr_debug_dump(zr_engine* e, int32_t what, void* host, size_t bytes)
   int64_t need = zr_debug_size(e, what);
   if (need < 0 || (size_t)need != bytes || (need > 0 && !host)) return fail(e, ZR_ERR_ARG, "bad dump request");
   if (need == 0) return ZR_OK;
+  if (what == ZR_DUMP_SORTER || what == ZR_DUMP_ORDER || what == ZR_DUMP_BASE_OFFSET)
+    if (int rc_order = user_order(e)) return rc_order;
   hipStream_t s = e->stream;
   const uint32_t n = (uint32_t)e->n, A = e->A, nn = e->S * 32;
   ZR_HIP(e, hipStreamSynchronize(s));
