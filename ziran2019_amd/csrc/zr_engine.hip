@@ -74,9 +74,11 @@ struct ColliderSet {
   DevCollider c[kMaxColliders];
 };
 
-// device counters: the first CNT_SORT are zeroed by every sort; CNT_ADJ_BAD
-// and CNT_CFL_RUN (the CFL flags of every step since it was last cleared)
-// are cleared by the calls that read them
+// device counters of a sort and its step, in two banks: a sort uses one and
+// zeroes the other for the next.  CNT_ADJ_BAD and CNT_CFL_RUN (the CFL flags
+// of every step since it was last cleared) lie beside the banks and are
+// cleared by the calls that read them; the host's mirror holds the bank, the
+// two and the number of the publication.
 enum {
   CNT_GROUPS = 0,
   CNT_SLOTS = 1,
@@ -86,10 +88,25 @@ enum {
   CNT_BREAKS = 5,   // sampled groups' places where the order is not consecutive
   CNT_SAMPLED = 6,  // their particles
   CNT_SORT = 7,
-  CNT_ADJ_BAD = 7,
-  CNT_CFL_RUN = 8,
-  CNT_N = 10
+  CNT_ADJ_BAD = 8,
+  CNT_CFL_RUN = 9,
+  CNT_SEQ = 10,
+  CNT_N = 11
 };
+constexpr int kBank = 16;  // words between the banks; the two others follow both
+enum { RUN_ADJ_BAD = 0, RUN_CFL = 1 };
+
+// the counters to the host's pinned mirror, then the publication's number
+__global__ void k_publish(const uint32_t* __restrict__ bank, const uint32_t* __restrict__ run, uint32_t* host,
+                          uint32_t seq)
+{
+  const uint32_t t = threadIdx.x;
+  if (t < CNT_SORT) __hip_atomic_store(host + t, bank[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (t == CNT_ADJ_BAD || t == CNT_CFL_RUN)
+    __hip_atomic_store(host + t, run[t - CNT_ADJ_BAD], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __threadfence_system();
+  if (t == 0) __hip_atomic_store(host + CNT_SEQ, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // ---------------------------------------------------------------------------
 // collisions: AnalyticCollisionObject moving as x = R s X + b(t)
@@ -204,13 +221,13 @@ __device__ __forceinline__ void trial_collision(const ColliderSet& cs, int fr, c
 // ---------------------------------------------------------------------------
 // binning and sort (MpmSimulationBase.cpp:1032-1103)
 // ---------------------------------------------------------------------------
-// (and zeroes the sort's counters)
+// the dense page tables are clean between sorts: the sort resets what it
+// touched once its lists no longer need them
 __global__ void k_reset_tables(const uint32_t* group_page, uint32_t ngroups, const uint32_t* slot_page, uint32_t nslots,
                                uint32_t* page_count, int32_t* page_group, uint32_t* page_bits, uint32_t* page_sum,
-                               uint32_t* page_touch, int32_t* page_slot, uint32_t* counters)
+                               uint32_t* page_touch, int32_t* page_slot)
 {
   uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (counters && t < CNT_SORT) counters[t] = 0u;
   if (t < ngroups) {
     uint32_t p = group_page[t];
     page_count[p] = 0u;
@@ -329,6 +346,102 @@ __global__ __launch_bounds__(256) void k_list_groups(const uint32_t* page_sum, u
   }
 }
 
+// the same listing and the groups' first particles (the prefix sums of the
+// page counts) in one block, for extents of at most kListMax summary words
+// (2^9 nodes per axis): four launches and their gaps on the step's critical
+// path against one.  140,608 particles: 17.4 us of kernels to 7.3; 2.1M: 25 to
+// 24
+constexpr uint32_t kListMax = 4096;
+__global__ __launch_bounds__(1024) void k_list_pages(const uint32_t* __restrict__ page_sum, uint32_t nsum,
+                                                     const uint32_t* __restrict__ page_bits,
+                                                     const uint32_t* __restrict__ page_count, uint32_t* group_page,
+                                                     int32_t* __restrict__ page_group,
+                                                     uint32_t* __restrict__ group_start, uint32_t* counters)
+{
+  __shared__ uint16_t words[kListMax];  // the summary words that are not zero
+  __shared__ uint32_t base[kListMax];   // pages under each, then before each
+  __shared__ uint32_t smem[16];
+  const uint32_t tid = threadIdx.x, lane = tid & 31u;
+  uint32_t total;
+  {
+    const uint32_t q = (nsum + 1023u) / 1024u;
+    uint32_t set = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k)
+      if (k < q && tid * q + k < nsum && page_sum[tid * q + k]) set |= 1u << k;
+    uint32_t pos = block_exclusive_scan<1024>((uint32_t)__popc(set), total, smem);
+    while (set) {
+      words[pos++] = (uint16_t)(tid * q + (uint32_t)__builtin_ctz(set));
+      set &= set - 1u;
+    }
+  }
+  const uint32_t nw = total;
+  __syncthreads();
+  for (uint32_t i = tid >> 5; i < nw; i += 32u) {
+    const uint32_t w = words[i];
+    uint32_t c = ((page_sum[w] >> lane) & 1u) ? (uint32_t)__popc(page_bits[w * 32u + lane]) : 0u;
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) c += __shfl_xor(c, off, 32);
+    if (lane == 0) base[i] = c;
+  }
+  __syncthreads();
+  {
+    const uint32_t q = (nw + 1023u) / 1024u, b = tid * q;
+    uint32_t c = 0;
+    for (uint32_t k = 0; k < q; ++k)
+      if (b + k < nw) c += base[b + k];
+    uint32_t off = block_exclusive_scan<1024>(c, total, smem);
+    for (uint32_t k = 0; k < q; ++k)
+      if (b + k < nw) {
+        const uint32_t t = base[b + k];
+        base[b + k] = off;
+        off += t;
+      }
+  }
+  const uint32_t A = total;
+  if (tid == 0) counters[CNT_GROUPS] = A;
+  __syncthreads();
+  for (uint32_t i = tid >> 5; i < nw; i += 32u) {
+    const uint32_t w = words[i] * 32u + lane;
+    uint32_t bits = ((page_sum[words[i]] >> lane) & 1u) ? page_bits[w] : 0u;
+    const uint32_t c = (uint32_t)__popc(bits);
+    uint32_t incl = c;
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) {
+      const uint32_t t = __shfl_up(incl, off, 32);
+      if (lane >= (uint32_t)off) incl += t;
+    }
+    uint32_t g = base[i] + incl - c;
+    while (bits) {
+      const uint32_t pc = w * 32u + (uint32_t)__builtin_ctz(bits);
+      bits &= bits - 1u;
+      group_page[g] = pc;
+      page_group[pc] = (int32_t)g;
+      ++g;
+    }
+  }
+  __syncthreads();
+  uint32_t carry = 0;
+  for (uint32_t b0 = 0; b0 < A; b0 += 4096u) {
+    uint32_t v[4], c = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+      const uint32_t g = b0 + tid * 4u + k;
+      v[k] = g < A ? page_count[group_page[g]] : 0u;
+      c += v[k];
+    }
+    uint32_t off = carry + block_exclusive_scan<1024>(c, total, smem);
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+      const uint32_t g = b0 + tid * 4u + k;
+      if (g < A) group_start[g] = off;
+      off += v[k];
+    }
+    carry += total;
+  }
+  if (tid == 0) group_start[A] = carry;
+}
+
 // the group count the kernels after the page listing stop at: the
 // device-side count, or the launch's hint when that is smaller (the host
 // then repeats those kernels at the exact count)
@@ -359,14 +472,16 @@ struct LdFirstTouch {
 
 // a particle's sort key: cell within the page (5 bits) | the caller's index
 // (27 bits) | its place in the engine's arrays (32 bits)
-// (thread 0 also closes group_start with the particle total)
+// (thread 0 also closes group_start with the particle total, where it is
+// given, and the first threads zero the next sort's counters)
 __global__ void k_scatter(uint32_t n, const uint32_t* p_page, const uint32_t* p_re, const int32_t* page_group,
                           uint32_t* group_start, uint64_t* keys, GroupBound gb, const uint32_t* total,
-                          const uint32_t* uid)
+                          const uint32_t* uid, uint32_t* next_counters)
 {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t ng = gb.get();
-  if (i == 0) group_start[ng] = *total;
+  if (total && i == 0) group_start[ng] = *total;
+  if (i < CNT_SORT) next_counters[i] = 0u;
   if (i >= n) return;
   uint32_t re = p_re[i];
   int32_t g = page_group[p_page[i]];
@@ -380,12 +495,17 @@ __global__ void k_scatter(uint32_t n, const uint32_t* p_page, const uint32_t* p_
 // counters), and each particle's place in its cell's bucket is the number of
 // the bucket's caller's indices below its own;
 // and records where each cell's run begins within the group (cell_off,
-// 32 entries per group), for the transfers that work cell by cell
+// 32 entries per group), for the transfers that work cell by cell.
+// Its first threads touch the group's pages: SPGrid_Page_Map::Set_Page over
+// the 2x2x2 page neighbourhood in the reference loop order i(x), j(y), k(z)
+// (MpmSimulationBase.cpp:1081-1090), the first touch kept by atomicMin
 __global__ __launch_bounds__(256) void k_sort_groups(const uint64_t* __restrict__ keys,
                                                      const uint32_t* __restrict__ group_start,
                                                      uint32_t* order,
                                                      uint32_t* __restrict__ cell_off, GroupBound gb,
-                                                     uint32_t* counters)
+                                                     uint32_t* counters, const uint32_t* __restrict__ group_page,
+                                                     uint32_t* __restrict__ touch_page,
+                                                     uint32_t* __restrict__ page_touch)
 {
   __shared__ uint32_t bucket[kSortLds];  // caller's indices by cell, unordered within a cell
   __shared__ uint32_t pidx[kSortLds];    // caller's index of each key position
@@ -399,6 +519,14 @@ __global__ __launch_bounds__(256) void k_sort_groups(const uint64_t* __restrict_
   const uint32_t start = group_start[g];
   const uint32_t n = group_start[g + 1] - start;
   if (tid < 32) cnt[tid] = 0u;
+  if (tid < 8) {
+    uint32_t px, py, pz;
+    page_decode(group_page[g], px, py, pz);
+    const uint32_t t = 8u * g + (uint32_t)tid;
+    const uint32_t q = page_encode(px + (tid >> 2), py + ((tid >> 1) & 1), pz + (tid & 1));
+    touch_page[t] = q;
+    atomicMin(&page_touch[q], t);
+  }
   __syncthreads();
   const bool in_lds = n <= (uint32_t)kSortLds;
   for (uint32_t k = tid; k < n; k += 256) {
@@ -464,20 +592,6 @@ __global__ __launch_bounds__(256) void k_sort_groups(const uint64_t* __restrict_
   }
 }
 
-// SPGrid_Page_Map::Set_Page over the 2x2x2 page neighbourhood of each group in
-// the reference loop order i(x), j(y), k(z) (MpmSimulationBase.cpp:1081-1090)
-__global__ void k_touch(GroupBound gb, const uint32_t* group_page, uint32_t* touch_page, uint32_t* page_touch)
-{
-  uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 8u * gb.get()) return;
-  uint32_t g = t >> 3, o = t & 7u;
-  uint32_t px, py, pz;
-  page_decode(group_page[g], px, py, pz);
-  uint32_t q = page_encode(px + (o >> 2), py + ((o >> 1) & 1u), pz + (o & 1u));
-  touch_page[t] = q;
-  atomicMin(&page_touch[q], t);
-}
-
 __global__ void k_assign_slots(GroupBound gb, const uint32_t* touch_page, const uint32_t* page_touch,
                                const uint32_t* touch_slot, uint32_t* slot_page, int32_t* page_slot)
 {
@@ -490,29 +604,84 @@ __global__ void k_assign_slots(GroupBound gb, const uint32_t* touch_page, const 
   page_slot[q] = (int32_t)s;
 }
 
-// the 8 neighbour page slots of every group, in touch order (o = 4a + 2b + c)
-__global__ void k_group_slots(GroupBound gb, const uint32_t* touch_page, const int32_t* page_slot,
-                              int32_t* group_nslot)
+// the group whose staged tile overlaps slot page q from q - (a, b, c), o =
+// 4a + 2b + c (-1 when absent)
+__device__ __forceinline__ int32_t slot_source(uint32_t q, uint32_t o, const int32_t* page_group)
 {
-  uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 8u * gb.get()) return;
-  group_nslot[t] = page_slot[touch_page[t]];
-}
-
-// the <= 8 groups whose staged tiles overlap each slot page (o = 4a + 2b + c
-// for the source page q - (a, b, c); -1 when absent)
-__global__ void k_slot_sources(uint32_t nslots, const uint32_t* slot_page, const int32_t* page_group,
-                               int32_t* slot_src)
-{
-  uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 8u * nslots) return;
-  const uint32_t s = t >> 3, o = t & 7u;
   const uint32_t a = o >> 2, b = (o >> 1) & 1u, c = o & 1u;
   uint32_t qx, qy, qz;
-  page_decode(slot_page[s], qx, qy, qz);
-  int32_t src = -1;
-  if (a <= qx && b <= qy && c <= qz) src = page_group[page_encode(qx - a, qy - b, qz - c)];
-  slot_src[t] = src;
+  page_decode(q, qx, qy, qz);
+  return a <= qx && b <= qy && c <= qz ? page_group[page_encode(qx - a, qy - b, qz - c)] : -1;
+}
+
+// the 8 neighbour page slots of every group, in touch order, and the <= 8
+// source groups of every slot
+__global__ void k_slot_tables(uint32_t ngroups, uint32_t nslots, const uint32_t* __restrict__ touch_page,
+                              const int32_t* __restrict__ page_slot, int32_t* __restrict__ group_nslot,
+                              const uint32_t* __restrict__ slot_page, const int32_t* __restrict__ page_group,
+                              int32_t* __restrict__ slot_src)
+{
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < 8u * ngroups) group_nslot[t] = page_slot[touch_page[t]];
+  if (t < 8u * nslots) slot_src[t] = slot_source(slot_page[t >> 3], t & 7u, page_group);
+}
+
+// The slots (pages in order of their first touch), both tables and the reset
+// of the dense page tables in one block, for at most kSlotsMax groups: five
+// launches and the host's look at the slot count between them against one.
+// Stops at a group count above the hint or a slot count above the buffers'
+// (the host then repeats the rest in the kernels above).  140,608 particles
+// (700 groups): 15.6 us against 18.5 of kernels, five launches and a wait.
+// Above kSlotsMax the grid-wide kernels: 16 touches per thread is what stays
+// in registers, and one block takes a microsecond per 45 groups
+constexpr uint32_t kSlotsMax = 2048;
+__global__ __launch_bounds__(1024) void k_slots(const uint32_t* __restrict__ group_page, uint32_t hint, uint32_t smax,
+                                                const uint32_t* __restrict__ touch_page, uint32_t* page_touch,
+                                                int32_t* page_slot, uint32_t* slot_page,
+                                                int32_t* __restrict__ group_nslot, int32_t* __restrict__ slot_src,
+                                                uint32_t* page_count, int32_t* page_group, uint32_t* page_bits,
+                                                uint32_t* page_sum, uint32_t* counters)
+{
+  __shared__ uint32_t smem[16];
+  const uint32_t tid = threadIdx.x;
+  const uint32_t A = counters[CNT_GROUPS];
+  if (A > hint) return;
+  const uint32_t T = 8u * A, q = (T + 1023u) / 1024u, t0 = tid * q;
+  uint32_t page[16], first = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 16u; ++k) page[k] = k < q && t0 + k < T ? touch_page[t0 + k] : kNone;
+#pragma unroll
+  for (uint32_t k = 0; k < 16u; ++k)
+    if (page[k] != kNone && page_touch[page[k]] == t0 + k) first |= 1u << k;
+  uint32_t S;
+  uint32_t s = block_exclusive_scan<1024>((uint32_t)__popc(first), S, smem);
+#pragma unroll
+  for (uint32_t k = 0; k < 16u; ++k)
+    if ((first >> k) & 1u) {
+      slot_page[s] = page[k];
+      page_slot[page[k]] = (int32_t)s;
+      ++s;
+    }
+  if (tid == 0) counters[CNT_SLOTS] = S;
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < 16u; ++k)
+    if (page[k] != kNone) group_nslot[t0 + k] = page_slot[page[k]];
+  if (S > smax) return;
+  for (uint32_t t = tid; t < 8u * S; t += 1024u) slot_src[t] = slot_source(slot_page[t >> 3], t & 7u, page_group);
+  __syncthreads();
+  for (uint32_t g = tid; g < A; g += 1024u) {
+    const uint32_t p = group_page[g];
+    page_count[p] = 0u;
+    page_group[p] = -1;
+    page_bits[p >> 5] = 0u;
+    page_sum[p >> 10] = 0u;
+  }
+  for (uint32_t k = tid; k < S; k += 1024u) {
+    const uint32_t p = slot_page[k];
+    page_touch[p] = kNone;
+    page_slot[p] = -1;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -932,9 +1101,10 @@ template <bool MLS>
 __global__ __launch_bounds__(g2p_threads<MLS>()) void k_g2p(ParticlesView P, const uint32_t* __restrict__ order,
                                                  const uint32_t* __restrict__ group_start,
                                                  const uint32_t* __restrict__ group_page,
-                                                 const int32_t* __restrict__ page_slot, const double* __restrict__ gvs,
-                                                 int64_t gstride, double dx, double inv_dx, double Dinv, double dt,
-                                                 double cfl, uint32_t* counters)
+                                                 const int32_t* __restrict__ group_nslot,
+                                                 const double* __restrict__ gvs, int64_t gstride, double dx,
+                                                 double inv_dx, double Dinv, double dt, double cfl, uint32_t* counters,
+                                                 uint32_t* run)
 {
   __shared__ double tv[3 * kTileNodes];
   __shared__ int32_t nslot[8];
@@ -944,7 +1114,7 @@ __global__ __launch_bounds__(g2p_threads<MLS>()) void k_g2p(ParticlesView P, con
   const uint32_t n = group_start[g + 1] - start;
   uint32_t px, py, pz;
   page_decode(group_page[g], px, py, pz);
-  if (tid < 8) nslot[tid] = page_slot[page_encode(px + (tid >> 2), py + ((tid >> 1) & 1), pz + (tid & 1))];
+  if (tid < 8) nslot[tid] = group_nslot[8 * (size_t)g + tid];
   __syncthreads();
   constexpr int NT = g2p_threads<MLS>();
   for (int t = tid; t < kTileNodes; t += NT) {
@@ -1039,7 +1209,7 @@ __global__ __launch_bounds__(g2p_threads<MLS>()) void k_g2p(ParticlesView P, con
   }
   if (flags) {
     atomicOr(&counters[CNT_CFL], flags);
-    atomicOr(&counters[CNT_CFL_RUN], flags);
+    atomicOr(&run[RUN_CFL], flags);
   }
 }
 
@@ -1424,7 +1594,11 @@ struct zr_engine {
 
   uint32_t* scan_tmp = nullptr;
   size_t scan_cap = 0;
-  uint32_t* dcount = nullptr;
+  uint32_t* dbase = nullptr;   // the counters' two banks and the two counters beside them
+  uint32_t* dcount = nullptr;  // the current bank
+  uint32_t* drun = nullptr;    // RUN_ADJ_BAD, RUN_CFL
+  uint32_t seq = 0;            // publications of the counters so far
+  bool tables_clean = true;    // nothing left in the dense page tables by a sort that failed
   // evalMaxParticleSpeed: 7 block maxima per block, then the 7 results
   double* speed = nullptr;
   uint32_t* hcount = nullptr;
@@ -1471,8 +1645,6 @@ struct zr_engine {
   std::vector<Spare> alt;
   double disorder = 0.0;
   size_t cell_cap = 0;           // groups
-  // the CFL flag counter is zero (the sort clears every counter; only G2P sets it)
-  bool cfl_clear = false;
   // inside a rollout: a step does not wait for its CFL flags; the next
   // step's sort reads them (CNT_CFL_RUN) and stops the rollout there
   bool defer_cfl = false;
@@ -1593,10 +1765,25 @@ int prof_mark(zr_engine* e, int k)
   return ZR_OK;
 }
 
+// The counters on the host, after all the work enqueued so far.  A kernel
+// stores them in pinned memory and the host watches for its number: a device
+// to host copy and a stream synchronisation take some 10 us more per wait.
+// The stream is asked now and then, so that a failed kernel ends the wait.
 int sync_counts(zr_engine* e)
 {
-  ZR_HIP(e, hipMemcpyAsync(e->hcount, e->dcount, CNT_N * sizeof(uint32_t), hipMemcpyDeviceToHost, e->stream));
-  ZR_HIP(e, hipStreamSynchronize(e->stream));
+  const uint32_t seq = ++e->seq;
+  k_publish<<<1, 64, 0, e->stream>>>(e->dcount, e->drun, e->hcount, seq);
+  ZR_LAUNCH_CHECK(e);
+  for (uint32_t spins = 1; __atomic_load_n(e->hcount + CNT_SEQ, __ATOMIC_ACQUIRE) != seq; ++spins) {
+    if (spins % 8192u == 0u) {
+      const hipError_t st = hipStreamQuery(e->stream);
+      if (st == hipErrorNotReady) continue;
+      if (st != hipSuccess) return fail(e, ZR_ERR_HIP, std::string("waiting for the step: ") + hipGetErrorString(st));
+      if (__atomic_load_n(e->hcount + CNT_SEQ, __ATOMIC_ACQUIRE) != seq)
+        return fail(e, ZR_ERR_HIP, "the step's counters did not arrive");
+    }
+    __builtin_ia32_pause();
+  }
   return ZR_OK;
 }
 
@@ -1736,16 +1923,22 @@ int ensure_grid(zr_engine* e)
   return ZR_OK;
 }
 
-// the sort after the page listing, for at most `hint` groups (GroupBound)
+// the sort after the page listing, for at most `hint` groups (GroupBound):
+// particles into their groups, the groups' order and their pages' touches
 int sort_groups(zr_engine* e, uint32_t hint)
 {
   hipStream_t s = e->stream;
   const uint32_t n = (uint32_t)e->n;
   const GroupBound gb{ e->dcount + CNT_GROUPS, hint };
-  int rc = run_scan(e, LdGroupCount{ e->group_count, gb }, hint, e->group_start, e->dcount + CNT_TOTAL);
-  if (rc) return rc;
+  const bool listed = e->nsum <= kListMax;  // k_list_pages has written group_start
+  if (!listed) {
+    int rc = run_scan(e, LdGroupCount{ e->group_count, gb }, hint, e->group_start, e->dcount + CNT_TOTAL);
+    if (rc) return rc;
+  }
+  uint32_t* const next = e->dcount == e->dbase ? e->dbase + kBank : e->dbase;
   k_scatter<<<blocks_for(n, 256), 256, 0, s>>>(n, e->p_page, e->p_re, e->page_group, e->group_start, e->keys, gb,
-                                               e->dcount + CNT_TOTAL, e->permuted ? e->uid : nullptr);
+                                               listed ? nullptr : e->dcount + CNT_TOTAL,
+                                               e->permuted ? e->uid : nullptr, next);
   if (e->cell_cap < hint) {
     dfree(e->cell_off);
     e->cell_cap = 0;
@@ -1753,16 +1946,34 @@ int sort_groups(zr_engine* e, uint32_t hint)
     ZR_HIP(e, hipMalloc(&e->cell_off, 32 * cap * sizeof(uint32_t)));
     e->cell_cap = cap;
   }
-  k_sort_groups<<<hint, 256, 0, s>>>(e->keys, e->group_start, e->order, e->cell_off, gb, e->dcount);
-  k_touch<<<blocks_for(8ull * hint, 256), 256, 0, s>>>(gb, e->group_page, e->touch_page, e->page_touch);
+  k_sort_groups<<<hint, 256, 0, s>>>(e->keys, e->group_start, e->order, e->cell_off, gb, e->dcount, e->group_page,
+                                     e->touch_page, e->page_touch);
   ZR_LAUNCH_CHECK(e);
-  rc = run_scan(e, LdFirstTouch{ e->touch_page, e->page_touch, gb }, 8u * hint, e->touch_slot,
-                e->dcount + CNT_SLOTS);
+  return ZR_OK;
+}
+
+// the touched pages' slots in order of first touch
+int assign_slots(zr_engine* e, uint32_t hint)
+{
+  const GroupBound gb{ e->dcount + CNT_GROUPS, hint };
+  int rc = run_scan(e, LdFirstTouch{ e->touch_page, e->page_touch, gb }, 8u * hint, e->touch_slot,
+                    e->dcount + CNT_SLOTS);
   if (rc) return rc;
-  k_assign_slots<<<blocks_for(8ull * hint, 256), 256, 0, s>>>(gb, e->touch_page, e->page_touch, e->touch_slot,
-                                                             e->slot_page, e->page_slot);
-  k_group_slots<<<blocks_for(8ull * hint, 256), 256, 0, s>>>(gb, e->touch_page, e->page_slot, e->group_nslot);
+  k_assign_slots<<<blocks_for(8ull * hint, 256), 256, 0, e->stream>>>(gb, e->touch_page, e->page_touch,
+                                                                      e->touch_slot, e->slot_page, e->page_slot);
   ZR_LAUNCH_CHECK(e);
+  return ZR_OK;
+}
+
+int reset_tables(zr_engine* e)
+{
+  const uint32_t rst = e->A > e->S ? e->A : e->S;
+  if (rst)
+    k_reset_tables<<<blocks_for(rst, 256), 256, 0, e->stream>>>(e->group_page, e->A, e->slot_page, e->S,
+                                                                e->page_count, e->page_group, e->page_bits,
+                                                                e->page_sum, e->page_touch, e->page_slot);
+  ZR_LAUNCH_CHECK(e);
+  e->tables_clean = true;
   return ZR_OK;
 }
 
@@ -1872,27 +2083,30 @@ int do_sort(zr_engine* e, zr_step_stats* st)
   if (e->n <= 0) return fail(e, ZR_ERR_STATE, "no particles uploaded");
   const uint32_t n = (uint32_t)e->n;
   hipStream_t s = e->stream;
-  // clear the dense tables touched by the previous sort
-  uint32_t rst = e->A > e->S ? e->A : e->S;
-  const uint32_t nrst = rst > (uint32_t)CNT_N ? rst : (uint32_t)CNT_N;
   e->sorted = e->rasterised = e->updated = false;
-  e->cfl_clear = true;
+  int rc = ZR_OK;
+  if (!e->tables_clean) {  // a sort that failed left its entries
+    rc = reset_tables(e);
+    if (rc) return rc;
+  }
+  e->dcount = e->dcount == e->dbase ? e->dbase + kBank : e->dbase;
+  e->tables_clean = false;
+  e->A = e->S = 0;
   prof_mark(e, ZR_PROF_SORT);
-  k_reset_tables<<<blocks_for(nrst, 256), 256, 0, s>>>(e->group_page, e->A, e->slot_page, e->S, e->page_count,
-                                                      e->page_group, e->page_bits, e->page_sum, e->page_touch,
-                                                      e->page_slot, e->dcount);
   k_bin<<<blocks_for(n, 256), 256, 0, s>>>(e->x, e->n, n, 1.0 / e->cfg.dx, (int)e->lim, e->page_count, e->page_bits,
                                            e->page_sum, e->p_page, e->p_re, e->dcount);
   ZR_LAUNCH_CHECK(e);
-  uint32_t nbs = (e->nsum + 7u) / 8u;
-  if (nbs > 2048u) nbs = 2048u;
-  k_sum_counts<<<nbs, 256, 0, s>>>(e->page_sum, e->nsum, e->page_bits, e->page_sumcnt);
-  int rc = run_scan(e, LdArray{ e->page_sumcnt }, e->nsum, e->sum_base, e->dcount + CNT_GROUPS);
-  if (rc) return rc;
-  {
-    const uint32_t nb = nbs;
-    k_list_groups<<<nb, 256, 0, s>>>(e->page_sum, e->nsum, e->page_bits, e->sum_base, e->page_count, e->group_page,
-                                     e->page_group, e->group_count);
+  if (e->nsum <= kListMax) {
+    k_list_pages<<<1, 1024, 0, s>>>(e->page_sum, e->nsum, e->page_bits, e->page_count, e->group_page, e->page_group,
+                                    e->group_start, e->dcount);
+  } else {
+    uint32_t nbs = (e->nsum + 7u) / 8u;
+    if (nbs > 2048u) nbs = 2048u;
+    k_sum_counts<<<nbs, 256, 0, s>>>(e->page_sum, e->nsum, e->page_bits, e->page_sumcnt);
+    rc = run_scan(e, LdArray{ e->page_sumcnt }, e->nsum, e->sum_base, e->dcount + CNT_GROUPS);
+    if (rc) return rc;
+    k_list_groups<<<nbs, 256, 0, s>>>(e->page_sum, e->nsum, e->page_bits, e->sum_base, e->page_count, e->group_page,
+                                      e->page_group, e->group_count);
   }
   ZR_LAUNCH_CHECK(e);
   // group sizes, in-page order and slots: launched for a hint of the group
@@ -1906,9 +2120,8 @@ int do_sort(zr_engine* e, zr_step_stats* st)
     if (rc) return rc;
     hint = e->hcount[CNT_GROUPS];
     if (e->hcount[CNT_DOMAIN]) {
-      // tables hold clamped entries; keep A so the next sort clears them
+      // the tables hold clamped entries; A is kept so that the next sort clears them
       e->A = hint;
-      e->S = 0;
       return fail(e, ZR_ERR_DOMAIN, "particle base node outside [0, 2^grid_log2 - 8]");
     }
   }
@@ -1916,23 +2129,37 @@ int do_sort(zr_engine* e, zr_step_stats* st)
   if (hint == 0) hint = 1;
   rc = sort_groups(e, hint);
   if (rc) return rc;
+  // the slots and their tables in one block, or grid-wide kernels that need
+  // the slot count
+  const bool one_block = hint <= kSlotsMax && e->slot_src;
+  const uint32_t smax = (uint32_t)(e->grid_cap / 32);
+  if (one_block) {
+    k_slots<<<1, 1024, 0, s>>>(e->group_page, hint, smax, e->touch_page, e->page_touch, e->page_slot, e->slot_page,
+                               e->group_nslot, e->slot_src, e->page_count, e->page_group, e->page_bits, e->page_sum,
+                               e->dcount);
+    ZR_LAUNCH_CHECK(e);
+  } else {
+    rc = assign_slots(e, hint);
+    if (rc) return rc;
+  }
   prof_mark(e, ZR_PROF_SORT);
   rc = sync_counts(e);
   if (rc) return rc;
   const uint32_t A = e->hcount[CNT_GROUPS];
+  const bool exact = A <= hint;
+  bool tables = one_block && exact && e->hcount[CNT_SLOTS] <= smax;  // k_slots went through
+  e->tables_clean = tables;
   e->A = A;
   e->S = e->hcount[CNT_SLOTS];
-  if (e->hcount[CNT_DOMAIN]) {
-    // tables hold clamped entries; A and S are kept so the next sort clears them
-    return fail(e, ZR_ERR_DOMAIN, "particle base node outside [0, 2^grid_log2 - 8]");
-  }
-  if (A > hint) {
+  if (!exact) {
     rc = sort_groups(e, A);
-    if (rc) return rc;
-    rc = sync_counts(e);
+    if (!rc) rc = assign_slots(e, A);
+    if (!rc) rc = sync_counts(e);
     if (rc) return rc;
     e->S = e->hcount[CNT_SLOTS];
   }
+  if (e->hcount[CNT_DOMAIN])  // (the tables' clamped entries are cleared by the next sort, if not yet)
+    return fail(e, ZR_ERR_DOMAIN, "particle base node outside [0, 2^grid_log2 - 8]");
   e->a_hint = A + A / 4 + 64 < n ? A + A / 4 + 64 : n;
   // a rollout's earlier step asked for a restart: the particles are those
   // after that step (a sort moves none)
@@ -1954,9 +2181,13 @@ int do_sort(zr_engine* e, zr_step_stats* st)
   }
   rc = ensure_grid(e);
   if (rc) return rc;
-  if (e->S) {
-    k_slot_sources<<<blocks_for(8ull * e->S, 256), 256, 0, s>>>(e->S, e->slot_page, e->page_group, e->slot_src);
+  if (!tables) {
+    const uint32_t m = 8u * (A > e->S ? A : e->S);
+    k_slot_tables<<<blocks_for(m, 256), 256, 0, s>>>(A, e->S, e->touch_page, e->page_slot, e->group_nslot,
+                                                     e->slot_page, e->page_group, e->slot_src);
     ZR_LAUNCH_CHECK(e);
+    rc = reset_tables(e);
+    if (rc) return rc;
   }
   e->sorted = true;
   if (st) {
@@ -2049,19 +2280,17 @@ int do_g2p(zr_engine* e, double dt, zr_step_stats* st, bool mls)
 {
   if (!e->updated) return fail(e, ZR_ERR_STATE, "gridToParticles before the grid update");
   const double dx = e->cfg.dx;
-  if (!e->cfl_clear) ZR_HIP(e, hipMemsetAsync(e->dcount + CNT_CFL, 0, sizeof(uint32_t), e->stream));
-  e->cfl_clear = false;
   ParticlesView pv = pview(e);
   pv.gradv = e->g2p_gradv;
   prof_mark(e, ZR_PROF_G2P);
   if (mls)
-    k_g2p<true><<<e->A, g2p_threads<true>(), 0, e->stream>>>(pview(e), e->order, e->group_start, e->group_page, e->page_slot, e->gvs,
+    k_g2p<true><<<e->A, g2p_threads<true>(), 0, e->stream>>>(pview(e), e->order, e->group_start, e->group_page, e->group_nslot, e->gvs,
                                              (int64_t)e->grid_cap, dx, 1.0 / dx, 4.0 / (dx * dx), dt, e->cfg.cfl,
-                                             e->dcount);
+                                             e->dcount, e->drun);
   else
-    k_g2p<false><<<e->A, g2p_threads<false>(), 0, e->stream>>>(pv, e->order, e->group_start, e->group_page, e->page_slot,
+    k_g2p<false><<<e->A, g2p_threads<false>(), 0, e->stream>>>(pv, e->order, e->group_start, e->group_page, e->group_nslot,
                                               e->gvs, (int64_t)e->grid_cap, dx, 1.0 / dx, 4.0 / (dx * dx), dt,
-                                              e->cfg.cfl, e->dcount);
+                                              e->cfg.cfl, e->dcount, e->drun);
   ZR_LAUNCH_CHECK(e);
   if (mls && e->visco) {  // the viscoelastic helper's evolveStrain with gradV = C
     k_visco_strain<<<blocks_for((uint64_t)e->n, 256), 256, 0, e->stream>>>(
@@ -2264,7 +2493,7 @@ int adjoint_kernels(zr_engine* e, double dt, const AdjTables& t)
   if (nn) {
     k_adj_grid<<<blocks_for(nn, 256), 256, 0, s>>>(nn, t.slot_page, t.slot_src, e->stage, G, e->adj_grid, dx, dt,
                                                    e->cfg.gravity[0], e->cfg.gravity[1], e->cfg.gravity[2],
-                                                   collider_set(e, dt), e->dcount + CNT_ADJ_BAD);
+                                                   collider_set(e, dt), e->drun + RUN_ADJ_BAD);
     ZR_LAUNCH_CHECK(e);
   }
   k_adj_p2g<<<t.A, 256, 0, s>>>(pview(e), A, t.order, t.group_start, t.group_page, t.group_nslot, e->adj_grid,
@@ -2774,7 +3003,7 @@ int be_state_residual(zr_engine* e, bool jac = false)
   prof_mark(e, ZR_PROF_STATE);
   if (jac)
     k_be_state<T, true><<<e->A, 256, 0, e->stream>>>(pview(e), hvp_cache<T>(e), e->order, e->group_start,
-                                                     e->group_page, e->page_slot, e->ivn, e->idv,
+                                                     e->group_page, e->group_nslot, e->ivn, e->idv,
                                                      (int64_t)e->grid_cap, dx, 1.0 / dx, dt, e->stage, co, e->jstage);
   else {
     // the same state in three passes (k_be_grad, k_be_svd, k_be_scatter):
@@ -2787,7 +3016,7 @@ int be_state_residual(zr_engine* e, bool jac = false)
       e->be_fb_cap = N;
     }
     const HvpCache<T> hc = hvp_cache<T>(e);
-    k_be_grad<T><<<e->A, 256, 0, e->stream>>>(pview(e), hc, e->order, e->group_start, e->group_page, e->page_slot,
+    k_be_grad<T><<<e->A, 256, 0, e->stream>>>(pview(e), hc, e->order, e->group_start, e->group_page, e->group_nslot,
                                               e->ivn, e->idv, (int64_t)e->grid_cap, 1.0 / dx, dt, e->be_fb, co);
     k_be_svd<T><<<blocks_for(N, 256), 256, 0, e->stream>>>(pview(e), hc, e->order, (uint32_t)N, e->be_fb);
     k_be_scatter<<<e->A, 256, 0, e->stream>>>(pview(e), e->order, e->group_start, e->group_page, hc.stride,
@@ -3165,10 +3394,15 @@ int zr_create(const zr_config* cfg, zr_engine** out)
             hipMalloc(&e->page_sum, e->nsum * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&e->page_sumcnt, e->nsum * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&e->sum_base, (e->nsum + 1) * sizeof(uint32_t)) == hipSuccess &&
-            hipMalloc(&e->dcount, CNT_N * sizeof(uint32_t)) == hipSuccess &&
+            hipMalloc(&e->dbase, 3 * kBank * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&e->ticket, sizeof(uint32_t)) == hipSuccess &&
             hipHostMalloc(&e->hcount, CNT_N * sizeof(uint32_t)) == hipSuccess;
-  ok = ok && hipMemset(e->dcount, 0, CNT_N * sizeof(uint32_t)) == hipSuccess;
+  ok = ok && hipMemset(e->dbase, 0, 3 * kBank * sizeof(uint32_t)) == hipSuccess;
+  if (ok) {
+    e->dcount = e->dbase;
+    e->drun = e->dbase + 2 * kBank;
+    memset(e->hcount, 0, CNT_N * sizeof(uint32_t));
+  }
   ok = ok && hipMemset(e->page_count, 0, e->ndense * sizeof(uint32_t)) == hipSuccess &&
        hipMemset(e->page_group, 0xff, e->ndense * sizeof(int32_t)) == hipSuccess &&
        hipMemset(e->page_touch, 0xff, e->ndense * sizeof(uint32_t)) == hipSuccess &&
@@ -3193,7 +3427,7 @@ void zr_destroy(zr_engine* e)
   free_particles(e);
   dfree(e->page_count); dfree(e->page_group); dfree(e->page_touch); dfree(e->page_slot); dfree(e->page_bits);
   dfree(e->page_sum); dfree(e->page_sumcnt); dfree(e->sum_base); dfree(e->stage); dfree(e->gm); dfree(e->gv); dfree(e->gf); dfree(e->gvs);
-  dfree(e->scan_tmp); dfree(e->cell_off); dfree(e->speed); dfree(e->dcount); dfree(e->ticket); dfree(e->slot_src);
+  dfree(e->scan_tmp); dfree(e->cell_off); dfree(e->speed); dfree(e->dbase); dfree(e->ticket); dfree(e->slot_src);
   dfree(e->ivn); dfree(e->idv); dfree(e->ir); dfree(e->ix); dfree(e->irc); dfree(e->iq); dfree(e->ip); dfree(e->iap);
   dfree(e->partial); dfree(e->partial2); dfree(e->sc); dfree(e->ci); dfree(e->hvp_ctr); dfree(e->hvp_bounds); dfree(e->hvp_order); dfree(e->cell_order); dfree(e->jstage); dfree(e->pinv); dfree(e->collided); dfree(e->c64); dfree(e->c32); dfree(e->ccell);
   dfree(e->pf_node); dfree(e->pf_partial); dfree(e->adj_grid); dfree(e->admm_node); dfree(e->admm_coll); dfree(e->act); dfree(e->act_scan); dfree(e->be_fb); dfree(e->admm_c32); dfree(e->admm_cell32); dfree(e->admm_node32);
@@ -3358,17 +3592,13 @@ int zr_upload_particles(zr_engine* e, const zr_particles* p)
   if (p->n > 0 && (!p->X || !p->V || !p->C || !p->F || !p->mass || !p->vol || !p->mu || !p->lambda))
     return fail(e, ZR_ERR_ARG, "all particle attributes are required");
   ZR_HIP(e, hipStreamSynchronize(e->stream));
-  // reset tables owned by the previous particle set
-  if (e->A || e->S) {
-    uint32_t rst = e->A > e->S ? e->A : e->S;
-    k_reset_tables<<<blocks_for(rst, 256), 256, 0, e->stream>>>(e->group_page, e->A, e->slot_page, e->S,
-                                                                e->page_count, e->page_group, e->page_bits,
-                                                                e->page_sum, e->page_touch, e->page_slot,
-                                                                nullptr);
-    ZR_LAUNCH_CHECK(e);
+  // clear what a failed sort of the previous particle set left in the tables
+  if (!e->tables_clean) {
+    int rc = reset_tables(e);
+    if (rc) return rc;
     ZR_HIP(e, hipStreamSynchronize(e->stream));
-    e->A = e->S = 0;
   }
+  e->A = e->S = 0;
   free_particles(e);
   e->sorted = e->rasterised = e->updated = false;
   const int64_t n = p->n;
@@ -3728,7 +3958,7 @@ int zr_adjoint_step(zr_engine* e, double dt)
   if (!adjoint_supported(e)) return ZR_ERR_ARG;
   if (!e->adj || e->adj_n != e->n) return fail(e, ZR_ERR_STATE, "zr_adjoint_set was not called");
   if (int rc_order = user_order(e)) return rc_order;
-  ZR_HIP(e, hipMemsetAsync(e->dcount + CNT_ADJ_BAD, 0, sizeof(uint32_t), e->stream));
+  ZR_HIP(e, hipMemsetAsync(e->drun + RUN_ADJ_BAD, 0, sizeof(uint32_t), e->stream));
   return do_adjoint_step(e, dt, true);
 }
 
@@ -3835,7 +4065,7 @@ int zr_rollout_forward(zr_engine* e, int32_t steps, double dt, int32_t every, in
   if (!e) return ZR_ERR_ARG;
   if (steps < 0 || every < 1 || slot0 < 0 || !(dt > 0.0)) return fail(e, ZR_ERR_ARG, "bad rollout arguments");
   if (int rc_order = user_order(e)) return rc_order;
-  ZR_HIP(e, hipMemsetAsync(e->dcount + CNT_CFL_RUN, 0, sizeof(uint32_t), e->stream));
+  ZR_HIP(e, hipMemsetAsync(e->drun + RUN_CFL, 0, sizeof(uint32_t), e->stream));
   DeferCfl defer(e);
   for (int32_t k = 0; k < steps; ++k) {
     if (k % every == 0) {
@@ -3858,8 +4088,8 @@ int zr_rollout_backward(zr_engine* e, int32_t steps, double dt, int32_t every, i
   if (!adjoint_supported(e)) return ZR_ERR_ARG;
   if (!e->adj || e->adj_n != e->n) return fail(e, ZR_ERR_STATE, "zr_adjoint_set was not called");
   if (int rc_order = user_order(e)) return rc_order;
-  static_assert(CNT_CFL_RUN == CNT_ADJ_BAD + 1, "cleared together");
-  ZR_HIP(e, hipMemsetAsync(e->dcount + CNT_ADJ_BAD, 0, 2 * sizeof(uint32_t), e->stream));
+  static_assert(RUN_ADJ_BAD == 0 && RUN_CFL == 1, "cleared together");
+  ZR_HIP(e, hipMemsetAsync(e->drun, 0, 2 * sizeof(uint32_t), e->stream));
   DeferCfl defer(e);
   const int32_t nseg = (steps + every - 1) / every;
   for (int32_t seg = nseg - 1; seg >= 0; --seg) {

@@ -137,33 +137,6 @@ __device__ __forceinline__ void project_node(const ColliderSet& cs, const double
   }
 }
 
-// sum of the <= 8 staged tiles overlapping node (slot page q, element e)
-template <int NF, class T>
-__device__ __forceinline__ void sum_tiles(const T* stage, const int32_t* page_group, uint32_t qx, uint32_t qy,
-                                          uint32_t qz, int ex, int ey, int ez, T acc[NF])
-{
-  constexpr int stride = NF * kTileNodes;
-#pragma unroll
-  for (int f = 0; f < NF; ++f) acc[f] = (T)0;
-  for (int a = 0; a < 2; ++a) {
-    if (a > (int)qx) break;
-    const int tx = ex + 2 * a;
-    for (int b = 0; b < 2; ++b) {
-      const int ty = ey + 4 * b;
-      if (ty >= kTileY || b > (int)qy) break;
-      for (int c = 0; c < 2; ++c) {
-        const int tz = ez + 4 * c;
-        if (tz >= kTileZ || c > (int)qz) break;
-        const int32_t src = page_group[page_encode(qx - a, qy - b, qz - c)];
-        if (src < 0) continue;
-        const T* base = stage + (size_t)src * stride + (tx * kTileY + ty) * kTileZ + tz;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) acc[f] += base[f * kTileNodes];
-      }
-    }
-  }
-}
-
 // sum of the <= 8 staged tiles overlapping a node, from the slot's
 // precomputed source groups (o = 4a + 2b + c, -1 when absent)
 template <int NF, class T>
@@ -240,14 +213,14 @@ __device__ __forceinline__ void node_pos(const NodeCoord& c, double dx, double x
   xi[2] = (double)(4 * (int)c.qz + c.ez) * dx;
 }
 
-// v* of the 4x6x6 footprint of group page (px,py,pz) -> LDS, summing up to two
-// node vectors (vn + dv); the 8 neighbour slots are looked up once
+// v* of the 4x6x6 footprint of a group -> LDS, summing up to two node vectors
+// (vn + dv), through the group's 8 neighbour slots
 template <class T, class TS>
-__device__ __forceinline__ void load_tile3(uint32_t px, uint32_t py, uint32_t pz, const int32_t* page_slot,
-                                           const TS* a, const TS* b, int64_t stride, T* tv, int32_t* nslot)
+__device__ __forceinline__ void load_tile3(const int32_t* gslot, const TS* a, const TS* b, int64_t stride, T* tv,
+                                           int32_t* nslot)
 {
   const int tid = threadIdx.x;
-  if (tid < 8) nslot[tid] = page_slot[page_encode(px + (tid >> 2), py + ((tid >> 1) & 1), pz + (tid & 1))];
+  if (tid < 8) nslot[tid] = gslot[tid];
   __syncthreads();
   for (int t = tid; t < kTileNodes; t += blockDim.x) {
     const int tx = t / (kTileY * kTileZ), ty = (t / kTileZ) % kTileY, tz = t % kTileZ;
@@ -433,7 +406,8 @@ __global__ __launch_bounds__(256) void k_be_state(ParticlesView P, HvpCache<T> c
                                                   const uint32_t* __restrict__ order,
                                                   const uint32_t* __restrict__ group_start,
                                                   const uint32_t* __restrict__ group_page,
-                                                  const int32_t* __restrict__ page_slot, const double* __restrict__ vn,
+                                                  const int32_t* __restrict__ group_nslot,
+                                                  const double* __restrict__ vn,
                                                   const double* __restrict__ dv, int64_t gstride, double dx,
                                                   double inv_dx, double dt, double* __restrict__ stage,
                                                   uint8_t* __restrict__ cell_order, double* __restrict__ dstage)
@@ -453,7 +427,7 @@ __global__ __launch_bounds__(256) void k_be_state(ParticlesView P, HvpCache<T> c
   const uint32_t n = group_start[g + 1] - start;
   uint32_t px, py, pz;
   page_decode(group_page[g], px, py, pz);
-  load_tile3(px, py, pz, page_slot, vn, dv, gstride, tv, nslot);
+  load_tile3(group_nslot + 8 * (size_t)g, vn, dv, gstride, tv, nslot);
   const int ox = 2 * (int)px, oy = 4 * (int)py, oz = 4 * (int)pz;
   double* wt = tile + (tid >> 6) * kImpStage;
   double* wd = dtile + (JAC ? (tid >> 6) * kImpStage : 0);
@@ -642,7 +616,7 @@ __global__ __launch_bounds__(256) void k_be_grad(ParticlesView P, HvpCache<T> ca
                                                  const uint32_t* __restrict__ order,
                                                  const uint32_t* __restrict__ group_start,
                                                  const uint32_t* __restrict__ group_page,
-                                                 const int32_t* __restrict__ page_slot,
+                                                 const int32_t* __restrict__ group_nslot,
                                                  const double* __restrict__ vn, const double* __restrict__ dv,
                                                  int64_t gstride, double inv_dx, double dt, double* __restrict__ fb,
                                                  uint8_t* __restrict__ cell_order)
@@ -657,7 +631,7 @@ __global__ __launch_bounds__(256) void k_be_grad(ParticlesView P, HvpCache<T> ca
   const uint32_t n = group_start[g + 1] - start;
   uint32_t px, py, pz;
   page_decode(group_page[g], px, py, pz);
-  load_tile3(px, py, pz, page_slot, vn, dv, gstride, tv, nslot);
+  load_tile3(group_nslot + 8 * (size_t)g, vn, dv, gstride, tv, nslot);
   const int ox = 2 * (int)px, oy = 4 * (int)py, oz = 4 * (int)pz;
   const uint32_t perm = (uint32_t)((tid & 31) * 8 + (tid >> 5));
   const int64_t S = P.stride, CS = cache.stride;
