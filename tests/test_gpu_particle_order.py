@@ -139,3 +139,34 @@ def test_checkpoint_of_a_moved_set():
         e.advanceOneTimeStep(1e-4)
     _same(e.download(), moved)
     e.close()
+
+
+@pytest.mark.parametrize("n", [1, 7, 21845, 21846, 70001, 700001])
+def test_transfers_around_the_window_size(n):
+    """Uploads and downloads cut into windows of 2^19 values: one window (kernel
+    to pinned memory), its edge (24 values per particle down, 28 up), several
+    windows per array, and the same engine again with as many particles and
+    with others."""
+    rng = np.random.default_rng(n)
+
+    def scene():
+        s = {k: rng.normal(size=(n, c)) for k, c in (("V", 3), ("C", 9), ("F", 9))}
+        s.update({k: 1 + rng.random(n) for k in ("mass", "vol", "mu", "lam")})
+        s["X"] = 0.2 + 0.5 * rng.random((n, 3))
+        return s
+
+    e = MpmEngine(dx=1.0 / 64)
+    for s in (scene(), scene()):
+        e.upload(s)
+        e.checkpoint_save(0)
+        _same(e.download(), {k: s[k] for k in ("X", "V", "C", "F")})
+        _same(e.download(("X",)), {"X": s["X"]})
+        a = dict(X=s["V"], V=s["X"], C=s["F"], F=s["C"], mu=s["mass"], lam=s["vol"])
+        e.adjoint_set(**a)
+        _same(e.adjoint_get(), a)
+        e.adjoint_set(X=s["V"])
+        got = e.adjoint_get(("X", "F", "mu"))
+        _same(got, dict(X=s["V"], F=np.zeros((n, 9)), mu=np.zeros(n)))
+    e.upload({k: np.asarray(v)[: max(1, n // 2)] for k, v in s.items()})
+    _same(e.download(), {k: s[k][: max(1, n // 2)] for k in ("X", "V", "C", "F")})
+    e.close()

@@ -49,7 +49,7 @@ class Rollout:
         eng.set_colliders(self.colliders)
         eng.set_time(0.0)
         eng.rollout_forward(self.steps, self.dt, self.every, 0)
-        return eng.download()["X"]
+        return eng.download(("X",))["X"]
 
     def backward(self, gX, gV=None):
         """Gradients (dE (n,), dV0 (n, 3)) of a loss whose gradient in the
@@ -60,7 +60,7 @@ class Rollout:
         # steps' inputs into the scratch slots, then the adjoint steps in
         # reverse (zr_rollout_backward)
         eng.rollout_backward(self.steps, self.dt, self.every, 0, self.nseg)
-        a = eng.adjoint_get()
+        a = eng.adjoint_get(("V", "mu", "lam"))
         nu = self.nu
         gE = a["mu"] / (2.0 * (1.0 + nu)) + a["lam"] * nu / ((1.0 + nu) * (1.0 - 2.0 * nu))
         return gE, a["V"]

@@ -26,7 +26,9 @@
 #include <string>
 #include <vector>
 #include <array>
+#include <atomic>
 #include <mutex>
+#include <thread>
 #include <type_traits>
 
 #include "../../include/zr_mpm.h"
@@ -51,6 +53,7 @@ constexpr int g2p_threads() { return MLS ? 256 : 128; }
 constexpr int kP2GFields = 7;                          // m, mv[3], f[3]
 constexpr int kStageStride = kP2GFields * kTileNodes;  // doubles per group
 constexpr int kMaxColliders = 8;
+constexpr int kIoThreads = 8;  // threads of a host transfer
 constexpr int kSortLds = 2048;  // particles per page sorted in LDS
 constexpr uint32_t kMoveMin = 65536;  // fewer particles are not moved
 constexpr double kDisorder = 1.0;
@@ -1398,25 +1401,6 @@ __global__ __launch_bounds__(256) void k_visco_strain(uint32_t n, const double* 
 // ---------------------------------------------------------------------------
 // layout conversion and introspection
 // ---------------------------------------------------------------------------
-__global__ void k_aos_to_soa(const double* __restrict__ aos, double* __restrict__ soa, uint32_t n, int ncomp, int64_t stride)
-{
-  uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (uint64_t)n * ncomp) return;
-  uint32_t i = (uint32_t)(t / ncomp);
-  int c = (int)(t % ncomp);
-  soa[c * stride + i] = aos[t];
-}
-// uid: the caller's index of each place (null: the same)
-__global__ void k_soa_to_aos(const double* __restrict__ soa, double* __restrict__ aos, uint32_t n, int ncomp,
-                             int64_t stride, const uint32_t* __restrict__ uid)
-{
-  uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (uint64_t)n * ncomp) return;
-  uint32_t i = (uint32_t)(t / ncomp);
-  int c = (int)(t % ncomp);
-  aos[uid ? (uint64_t)uid[i] * ncomp + c : t] = soa[c * stride + i];
-}
-
 // Moves every per-particle array to another order in one launch: thread k
 // copies each row's element from[k] -> k (gather), or k -> to[k] (scatter)
 constexpr int kMoveArrays = 32;
@@ -1550,6 +1534,9 @@ struct zr_engine {
   size_t adj_grid_cap = 0;
   std::vector<double*> ckpt;
   std::vector<double> ckpt_time;
+  // buffers that an upload of as many particles keeps for the next use
+  std::vector<double*> ckpt_spare;
+  double* adj_spare = nullptr;
   // a backward rollout's recomputed steps: the sort tables and grid of each
   // (StepRecord), so that its adjoint step need not sort and rasterise again
   struct StepRecord {
@@ -1636,6 +1623,10 @@ struct zr_engine {
   // second copy of each per-particle array that a move writes to (the two
   // swap); disorder: sum over the steps since the last move of the share of
   // particles not next to their predecessor in the sort's order.
+  // host transfers: device windows, one per thread, and their events
+  double* io_dev = nullptr;
+  int io_threads = 0;
+  hipEvent_t io_ev[kIoThreads] = {};
   bool permuted = false;
   uint32_t* uid = nullptr;
   struct Spare {
@@ -1787,12 +1778,37 @@ int sync_counts(zr_engine* e)
   return ZR_OK;
 }
 
-void free_particles(zr_engine* e)
+// forgets the particles and all that belongs to them; keep: the arrays of an
+// upload that brings as many stay allocated (as do those of the checkpoints
+// and adjoints, whose contents are forgotten all the same)
+void free_particles(zr_engine* e, bool keep = false)
 {
-  dfree(e->x); dfree(e->v); dfree(e->C); dfree(e->F); dfree(e->m); dfree(e->vol); dfree(e->mu); dfree(e->lam);
-  dfree(e->p_page); dfree(e->p_re); dfree(e->order); dfree(e->keys);
-  dfree(e->group_page); dfree(e->group_count); dfree(e->group_start);
-  dfree(e->touch_page); dfree(e->touch_slot); dfree(e->slot_page); dfree(e->group_nslot);
+  if (keep) {
+    for (auto& c : e->ckpt)
+      if (c) e->ckpt_spare.push_back(c);
+    if (e->adj) std::swap(e->adj, e->adj_spare);
+    dfree(e->adj);
+  } else {
+    dfree(e->x); dfree(e->v); dfree(e->C); dfree(e->F); dfree(e->m); dfree(e->vol); dfree(e->mu); dfree(e->lam);
+    dfree(e->p_page); dfree(e->p_re); dfree(e->order); dfree(e->keys);
+    dfree(e->group_page); dfree(e->group_count); dfree(e->group_start);
+    dfree(e->touch_page); dfree(e->touch_slot); dfree(e->slot_page); dfree(e->group_nslot);
+    for (auto& c : e->ckpt) dfree(c);
+    for (auto& c : e->ckpt_spare) dfree(c);
+    e->ckpt_spare.clear();
+    for (auto& r : e->step_rec) dfree(r.buf);
+    e->step_rec.clear();
+    for (auto& a : e->alt) dfree(a.p);
+    e->alt.clear();
+    dfree(e->uid);
+    dfree(e->adj);
+    dfree(e->adj_spare);
+  }
+  e->ckpt.clear();
+  e->ckpt_time.clear();
+  e->permuted = false;
+  e->disorder = 0.0;
+  e->adj_n = 0;
   dfree(e->mat); dfree(e->pparam); dfree(e->pstate); dfree(e->gdeg); dfree(e->broken);
   e->has_models = e->has_plastic = false;
   e->uniform_model = ZR_MODEL_FIXED_COROTATED;
@@ -1801,21 +1817,9 @@ void free_particles(zr_engine* e)
   dfree(e->pf_c); dfree(e->pf_H); dfree(e->pf_l0); dfree(e->pf_osc); dfree(e->pf_Fp); dfree(e->pf_Hmax);
   dfree(e->pf_k); dfree(e->pf_vol); dfree(e->pf_allow);
   e->pf_on = false;
-  for (auto& a : e->alt) dfree(a.p);
-  e->alt.clear();
-  dfree(e->uid);
-  e->permuted = false;
-  e->disorder = 0.0;
-  dfree(e->adj);
-  e->adj_n = 0;
   dfree(e->admm_p);
   e->admm_n = 0;
   e->admm_steps = 0;
-  for (auto& c : e->ckpt) dfree(c);
-  e->ckpt.clear();
-  e->ckpt_time.clear();
-  for (auto& r : e->step_rec) dfree(r.buf);
-  e->step_rec.clear();
   e->n = 0;
 }
 
@@ -2328,6 +2332,8 @@ int ensure_scalars(zr_engine* e)
   return ZR_OK;
 }
 
+#include "zr_transfer.hpp"
+
 // ----------------------------------------------------------- phase field
 PfParticles pf_view(zr_engine* e)
 {
@@ -2416,8 +2422,11 @@ int ensure_adjoint(zr_engine* e)
 {
   if (e->adj_n != e->n) {
     dfree(e->adj);
-    ZR_HIP(e, hipMalloc(&e->adj, kAdjRows * (size_t)e->n * sizeof(double)));
-    ZR_HIP(e, hipMemset(e->adj, 0, kAdjRows * (size_t)e->n * sizeof(double)));
+    if (e->adj_spare)
+      std::swap(e->adj, e->adj_spare);  // as large: kept by the upload
+    else
+      ZR_HIP(e, hipMalloc(&e->adj, kAdjRows * (size_t)e->n * sizeof(double)));
+    ZR_HIP(e, hipMemsetAsync(e->adj, 0, kAdjRows * (size_t)e->n * sizeof(double), e->stream));
     e->adj_n = e->n;
   }
   return ZR_OK;
@@ -3357,6 +3366,7 @@ int zr_create(const zr_config* cfg, zr_engine** out)
       (cfg->precision != ZR_FP64 && cfg->precision != ZR_FP32_REFINED) || cfg->transfer != ZR_TRANSFER_MLS)
     return ZR_ERR_ARG;
   zr_engine* e = new zr_engine();
+  pinned_acquire();
   e->cfg = *cfg;
   e->L = (uint32_t)cfg->grid_log2;
   e->lim = (1u << e->L) - 8u;
@@ -3365,6 +3375,7 @@ int zr_create(const zr_config* cfg, zr_engine** out)
   e->nsum = (e->nwords + 31u) / 32u;
   hipError_t st = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
   if (st != hipSuccess) {
+    pinned_release();
     delete e;
     return ZR_ERR_HIP;
   }
@@ -3380,6 +3391,7 @@ int zr_create(const zr_config* cfg, zr_engine** out)
         ncu <= 0 ||
         b32 <= 0 || b64 <= 0) {
       (void)hipStreamDestroy(e->stream);
+      pinned_release();
       delete e;
       return ZR_ERR_HIP;
     }
@@ -3396,7 +3408,7 @@ int zr_create(const zr_config* cfg, zr_engine** out)
             hipMalloc(&e->sum_base, (e->nsum + 1) * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&e->dbase, 3 * kBank * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&e->ticket, sizeof(uint32_t)) == hipSuccess &&
-            hipHostMalloc(&e->hcount, CNT_N * sizeof(uint32_t)) == hipSuccess;
+            hipHostMalloc(&e->hcount, CNT_N * sizeof(uint32_t), hipHostMallocCoherent) == hipSuccess;
   ok = ok && hipMemset(e->dbase, 0, 3 * kBank * sizeof(uint32_t)) == hipSuccess;
   if (ok) {
     e->dcount = e->dbase;
@@ -3438,7 +3450,11 @@ void zr_destroy(zr_engine* e)
   for (auto& v : e->prof_ev)
     for (auto h : v) (void)hipEventDestroy(h);
   if (e->hcount) (void)hipHostFree(e->hcount);
+  dfree(e->io_dev);
+  for (auto& h : e->io_ev)
+    if (h) (void)hipEventDestroy(h);
   if (e->stream) (void)hipStreamDestroy(e->stream);
+  pinned_release();
   delete e;
 }
 
@@ -3599,53 +3615,37 @@ int zr_upload_particles(zr_engine* e, const zr_particles* p)
     ZR_HIP(e, hipStreamSynchronize(e->stream));
   }
   e->A = e->S = 0;
-  free_particles(e);
-  e->sorted = e->rasterised = e->updated = false;
   const int64_t n = p->n;
+  const bool keep = n > 0 && n == e->n && e->x;
+  free_particles(e, keep);
+  e->sorted = e->rasterised = e->updated = false;
   e->n = n;
   if (n == 0) return ZR_OK;
   size_t N = (size_t)n;
-  ZR_HIP(e, hipMalloc(&e->x, 3 * N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->v, 3 * N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->C, 9 * N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->F, 9 * N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->m, N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->vol, N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->mu, N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->lam, N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->p_page, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->p_re, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->order, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->keys, N * sizeof(uint64_t)));
-  ZR_HIP(e, hipMalloc(&e->group_page, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->group_count, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->group_start, (N + 1) * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->touch_page, 8 * N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->touch_slot, 8 * N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->slot_page, 8 * N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->group_nslot, 8 * N * sizeof(int32_t)));
-  double* tmp = nullptr;
-  ZR_HIP(e, hipMalloc(&tmp, 9 * N * sizeof(double)));
-  struct Item {
-    const double* src;
-    double* dst;
-    int nc;
-  } items[] = { { p->X, e->x, 3 }, { p->V, e->v, 3 }, { p->C, e->C, 9 }, { p->F, e->F, 9 },
-                { p->mass, e->m, 1 }, { p->vol, e->vol, 1 }, { p->mu, e->mu, 1 }, { p->lambda, e->lam, 1 } };
-  for (auto& it : items) {
-    hipError_t st = hipMemcpyAsync(tmp, it.src, it.nc * N * sizeof(double), hipMemcpyHostToDevice, e->stream);
-    if (st == hipSuccess) {
-      k_aos_to_soa<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(tmp, it.dst, (uint32_t)N, it.nc, n);
-      st = hipGetLastError();
-    }
-    if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
-    if (st != hipSuccess) {
-      (void)hipFree(tmp);
-      return fail(e, ZR_ERR_HIP, std::string("upload: ") + hipGetErrorString(st));
-    }
+  if (!keep) {
+    ZR_HIP(e, hipMalloc(&e->x, 3 * N * sizeof(double)));
+    ZR_HIP(e, hipMalloc(&e->v, 3 * N * sizeof(double)));
+    ZR_HIP(e, hipMalloc(&e->C, 9 * N * sizeof(double)));
+    ZR_HIP(e, hipMalloc(&e->F, 9 * N * sizeof(double)));
+    ZR_HIP(e, hipMalloc(&e->m, N * sizeof(double)));
+    ZR_HIP(e, hipMalloc(&e->vol, N * sizeof(double)));
+    ZR_HIP(e, hipMalloc(&e->mu, N * sizeof(double)));
+    ZR_HIP(e, hipMalloc(&e->lam, N * sizeof(double)));
+    ZR_HIP(e, hipMalloc(&e->p_page, N * sizeof(uint32_t)));
+    ZR_HIP(e, hipMalloc(&e->p_re, N * sizeof(uint32_t)));
+    ZR_HIP(e, hipMalloc(&e->order, N * sizeof(uint32_t)));
+    ZR_HIP(e, hipMalloc(&e->keys, N * sizeof(uint64_t)));
+    ZR_HIP(e, hipMalloc(&e->group_page, N * sizeof(uint32_t)));
+    ZR_HIP(e, hipMalloc(&e->group_count, N * sizeof(uint32_t)));
+    ZR_HIP(e, hipMalloc(&e->group_start, (N + 1) * sizeof(uint32_t)));
+    ZR_HIP(e, hipMalloc(&e->touch_page, 8 * N * sizeof(uint32_t)));
+    ZR_HIP(e, hipMalloc(&e->touch_slot, 8 * N * sizeof(uint32_t)));
+    ZR_HIP(e, hipMalloc(&e->slot_page, 8 * N * sizeof(uint32_t)));
+    ZR_HIP(e, hipMalloc(&e->group_nslot, 8 * N * sizeof(int32_t)));
   }
-  ZR_HIP(e, hipFree(tmp));
-  return ZR_OK;
+  const HostArray items[] = { { p->X, e->x, 3 },    { p->V, e->v, 3 },     { p->C, e->C, 9 },   { p->F, e->F, 9 },
+                              { p->mass, e->m, 1 }, { p->vol, e->vol, 1 }, { p->mu, e->mu, 1 }, { p->lambda, e->lam, 1 } };
+  return transfer_arrays(e, items, 8, false, false);
 }
 
 int zr_download_particles(zr_engine* e, zr_particles* p)
@@ -3653,29 +3653,9 @@ int zr_download_particles(zr_engine* e, zr_particles* p)
   if (!e || !p) return fail(e, ZR_ERR_ARG, "bad particle view");
   if (p->n != e->n) return fail(e, ZR_ERR_ARG, "particle count mismatch");
   if (e->n == 0) return ZR_OK;
-  size_t N = (size_t)e->n;
-  double* tmp = nullptr;
-  ZR_HIP(e, hipMalloc(&tmp, 9 * N * sizeof(double)));
-  struct Item {
-    double* dst;
-    const double* src;
-    int nc;
-  } items[] = { { p->X, e->x, 3 }, { p->V, e->v, 3 }, { p->C, e->C, 9 }, { p->F, e->F, 9 },
-                { p->mass, e->m, 1 }, { p->vol, e->vol, 1 }, { p->mu, e->mu, 1 }, { p->lambda, e->lam, 1 } };
-  for (auto& it : items) {
-    if (!it.dst) continue;
-    k_soa_to_aos<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(it.src, tmp, (uint32_t)N, it.nc, e->n,
-                                                                              e->permuted ? e->uid : nullptr);
-    hipError_t st = hipGetLastError();
-    if (st == hipSuccess) st = hipMemcpyAsync(it.dst, tmp, it.nc * N * sizeof(double), hipMemcpyDeviceToHost, e->stream);
-    if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
-    if (st != hipSuccess) {
-      (void)hipFree(tmp);
-      return fail(e, ZR_ERR_HIP, std::string("download: ") + hipGetErrorString(st));
-    }
-  }
-  ZR_HIP(e, hipFree(tmp));
-  return ZR_OK;
+  const HostArray items[] = { { p->X, e->x, 3 },    { p->V, e->v, 3 },     { p->C, e->C, 9 },   { p->F, e->F, 9 },
+                              { p->mass, e->m, 1 }, { p->vol, e->vol, 1 }, { p->mu, e->mu, 1 }, { p->lambda, e->lam, 1 } };
+  return transfer_arrays(e, items, 8, true, true);
 }
 
 int zr_set_materials(zr_engine* e, const zr_materials* mt)
@@ -3890,33 +3870,13 @@ int zr_adjoint_set(zr_engine* e, const zr_particles_adjoint* a)
   if (rc) return rc;
   const size_t N = (size_t)e->n;
   AdjointView A = adj_view(e);
-  double* tmp = nullptr;
-  ZR_HIP(e, hipMalloc(&tmp, 9 * N * sizeof(double)));
-  struct Item {
-    const double* src;
-    double* dst;
-    int nc;
-  } items[] = { { a->X, A.x, 3 }, { a->V, A.v, 3 }, { a->C, A.C, 9 }, { a->F, A.F, 9 }, { a->mu, A.mu, 1 },
-                { a->lambda, A.lam, 1 } };
-  for (auto& it : items) {
-    hipError_t st;
-    if (it.src) {
-      st = hipMemcpyAsync(tmp, it.src, it.nc * N * sizeof(double), hipMemcpyHostToDevice, e->stream);
-      if (st == hipSuccess) {
-        k_aos_to_soa<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(tmp, it.dst, (uint32_t)N, it.nc,
-                                                                                  e->n);
-        st = hipGetLastError();
-      }
-    } else {
-      st = hipMemsetAsync(it.dst, 0, it.nc * N * sizeof(double), e->stream);
-    }
-    if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
-    if (st != hipSuccess) {
-      (void)hipFree(tmp);
-      return fail(e, ZR_ERR_HIP, std::string("adjoint upload: ") + hipGetErrorString(st));
-    }
-  }
-  ZR_HIP(e, hipFree(tmp));
+  const HostArray items[] = { { a->X, A.x, 3 }, { a->V, A.v, 3 },   { a->C, A.C, 9 },
+                              { a->F, A.F, 9 }, { a->mu, A.mu, 1 }, { a->lambda, A.lam, 1 } };
+  for (auto& it : items)
+    if (!it.host) ZR_HIP(e, hipMemsetAsync(it.dev, 0, it.nc * N * sizeof(double), e->stream));
+  rc = transfer_arrays(e, items, 6, false, false);
+  if (rc) return rc;
+  ZR_HIP(e, hipStreamSynchronize(e->stream));
   return ZR_OK;
 }
 
@@ -3926,29 +3886,10 @@ int zr_adjoint_get(zr_engine* e, zr_particles_adjoint* a)
   if (a->n != e->n) return fail(e, ZR_ERR_ARG, "adjoint count differs from the particle count");
   if (e->n == 0) return ZR_OK;
   if (!e->adj) return fail(e, ZR_ERR_STATE, "no adjoint was set");
-  const size_t N = (size_t)e->n;
   AdjointView A = adj_view(e);
-  double* tmp = nullptr;
-  ZR_HIP(e, hipMalloc(&tmp, 9 * N * sizeof(double)));
-  struct Item {
-    double* dst;
-    const double* src;
-    int nc;
-  } items[] = { { a->X, A.x, 3 }, { a->V, A.v, 3 }, { a->C, A.C, 9 }, { a->F, A.F, 9 }, { a->mu, A.mu, 1 },
-                { a->lambda, A.lam, 1 } };
-  for (auto& it : items) {
-    if (!it.dst) continue;
-    k_soa_to_aos<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(it.src, tmp, (uint32_t)N, it.nc, e->n, nullptr);
-    hipError_t st = hipGetLastError();
-    if (st == hipSuccess) st = hipMemcpyAsync(it.dst, tmp, it.nc * N * sizeof(double), hipMemcpyDeviceToHost, e->stream);
-    if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
-    if (st != hipSuccess) {
-      (void)hipFree(tmp);
-      return fail(e, ZR_ERR_HIP, std::string("adjoint download: ") + hipGetErrorString(st));
-    }
-  }
-  ZR_HIP(e, hipFree(tmp));
-  return ZR_OK;
+  const HostArray items[] = { { a->X, A.x, 3 }, { a->V, A.v, 3 },   { a->C, A.C, 9 },
+                              { a->F, A.F, 9 }, { a->mu, A.mu, 1 }, { a->lambda, A.lam, 1 } };
+  return transfer_arrays(e, items, 6, true, false);
 }
 
 int zr_adjoint_step(zr_engine* e, double dt)
@@ -3965,7 +3906,7 @@ int zr_adjoint_step(zr_engine* e, double dt)
 namespace {
 // the checkpoint arrays X, V, C, F and a 24n-double checkpoint, copied in
 // one pass (to: state -> checkpoint, else back), the checkpoint in the
-// caller's order (uid as in k_soa_to_aos)
+// caller's order (uid: the caller's index of each place; null: the same)
 __global__ __launch_bounds__(256) void k_ckpt_copy(double* x, double* v, double* C, double* F, double* c, uint32_t n,
                                                    int to, const uint32_t* __restrict__ uid)
 {
@@ -3996,6 +3937,10 @@ int ckpt_save(zr_engine* e, int32_t slot)
   if ((size_t)slot >= e->ckpt.size()) {
     e->ckpt.resize((size_t)slot + 1, nullptr);
     e->ckpt_time.resize((size_t)slot + 1, 0.0);
+  }
+  if (!e->ckpt[slot] && N && !e->ckpt_spare.empty()) {
+    e->ckpt[slot] = e->ckpt_spare.back();
+    e->ckpt_spare.pop_back();
   }
   if (!e->ckpt[slot]) ZR_HIP(e, hipMalloc(&e->ckpt[slot], 24 * (N ? N : 1) * sizeof(double)));
   if (N) {
@@ -4165,29 +4110,9 @@ int zr_get_admm_state(zr_engine* e, double* F, double* y, double* omega)
 {
   if (!e) return ZR_ERR_ARG;
   if (!e->admm_p || e->admm_n != e->n) return fail(e, ZR_ERR_STATE, "no ADMM step has run");
-  if (int rc_order = user_order(e)) return rc_order;
   const size_t N = (size_t)e->n;
-  double* tmp = nullptr;
-  ZR_HIP(e, hipMalloc(&tmp, 9 * N * sizeof(double)));
-  struct Item {
-    double* dst;
-    const double* src;
-    int nc;
-  } items[] = { { F, e->admm_p, 9 }, { y, e->admm_p + 9 * N, 9 }, { omega, e->admm_p + 18 * N, 1 } };
-  for (auto& it : items) {
-    if (!it.dst) continue;
-    k_soa_to_aos<<<blocks_for((uint64_t)N * it.nc, 256), 256, 0, e->stream>>>(it.src, tmp, (uint32_t)N, it.nc, e->n, nullptr);
-    hipError_t stt = hipGetLastError();
-    if (stt == hipSuccess)
-      stt = hipMemcpyAsync(it.dst, tmp, it.nc * N * sizeof(double), hipMemcpyDeviceToHost, e->stream);
-    if (stt == hipSuccess) stt = hipStreamSynchronize(e->stream);
-    if (stt != hipSuccess) {
-      (void)hipFree(tmp);
-      return fail(e, ZR_ERR_HIP, std::string("admm download: ") + hipGetErrorString(stt));
-    }
-  }
-  ZR_HIP(e, hipFree(tmp));
-  return ZR_OK;
+  const HostArray items[] = { { F, e->admm_p, 9 }, { y, e->admm_p + 9 * N, 9 }, { omega, e->admm_p + 18 * N, 1 } };
+  return transfer_arrays(e, items, 3, true, true);
 }
 
 int zr_sort_particles_and_pollute_grid(zr_engine* e, zr_step_stats* st)

@@ -502,11 +502,11 @@ class MpmEngine:
         a = ZrParticlesAdjoint(n, *[_dptr(x) for x in arrs])
         self._check(self.L.zr_adjoint_set(self.h, ctypes.byref(a)), "adjoint_set")
 
-    def adjoint_get(self):
+    def adjoint_get(self, keys=("X", "V", "C", "F", "mu", "lam")):
         n = self.n
-        out = dict(X=np.zeros((n, 3)), V=np.zeros((n, 3)), C=np.zeros((n, 9)), F=np.zeros((n, 9)), mu=np.zeros(n),
-                   lam=np.zeros(n))
-        a = ZrParticlesAdjoint(n, *[_dptr(out[k]) for k in ("X", "V", "C", "F", "mu", "lam")])
+        nc = dict(X=3, V=3, C=9, F=9, mu=1, lam=1)
+        out = {k: np.empty((n, nc[k]) if nc[k] > 1 else n) for k in keys}
+        a = ZrParticlesAdjoint(n, *[_dptr(out.get(k)) for k in nc])
         self._check(self.L.zr_adjoint_get(self.h, ctypes.byref(a)), "adjoint_get")
         return out
 
@@ -543,12 +543,13 @@ class MpmEngine:
         self._check(self.L.zr_get_materials(self.h, ctypes.byref(mt)), "get_materials")
         return dict(plastic_state=st, degradation=g, broken=b)
 
-    def download(self):
+    def download(self, keys=("X", "V", "C", "F")):
         n = self.n
-        X = np.zeros(3 * n); V = np.zeros(3 * n); C = np.zeros(9 * n); F = np.zeros(9 * n)
-        p = ZrParticles(n, _dptr(X), _dptr(V), _dptr(C), _dptr(F), None, None, None, None)
+        nc = dict(X=3, V=3, C=9, F=9)
+        out = {k: np.empty((n, nc[k])) for k in keys}
+        p = ZrParticles(n, *[_dptr(out.get(k)) for k in nc], None, None, None, None)
         self._check(self.L.zr_download_particles(self.h, ctypes.byref(p)), "zr_download_particles")
-        return dict(X=X.reshape(n, 3), V=V.reshape(n, 3), C=C.reshape(n, 9), F=F.reshape(n, 9))
+        return out
 
     # ------------------------------------------------------- restart state
     def write_state(self, f):
@@ -580,7 +581,7 @@ class MpmEngine:
         MpmSimulationBase::writeState calls when write_partio is set: every
         particle's position in a .bgeo file (ziran2019_amd/partio.py)."""
         from . import partio
-        partio.write_bgeo(f, self.download()["X"])
+        partio.write_bgeo(f, self.download(("X",))["X"])
 
     def write_phase_field_partio(self, f):
         """The fracture project's frame output (Projects/fracture/
@@ -588,7 +589,7 @@ class MpmEngine:
         1 / one_over_sigma_c (the reciprocal of the float-rounded value),
         1 for particles without a phase field."""
         from . import partio
-        X = self.download()["X"]
+        X = self.download(("X",))["X"]
         pf, sc = np.ones(len(X)), np.ones(len(X))
         if getattr(self, "_pf", None) is not None:
             pf = self.get_phase_field()["c"]
