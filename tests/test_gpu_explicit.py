@@ -294,3 +294,41 @@ def test_empty_upload_is_a_state_error():
     with pytest.raises(ZrError):
         eng.advanceOneTimeStep(1e-4)
     eng.close()
+
+
+def test_step_beyond_the_last_steps_counts():
+    """A step is launched for as many groups and slots as the last one had,
+    with headroom; particles that spread to many more pages within one step of
+    the sort (their positions uploaded anew between the steps keep the engine's
+    buffers) and particles that leave the domain leave the launch without
+    effect, and the step is repeated or refused."""
+    rng = np.random.default_rng(12)
+    n = 3000
+    s = scenes.cube_scene_small(seed=3, ncells=8)
+    s = {k: (np.ascontiguousarray(np.asarray(v)[:n]) if k in ("X", "V", "C", "F", "mass", "vol", "mu", "lam") else v)
+         for k, v in s.items()}
+    spread = dict(s, X=0.2 + 0.6 * rng.random((n, 3)))
+    for first, second in ((s, spread), (spread, s)):
+        eng, _ = make_pair(first)
+        eng.advanceOneTimeStep(1e-4)
+        eng.advanceOneTimeStep(1e-4)
+        eng.upload(second)  # the launch hints stay those of the first set
+        ora = make_pair(second)[1]
+        for _ in range(3):
+            eng.advanceOneTimeStep(1e-4)
+            ora.step(1e-4)
+        out = eng.download()
+        X, V, C, F = ora.get_particles()
+        for k, r in (("X", X), ("V", V), ("C", C), ("F", F)):
+            assert rel_err(out[k], r) < 1e-10, k
+        gone = dict(second, X=second["X"].copy())
+        gone["X"][n // 2] = (-0.5, 0.5, 0.5)
+        eng.upload(gone)
+        t = eng.time
+        with pytest.raises(ZrError, match="outside"):
+            eng.advanceOneTimeStep(1e-4)
+        assert eng.time == t
+        assert np.array_equal(eng.download()["X"], gone["X"])
+        eng.upload(second)
+        eng.advanceOneTimeStep(1e-4)
+        eng.close()
