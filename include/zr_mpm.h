@@ -255,8 +255,8 @@ typedef struct zr_implicit_opts {
   double cg_tolerance;           /* absolute cap of the CG local tolerance */
   double cg_relative_tolerance;  /* <= 0: Newton-adaptive (reference behaviour) */
   int32_t precision;             /* ZR_FP64 or ZR_FP32_REFINED */
-  int32_t cg_check_interval;     /* CG iterations between host polls of the
-                                    device-side termination flag (0: 8) */
+  int32_t cg_check_interval;     /* most iterations issued past the last one
+                                    known to have run (0 or above 2: 2) */
   int32_t preconditioner;        /* ZR_PRECOND_MASS or ZR_PRECOND_JACOBI */
   int32_t solver;                /* ZR_SOLVER_CG or ZR_SOLVER_MINRES */
 } zr_implicit_opts;

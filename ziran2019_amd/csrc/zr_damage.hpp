@@ -305,10 +305,14 @@ enum { PFR_INIT = 0, PFR_ALPHA = 1, PFR_CHECK = 2 };
 
 // one-block ordered sums of the partials and the CG scalar logic
 __global__ __launch_bounds__(256) void k_pf_reduce(const double* __restrict__ partial, uint32_t nb, double* sc,
-                                                   int32_t* ci, int mode, double cg_relative, PfScalars ps)
+                                                   int32_t* ci, int mode, double cg_relative, PfScalars ps,
+                                                   SolveMark mark)
 {
   __shared__ double smem[4];
-  if (mode != PFR_INIT && ci[CI_DONE]) return;
+  if (mode != PFR_INIT && ci[CI_DONE]) {
+    if (threadIdx.x == 0) mark_solve(mark, ci[CI_ITERS], 1);
+    return;
+  }
   const double a0 = thread_partials256(partial, nb);
   const double a1 = mode != PFR_ALPHA ? thread_partials256(partial + nb, nb) : 0.0;
   const double s0 = block_sum256(a0, smem);
@@ -331,10 +335,12 @@ __global__ __launch_bounds__(256) void k_pf_reduce(const double* __restrict__ pa
     if (norm < ps.tol || norm < sc[PF_REL] || it == ps.max_it) {
       ci[CI_DONE] = 1;
       ci[CI_ITERS] = it;
+      mark_solve(mark, it, 1);
     } else {
       sc[PF_BETA] = s1 / sc[PF_RHO];
       sc[PF_RHO] = s1;
       ci[CI_PF_IT] = it + 1;
+      mark_solve(mark, it, 0);
     }
   }
 }

@@ -1560,7 +1560,7 @@ __global__ __launch_bounds__(256) void k_cg_ap(uint32_t nn, const uint32_t* __re
                                                NodeVec<T> ap, double dx, double dt, ColliderSet cs,
                                                int project, double* __restrict__ partial, const double* sc,
                                                const int32_t* ci, uint32_t* __restrict__ hvp_ctr,
-                                               const uint32_t* __restrict__ act, uint32_t nact)
+                                               const uint32_t* __restrict__ act, uint32_t nact, SolveMark mark)
 {
   // the operator apply this kernel follows has drained its work counters
   if (blockIdx.x == 0 && threadIdx.x < kHvpCounters) hvp_ctr[kHvpCounterStride * threadIdx.x] = 0u;
@@ -1589,7 +1589,9 @@ __global__ __launch_bounds__(256) void k_cg_ap(uint32_t nn, const uint32_t* __re
     }
   };
   if (t0 < count) fetch(act ? act[t0] : t0);
-  if (ci && ci[CI_DONE]) return;
+  const int32_t ended = ci ? ci[CI_DONE] : 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) mark_solve(mark, 0, ended);
+  if (ended) return;
   double contrib = 0.0;
   const T beta = q.p ? (T)sc[SC_BETA] : (T)0;
   for (uint32_t t = t0; t < count; t += tstep) {

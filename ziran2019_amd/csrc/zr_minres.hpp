@@ -34,10 +34,17 @@ enum { MR_INIT = 0, MR_ALPHA = 1, MR_GIVENS = 2 };
 // the MINRES scalar logic (Minres.h:75-178) in one thread after an ordered sum
 __global__ __launch_bounds__(256) void k_minres_reduce(const double* __restrict__ partial, uint32_t nb, double* sc,
                                                        int32_t* ai, int mode, double tol, double rel, int it,
-                                                       int max_it)
+                                                       int max_it, SolveMark mark)
 {
   __shared__ double smem[4];
-  if (mode != MR_INIT && ai[AI_DONE]) return;
+  const int32_t ended = mode != MR_INIT ? ai[AI_DONE] : 0;
+  // the update of this iteration still runs when the convergence flag is
+  // raised by its Givens step
+  if (mode == MR_ALPHA && threadIdx.x == 0) ai[AI_DONE + 2] = ended;
+  if (ended) {
+    if (threadIdx.x == 0) mark_solve(mark, ai[AI_ITERS], 1);
+    return;
+  }
   const double acc = thread_partials256(partial, nb);
   const double v = block_sum256(acc, smem);
   if (threadIdx.x != 0) return;
@@ -58,6 +65,7 @@ __global__ __launch_bounds__(256) void k_minres_reduce(const double* __restrict_
     ai[AI_DONE + 2] = ai[AI_DONE];
   } else if (mode == MR_ALPHA) {
     sc[AD_ALPHA] = v;
+    sc[AD_BETA_K] = sc[AD_BETA_KP1];  // (an iteration's first step over the scalars)
   } else {
     const double bb = v > 0.0 ? v : 0.0;
     const double beta_kp1 = sqrt(bb);
@@ -93,18 +101,10 @@ __global__ __launch_bounds__(256) void k_minres_reduce(const double* __restrict_
     const double res = lt[1] < 0.0 ? -lt[1] : lt[1];
     sc[AD_RES] = res;
     ai[AI_ITERS] = it + 1;
-    if (res < sc[AD_LTOL] || it + 1 >= max_it) ai[AI_DONE] = 1;
+    const bool done = res < sc[AD_LTOL] || it + 1 >= max_it;
+    if (done) ai[AI_DONE] = 1;
+    mark_solve(mark, it + 1, done);
   }
-}
-
-// the start of each MINRES iteration: beta_k = beta_{k+1}; the update of this
-// iteration still runs when the convergence flag is raised by its Givens step
-__global__ void k_minres_begin(double* sc, int32_t* ai)
-{
-  if (threadIdx.x != 0) return;
-  ai[AI_DONE + 2] = ai[AI_DONE];
-  if (ai[AI_DONE]) return;
-  sc[AD_BETA_K] = sc[AD_BETA_KP1];
 }
 
 // ---- the implicit Newton step's MINRES (BackwardEuler::computeStep with the
