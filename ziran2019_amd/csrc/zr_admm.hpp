@@ -447,33 +447,6 @@ __device__ __forceinline__ void admm_tile3(const int32_t* gslot, const double* g
   __syncthreads();
 }
 
-// G = sum_i v_i grad w_i^T over the tile
-__device__ __forceinline__ void admm_grad_tile(const double* tv, const double w[3][3], const double dw[3][3],
-                                               double inv_dx, int lx, int ly, int lz, double G[3][3])
-{
-#pragma unroll
-  for (int r = 0; r < 3; ++r)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) G[r][c] = 0.0;
-#pragma unroll
-  for (int a = 0; a < 3; ++a)
-#pragma unroll
-    for (int b = 0; b < 3; ++b)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        double gw[3];
-        wgrad(w, dw, inv_dx, a, b, c, gw);
-        const int t = ((lx + a) * kTileY + (ly + b)) * kTileZ + (lz + c);
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-          const double v = tv[r * kTileNodes + t];
-          G[r][0] += v * gw[0];
-          G[r][1] += v * gw[1];
-          G[r][2] += v * gw[2];
-        }
-      }
-}
-
 __device__ __forceinline__ void load_F(const double* F, int64_t S, uint32_t i, double M[3][3])
 {
 #pragma unroll
@@ -482,12 +455,46 @@ __device__ __forceinline__ void load_F(const double* F, int64_t S, uint32_t i, d
     for (int r = 0; r < 3; ++r) M[r][c] = F[(c * 3 + r) * S + i];
 }
 
+// D += k (G F) F^T
+template <class T>
+__device__ __forceinline__ void add_operator_term(T k, const T G[3][3], const T F[3][3], T D[3][3])
+{
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    T y[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) y[c] = k * (G[r][0] * F[0][c] + G[r][1] * F[1][c] + G[r][2] * F[2][c]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) D[r][c] += y[0] * F[c][0] + y[1] * F[c][1] + y[2] * F[c][2];
+  }
+}
+
+// D += k U diag(z - sigma) V^T F^T
+__device__ __forceinline__ void admm_residual_term(double k, const M3<double>& u, const double z[3],
+                                                   const double sg[3], const M3<double>& v, const double F[3][3],
+                                                   double D[3][3])
+{
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const double t = k * (z[d] - sg[d]);
+    double q[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) q[c] = F[c][0] * v.a[0][d] + F[c][1] * v.a[1][d] + F[c][2] * v.a[2][d];
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) D[r][c] = fma(u.a[r][d] * t, q[c], D[r][c]);
+  }
+}
+
 // FStepSolve's viscoelastic branch (:566-611): F2 = U diag(z) V^T with z the
 // Newton solution (at most 20 iterations) of
 // vol dE(zp(z)) + rho omega2^2 (z - sigma) = 0, sigma the singular values of
-// FFn - y2 / (rho omega2) + dt G FFn, G = grad(vn + dv)
+// FFn - y2 / (rho omega2) + dt G FFn, G = grad(vn + dv); its term of the
+// global step's right side is added to D
 __device__ __forceinline__ void admm_visco_fstep(const AdmmParticles& A, int64_t S, uint32_t i, double vol,
-                                                 const double G[3][3], double dt, double rho, double local_tol)
+                                                 const double G[3][3], double dt, double rho, double local_tol,
+                                                 double D[3][3])
 {
   double Fv[3][3];
   load_F(A.fneq, S, i, Fv);
@@ -517,8 +524,8 @@ __device__ __forceinline__ void admm_visco_fstep(const AdmmParticles& A, int64_t
   }
   const double mu = A.mu2[i], lam = A.lam2[i], coeff = rho * om * om;
   for (int it = 0; it < 20; ++it) {
-    double zp[3], D[3][3], dE[3], ddE[3][3], gg[3], H[3][3], Hi[3][3];
-    admm_visco_map(mu, lam, A.visc_d, A.visc_v, dt, z, zp, D);
+    double zp[3], Dz[3][3], dE[3], ddE[3][3], gg[3], H[3][3], Hi[3][3];
+    admm_visco_map(mu, lam, A.visc_d, A.visc_v, dt, z, zp, Dz);
     hencky_dE(mu, lam, zp, dE);
     hencky_ddE(mu, lam, zp, ddE);
 #pragma unroll
@@ -526,7 +533,7 @@ __device__ __forceinline__ void admm_visco_fstep(const AdmmParticles& A, int64_t
       gg[a] = vol * dE[a] + coeff * (z[a] - sg[a]);
 #pragma unroll
       for (int bb = 0; bb < 3; ++bb)
-        H[a][bb] = vol * (ddE[a][0] * D[0][bb] + ddE[a][1] * D[1][bb] + ddE[a][2] * D[2][bb]) + (a == bb ? coeff : 0.0);
+        H[a][bb] = vol * (ddE[a][0] * Dz[0][bb] + ddE[a][1] * Dz[1][bb] + ddE[a][2] * Dz[2][bb]) + (a == bb ? coeff : 0.0);
     }
     inv3(H, Hi);
     double sn = 0.0;
@@ -543,6 +550,10 @@ __device__ __forceinline__ void admm_visco_fstep(const AdmmParticles& A, int64_t
 #pragma unroll
     for (int c = 0; c < 3; ++c)
       A.F2[(c * 3 + r) * S + i] = u.a[r][0] * z[0] * v.a[c][0] + u.a[r][1] * z[1] * v.a[c][1] + u.a[r][2] * z[2] * v.a[c][2];
+  uint32_t ir = i;  // FFn from memory again, as in admm_local_step
+  asm volatile("" : "+v"(ir));
+  load_F(A.fneq, S, ir, Fv);
+  admm_residual_term(dt * coeff, u, z, sg, v, Fv, D);
 }
 
 
@@ -588,7 +599,7 @@ __global__ __launch_bounds__(256) void k_admm_init_particles(ParticlesView P, Ad
     const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
     if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
     double G[3][3], Fn[3][3];
-    admm_grad_tile(tv, w, dw, inv_dx, lx, ly, lz, G);
+    grad_from_tile(tv, (lx * kTileY + ly) * kTileZ + lz, w, dw, inv_dx, G);
     load_F(P.F, S, i, Fn);
     M3<double> f, u, v;
 #pragma unroll
@@ -672,12 +683,13 @@ __global__ __launch_bounds__(256) void k_admm_diag(uint32_t nn, const int32_t* _
 }
 
 // the local step of particle i (FStepSolve, AdmmSimulationFoam.h:507-615)
-// given G = grad(vn + dv) at the particle
+// given G = grad(vn + dv) at the particle; leaves in G the particle's term of
+// the global step's residual (see k_admm_flocal)
 template <bool VISCO>
 __device__ __forceinline__ void admm_local_step(const ParticlesView& P, const AdmmParticles& A,
                                                 const int32_t* __restrict__ mat, const double* __restrict__ pparam,
-                                                const double* __restrict__ pstate, uint32_t i, const double G[3][3],
-                                                double dt, double rho, double local_tol)
+                                                const double* __restrict__ pstate, uint32_t i, double G[3][3], double dt,
+                                                double rho, double local_tol)
 {
   const int64_t S = P.stride;
   double Fn[3][3];
@@ -748,7 +760,17 @@ __device__ __forceinline__ void admm_local_step(const ParticlesView& P, const Ad
 #pragma unroll
     for (int c = 0; c < 3; ++c)
       A.F[(c * 3 + r) * S + i] = u.a[r][0] * z[0] * v.a[c][0] + u.a[r][1] * z[1] * v.a[c][1] + u.a[r][2] * z[2] * v.a[c][2];
-  if constexpr (VISCO) admm_visco_fstep(A, S, i, vol, G, dt, rho, local_tol);
+  double T[3][3] = { { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 } };
+  // Fn again from memory rather than held across the iterations
+  uint32_t ir = i;
+  asm volatile("" : "+v"(ir));
+  load_F(P.F, S, ir, Fn);
+  admm_residual_term(dt * coeff, u, z, sg, v, Fn, T);
+  if constexpr (VISCO) admm_visco_fstep(A, S, i, vol, G, dt, rho, local_tol, T);
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) G[r][c] = T[r][c];
 }
 
 // FStepSolve (:507-615): F = U diag(z) V^T with z the Newton solution of
@@ -757,8 +779,19 @@ __device__ __forceinline__ void admm_local_step(const ParticlesView& P, const Ad
 // branch's F2.  In two passes, so that the SVD and the Newton iterations run
 // in a kernel without the tile (134 VGPRs, 3 waves/SIMD, against one kernel
 // of 256 VGPRs with spills): k_admm_fgrad writes grad(vn + dv) of every
-// particle (9 rows of n, particle order), k_admm_flocal runs the local step
-// per particle from it
+// particle (9 rows of n, sorted order), k_admm_flocal runs the local step
+// per particle from it and leaves the particle's term of the global step's
+// residual at the current dv in its place.
+//
+// dvStep solves (M + K) dv = b (:167-206) with K the sum of
+// rho omega^2 dt^2 (grad(dv) Fn) Fn^T grad w and b the sum of
+// dt rho omega^2 (F - Fn + y / (rho omega) - dt grad(vn) Fn) Fn^T grad w plus
+// dt M g, from the current dv.  The residual it starts from, b - (M + K) dv,
+// takes grad(vn) and grad(dv) together, which is the local step's G, and the
+// bracket becomes F - (Fn - y / (rho omega) + dt G Fn) = U diag(z - sigma) V^T.
+// So the local step knows the term, and neither b nor K dv needs a pass with
+// a gather of its own (2.1M particles: 303 us and, in FP32, 166 us; now
+// k_be_scatter's).
 __global__ __launch_bounds__(256) void k_admm_fgrad(ParticlesView P, AdmmNodes N, const uint32_t* __restrict__ order,
                                                     const uint32_t* __restrict__ group_start,
                                                     const uint32_t* __restrict__ group_page,
@@ -786,11 +819,11 @@ __global__ __launch_bounds__(256) void k_admm_fgrad(ParticlesView P, AdmmNodes N
     const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
     if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
     double G[3][3];
-    admm_grad_tile(tv, w, dw, inv_dx, lx, ly, lz, G);
+    grad_from_tile(tv, (lx * kTileY + ly) * kTileZ + lz, w, dw, inv_dx, G);
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int r = 0; r < 3; ++r) gs[(c * 3 + r) * S + i] = G[r][c];
+      for (int r = 0; r < 3; ++r) gs[(c * 3 + r) * S + start + j] = G[r][c];
   }
 }
 
@@ -798,35 +831,38 @@ template <bool VISCO>
 __global__ __launch_bounds__(256) void k_admm_flocal(ParticlesView P, AdmmParticles A,
                                                      const int32_t* __restrict__ mat,
                                                      const double* __restrict__ pparam,
-                                                     const double* __restrict__ pstate, uint32_t n,
-                                                     const double* __restrict__ gs, double dt, double rho,
-                                                     double local_tol)
+                                                     const double* __restrict__ pstate,
+                                                     const uint32_t* __restrict__ order, uint32_t n,
+                                                     double* __restrict__ gs, double dt, double rho, double local_tol)
 {
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i >= n) return;
+  const uint32_t ks = blockIdx.x * 256u + threadIdx.x;
+  if (ks >= n) return;
   const int64_t S = P.stride;
   double G[3][3];
 #pragma unroll
   for (int c = 0; c < 3; ++c)
 #pragma unroll
-    for (int r = 0; r < 3; ++r) G[r][c] = gs[(c * 3 + r) * S + i];
-  admm_local_step<VISCO>(P, A, mat, pparam, pstate, i, G, dt, rho, local_tol);
+    for (int r = 0; r < 3; ++r) G[r][c] = gs[(c * 3 + r) * S + ks];
+  admm_local_step<VISCO>(P, A, mat, pparam, pstate, order[ks], G, dt, rho, local_tol);
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int r = 0; r < 3; ++r) gs[(c * 3 + r) * S + ks] = G[r][c];
 }
 
-// dvStep rhs scatter (:167-205): dt rho omega^2 (F - Fn + y/(rho omega) - dt grad(vn) Fn) Fn^T grad w
-// MODE 0; the operator's particle term c_p (grad(x) Fn) Fn^T grad w: MODE 1;
-// VISCO adds the viscoelastic branch's terms with F2, y2, omega2 and FFn
-template <int MODE, bool VISCO>
-__global__ __launch_bounds__(256) void k_admm_scatter(ParticlesView P, AdmmParticles A, AdmmNodes N,
-                                                      const double* __restrict__ xvec,
-                                                      const uint32_t* __restrict__ order,
-                                                      const uint32_t* __restrict__ group_start,
-                                                      const uint32_t* __restrict__ group_page,
-                                                      const int32_t* __restrict__ group_nslot,
-                                                      const double* __restrict__ gm, double* stage, double dt,
-                                                      double rho, double inv_dx, const int32_t* ai)
+// the global operator's particle term c_p (grad(x) Fn) Fn^T grad w in FP64,
+// c_p = rho omega^2 dt^2; VISCO adds the viscoelastic branch's with FFn
+template <bool VISCO>
+__global__ __launch_bounds__(256) void k_admm_op64(ParticlesView P, AdmmParticles A, AdmmNodes N,
+                                                   const double* __restrict__ xvec,
+                                                   const uint32_t* __restrict__ order,
+                                                   const uint32_t* __restrict__ group_start,
+                                                   const uint32_t* __restrict__ group_page,
+                                                   const int32_t* __restrict__ group_nslot,
+                                                   const double* __restrict__ gm, double* stage, double dt,
+                                                   double rho, double inv_dx, const int32_t* ai)
 {
-  if (MODE == 1 && ai[AI_DONE]) return;
+  if (ai[AI_DONE]) return;
   constexpr int SS = 3 * kTileNodes;
   __shared__ double tv[3 * kTileNodes];
   __shared__ double tile[4 * SS];
@@ -834,7 +870,7 @@ __global__ __launch_bounds__(256) void k_admm_scatter(ParticlesView P, AdmmParti
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;
   for (int k = tid; k < 4 * SS; k += 256) tile[k] = 0.0;
-  admm_tile3(group_nslot + 8 * (size_t)g, gm, MODE == 0 ? N.vn : xvec, nullptr, N.stride, tv, nslot);
+  admm_tile3(group_nslot + 8 * (size_t)g, gm, xvec, nullptr, N.stride, tv, nslot);
   const uint32_t start = group_start[g];
   const uint32_t n = group_start[g + 1] - start;
   uint32_t px, py, pz;
@@ -854,63 +890,19 @@ __global__ __launch_bounds__(256) void k_admm_scatter(ParticlesView P, AdmmParti
     for (int d = 0; d < 3; ++d) b[d] = bspline_wdw(xp[d] * inv_dx, w[d], dw[d]);
     const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
     if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
-    double G[3][3], Fn[3][3], Y[3][3];
-    admm_grad_tile(tv, w, dw, inv_dx, lx, ly, lz, G);
+    const int t0 = (lx * kTileY + ly) * kTileZ + lz;
+    double G[3][3], Fn[3][3];
+    grad_from_tile(tv, t0, w, dw, inv_dx, G);
     load_F(P.F, S, i, Fn);
     const double om = A.om[i];
-    const double c2 = MODE == 0 ? dt * rho * om * om : rho * om * om * dt * dt;
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const double gf = G[r][0] * Fn[0][c] + G[r][1] * Fn[1][c] + G[r][2] * Fn[2][c];
-        if (MODE == 0)
-          Y[r][c] = c2 * (A.F[(c * 3 + r) * S + i] - Fn[r][c] + A.y[(c * 3 + r) * S + i] / (om * rho) - dt * gf);
-        else
-          Y[r][c] = c2 * gf;
-      }
-    double Fv[3][3], Y2[3][3];
+    double D[3][3] = { { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 } };
+    add_operator_term(rho * om * om * dt * dt, G, Fn, D);
     if constexpr (VISCO) {
-      load_F(A.fneq, S, i, Fv);
+      load_F(A.fneq, S, i, Fn);
       const double om2 = A.om2[i];
-      const double c22 = MODE == 0 ? dt * rho * om2 * om2 : rho * om2 * om2 * dt * dt;
-#pragma unroll
-      for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const double gf = G[r][0] * Fv[0][c] + G[r][1] * Fv[1][c] + G[r][2] * Fv[2][c];
-          if (MODE == 0)
-            Y2[r][c] = c22 * (A.F2[(c * 3 + r) * S + i] - Fv[r][c] + A.y2[(c * 3 + r) * S + i] / (om2 * rho) - dt * gf);
-          else
-            Y2[r][c] = c22 * gf;
-        }
+      add_operator_term(rho * om2 * om2 * dt * dt, G, Fn, D);
     }
-    opaque_weights(w, dw);
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int bb = 0; bb < 3; ++bb)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          double gw[3], fg[3];
-          wgrad(w, dw, inv_dx, a, bb, c, gw);
-#pragma unroll
-          for (int d = 0; d < 3; ++d) fg[d] = Fn[0][d] * gw[0] + Fn[1][d] * gw[1] + Fn[2][d] * gw[2];
-          const int t = ((lx + a) * kTileY + (ly + bb)) * kTileZ + (lz + c);
-          if constexpr (VISCO) {
-            double fg2[3];
-#pragma unroll
-            for (int d = 0; d < 3; ++d) fg2[d] = Fv[0][d] * gw[0] + Fv[1][d] * gw[1] + Fv[2][d] * gw[2];
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-              atomicAdd(&wt[r * kTileNodes + t], (Y[r][0] * fg[0] + Y[r][1] * fg[1] + Y[r][2] * fg[2]) +
-                                                     (Y2[r][0] * fg2[0] + Y2[r][1] * fg2[1] + Y2[r][2] * fg2[2]));
-          } else {
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-              atomicAdd(&wt[r * kTileNodes + t], Y[r][0] * fg[0] + Y[r][1] * fg[1] + Y[r][2] * fg[2]);
-          }
-        }
+    scatter_grad(wt, t0, w, dw, inv_dx, D);
   }
   __syncthreads();
   double* out = stage + (size_t)g * SS;
@@ -929,34 +921,16 @@ __device__ __forceinline__ void admm_project_node(const AdmmNodes& N, uint32_t k
   r[2] = t[2];
 }
 
-// rhs = dt m g + staged sums (:167-173,206-209)
-__global__ __launch_bounds__(256) void k_admm_rhs(uint32_t nn, const int32_t* __restrict__ slot_src,
-                                                  const double* __restrict__ stage, const double* __restrict__ gm,
-                                                  double* rhs, int64_t S, double dt, double gx, double gy, double gz)
-{
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
-  if (k >= nn) return;
-  double f[3] = { 0.0, 0.0, 0.0 };
-  const double m = gm[k];
-  if (m != 0.0) {
-    const uint32_t e = k & 31u;
-    sum_tiles_src<3>(stage, slot_src + 8 * (size_t)(k >> 5), (int)(e >> 4), (int)((e >> 2) & 3u), (int)(e & 3u), f);
-    f[0] += dt * m * gx;
-    f[1] += dt * m * gy;
-    f[2] += dt * m * gz;
-  }
-  for (int d = 0; d < 3; ++d) rhs[d * S + k] = f[d];
-}
-
-// MINRES start (Minres.h:40-101): q = P(b - A x), z = q / diag, partial z.q;
+// MINRES start (Minres.h:40-101): q = P(b - A x) with x = dv, from the staged
+// sums of the local step's terms (see k_admm_flocal): dt m g + sums - m dv;
+// z = q / diag, partial z.q;
 // m_k, m_{k-1} and q_k start at zero (Minres::reinitialize)
 // (T: the precision the Krylov vectors are stored in; arithmetic in FP64)
 template <class T>
 __global__ __launch_bounds__(256) void k_minres_init(uint32_t nn, const int32_t* __restrict__ slot_src,
                                                      const double* __restrict__ stage, const double* __restrict__ gm,
-                                                     AdmmNodes N, const double* __restrict__ b,
-                                                     const double* __restrict__ x, T* q, T* z, T* zero0, T* zero1,
-                                                     T* zero2, double* partial)
+                                                     AdmmNodes N, double dt, double gx, double gy, double gz, T* q,
+                                                     T* z, T* zero0, T* zero1, T* zero2, double* partial)
 {
   const uint32_t k = blockIdx.x * 256u + threadIdx.x;
   const int64_t S = N.stride;
@@ -968,7 +942,8 @@ __global__ __launch_bounds__(256) void k_minres_init(uint32_t nn, const int32_t*
       const uint32_t e = k & 31u;
       double f[3];
       sum_tiles_src<3>(stage, slot_src + 8 * (size_t)(k >> 5), (int)(e >> 4), (int)((e >> 2) & 3u), (int)(e & 3u), f);
-      for (int d = 0; d < 3; ++d) r[d] = b[d * S + k] - (m * x[d * S + k] + f[d]);
+      const double gr[3] = { gx, gy, gz };
+      for (int d = 0; d < 3; ++d) r[d] = dt * m * gr[d] + f[d] - m * N.dv[d * S + k];
       admm_project_node(N, k, r);
       const double dg = N.diag[k];
       for (int d = 0; d < 3; ++d) {
@@ -1124,13 +1099,11 @@ __global__ __launch_bounds__(256) void k_admm_cache32(ParticlesView P, AdmmParti
   }
 }
 
-// the global operator's particle term in FP32 (k_admm_scatter<1>'s sums):
-// c_p (grad(x) Fn) Fn^T grad w (+ the viscoelastic branch's term with FFn),
-// x given in precision TX
-template <bool VISCO, class TX>
+// the global operator's particle term in FP32 (k_admm_op64's sums)
+template <bool VISCO>
 __global__ __launch_bounds__(256) void k_admm_op32(AdmmCache32 C, const uint32_t* __restrict__ group_start,
                                                    const int32_t* __restrict__ group_nslot,
-                                                   const double* __restrict__ gm, const TX* __restrict__ xvec,
+                                                   const double* __restrict__ gm, const float* __restrict__ xvec,
                                                    int64_t NS, double* stage, float inv_dx, const int32_t* ai)
 {
   if (ai[AI_DONE]) return;
@@ -1149,7 +1122,7 @@ __global__ __launch_bounds__(256) void k_admm_op32(AdmmCache32 C, const uint32_t
     const int64_t node = (int64_t)sl * 32 + elem_of(tx, ty, tz);
     const bool on = sl >= 0 && gm[node] != 0.0;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) tv[d * kTileNodes + t] = on ? (float)xvec[d * NS + node] : 0.0f;
+    for (int d = 0; d < 3; ++d) tv[d * kTileNodes + t] = on ? xvec[d * NS + node] : 0.0f;
   }
   __syncthreads();
   const uint32_t start = group_start[g];
@@ -1166,70 +1139,23 @@ __global__ __launch_bounds__(256) void k_admm_op32(AdmmCache32 C, const uint32_t
     float w[3][3], dw[3][3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) bspline_frac(C.frac[d * CS + ks], w[d], dw[d]);
-    float G[3][3] = { { 0.f } };
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int bb = 0; bb < 3; ++bb)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          float gw[3];
-          wgradT(w, dw, inv_dx, a, bb, c, gw);
-          const int t = ((lx + a) * kTileY + (ly + bb)) * kTileZ + (lz + c);
-#pragma unroll
-          for (int r = 0; r < 3; ++r) {
-            const float v = tv[r * kTileNodes + t];
-            G[r][0] += v * gw[0];
-            G[r][1] += v * gw[1];
-            G[r][2] += v * gw[2];
-          }
-        }
-    float Fn[3][3], Y[3][3];
+    const int t0 = (lx * kTileY + ly) * kTileZ + lz;
+    float G[3][3], Fn[3][3];
+    grad_from_tile(tv, t0, w, dw, inv_dx, G);
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
       for (int r = 0; r < 3; ++r) Fn[r][c] = C.F[(c * 3 + r) * CS + ks];
-    const float cp = C.cp[ks];
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) Y[r][c] = cp * (G[r][0] * Fn[0][c] + G[r][1] * Fn[1][c] + G[r][2] * Fn[2][c]);
-    float Fv[3][3], Y2[3][3];
+    float D[3][3] = { { 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f } };
+    add_operator_term(C.cp[ks], G, Fn, D);
     if constexpr (VISCO) {
 #pragma unroll
       for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int r = 0; r < 3; ++r) Fv[r][c] = C.F2[(c * 3 + r) * CS + ks];
-      const float cp2 = C.cp2[ks];
-#pragma unroll
-      for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) Y2[r][c] = cp2 * (G[r][0] * Fv[0][c] + G[r][1] * Fv[1][c] + G[r][2] * Fv[2][c]);
+        for (int r = 0; r < 3; ++r) Fn[r][c] = C.F2[(c * 3 + r) * CS + ks];
+      add_operator_term(C.cp2[ks], G, Fn, D);
     }
-    opaque_weights(w, dw);
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int bb = 0; bb < 3; ++bb)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          float gw[3], fg[3];
-          wgradT(w, dw, inv_dx, a, bb, c, gw);
-#pragma unroll
-          for (int d = 0; d < 3; ++d) fg[d] = Fn[0][d] * gw[0] + Fn[1][d] * gw[1] + Fn[2][d] * gw[2];
-          const int t = ((lx + a) * kTileY + (ly + bb)) * kTileZ + (lz + c);
-#pragma unroll
-          for (int r = 0; r < 3; ++r) {
-            float val = Y[r][0] * fg[0] + Y[r][1] * fg[1] + Y[r][2] * fg[2];
-            if constexpr (VISCO) {
-              float fg2[3];
-#pragma unroll
-              for (int d = 0; d < 3; ++d) fg2[d] = Fv[0][d] * gw[0] + Fv[1][d] * gw[1] + Fv[2][d] * gw[2];
-              val += Y2[r][0] * fg2[0] + Y2[r][1] * fg2[1] + Y2[r][2] * fg2[2];
-            }
-            atomicAdd(&wt[r * kTileNodes + t], (double)val);
-          }
-        }
+    scatter_grad(wt, t0, w, dw, inv_dx, D);
   }
   __syncthreads();
   double* out = stage + (size_t)g * SS;
@@ -1268,7 +1194,7 @@ __global__ __launch_bounds__(256) void k_admm_ustep(ParticlesView P, AdmmParticl
     const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
     if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
     double G[3][3], Fn[3][3];
-    admm_grad_tile(tv, w, dw, inv_dx, lx, ly, lz, G);
+    grad_from_tile(tv, (lx * kTileY + ly) * kTileZ + lz, w, dw, inv_dx, G);
     load_F(P.F, S, i, Fn);
     const double om = A.om[i];
 #pragma unroll
@@ -1405,9 +1331,4 @@ __global__ __launch_bounds__(256) void k_admm_lastdv(ParticlesView P, AdmmPartic
         }
     for (int d = 0; d < 3; ++d) A.last[d * S + i] = acc[d] / (ws * dt);
   }
-}
-
-__global__ void k_admm_reset_flags(int32_t* ai)
-{
-  if (threadIdx.x < AI_N) ai[threadIdx.x] = 0;
 }

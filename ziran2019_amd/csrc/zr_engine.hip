@@ -2821,12 +2821,12 @@ int advance_recorded(zr_engine* e, double dt, zr_engine::StepRecord& r)
 }
 
 // ------------------------------------------------------------------- ADMM
-constexpr int kAdmmNodeRows = 3 + 3 + 9 + 1 + 3 + 9 + 3 + 9;  // vn dv proj diag rhs q(3) z m(3)
+constexpr int kAdmmNodeRows = 3 + 3 + 9 + 1 + 9 + 3 + 9;  // vn dv proj diag q(3) z m(3)
 
 // the global operator's particle term of x into the staged tiles: the FP64
 // scatter from the particle arrays, or the FP32 apply over the sorted cache
 struct AdmmOp {
-  bool fp32, visco;
+  bool visco;
   ParticlesView P;
   AdmmParticles Ap;
   AdmmNodes Nd;
@@ -2834,41 +2834,31 @@ struct AdmmOp {
   double dt, rho, inv_dx;
 };
 
-template <class TX>
-void admm_apply(zr_engine* e, const AdmmOp& op, const TX* x)
+void admm_apply(zr_engine* e, const AdmmOp& op, const float* x)
 {
-  hipStream_t s = e->stream;
-  if (op.fp32) {
-    if (op.visco)
-      k_admm_op32<true, TX><<<e->A, 256, 0, s>>>(op.C, e->group_start, e->group_nslot, e->gm, x, op.Nd.stride,
-                                                 e->stage, (float)op.inv_dx, e->ci);
-    else
-      k_admm_op32<false, TX><<<e->A, 256, 0, s>>>(op.C, e->group_start, e->group_nslot, e->gm, x, op.Nd.stride,
-                                                  e->stage, (float)op.inv_dx, e->ci);
-  } else if constexpr (std::is_same<TX, double>::value) {
-    if (op.visco)
-      k_admm_scatter<1, true><<<e->A, 256, 0, s>>>(op.P, op.Ap, op.Nd, x, e->order, e->group_start, e->group_page,
-                                                   e->group_nslot, e->gm, e->stage, op.dt, op.rho, op.inv_dx, e->ci);
-    else
-      k_admm_scatter<1, false><<<e->A, 256, 0, s>>>(op.P, op.Ap, op.Nd, x, e->order, e->group_start, e->group_page,
-                                                    e->group_nslot, e->gm, e->stage, op.dt, op.rho, op.inv_dx, e->ci);
-  }
+  auto k = op.visco ? k_admm_op32<true> : k_admm_op32<false>;
+  k<<<e->A, 256, 0, e->stream>>>(op.C, e->group_start, e->group_nslot, e->gm, x, op.Nd.stride, e->stage,
+                                 (float)op.inv_dx, e->ci);
+}
+void admm_apply(zr_engine* e, const AdmmOp& op, const double* x)
+{
+  auto k = op.visco ? k_admm_op64<true> : k_admm_op64<false>;
+  k<<<e->A, 256, 0, e->stream>>>(op.P, op.Ap, op.Nd, x, e->order, e->group_start, e->group_page, e->group_nslot, e->gm,
+                                 e->stage, op.dt, op.rho, op.inv_dx, e->ci);
 }
 
 // Minres::solve (Minres.h:69-149) on the global system for dv (FP64), the
 // Krylov vectors in precision T (the seven vectors rotate by pointer)
 template <class T>
-int admm_minres(zr_engine* e, const AdmmOp& op, const double* rhs, T* const qb[3], T* zb, T* const mb[3],
+int admm_minres(zr_engine* e, const AdmmOp& op, T* const qb[3], T* zb, T* const mb[3],
                 const zr_admm_opts* o, uint32_t nn, uint32_t nbn, int& iters)
 {
   hipStream_t s = e->stream;
   const AdmmNodes& Nd = op.Nd;
   const int64_t C = Nd.stride;
-  k_admm_reset_flags<<<1, 64, 0, s>>>(e->ci);
-  admm_apply<double>(e, op, Nd.dv);
   T *q = qb[2], *qk = qb[1], *qkm1 = qb[0], *z = zb, *mk = mb[2], *mkm1 = mb[1], *mkm2 = mb[0];
-  k_minres_init<T><<<nbn, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, Nd, rhs, Nd.dv, q, z, mk, mkm1, qk,
-                                       e->partial);
+  k_minres_init<T><<<nbn, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, Nd, op.dt, e->cfg.gravity[0],
+                                       e->cfg.gravity[1], e->cfg.gravity[2], q, z, mk, mkm1, qk, e->partial);
   k_minres_reduce<<<1, 256, 0, s>>>(e->partial, nbn, e->sc, e->ci, MR_INIT, o->global_tolerance, 0.5, 0,
                                     o->minres_max_iterations, SolveMark{});
   k_minres_scale<T><<<nbn, 256, 0, s>>>(nn, e->gm, C, q, z, e->sc, e->ci);
@@ -2886,7 +2876,7 @@ int admm_minres(zr_engine* e, const AdmmOp& op, const double* rhs, T* const qb[3
     qkm1 = qk;
     qk = q;
     q = t;
-    admm_apply<T>(e, op, mk);
+    admm_apply(e, op, mk);
     k_minres_apply<T><<<nbn, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, Nd, mk, q, e->ci, e->partial);
     k_minres_reduce<<<1, 256, 0, s>>>(e->partial, nbn, e->sc, e->ci, MR_ALPHA, 0.0, 0.0, k, o->minres_max_iterations,
                                       SolveMark{});
@@ -2937,10 +2927,9 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
   const int64_t C = (int64_t)e->admm_cap;
   double* base = e->admm_node;
   AdmmNodes Nd{ base, base + 3 * C, base + 6 * C, e->admm_coll, base + 15 * C, C };
-  double* rhs = base + 16 * C;
-  double* qb[3] = { base + 19 * C, base + 22 * C, base + 25 * C };
-  double* zb = base + 28 * C;
-  double* mb[3] = { base + 31 * C, base + 34 * C, base + 37 * C };
+  double* qb[3] = { base + 16 * C, base + 19 * C, base + 22 * C };
+  double* zb = base + 25 * C;
+  double* mb[3] = { base + 28 * C, base + 31 * C, base + 34 * C };
   double* pa = e->admm_p;
   AdmmParticles Ap{ pa, pa + 9 * N, pa + 18 * N, pa + 19 * N, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                     e->visc_d, e->visc_v };
@@ -2975,7 +2964,7 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
   // the FP32-bulk global step: per-particle operator data in FP32, sorted,
   // and FP32 Krylov vectors
   const bool fp32 = o->precision == ZR_FP32_REFINED;
-  AdmmOp op{ fp32, visco, P, Ap, Nd, AdmmCache32{}, dt, rho, inv_dx };
+  AdmmOp op{ visco, P, Ap, Nd, AdmmCache32{}, dt, rho, inv_dx };
   float *qb32[3] = { nullptr, nullptr, nullptr }, *zb32 = nullptr, *mb32[3] = { nullptr, nullptr, nullptr };
   if (fp32) {
     const size_t rows = visco ? 23 : 13;
@@ -3011,7 +3000,7 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
                                                                         rho, dt);
     ZR_LAUNCH_CHECK(e);
   }
-  // the local step's per-particle grad(vn + dv) (9 rows of n)
+  // the local step's per-particle grad(vn + dv), then its residual term (9 rows of n)
   if (e->be_fb_cap < N) {
     dfree(e->be_fb);
     e->be_fb_cap = 0;
@@ -3024,24 +3013,17 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
     k_admm_collide<<<nbn, 256, 0, s>>>(nn, e->slot_page, e->gm, Nd, dx, cs);
     k_admm_fgrad<<<e->A, 256, 0, s>>>(P, Nd, e->order, e->group_start, e->group_page, e->group_nslot, e->gm, inv_dx,
                                       e->be_fb);
-    if (visco) {
-      k_admm_flocal<true><<<npb, 256, 0, s>>>(P, Ap, mat, e->pparam, e->pstate, (uint32_t)n, e->be_fb, dt, rho,
-                                              o->local_tolerance);
-      k_admm_scatter<0, true><<<e->A, 256, 0, s>>>(P, Ap, Nd, nullptr, e->order, e->group_start, e->group_page,
-                                                   e->group_nslot, e->gm, e->stage, dt, rho, inv_dx, e->ci);
-    } else {
-      k_admm_flocal<false><<<npb, 256, 0, s>>>(P, Ap, mat, e->pparam, e->pstate, (uint32_t)n, e->be_fb, dt, rho,
-                                               o->local_tolerance);
-      k_admm_scatter<0, false><<<e->A, 256, 0, s>>>(P, Ap, Nd, nullptr, e->order, e->group_start, e->group_page,
-                                                    e->group_nslot, e->gm, e->stage, dt, rho, inv_dx, e->ci);
+    {
+      auto k = visco ? k_admm_flocal<true> : k_admm_flocal<false>;
+      k<<<npb, 256, 0, s>>>(P, Ap, mat, e->pparam, e->pstate, e->order, (uint32_t)n, e->be_fb, dt, rho,
+                            o->local_tolerance);
     }
-    k_admm_rhs<<<nbn, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, rhs, C, dt, e->cfg.gravity[0],
-                                   e->cfg.gravity[1], e->cfg.gravity[2]);
+    k_be_scatter<<<e->A, 256, 0, s>>>(P, e->order, e->group_start, e->group_page, n, inv_dx, e->be_fb, e->stage);
     // MINRES on the global system, warm-started from dv (Minres.h:69-149),
     // relative tolerance min(0.5, sqrt(max(1, 1e-6))) = 0.5 (:785-787)
     int its = 0;
-    int rc2 = fp32 ? admm_minres<float>(e, op, rhs, qb32, zb32, mb32, o, nn, nbn, its)
-                   : admm_minres<double>(e, op, rhs, qb, zb, mb, o, nn, nbn, its);
+    int rc2 = fp32 ? admm_minres<float>(e, op, qb32, zb32, mb32, o, nn, nbn, its)
+                   : admm_minres<double>(e, op, qb, zb, mb, o, nn, nbn, its);
     if (rc2) return rc2;
     total_minres += its;
     if (visco)
