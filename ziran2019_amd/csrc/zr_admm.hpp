@@ -853,60 +853,65 @@ __global__ __launch_bounds__(256) void k_admm_flocal(ParticlesView P, AdmmPartic
 // the global operator's particle term c_p (grad(x) Fn) Fn^T grad w in FP64,
 // c_p = rho omega^2 dt^2; VISCO adds the viscoelastic branch's with FFn
 template <bool VISCO>
-__global__ __launch_bounds__(256) void k_admm_op64(ParticlesView P, AdmmParticles A, AdmmNodes N,
+__global__ __launch_bounds__(kSumThreads, 4) void k_admm_op64(ParticlesView P, AdmmParticles A, AdmmNodes N,
                                                    const double* __restrict__ xvec,
                                                    const uint32_t* __restrict__ order,
                                                    const uint32_t* __restrict__ group_start,
+                                                   const uint32_t* __restrict__ cell_off,
                                                    const uint32_t* __restrict__ group_page,
                                                    const int32_t* __restrict__ group_nslot,
                                                    const double* __restrict__ gm, double* stage, double dt,
                                                    double rho, double inv_dx, const int32_t* ai)
 {
   if (ai[AI_DONE]) return;
-  constexpr int SS = 3 * kTileNodes;
   __shared__ double tv[3 * kTileNodes];
-  __shared__ double tile[4 * SS];
   __shared__ int32_t nslot[8];
+  __shared__ CellSums cs;
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;
-  for (int k = tid; k < 4 * SS; k += 256) tile[k] = 0.0;
-  admm_tile3(group_nslot + 8 * (size_t)g, gm, xvec, nullptr, N.stride, tv, nslot);
   const uint32_t start = group_start[g];
   const uint32_t n = group_start[g + 1] - start;
+  cell_sums_begin(cs, cell_off + 32 * (size_t)g, n);
+  admm_tile3(group_nslot + 8 * (size_t)g, gm, xvec, nullptr, N.stride, tv, nslot);
   uint32_t px, py, pz;
   page_decode(group_page[g], px, py, pz);
   const int ox = 2 * (int)px, oy = 4 * (int)py, oz = 4 * (int)pz;
   const int64_t S = P.stride;
-  double* wt = tile + (tid >> 6) * SS;
-  const uint32_t perm = (uint32_t)((tid & 31) * 8 + (tid >> 5));
-  for (uint32_t j0 = 0; j0 < n; j0 += 256) {
-    const uint32_t j = j0 + perm;
-    if (j >= n) continue;
-    const uint32_t i = order[start + j];
-    const double xp[3] = { P.x[i], P.x[S + i], P.x[2 * S + i] };
-    double w[3][3], dw[3][3];
-    int b[3];
+  double acc[3][3] = { { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 } };
+  for (uint32_t c0 = 0; c0 < n; c0 += kSumChunk) {
+    const uint32_t count = n - c0 < (uint32_t)kSumChunk ? n - c0 : (uint32_t)kSumChunk;
+    if ((uint32_t)tid < count) {
+      const uint32_t i = order[start + c0 + tid];
+      double w[3][3], dw[3][3], f[3];
+      int b[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) b[d] = bspline_wdw(xp[d] * inv_dx, w[d], dw[d]);
-    const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
-    if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
-    const int t0 = (lx * kTileY + ly) * kTileZ + lz;
-    double G[3][3], Fn[3][3];
-    grad_from_tile(tv, t0, w, dw, inv_dx, G);
-    load_F(P.F, S, i, Fn);
-    const double om = A.om[i];
-    double D[3][3] = { { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 } };
-    add_operator_term(rho * om * om * dt * dt, G, Fn, D);
-    if constexpr (VISCO) {
-      load_F(A.fneq, S, i, Fn);
-      const double om2 = A.om2[i];
-      add_operator_term(rho * om2 * om2 * dt * dt, G, Fn, D);
+      for (int d = 0; d < 3; ++d) {
+        const double xi = P.x[d * S + i] * inv_dx;
+        b[d] = int_floor(xi - 0.5);
+        f[d] = xi - (double)b[d];
+        bspline_frac(f[d], w[d], dw[d]);
+      }
+      double D[3][3] = { { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 } };
+      const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
+      if ((unsigned)lx <= 1u && (unsigned)ly <= 3u && (unsigned)lz <= 3u) {
+        double G[3][3], Fn[3][3];
+        grad_from_tile(tv, (lx * kTileY + ly) * kTileZ + lz, w, dw, inv_dx, G);
+        load_F(P.F, S, i, Fn);
+        const double om = A.om[i], k = rho * dt * dt * inv_dx;
+        add_operator_term(k * om * om, G, Fn, D);
+        if constexpr (VISCO) {
+          load_F(A.fneq, S, i, Fn);
+          const double om2 = A.om2[i];
+          add_operator_term(k * om2 * om2, G, Fn, D);
+        }
+      }
+      cell_sums_put(cs, tid, D, f);
     }
-    scatter_grad(wt, t0, w, dw, inv_dx, D);
+    __syncthreads();
+    cell_sums_chunk(cs, c0, count, acc);
+    __syncthreads();
   }
-  __syncthreads();
-  double* out = stage + (size_t)g * SS;
-  for (int k = tid; k < SS; k += 256) out[k] = tile[k] + tile[SS + k] + tile[2 * SS + k] + tile[3 * SS + k];
+  cell_sums_store(cs, acc, stage + (size_t)g * (3 * kTileNodes));
 }
 
 __device__ __forceinline__ void admm_project_node(const AdmmNodes& N, uint32_t k, double r[3])
@@ -1057,9 +1062,8 @@ __global__ __launch_bounds__(256) void k_minres_scale(uint32_t nn, const double*
 // ---- the FP32-bulk global step (configuration 3: FP32 bulk, FP64 SVD and
 // projection): the operator's per-particle data in FP32, in sorted order,
 // formed once per step after initStep; the operator apply reads it
-// coalesced, gathers and forms its terms in FP32, and adds them into the
-// FP64 LDS tiles (FP32 LDS adds are far slower on this part); the Krylov
-// vectors are FP32, their inner products and the solution dv FP64.
+// coalesced, gathers and forms its terms in FP32, and sums them in FP64; the
+// Krylov vectors are FP32, their inner products and the solution dv FP64.
 struct AdmmCache32 {
   float* frac;     // [3][n] x / dx - base node
   float* F;        // [9][n] Fn, column-major
@@ -1101,22 +1105,24 @@ __global__ __launch_bounds__(256) void k_admm_cache32(ParticlesView P, AdmmParti
 
 // the global operator's particle term in FP32 (k_admm_op64's sums)
 template <bool VISCO>
-__global__ __launch_bounds__(256) void k_admm_op32(AdmmCache32 C, const uint32_t* __restrict__ group_start,
+__global__ __launch_bounds__(kSumThreads, 5) void k_admm_op32(AdmmCache32 C, const uint32_t* __restrict__ group_start,
+                                                   const uint32_t* __restrict__ cell_off,
                                                    const int32_t* __restrict__ group_nslot,
                                                    const double* __restrict__ gm, const float* __restrict__ xvec,
                                                    int64_t NS, double* stage, float inv_dx, const int32_t* ai)
 {
   if (ai[AI_DONE]) return;
-  constexpr int SS = 3 * kTileNodes;
   __shared__ float tv[3 * kTileNodes];
-  __shared__ double tile[4 * SS];
   __shared__ int32_t nslot[8];
+  __shared__ CellSums cs;
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;
-  for (int k = tid; k < 4 * SS; k += 256) tile[k] = 0.0;
+  const uint32_t start = group_start[g];
+  const uint32_t n = group_start[g + 1] - start;
+  cell_sums_begin(cs, cell_off + 32 * (size_t)g, n);
   if (tid < 8) nslot[tid] = group_nslot[8 * (size_t)g + tid];
   __syncthreads();
-  for (int t = tid; t < kTileNodes; t += 256) {
+  for (int t = tid; t < kTileNodes; t += kSumThreads) {
     const int tx = t / (kTileY * kTileZ), ty = (t / kTileZ) % kTileY, tz = t % kTileZ;
     const int32_t sl = nslot[((tx >> 1) << 2) | ((ty >> 2) << 1) | (tz >> 2)];
     const int64_t node = (int64_t)sl * 32 + elem_of(tx, ty, tz);
@@ -1125,41 +1131,49 @@ __global__ __launch_bounds__(256) void k_admm_op32(AdmmCache32 C, const uint32_t
     for (int d = 0; d < 3; ++d) tv[d * kTileNodes + t] = on ? xvec[d * NS + node] : 0.0f;
   }
   __syncthreads();
-  const uint32_t start = group_start[g];
-  const uint32_t n = group_start[g + 1] - start;
   const int64_t CS = C.stride;
-  double* wt = tile + (tid >> 6) * SS;
-  const uint32_t perm = (uint32_t)((tid & 31) * 8 + (tid >> 5));
-  for (uint32_t j0 = 0; j0 < n; j0 += 256) {
-    const uint32_t j = j0 + perm;
-    if (j >= n) continue;
-    const uint32_t ks = start + j;
-    const uint32_t e = C.cell[ks];
-    const int lx = (int)(e >> 4), ly = (int)((e >> 2) & 3u), lz = (int)(e & 3u);
-    float w[3][3], dw[3][3];
+  double acc[3][3] = { { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 } };
+  for (uint32_t c0 = 0; c0 < n; c0 += kSumChunk) {
+    const uint32_t count = n - c0 < (uint32_t)kSumChunk ? n - c0 : (uint32_t)kSumChunk;
+    if ((uint32_t)tid < count) {
+      const uint32_t ks = start + c0 + tid;
+      const uint32_t e = C.cell[ks];
+      const int lx = (int)(e >> 4), ly = (int)((e >> 2) & 3u), lz = (int)(e & 3u);
+      float w[3][3], dw[3][3], f[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) bspline_frac(C.frac[d * CS + ks], w[d], dw[d]);
-    const int t0 = (lx * kTileY + ly) * kTileZ + lz;
-    float G[3][3], Fn[3][3];
-    grad_from_tile(tv, t0, w, dw, inv_dx, G);
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int r = 0; r < 3; ++r) Fn[r][c] = C.F[(c * 3 + r) * CS + ks];
-    float D[3][3] = { { 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f } };
-    add_operator_term(C.cp[ks], G, Fn, D);
-    if constexpr (VISCO) {
+      for (int d = 0; d < 3; ++d) {
+        f[d] = C.frac[d * CS + ks];
+        bspline_frac(f[d], w[d], dw[d]);
+      }
+      float G[3][3], Fn[3][3];
+      grad_from_tile(tv, (lx * kTileY + ly) * kTileZ + lz, w, dw, inv_dx, G);
 #pragma unroll
       for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int r = 0; r < 3; ++r) Fn[r][c] = C.F2[(c * 3 + r) * CS + ks];
-      add_operator_term(C.cp2[ks], G, Fn, D);
+        for (int r = 0; r < 3; ++r) Fn[r][c] = C.F[(c * 3 + r) * CS + ks];
+      float D[3][3] = { { 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f }, { 0.f, 0.f, 0.f } };
+      add_operator_term(C.cp[ks], G, Fn, D);
+      if constexpr (VISCO) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int r = 0; r < 3; ++r) Fn[r][c] = C.F2[(c * 3 + r) * CS + ks];
+        add_operator_term(C.cp2[ks], G, Fn, D);
+      }
+      double D64[3][3], f64[3];
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) D64[r][c] = (double)(inv_dx * D[r][c]);
+        f64[r] = (double)f[r];
+      }
+      cell_sums_put(cs, tid, D64, f64);
     }
-    scatter_grad(wt, t0, w, dw, inv_dx, D);
+    __syncthreads();
+    cell_sums_chunk(cs, c0, count, acc);
+    __syncthreads();
   }
-  __syncthreads();
-  double* out = stage + (size_t)g * SS;
-  for (int k = tid; k < SS; k += 256) out[k] = tile[k] + tile[SS + k] + tile[2 * SS + k] + tile[3 * SS + k];
+  cell_sums_store(cs, acc, stage + (size_t)g * (3 * kTileNodes));
 }
 
 

@@ -2837,14 +2837,14 @@ struct AdmmOp {
 void admm_apply(zr_engine* e, const AdmmOp& op, const float* x)
 {
   auto k = op.visco ? k_admm_op32<true> : k_admm_op32<false>;
-  k<<<e->A, 256, 0, e->stream>>>(op.C, e->group_start, e->group_nslot, e->gm, x, op.Nd.stride, e->stage,
+  k<<<e->A, kSumThreads, 0, e->stream>>>(op.C, e->group_start, e->cell_off, e->group_nslot, e->gm, x, op.Nd.stride, e->stage,
                                  (float)op.inv_dx, e->ci);
 }
 void admm_apply(zr_engine* e, const AdmmOp& op, const double* x)
 {
   auto k = op.visco ? k_admm_op64<true> : k_admm_op64<false>;
-  k<<<e->A, 256, 0, e->stream>>>(op.P, op.Ap, op.Nd, x, e->order, e->group_start, e->group_page, e->group_nslot, e->gm,
-                                 e->stage, op.dt, op.rho, op.inv_dx, e->ci);
+  k<<<e->A, kSumThreads, 0, e->stream>>>(op.P, op.Ap, op.Nd, x, e->order, e->group_start, e->cell_off, e->group_page,
+                                 e->group_nslot, e->gm, e->stage, op.dt, op.rho, op.inv_dx, e->ci);
 }
 
 // Minres::solve (Minres.h:69-149) on the global system for dv (FP64), the
@@ -3018,7 +3018,7 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
       k<<<npb, 256, 0, s>>>(P, Ap, mat, e->pparam, e->pstate, e->order, (uint32_t)n, e->be_fb, dt, rho,
                             o->local_tolerance);
     }
-    k_be_scatter<<<e->A, 256, 0, s>>>(P, e->order, e->group_start, e->group_page, n, inv_dx, e->be_fb, e->stage);
+    k_be_scatter<<<e->A, kSumThreads, 0, s>>>(P, e->order, e->group_start, e->cell_off, n, inv_dx, e->be_fb, e->stage);
     // MINRES on the global system, warm-started from dv (Minres.h:69-149),
     // relative tolerance min(0.5, sqrt(max(1, 1e-6))) = 0.5 (:785-787)
     int its = 0;
@@ -3165,7 +3165,7 @@ int be_state_residual(zr_engine* e, bool jac = false)
     k_be_grad<T><<<e->A, 256, 0, e->stream>>>(pview(e), hc, e->order, e->group_start, e->group_page, e->group_nslot,
                                               e->ivn, e->idv, (int64_t)e->grid_cap, 1.0 / dx, dt, e->be_fb, co);
     k_be_svd<T><<<blocks_for(N, 256), 256, 0, e->stream>>>(pview(e), hc, e->order, (uint32_t)N, e->be_fb);
-    k_be_scatter<<<e->A, 256, 0, e->stream>>>(pview(e), e->order, e->group_start, e->group_page, hc.stride,
+    k_be_scatter<<<e->A, kSumThreads, 0, e->stream>>>(pview(e), e->order, e->group_start, e->cell_off, hc.stride,
                                               1.0 / dx, e->be_fb, e->stage);
   }
   ZR_LAUNCH_CHECK(e);

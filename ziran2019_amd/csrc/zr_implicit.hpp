@@ -341,27 +341,6 @@ __device__ __forceinline__ void grad_from_tile(const T* tv, int t0, const T w[3]
     G[r][2] = inv_dx * (w[0][0] * W[0] + w[0][1] * W[1] + w[0][2] * W[2]);
   }
 }
-// its transpose: D grad w_i added to the 27 nodes of the wave's tile, the
-// x y products once for the three z offsets (270 operations; 81 LDS adds)
-template <class T>
-__device__ __forceinline__ void scatter_grad(double* wt, int t0, const T w[3][3], const T dw[3][3], T inv_dx,
-                                             const T D[3][3])
-{
-#pragma unroll
-  for (int a = 0; a < 3; ++a)
-#pragma unroll
-    for (int b = 0; b < 3; ++b) {
-      const T wa = inv_dx * w[0][a], da = inv_dx * dw[0][a];
-      const T x0 = da * w[1][b], x1 = wa * dw[1][b], x2 = wa * w[1][b];
-      double* q = wt + t0 + (a * kTileY + b) * kTileZ;
-#pragma unroll
-      for (int r = 0; r < 3; ++r) {
-        const T A = D[r][0] * x0 + D[r][1] * x1, B = D[r][2] * x2;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) atomicAdd(q + r * kTileNodes + c, (double)(A * w[2][c] + B * dw[2][c]));
-      }
-    }
-}
 // a scatter after a gather recomputes the 27 weight gradients from the 1-D
 // weights rather than holding them from the gather (register budget)
 template <class T>
@@ -651,6 +630,175 @@ __global__ __launch_bounds__(256) void k_be_state(ParticlesView P, HvpCache<T> c
   }
 }
 
+constexpr int kAB = 9;        // (a, b) stencil offsets; c is handled inside a task
+
+// Node-major layout of the per-(cell, a, b, c) partial sums of the operator
+// apply: tile node t = (tx, ty, tz) owns n(t) = na(tx) nb(ty) nb(tz)
+// consecutive entries from off(t), one per stencil offset (a, b, c) whose
+// source cell t - (a, b, c) lies in the page, ordered by a, then b, then c.
+// Per axis: na = {1,2,2,1} (2 cells), nb = {1,2,3,3,2,1} (4 cells), with
+// prefix sums {0,1,3,5} and {0,1,3,6,9,11}; 864 entries in all.
+constexpr int hvp_na(int tx) { return (0x1221 >> (4 * tx)) & 15; }
+constexpr int hvp_nb(int ty) { return (0x123321 >> (4 * ty)) & 15; }
+constexpr int hvp_node_off(int tx, int ty, int tz)
+{
+  return ((0x5310 >> (4 * tx)) & 15) * 144 +
+         hvp_na(tx) * (((0xB96310 >> (4 * ty)) & 15) * 12 + hvp_nb(ty) * ((0xB96310 >> (4 * tz)) & 15));
+}
+constexpr int hvp_slot(int tx, int ty, int tz, int a, int b, int c)
+{
+  return hvp_node_off(tx, ty, tz) +
+         ((a - (tx > 1 ? tx - 1 : 0)) * hvp_nb(ty) + (b - (ty > 3 ? ty - 3 : 0))) * hvp_nb(tz) +
+         (c - (tz > 3 ? tz - 3 : 0));
+}
+
+// slots of task (cell e, a, b)'s three c offsets, 10 bits each
+struct HvpTaskSlots {
+  uint32_t v[kCells * kAB];
+};
+constexpr HvpTaskSlots hvp_task_slots()
+{
+  HvpTaskSlots t{};
+  for (int task = 0; task < kCells * kAB; ++task) {
+    const int e = task / kAB, a = (task % kAB) / 3, b = task % 3;
+    const int tx = (e & 1) + a, ty = ((e >> 1) & 3) + b, cz = (e >> 3) & 3;
+    uint32_t v = 0;
+    for (int c = 0; c < 3; ++c) v |= (uint32_t)hvp_slot(tx, ty, cz + c, a, b, c) << (10 * c);
+    t.v[task] = v;
+  }
+  return t;
+}
+// every entry of the layout belongs to exactly one (task, c)
+constexpr bool hvp_task_slots_valid()
+{
+  const HvpTaskSlots t = hvp_task_slots();
+  int hits[kCells * kAB * 3] = {};
+  for (int task = 0; task < kCells * kAB; ++task)
+    for (int c = 0; c < 3; ++c) {
+      const uint32_t k = (t.v[task] >> (10 * c)) & 1023u;
+      if (k >= (uint32_t)(kCells * kAB * 3)) return false;
+      ++hits[k];
+    }
+  for (int k = 0; k < kCells * kAB * 3; ++k)
+    if (hits[k] != 1) return false;
+  return true;
+}
+static_assert(hvp_task_slots_valid(), "node-major layout is a bijection");
+static_assert(hvp_task_slots().v[0] == (0u | (2u << 10) | (5u << 20)), "slots of task (cell 0, a 0, b 0)");
+__constant__ HvpTaskSlots kHvpTaskSlots = hvp_task_slots();
+
+// Sums of D_p grad w_i over a group's particles without LDS adds, for any
+// per-particle matrix D (FP64).  The nine values of D and the three fractions
+// of a chunk's particles are staged in LDS; thread (cell, a, b) sums its
+// cell's particles (the sort's runs) for three nodes and three directions in
+// registers, forming the weights from the fractions; after the last chunk the
+// sums go into the node-major layout, over the rows, and a thread per node
+// adds its partials in order.  An LDS add per particle, node and direction
+// (81 of them) takes 12 cycles of the CU per particle at best; a task's
+// twelve LDS reads and 47 FP64 operations per particle (nine tasks) take
+// about 7 each.  Blocks of 320 threads, one for each of the 288 tasks, and
+// chunks of 304 particles, because eight particles per cell make groups of
+// 256 + some: with chunks of 256 a third of the groups went through a second
+// one for a few particles.  Measured, with LDS adds -> chunks of 256 -> so:
+// k_be_scatter 1M 82 -> 79 -> 74 us, 2.1M 146 -> 123 -> 110; k_admm_op32
+// 2.1M 119 -> 109 -> 108 (with the launches past the end of a solve).
+constexpr int kSumThreads = 320, kSumChunk = 304;
+constexpr int kSumStride = kSumChunk + 1;  // of the rows
+union CellSumsData {
+  double row[12 * kSumStride];               // D (row-major), then the fractions
+  double contrib[3][kCells * kAB * 3];
+};
+struct CellSums {
+  CellSumsData u;
+  uint32_t coff[kCells + 1];    // the cells' runs, in the sort's order of cells
+  int order[kCells];            // the cells by falling number of particles
+};
+static_assert(kCells * kAB <= kSumThreads && kSumChunk <= kSumThreads && kTileNodes <= kSumThreads,
+              "a thread per task, particle and node");
+// cell (bits x, y y, z z from the lowest) in the sort's order of cells
+__device__ __forceinline__ int sum_cell_slot(int e) { return ((e & 1) << 4) | (((e >> 1) & 3) << 2) | (e >> 3); }
+// the caller synchronises before the first chunk
+__device__ __forceinline__ void cell_sums_begin(CellSums& cs, const uint32_t* cell_off, uint32_t n)
+{
+  const int tid = threadIdx.x;
+  if (tid >= 64) return;
+  const uint32_t c = tid < kCells ? cell_off[tid] : n;
+  if (tid <= kCells) cs.coff[tid] = c;
+  const uint32_t next = (uint32_t)__shfl_down((int)c, 1, 64);
+  const int cnt = (int)(next - c);
+  int rank = 0;
+#pragma unroll
+  for (int k = 0; k < kCells; ++k) {
+    const int ck = __builtin_amdgcn_readlane(cnt, k);
+    rank += (ck > cnt || (ck == cnt && k < tid)) ? 1 : 0;
+  }
+  if (tid < kCells) cs.order[rank] = ((tid >> 4) & 1) | (((tid >> 2) & 3) << 1) | ((tid & 3) << 3);
+}
+__device__ __forceinline__ void cell_sums_put(CellSums& cs, int p, const double D[3][3], const double f[3])
+{
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) cs.u.row[(3 * r + c) * kSumStride + p] = D[r][c];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) cs.u.row[(9 + d) * kSumStride + p] = f[d];
+}
+// this thread's task's sums over the chunk [c0, c0 + count) of the group,
+// added to acc[c][r]; between barriers
+__device__ __forceinline__ void cell_sums_chunk(const CellSums& cs, uint32_t c0, uint32_t count, double acc[3][3])
+{
+  const int rk = (int)threadIdx.x / kAB, ab = (int)threadIdx.x - rk * kAB;
+  if (rk >= kCells) return;
+  const int e = cs.order[rk], a = ab / 3, b = ab - 3 * a;
+  const uint32_t b0 = cs.coff[sum_cell_slot(e)], b1 = cs.coff[sum_cell_slot(e) + 1];
+  const uint32_t jb = b0 > c0 ? b0 - c0 : 0u;
+  const uint32_t je = b1 > c0 ? (b1 - c0 < count ? b1 - c0 : count) : 0u;
+  const double sx = 1.5 - 0.5 * a, kx = a == 1 ? -1.0 : 0.5, ex = a == 1 ? 0.75 : 0.0;
+  const double sy = 1.5 - 0.5 * b, ky = b == 1 ? -1.0 : 0.5, ey = b == 1 ? 0.75 : 0.0;
+  for (uint32_t j = jb; j < je; ++j) {
+    const double* q = cs.u.row + j;
+    const double tx = q[9 * kSumStride] - sx, ty = q[10 * kSumStride] - sy, f2 = q[11 * kSumStride];
+    const double hx = kx * tx, hy = ky * ty;
+    const double wa = fma(hx, tx, ex), wb = fma(hy, ty, ey);
+    const double x0 = (hx + hx) * wb, x1 = wa * (hy + hy), x2 = wa * wb;
+    const double z0 = f2 - 1.5, z1 = f2 - 1.0, z2 = f2 - 0.5;
+    const double wc[3] = { 0.5 * z0 * z0, fma(-z1, z1, 0.75), 0.5 * z2 * z2 }, dc[3] = { z0, -2.0 * z1, z2 };
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      const double A = fma(q[(3 * r + 1) * kSumStride], x1, q[3 * r * kSumStride] * x0);
+      const double B = q[(3 * r + 2) * kSumStride] * x2;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) acc[c][r] = fma(B, dc[c], fma(A, wc[c], acc[c][r]));
+    }
+  }
+}
+// after a barrier: the group's sums into its staged tile
+__device__ __forceinline__ void cell_sums_store(CellSums& cs, const double acc[3][3], double* out)
+{
+  const int t = threadIdx.x;
+  const int rk = t / kAB, ab = t - rk * kAB;
+  if (rk < kCells) {
+    const uint32_t ts = kHvpTaskSlots.v[cs.order[rk] * kAB + ab];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int r = 0; r < 3; ++r) cs.u.contrib[r][(ts >> (10 * c)) & 1023u] = acc[c][r];
+  }
+  __syncthreads();
+  if (t >= kTileNodes) return;
+  const int tx = t / (kTileY * kTileZ), ty = (t / kTileZ) % kTileY, tz = t % kTileZ;
+  const int k0 = hvp_node_off(tx, ty, tz), nk = hvp_na(tx) * hvp_nb(ty) * hvp_nb(tz);
+  double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+  for (int k = k0; k < k0 + nk; ++k) {
+    a0 += cs.u.contrib[0][k];
+    a1 += cs.u.contrib[1][k];
+    a2 += cs.u.contrib[2][k];
+  }
+  out[t] = a0;
+  out[kTileNodes + t] = a1;
+  out[2 * kTileNodes + t] = a2;
+}
+
 // The Newton state of k_be_state<T, false> in three passes, so that the
 // SVD runs in a kernel of its own at a higher occupancy than the fused
 // kernel's one wave per SIMD:
@@ -788,110 +936,43 @@ __global__ __launch_bounds__(256) void k_be_svd(ParticlesView P, HvpCache<T> cac
       fb[(c * 3 + r) * CS + ks] = vol * (Pm[r][0] * Fn[c][0] + Pm[r][1] * Fn[c][1] + Pm[r][2] * Fn[c][2]);
 }
 
-__global__ __launch_bounds__(256) void k_be_scatter(ParticlesView P, const uint32_t* __restrict__ order,
+__global__ __launch_bounds__(kSumThreads) void k_be_scatter(ParticlesView P, const uint32_t* __restrict__ order,
                                                     const uint32_t* __restrict__ group_start,
-                                                    const uint32_t* __restrict__ group_page, int64_t cstride,
+                                                    const uint32_t* __restrict__ cell_off, int64_t cstride,
                                                     double inv_dx, const double* __restrict__ fb,
                                                     double* __restrict__ stage)
 {
-  __shared__ double tile[4 * kImpStage];
+  __shared__ CellSums cs;
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;
-  for (int k = tid; k < 4 * kImpStage; k += 256) tile[k] = 0.0;
   const uint32_t start = group_start[g];
   const uint32_t n = group_start[g + 1] - start;
-  uint32_t px, py, pz;
-  page_decode(group_page[g], px, py, pz);
-  const int ox = 2 * (int)px, oy = 4 * (int)py, oz = 4 * (int)pz;
-  __syncthreads();
-  double* wt = tile + (tid >> 6) * kImpStage;
-  const uint32_t perm = (uint32_t)((tid & 31) * 8 + (tid >> 5));
+  cell_sums_begin(cs, cell_off + 32 * (size_t)g, n);
   const int64_t S = P.stride;
-  for (uint32_t j0 = 0; j0 < n; j0 += 256) {
-    const uint32_t j = j0 + perm;
-    if (j >= n) continue;
-    const uint32_t i = order[start + j];
-    const uint32_t ks = start + j;
-    double w[3][3], dw[3][3];
-    int b[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const double xi = P.x[d * S + i] * inv_dx;
-      b[d] = int_floor(xi - 0.5);
-      bspline_frac(xi - (double)b[d], w[d], dw[d]);
-    }
-    const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
-    if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
-    const int t0 = (lx * kTileY + ly) * kTileZ + lz;
-    double vp[3][3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int r = 0; r < 3; ++r) vp[r][c] = fb[(c * 3 + r) * cstride + ks];
-    scatter_grad(wt, t0, w, dw, inv_dx, vp);
-  }
   __syncthreads();
-  double* out = stage + (size_t)g * kImpStage;
-  for (int k = tid; k < kImpStage; k += 256)
-    out[k] = tile[k] + tile[kImpStage + k] + tile[2 * kImpStage + k] + tile[3 * kImpStage + k];
-}
-
-constexpr int kAB = 9;        // (a, b) stencil offsets; c is handled inside a task
-
-// Node-major layout of the per-(cell, a, b, c) partial sums of the operator
-// apply: tile node t = (tx, ty, tz) owns n(t) = na(tx) nb(ty) nb(tz)
-// consecutive entries from off(t), one per stencil offset (a, b, c) whose
-// source cell t - (a, b, c) lies in the page, ordered by a, then b, then c.
-// Per axis: na = {1,2,2,1} (2 cells), nb = {1,2,3,3,2,1} (4 cells), with
-// prefix sums {0,1,3,5} and {0,1,3,6,9,11}; 864 entries in all.
-constexpr int hvp_na(int tx) { return (0x1221 >> (4 * tx)) & 15; }
-constexpr int hvp_nb(int ty) { return (0x123321 >> (4 * ty)) & 15; }
-constexpr int hvp_node_off(int tx, int ty, int tz)
-{
-  return ((0x5310 >> (4 * tx)) & 15) * 144 +
-         hvp_na(tx) * (((0xB96310 >> (4 * ty)) & 15) * 12 + hvp_nb(ty) * ((0xB96310 >> (4 * tz)) & 15));
-}
-constexpr int hvp_slot(int tx, int ty, int tz, int a, int b, int c)
-{
-  return hvp_node_off(tx, ty, tz) +
-         ((a - (tx > 1 ? tx - 1 : 0)) * hvp_nb(ty) + (b - (ty > 3 ? ty - 3 : 0))) * hvp_nb(tz) +
-         (c - (tz > 3 ? tz - 3 : 0));
-}
-
-// slots of task (cell e, a, b)'s three c offsets, 10 bits each
-struct HvpTaskSlots {
-  uint32_t v[kCells * kAB];
-};
-constexpr HvpTaskSlots hvp_task_slots()
-{
-  HvpTaskSlots t{};
-  for (int task = 0; task < kCells * kAB; ++task) {
-    const int e = task / kAB, a = (task % kAB) / 3, b = task % 3;
-    const int tx = (e & 1) + a, ty = ((e >> 1) & 3) + b, cz = (e >> 3) & 3;
-    uint32_t v = 0;
-    for (int c = 0; c < 3; ++c) v |= (uint32_t)hvp_slot(tx, ty, cz + c, a, b, c) << (10 * c);
-    t.v[task] = v;
-  }
-  return t;
-}
-// every entry of the layout belongs to exactly one (task, c)
-constexpr bool hvp_task_slots_valid()
-{
-  const HvpTaskSlots t = hvp_task_slots();
-  int hits[kCells * kAB * 3] = {};
-  for (int task = 0; task < kCells * kAB; ++task)
-    for (int c = 0; c < 3; ++c) {
-      const uint32_t k = (t.v[task] >> (10 * c)) & 1023u;
-      if (k >= (uint32_t)(kCells * kAB * 3)) return false;
-      ++hits[k];
+  double acc[3][3] = { { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0 } };
+  for (uint32_t c0 = 0; c0 < n; c0 += kSumChunk) {
+    const uint32_t count = n - c0 < (uint32_t)kSumChunk ? n - c0 : (uint32_t)kSumChunk;
+    if ((uint32_t)tid < count) {
+      const uint32_t ks = start + c0 + tid, i = order[ks];
+      double f[3], D[3][3];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double xi = P.x[d * S + i] * inv_dx;
+        f[d] = xi - (double)int_floor(xi - 0.5);
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int r = 0; r < 3; ++r) D[r][c] = inv_dx * fb[(c * 3 + r) * cstride + ks];
+      cell_sums_put(cs, tid, D, f);
     }
-  for (int k = 0; k < kCells * kAB * 3; ++k)
-    if (hits[k] != 1) return false;
-  return true;
+    __syncthreads();
+    cell_sums_chunk(cs, c0, count, acc);
+    __syncthreads();
+  }
+  cell_sums_store(cs, acc, stage + (size_t)g * kImpStage);
 }
-static_assert(hvp_task_slots_valid(), "node-major layout is a bijection");
-static_assert(hvp_task_slots().v[0] == (0u | (2u << 10) | (5u << 20)), "slots of task (cell 0, a 0, b 0)");
-__constant__ HvpTaskSlots kHvpTaskSlots = hvp_task_slots();
 
 // particles per chunk of the operator apply, and the waves per SIMD its LDS
 // allows (the register budget is held to it)
