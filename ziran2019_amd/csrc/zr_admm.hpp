@@ -35,6 +35,7 @@ struct AdmmParticles {
 struct AdmmNodes {
   double* vn;      // [3][cap]
   double* dv;      // [3][cap]
+  double* dvp;     // [3][cap] dv before the last collision update, where coll is set
   double* proj;    // [9][cap] collision projection
   int32_t* coll;   // [cap]
   double* diag;    // [cap]
@@ -421,7 +422,10 @@ __global__ __launch_bounds__(256) void k_admm_collide(uint32_t nn, const uint32_
       hit = 1;
       for (int i = 0; i < 3; ++i)
         for (int j = 0; j < 3; ++j) N.proj[(3 * i + j) * S + k] = P[i][j];
-      for (int d = 0; d < 3; ++d) N.dv[d * S + k] = vi[d] - N.vn[d * S + k];
+      for (int d = 0; d < 3; ++d) {
+        N.dvp[d * S + k] = N.dv[d * S + k];
+        N.dv[d * S + k] = vi[d] - N.vn[d * S + k];
+      }
     }
   }
   N.coll[k] = hit;
@@ -487,18 +491,34 @@ __device__ __forceinline__ void admm_residual_term(double k, const M3<double>& u
   }
 }
 
+// uStep (:638-671): y += k (F - Fn - dt G Fn), k = rho omega
+__device__ __forceinline__ void admm_dual(const double* F, double* y, int64_t S, uint32_t i, const double G[3][3],
+                                          const double Fn[3][3], double dt, double k)
+{
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const double t = F[(c * 3 + r) * S + i] - Fn[r][c] -
+                       dt * (G[r][0] * Fn[0][c] + G[r][1] * Fn[1][c] + G[r][2] * Fn[2][c]);
+      y[(c * 3 + r) * S + i] += k * t;
+    }
+}
+
 // FStepSolve's viscoelastic branch (:566-611): F2 = U diag(z) V^T with z the
 // Newton solution (at most 20 iterations) of
 // vol dE(zp(z)) + rho omega2^2 (z - sigma) = 0, sigma the singular values of
 // FFn - y2 / (rho omega2) + dt G FFn, G = grad(vn + dv); its term of the
-// global step's right side is added to D
+// global step's right side is added to D.  First y2's update (see
+// k_admm_flocal) with G0, where it is due.
 __device__ __forceinline__ void admm_visco_fstep(const AdmmParticles& A, int64_t S, uint32_t i, double vol,
-                                                 const double G[3][3], double dt, double rho, double local_tol,
-                                                 double D[3][3])
+                                                 const double G[3][3], bool due, const double G0[3][3], double dt,
+                                                 double rho, double local_tol, double D[3][3])
 {
   double Fv[3][3];
   load_F(A.fneq, S, i, Fv);
   const double om = A.om2[i];
+  if (due) admm_dual(A.F2, A.y2, S, i, G0, Fv, dt, rho * om);
   M3<double> fd, u, v;
 #pragma unroll
   for (int r = 0; r < 3; ++r)
@@ -688,13 +708,14 @@ __global__ __launch_bounds__(256) void k_admm_diag(uint32_t nn, const int32_t* _
 template <bool VISCO>
 __device__ __forceinline__ void admm_local_step(const ParticlesView& P, const AdmmParticles& A,
                                                 const int32_t* __restrict__ mat, const double* __restrict__ pparam,
-                                                const double* __restrict__ pstate, uint32_t i, double G[3][3], double dt,
-                                                double rho, double local_tol)
+                                                const double* __restrict__ pstate, uint32_t i, double G[3][3], bool due,
+                                                const double G0[3][3], double dt, double rho, double local_tol)
 {
   const int64_t S = P.stride;
   double Fn[3][3];
   load_F(P.F, S, i, Fn);
   const double om = A.om[i];
+  if (due) admm_dual(A.F, A.y, S, i, G0, Fn, dt, rho * om);
   M3<double> fd, u, v;
 #pragma unroll
   for (int r = 0; r < 3; ++r)
@@ -766,12 +787,19 @@ __device__ __forceinline__ void admm_local_step(const ParticlesView& P, const Ad
   asm volatile("" : "+v"(ir));
   load_F(P.F, S, ir, Fn);
   admm_residual_term(dt * coeff, u, z, sg, v, Fn, T);
-  if constexpr (VISCO) admm_visco_fstep(A, S, i, vol, G, dt, rho, local_tol, T);
+  if constexpr (VISCO) admm_visco_fstep(A, S, i, vol, G, due, G0, dt, rho, local_tol, T);
 #pragma unroll
   for (int r = 0; r < 3; ++r)
 #pragma unroll
     for (int c = 0; c < 3; ++c) G[r][c] = T[r][c];
 }
+
+// grad(vn + dv) before the collision update (9 rows, sorted order), where it
+// differs from the one after it
+struct AdmmBefore {
+  double* gs;
+  uint8_t* differs;
+};
 
 // FStepSolve (:507-615): F = U diag(z) V^T with z the Newton solution of
 // vol dE(proj(z)) + rho omega^2 (z - sigma) = 0, sigma the singular values
@@ -792,17 +820,43 @@ __device__ __forceinline__ void admm_local_step(const ParticlesView& P, const Ad
 // So the local step knows the term, and neither b nor K dv needs a pass with
 // a gather of its own (2.1M particles: 303 us and, in FP32, 166 us; now
 // k_be_scatter's).
+//
+// uStep (:638-671) of the iteration before is made here too (`due`), where y,
+// F and Fn are at hand: its gradient is that of dv before the collision
+// update, which k_admm_fgrad forms beside the other for the groups whose tile
+// the update changed.  A pass of its own (k_admm_ustep, left for the last
+// iteration) took 188 us at 2.1M beside k_admm_fgrad's 71 and
+// k_admm_flocal's 312; the two take 87 and 390.
 __global__ __launch_bounds__(256) void k_admm_fgrad(ParticlesView P, AdmmNodes N, const uint32_t* __restrict__ order,
                                                     const uint32_t* __restrict__ group_start,
                                                     const uint32_t* __restrict__ group_page,
                                                     const int32_t* __restrict__ group_nslot,
                                                     const double* __restrict__ gm, double inv_dx,
-                                                    double* __restrict__ gs)
+                                                    double* __restrict__ gs, AdmmBefore before, int due)
 {
-  __shared__ double tv[3 * kTileNodes];
+  __shared__ double tv[3 * kTileNodes], tb[3 * kTileNodes];
   __shared__ int32_t nslot[8];
+  __shared__ int hit;
   const uint32_t g = blockIdx.x;
+  if (threadIdx.x == 0) hit = 0;
   admm_tile3(group_nslot + 8 * (size_t)g, gm, N.vn, N.dv, N.stride, tv, nslot);
+  if (due) {  // the tile before the collision update, where that differs
+    for (int t = threadIdx.x; t < kTileNodes; t += 256) {
+      const int tx = t / (kTileY * kTileZ), ty = (t / kTileZ) % kTileY, tz = t % kTileZ;
+      const int32_t sl = nslot[((tx >> 1) << 2) | ((ty >> 2) << 1) | (tz >> 2)];
+      const int64_t node = (int64_t)sl * 32 + elem_of(tx, ty, tz);
+      const bool on = sl >= 0 && gm[node] != 0.0 && N.coll[node] != 0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double now = tv[d * kTileNodes + t];
+        const double was = on ? N.vn[d * N.stride + node] + N.dvp[d * N.stride + node] : now;
+        tb[d * kTileNodes + t] = was;
+        if (was != now) hit = 1;
+      }
+    }
+    __syncthreads();
+  }
+  const bool two = due && hit;
   const uint32_t start = group_start[g];
   const uint32_t n = group_start[g + 1] - start;
   uint32_t px, py, pz;
@@ -810,20 +864,29 @@ __global__ __launch_bounds__(256) void k_admm_fgrad(ParticlesView P, AdmmNodes N
   const int ox = 2 * (int)px, oy = 4 * (int)py, oz = 4 * (int)pz;
   const int64_t S = P.stride;
   for (uint32_t j = threadIdx.x; j < n; j += 256) {
-    const uint32_t i = order[start + j];
+    const uint32_t i = order[start + j], ks = start + j;
     const double xp[3] = { P.x[i], P.x[S + i], P.x[2 * S + i] };
     double w[3][3], dw[3][3];
     int b[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) b[d] = bspline_wdw(xp[d] * inv_dx, w[d], dw[d]);
     const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
+    if (due) before.differs[ks] = two ? 1 : 0;
     if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
+    const int t0 = (lx * kTileY + ly) * kTileZ + lz;
     double G[3][3];
-    grad_from_tile(tv, (lx * kTileY + ly) * kTileZ + lz, w, dw, inv_dx, G);
+    grad_from_tile(tv, t0, w, dw, inv_dx, G);
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int r = 0; r < 3; ++r) gs[(c * 3 + r) * S + start + j] = G[r][c];
+      for (int r = 0; r < 3; ++r) gs[(c * 3 + r) * S + ks] = G[r][c];
+    if (two) {
+      grad_from_tile(tb, t0, w, dw, inv_dx, G);
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int r = 0; r < 3; ++r) before.gs[(c * 3 + r) * S + ks] = G[r][c];
+    }
   }
 }
 
@@ -833,17 +896,22 @@ __global__ __launch_bounds__(256) void k_admm_flocal(ParticlesView P, AdmmPartic
                                                      const double* __restrict__ pparam,
                                                      const double* __restrict__ pstate,
                                                      const uint32_t* __restrict__ order, uint32_t n,
-                                                     double* __restrict__ gs, double dt, double rho, double local_tol)
+                                                     double* __restrict__ gs, AdmmBefore before, int due, double dt,
+                                                     double rho, double local_tol)
 {
   const uint32_t ks = blockIdx.x * 256u + threadIdx.x;
   if (ks >= n) return;
   const int64_t S = P.stride;
-  double G[3][3];
+  double G[3][3], G0[3][3];
+  const double* g0 = due && before.differs[ks] ? before.gs : gs;
 #pragma unroll
   for (int c = 0; c < 3; ++c)
 #pragma unroll
-    for (int r = 0; r < 3; ++r) G[r][c] = gs[(c * 3 + r) * S + ks];
-  admm_local_step<VISCO>(P, A, mat, pparam, pstate, order[ks], G, dt, rho, local_tol);
+    for (int r = 0; r < 3; ++r) {
+      G[r][c] = gs[(c * 3 + r) * S + ks];
+      G0[r][c] = g0[(c * 3 + r) * S + ks];
+    }
+  admm_local_step<VISCO>(P, A, mat, pparam, pstate, order[ks], G, due != 0, G0, dt, rho, local_tol);
 #pragma unroll
   for (int c = 0; c < 3; ++c)
 #pragma unroll
@@ -851,7 +919,9 @@ __global__ __launch_bounds__(256) void k_admm_flocal(ParticlesView P, AdmmPartic
 }
 
 // the global operator's particle term c_p (grad(x) Fn) Fn^T grad w in FP64,
-// c_p = rho omega^2 dt^2; VISCO adds the viscoelastic branch's with FFn
+// c_p = rho omega^2 dt^2; VISCO adds the viscoelastic branch's with FFn.
+// (Four waves per SIMD, with 2 to 6 registers in scratch, so that three blocks
+// fit a CU: 40k 9.7 us, against 13.2 with two.)
 template <bool VISCO>
 __global__ __launch_bounds__(kSumThreads, 4) void k_admm_op64(ParticlesView P, AdmmParticles A, AdmmNodes N,
                                                    const double* __restrict__ xvec,
@@ -1210,27 +1280,10 @@ __global__ __launch_bounds__(256) void k_admm_ustep(ParticlesView P, AdmmParticl
     double G[3][3], Fn[3][3];
     grad_from_tile(tv, (lx * kTileY + ly) * kTileZ + lz, w, dw, inv_dx, G);
     load_F(P.F, S, i, Fn);
-    const double om = A.om[i];
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const double t = A.F[(c * 3 + r) * S + i] - Fn[r][c] -
-                         dt * (G[r][0] * Fn[0][c] + G[r][1] * Fn[1][c] + G[r][2] * Fn[2][c]);
-        A.y[(c * 3 + r) * S + i] += rho * om * t;
-      }
+    admm_dual(A.F, A.y, S, i, G, Fn, dt, rho * A.om[i]);
     if constexpr (VISCO) {
-      double Fv[3][3];
-      load_F(A.fneq, S, i, Fv);
-      const double om2 = A.om2[i];
-#pragma unroll
-      for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const double t = A.F2[(c * 3 + r) * S + i] - Fv[r][c] -
-                           dt * (G[r][0] * Fv[0][c] + G[r][1] * Fv[1][c] + G[r][2] * Fv[2][c]);
-          A.y2[(c * 3 + r) * S + i] += rho * om2 * t;
-        }
+      load_F(A.fneq, S, i, Fn);
+      admm_dual(A.F2, A.y2, S, i, G, Fn, dt, rho * A.om2[i]);
     }
   }
 }

@@ -1622,6 +1622,9 @@ struct zr_engine {
   // rows of n floats), element codes, and seven FP32 Krylov vectors
   float* admm_c32 = nullptr;
   uint8_t* admm_cell32 = nullptr;
+  double* admm_before = nullptr;  // AdmmBefore
+  uint8_t* admm_differs = nullptr;
+  size_t admm_before_cap = 0;
   size_t admm_c32_cap = 0, admm_c32_rows = 0;
   float* admm_node32 = nullptr;
   size_t admm_node32_cap = 0;
@@ -2821,7 +2824,7 @@ int advance_recorded(zr_engine* e, double dt, zr_engine::StepRecord& r)
 }
 
 // ------------------------------------------------------------------- ADMM
-constexpr int kAdmmNodeRows = 3 + 3 + 9 + 1 + 9 + 3 + 9;  // vn dv proj diag q(3) z m(3)
+constexpr int kAdmmNodeRows = 3 + 3 + 3 + 9 + 1 + 9 + 3 + 9;  // vn dv dvp proj diag q(3) z m(3)
 
 // the global operator's particle term of x into the staged tiles: the FP64
 // scatter from the particle arrays, or the FP32 apply over the sorted cache
@@ -2926,10 +2929,10 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
   }
   const int64_t C = (int64_t)e->admm_cap;
   double* base = e->admm_node;
-  AdmmNodes Nd{ base, base + 3 * C, base + 6 * C, e->admm_coll, base + 15 * C, C };
-  double* qb[3] = { base + 16 * C, base + 19 * C, base + 22 * C };
-  double* zb = base + 25 * C;
-  double* mb[3] = { base + 28 * C, base + 31 * C, base + 34 * C };
+  AdmmNodes Nd{ base, base + 3 * C, base + 6 * C, base + 9 * C, e->admm_coll, base + 18 * C, C };
+  double* qb[3] = { base + 19 * C, base + 22 * C, base + 25 * C };
+  double* zb = base + 28 * C;
+  double* mb[3] = { base + 31 * C, base + 34 * C, base + 37 * C };
   double* pa = e->admm_p;
   AdmmParticles Ap{ pa, pa + 9 * N, pa + 18 * N, pa + 19 * N, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                     e->visc_d, e->visc_v };
@@ -3007,15 +3010,25 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
     ZR_HIP(e, hipMalloc(&e->be_fb, 9 * N * sizeof(double)));
     e->be_fb_cap = N;
   }
+  if (e->admm_before_cap < N) {
+    dfree(e->admm_before);
+    dfree(e->admm_differs);
+    e->admm_before_cap = 0;
+    ZR_HIP(e, hipMalloc(&e->admm_before, 9 * N * sizeof(double)));
+    ZR_HIP(e, hipMalloc(&e->admm_differs, N));
+    e->admm_before_cap = N;
+  }
+  const AdmmBefore before{ e->admm_before, e->admm_differs };
   const uint32_t npb = blocks_for((uint64_t)n, 256);
   int total_minres = 0;
   for (int tim = 0; tim < o->admm_iterations; ++tim) {
     k_admm_collide<<<nbn, 256, 0, s>>>(nn, e->slot_page, e->gm, Nd, dx, cs);
+    const int due = tim > 0;  // the dual update of the iteration before
     k_admm_fgrad<<<e->A, 256, 0, s>>>(P, Nd, e->order, e->group_start, e->group_page, e->group_nslot, e->gm, inv_dx,
-                                      e->be_fb);
+                                      e->be_fb, before, due);
     {
       auto k = visco ? k_admm_flocal<true> : k_admm_flocal<false>;
-      k<<<npb, 256, 0, s>>>(P, Ap, mat, e->pparam, e->pstate, e->order, (uint32_t)n, e->be_fb, dt, rho,
+      k<<<npb, 256, 0, s>>>(P, Ap, mat, e->pparam, e->pstate, e->order, (uint32_t)n, e->be_fb, before, due, dt, rho,
                             o->local_tolerance);
     }
     k_be_scatter<<<e->A, kSumThreads, 0, s>>>(P, e->order, e->group_start, e->cell_off, n, inv_dx, e->be_fb, e->stage);
@@ -3026,13 +3039,10 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
                    : admm_minres<double>(e, op, qb, zb, mb, o, nn, nbn, its);
     if (rc2) return rc2;
     total_minres += its;
-    if (visco)
-      k_admm_ustep<true><<<e->A, 256, 0, s>>>(P, Ap, Nd, e->order, e->group_start, e->group_page, e->group_nslot,
-                                              e->gm, dt, rho, inv_dx);
-    else
-      k_admm_ustep<false><<<e->A, 256, 0, s>>>(P, Ap, Nd, e->order, e->group_start, e->group_page, e->group_nslot,
-                                               e->gm, dt, rho, inv_dx);
-    ZR_LAUNCH_CHECK(e);
+  }
+  if (o->admm_iterations > 0) {  // the last iteration's dual update
+    auto k = visco ? k_admm_ustep<true> : k_admm_ustep<false>;
+    k<<<e->A, 256, 0, s>>>(P, Ap, Nd, e->order, e->group_start, e->group_page, e->group_nslot, e->gm, dt, rho, inv_dx);
   }
   k_admm_finish_nodes<<<nbn, 256, 0, s>>>(nn, e->gm, Nd, e->gvs);
   k_admm_lastdv<<<e->A, 256, 0, s>>>(P, Ap, Nd, e->order, e->group_start, e->group_page, e->group_nslot, e->gm, dt,
@@ -3574,7 +3584,7 @@ void zr_destroy(zr_engine* e)
   dfree(e->scan_tmp); dfree(e->cell_off); dfree(e->speed); dfree(e->dbase); dfree(e->ticket); dfree(e->slot_src);
   dfree(e->ivn); dfree(e->idv); dfree(e->ir); dfree(e->ix); dfree(e->irc); dfree(e->iq); dfree(e->ip); dfree(e->iap);
   dfree(e->partial); dfree(e->partial2); dfree(e->sc); dfree(e->ci); dfree(e->hvp_ctr); dfree(e->hvp_bounds); dfree(e->hvp_order); dfree(e->cell_order); dfree(e->jstage); dfree(e->pinv); dfree(e->collided); dfree(e->c64); dfree(e->c32); dfree(e->ccell);
-  dfree(e->pf_node); dfree(e->pf_partial); dfree(e->adj_grid); dfree(e->admm_node); dfree(e->admm_coll); dfree(e->act); dfree(e->act_scan); dfree(e->be_fb); dfree(e->admm_c32); dfree(e->admm_cell32); dfree(e->admm_node32);
+  dfree(e->pf_node); dfree(e->pf_partial); dfree(e->adj_grid); dfree(e->admm_node); dfree(e->admm_coll); dfree(e->act); dfree(e->act_scan); dfree(e->be_fb); dfree(e->admm_c32); dfree(e->admm_cell32); dfree(e->admm_node32); dfree(e->admm_before); dfree(e->admm_differs);
   dfree(e->fx); dfree(e->frc); dfree(e->fq); dfree(e->fp); dfree(e->fap);
   dfree(e->mr64); dfree(e->mr32);
   if (e->hspeed) (void)hipHostFree(e->hspeed);
