@@ -1007,10 +1007,9 @@ __global__ __launch_bounds__(256) void k_minres_init(uint32_t nn, const int32_t*
                                                      AdmmNodes N, double dt, double gx, double gy, double gz, T* q,
                                                      T* z, T* zero0, T* zero1, T* zero2, double* partial)
 {
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
   const int64_t S = N.stride;
   double acc = 0.0;
-  if (k < nn) {
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
     double r[3] = { 0.0, 0.0, 0.0 }, zz[3] = { 0.0, 0.0, 0.0 };
     const double m = gm[k];
     if (m != 0.0) {
@@ -1042,14 +1041,13 @@ template <class T>
 __global__ __launch_bounds__(256) void k_minres_apply(uint32_t nn, const int32_t* __restrict__ slot_src,
                                                       const double* __restrict__ stage,
                                                       const double* __restrict__ gm, AdmmNodes N,
-                                                      const T* __restrict__ z, T* q, const int32_t* ai,
+                                                      const T* __restrict__ z, T* q, const int32_t* ai, int it,
                                                       double* partial)
 {
-  if (ai[AI_DONE]) return;
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+  if (ai[minres_flag(it)]) return;
   const int64_t S = N.stride;
   double acc = 0.0;
-  if (k < nn) {
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
     double r[3] = { 0.0, 0.0, 0.0 };
     const double m = gm[k];
     if (m != 0.0) {
@@ -1069,14 +1067,15 @@ __global__ __launch_bounds__(256) void k_minres_apply(uint32_t nn, const int32_t
 template <class T>
 __global__ __launch_bounds__(256) void k_minres_lanczos(uint32_t nn, const double* __restrict__ gm, AdmmNodes N,
                                                         T* q, const T* __restrict__ qk, const T* __restrict__ qkm1,
-                                                        T* z, const double* sc, const int32_t* ai, double* partial)
+                                                        T* z, const double* __restrict__ apartial, double* sc,
+                                                        const int32_t* ai, int it, double* partial)
 {
-  if (ai[AI_DONE]) return;
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+  if (ai[minres_flag(it)]) return;
+  const double alpha = minres_alpha(apartial, gridDim.x, sc), beta = minres_state(sc, it)[AS_BETA];
   const int64_t S = N.stride;
   double acc = 0.0;
-  if (k < nn && gm[k] != 0.0) {
-    const double alpha = sc[AD_ALPHA], beta = sc[AD_BETA_K];
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
+    if (gm[k] == 0.0) continue;
     const double dg = N.diag[k];
     for (int d = 0; d < 3; ++d) {
       double v = (double)q[d * S + k];
@@ -1095,37 +1094,46 @@ __global__ __launch_bounds__(256) void k_minres_lanczos(uint32_t nn, const doubl
 template <class T>
 __global__ __launch_bounds__(256) void k_minres_update(uint32_t nn, const double* __restrict__ gm, AdmmNodes N,
                                                        T* q, T* z, T* mk, const T* __restrict__ mkm1,
-                                                       const T* __restrict__ mkm2, double* x, const double* sc,
-                                                       const int32_t* ai)
+                                                       const T* __restrict__ mkm2, double* x,
+                                                       const double* __restrict__ partial, double* sc, int32_t* ai,
+                                                       int it, int max_it, SolveMark mark)
 {
-  if (ai[AI_DONE + 2]) return;  // finished before this iteration's Givens step
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
-  if (k >= nn || gm[k] == 0.0) return;
+  if (ai[minres_flag(it)]) {
+    minres_pass(ai, it, mark);
+    return;
+  }
+  const MinresStep st = minres_givens(partial, gridDim.x, sc, ai, it, max_it, mark);
   const int64_t S = N.stride;
-  const double bk = sc[AD_BETA_KP1], gamma = sc[AD_GAMMA], delta = sc[AD_DELTA], eps = sc[AD_EPS], tk = sc[AD_TK];
-  for (int d = 0; d < 3; ++d) {
-    if (bk > 0.0) {
-      q[d * S + k] = (T)((double)q[d * S + k] / bk);
-      z[d * S + k] = (T)((double)z[d * S + k] / bk);
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
+    if (gm[k] == 0.0) continue;
+    for (int d = 0; d < 3; ++d) {
+      if (st.beta > 0.0) {
+        q[d * S + k] = (T)((double)q[d * S + k] / st.beta);
+        z[d * S + k] = (T)((double)z[d * S + k] / st.beta);
+      }
+      const T m = (T)(((double)mk[d * S + k] - st.delta * (double)mkm1[d * S + k] -
+                       st.eps * (double)mkm2[d * S + k]) / st.gamma);
+      mk[d * S + k] = m;
+      x[d * S + k] += st.tk * (double)m;
     }
-    const T m = (T)(((double)mk[d * S + k] - delta * (double)mkm1[d * S + k] - eps * (double)mkm2[d * S + k]) / gamma);
-    mk[d * S + k] = m;
-    x[d * S + k] += tk * (double)m;
   }
 }
 
-// the start vectors divided by beta_1 = |r0|_P (Minres.h:95-98)
+// beta_1 = |r0|_P from the start's partials; the start vectors divided by it
+// (Minres.h:95-98)
 template <class T>
 __global__ __launch_bounds__(256) void k_minres_scale(uint32_t nn, const double* __restrict__ gm, int64_t S, T* q,
-                                                      T* z, const double* sc, const int32_t* ai)
+                                                      T* z, const double* __restrict__ partial, double* sc,
+                                                      int32_t* ai, double tol, double rel, int max_it)
 {
-  if (ai[AI_DONE]) return;
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
-  const double b = sc[AD_BETA_KP1];
-  if (k >= nn || gm[k] == 0.0 || !(b > 0.0)) return;
-  for (int d = 0; d < 3; ++d) {
-    q[d * S + k] = (T)((double)q[d * S + k] / b);
-    z[d * S + k] = (T)((double)z[d * S + k] / b);
+  double b;
+  if (minres_start(partial, gridDim.x, sc, ai, tol, rel, max_it, b) || !(b > 0.0)) return;
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
+    if (gm[k] == 0.0) continue;
+    for (int d = 0; d < 3; ++d) {
+      q[d * S + k] = (T)((double)q[d * S + k] / b);
+      z[d * S + k] = (T)((double)z[d * S + k] / b);
+    }
   }
 }
 

@@ -2442,6 +2442,7 @@ int ensure_scalars(zr_engine* e)
   if (!e->sc) {
     ZR_HIP(e, hipMalloc(&e->sc, SC_N * sizeof(double)));
     ZR_HIP(e, hipMalloc(&e->ci, CI_N * sizeof(int32_t)));
+    ZR_HIP(e, hipMalloc(&e->partial2, kCgBlocks * sizeof(double)));
     ZR_HIP(e, hipMalloc(&e->hvp_ctr, kHvpCounters * kHvpCounterStride * sizeof(uint32_t)));
     ZR_HIP(e, hipMemset(e->hvp_ctr, 0, kHvpCounters * kHvpCounterStride * sizeof(uint32_t)));
     ZR_HIP(e, hipMalloc(&e->hvp_bounds, 18 * sizeof(uint32_t)));
@@ -2837,38 +2838,39 @@ struct AdmmOp {
   double dt, rho, inv_dx;
 };
 
-void admm_apply(zr_engine* e, const AdmmOp& op, const float* x)
+// (gated by *done)
+void admm_apply(zr_engine* e, const AdmmOp& op, const float* x, const int32_t* done)
 {
   auto k = op.visco ? k_admm_op32<true> : k_admm_op32<false>;
   k<<<e->A, kSumThreads, 0, e->stream>>>(op.C, e->group_start, e->cell_off, e->group_nslot, e->gm, x, op.Nd.stride, e->stage,
-                                 (float)op.inv_dx, e->ci);
+                                 (float)op.inv_dx, done);
 }
-void admm_apply(zr_engine* e, const AdmmOp& op, const double* x)
+void admm_apply(zr_engine* e, const AdmmOp& op, const double* x, const int32_t* done)
 {
   auto k = op.visco ? k_admm_op64<true> : k_admm_op64<false>;
   k<<<e->A, kSumThreads, 0, e->stream>>>(op.P, op.Ap, op.Nd, x, e->order, e->group_start, e->cell_off, e->group_page,
-                                 e->group_nslot, e->gm, e->stage, op.dt, op.rho, op.inv_dx, e->ci);
+                                 e->group_nslot, e->gm, e->stage, op.dt, op.rho, op.inv_dx, done);
 }
 
 // Minres::solve (Minres.h:69-149) on the global system for dv (FP64), the
 // Krylov vectors in precision T (the seven vectors rotate by pointer)
 template <class T>
 int admm_minres(zr_engine* e, const AdmmOp& op, T* const qb[3], T* zb, T* const mb[3],
-                const zr_admm_opts* o, uint32_t nn, uint32_t nbn, int& iters)
+                const zr_admm_opts* o, uint32_t nn, int& iters)
 {
   hipStream_t s = e->stream;
   const AdmmNodes& Nd = op.Nd;
   const int64_t C = Nd.stride;
   T *q = qb[2], *qk = qb[1], *qkm1 = qb[0], *z = zb, *mk = mb[2], *mkm1 = mb[1], *mkm2 = mb[0];
-  k_minres_init<T><<<nbn, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, Nd, op.dt, e->cfg.gravity[0],
-                                       e->cfg.gravity[1], e->cfg.gravity[2], q, z, mk, mkm1, qk, e->partial);
-  k_minres_reduce<<<1, 256, 0, s>>>(e->partial, nbn, e->sc, e->ci, MR_INIT, o->global_tolerance, 0.5, 0,
-                                    o->minres_max_iterations, SolveMark{});
-  k_minres_scale<T><<<nbn, 256, 0, s>>>(nn, e->gm, C, q, z, e->sc, e->ci);
+  const uint32_t nb = std::min(blocks_for(nn, 256), kCgBlocks);
+  const int max_it = o->minres_max_iterations;
+  k_minres_init<T><<<nb, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, Nd, op.dt, e->cfg.gravity[0],
+                                      e->cfg.gravity[1], e->cfg.gravity[2], q, z, mk, mkm1, qk, e->partial);
+  k_minres_scale<T><<<nb, 256, 0, s>>>(nn, e->gm, C, q, z, e->partial, e->sc, e->ci, o->global_tolerance, 0.5, max_it);
   ZR_LAUNCH_CHECK(e);
   SolveWatch watch(e, kSolveAhead);
   int k = 0;
-  for (; k < o->minres_max_iterations && !watch.done; ++k) {
+  for (; k < max_it && !watch.done; ++k) {
     // m_{k-2} <- m_{k-1} <- m_k <- z; q_{k-1} <- q_k <- q_{k+1}
     T* t = mkm2;
     mkm2 = mkm1;
@@ -2879,14 +2881,11 @@ int admm_minres(zr_engine* e, const AdmmOp& op, T* const qb[3], T* zb, T* const 
     qkm1 = qk;
     qk = q;
     q = t;
-    admm_apply(e, op, mk);
-    k_minres_apply<T><<<nbn, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, Nd, mk, q, e->ci, e->partial);
-    k_minres_reduce<<<1, 256, 0, s>>>(e->partial, nbn, e->sc, e->ci, MR_ALPHA, 0.0, 0.0, k, o->minres_max_iterations,
-                                      SolveMark{});
-    k_minres_lanczos<T><<<nbn, 256, 0, s>>>(nn, e->gm, Nd, q, qk, qkm1, z, e->sc, e->ci, e->partial);
-    k_minres_reduce<<<1, 256, 0, s>>>(e->partial, nbn, e->sc, e->ci, MR_GIVENS, 0.0, 0.0, k,
-                                      o->minres_max_iterations, watch.mark(k));
-    k_minres_update<T><<<nbn, 256, 0, s>>>(nn, e->gm, Nd, q, z, mk, mkm1, mkm2, Nd.dv, e->sc, e->ci);
+    admm_apply(e, op, mk, e->ci + minres_flag(k));
+    k_minres_apply<T><<<nb, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, Nd, mk, q, e->ci, k, e->partial);
+    k_minres_lanczos<T><<<nb, 256, 0, s>>>(nn, e->gm, Nd, q, qk, qkm1, z, e->partial, e->sc, e->ci, k, e->partial2);
+    k_minres_update<T><<<nb, 256, 0, s>>>(nn, e->gm, Nd, q, z, mk, mkm1, mkm2, Nd.dv, e->partial2, e->sc, e->ci, k,
+                                          max_it, watch.mark(k));
     ZR_LAUNCH_CHECK(e);
     const int rc = watch.issued(k);
     if (rc) return rc;
@@ -3035,8 +3034,8 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
     // MINRES on the global system, warm-started from dv (Minres.h:69-149),
     // relative tolerance min(0.5, sqrt(max(1, 1e-6))) = 0.5 (:785-787)
     int its = 0;
-    int rc2 = fp32 ? admm_minres<float>(e, op, qb32, zb32, mb32, o, nn, nbn, its)
-                   : admm_minres<double>(e, op, qb, zb, mb, o, nn, nbn, its);
+    int rc2 = fp32 ? admm_minres<float>(e, op, qb32, zb32, mb32, o, nn, its)
+                   : admm_minres<double>(e, op, qb, zb, mb, o, nn, its);
     if (rc2) return rc2;
     total_minres += its;
   }
@@ -3079,7 +3078,6 @@ int ensure_implicit(zr_engine* e, int32_t prec)
     ZR_HIP(e, hipMalloc(&e->partial, nb * sizeof(double)));
     e->partial_cap = nb;
   }
-  if (!e->partial2) ZR_HIP(e, hipMalloc(&e->partial2, kCgBlocks * sizeof(double)));
   int rc = ensure_scalars(e);
   if (rc) return rc;
   const size_t n = (size_t)(e->n > 0 ? e->n : 1);
@@ -3320,11 +3318,10 @@ int be_minres(zr_engine* e, double rel, const zr_implicit_opts* o, int& iters)
   T *mk = ex, *mkm1 = ex + vs, *mkm2 = ex + 2 * vs;
   const NodeVec<T> pinv = nvT(e, e->jacobi ? reinterpret_cast<T*>(e->pinv) : (T*)nullptr);
   const int max_it = o->cg_max_iterations;
-  k_imr_init<T><<<nb, 256, 0, s>>>(nn, e->gm, nv(e, e->ir), nvT(e, V::x(e)), nvT(e, qkp1), nvT(e, z), nvT(e, qk),
-                                   nvT(e, mk), nvT(e, mkm1), pinv, e->partial);
-  k_minres_reduce<<<1, 256, 0, s>>>(e->partial, nb, e->sc, e->ci, MR_INIT, o->cg_tolerance, rel, 0, max_it,
-                                SolveMark{});
-  k_imr_scale<T><<<nb, 256, 0, s>>>(nn, e->gm, nvT(e, qkp1), nvT(e, z), e->sc, e->ci);
+  k_imr_init<T><<<ncg, 256, 0, s>>>(nn, e->gm, nv(e, e->ir), nvT(e, V::x(e)), nvT(e, qkp1), nvT(e, z), nvT(e, qk),
+                                    nvT(e, mk), nvT(e, mkm1), pinv, e->partial);
+  k_imr_scale<T><<<ncg, 256, 0, s>>>(nn, e->gm, nvT(e, qkp1), nvT(e, z), e->partial, e->sc, e->ci, o->cg_tolerance, rel,
+                                     max_it);
   ZR_LAUNCH_CHECK(e);
   SolveWatch watch(e, solve_ahead(o));
   int k = 0;
@@ -3339,14 +3336,12 @@ int be_minres(zr_engine* e, double rel, const zr_implicit_opts* o, int& iters)
     qk = qkp1;
     qkp1 = t;
     // q_{k+1} = P A m_k with the partials of alpha = m_k . q_{k+1}
-    int rc = be_apply<T>(e, nullptr, mk, qkp1, 1, e->ci, 0);
+    int rc = be_apply<T>(e, nullptr, mk, qkp1, 1, e->ci + minres_flag(k), 0);
     if (rc) return rc;
-    k_minres_reduce<<<1, 256, 0, s>>>(e->partial, ncg, e->sc, e->ci, MR_ALPHA, 0.0, 0.0, k, max_it, SolveMark{});
-    k_imr_lanczos<T><<<nb, 256, 0, s>>>(nn, e->gm, nvT(e, qkp1), nvT(e, qk), nvT(e, qkm1), nvT(e, z), pinv, e->sc,
-                                        e->ci, e->partial);
-    k_minres_reduce<<<1, 256, 0, s>>>(e->partial, nb, e->sc, e->ci, MR_GIVENS, 0.0, 0.0, k, max_it, watch.mark(k));
-    k_imr_update<T><<<nb, 256, 0, s>>>(nn, e->gm, nvT(e, qkp1), nvT(e, z), nvT(e, mk), nvT(e, mkm1),
-                                       nvT(e, mkm2), nvT(e, V::x(e)), e->sc, e->ci);
+    k_imr_lanczos<T><<<ncg, 256, 0, s>>>(nn, e->gm, nvT(e, qkp1), nvT(e, qk), nvT(e, qkm1), nvT(e, z), pinv, e->partial,
+                                         e->sc, e->ci, k, e->partial2);
+    k_imr_update<T><<<ncg, 256, 0, s>>>(nn, e->gm, nvT(e, qkp1), nvT(e, z), nvT(e, mk), nvT(e, mkm1), nvT(e, mkm2),
+                                        nvT(e, V::x(e)), e->partial2, e->sc, e->ci, k, max_it, watch.mark(k));
     ZR_LAUNCH_CHECK(e);
     rc = watch.issued(k);
     if (rc) return rc;

@@ -1,26 +1,37 @@
 // zr_minres.hpp -- Minres::solve (Lib/Ziran/Math/Linear/Minres.h:69-178) on
 // the device: the scalar recurrences (Lanczos alpha / beta, the Givens QR of
-// the tridiagonal, the residual estimate and the termination test) run in one
-// thread after an ordered block reduction, so the host only polls a flag.
-// Used by the ADMM global step and by the implicit Newton step.  Included by
-// zr_engine.hip inside its anonymous namespace after zr_implicit.hpp.
+// the tridiagonal, the residual estimate and the termination test) run in
+// every block of the node kernel that needs them, from the block partials of
+// the kernel before, so the host only watches a mark.  Used by the ADMM global
+// step and by the implicit Newton step.  Included by zr_engine.hip inside its
+// anonymous namespace after zr_implicit.hpp.
+//
+// An iteration is four launches: operator apply, A z with the partials of
+// alpha, the Lanczos step with those of beta, and the update.  One-block
+// kernels for the two sums and the scalars took 2.2 to 4.7 us each, with the
+// gaps to their neighbours a third of an iteration of 20k particles
+// (frames: 40k ADMM 11.6 -> 9.6 ms, 20k implicit
+// 9.2 -> 8.7).
 
-// device scalars (double) and flags (int32) of a MINRES solve
+// Device scalars (double) and flags (int32) of a MINRES solve.  The state
+// that an iteration hands to the next is kept twice, in turn, so that the
+// blocks of the update read one copy while block 0 writes the other.
 enum {
-  AD_RES = 0,      // MINRES residual (preconditioned norm)
-  AD_LTOL = 1,     // local tolerance
-  AD_ALPHA = 2,
-  AD_BETA_K = 3,
-  AD_BETA_KP1 = 4,
-  AD_GAMMA = 5,
-  AD_DELTA = 6,
-  AD_EPS = 7,
-  AD_TK = 8,
-  AD_LT0 = 9,      // last two Givens-transformed rhs components
-  AD_LT1 = 10,
-  AD_GK_C = 11, AD_GK_S = 12, AD_GKM1_C = 13, AD_GKM1_S = 14,
+  AD_LTOL = 0,     // local tolerance
+  AD_ALPHA = 1,
+  AD_STATE = 2,    // two of:
+  AS_BETA = 0,     // beta_{k+1}
+  AS_LT0 = 1,      // the last Givens-transformed right-hand side component
+  AS_GK_C = 2, AS_GK_S = 3, AS_GKM1_C = 4, AS_GKM1_S = 5,
+  AS_N = 6,
 };
-enum { AI_DONE = 0, AI_ITERS = 1, AI_N = 4 };
+static_assert(AD_STATE + 2 * AS_N <= SC_N, "the solvers' scalars");
+// whether the solve had ended before iteration k, at minres_flag(k)
+enum { AI_DONE = 0, AI_ITERS = 1 };
+constexpr int minres_flag(int k) { return AI_DONE + 2 * (k & 1); }
+static_assert(minres_flag(1) < CI_N, "the solvers' flags");
+
+__device__ __forceinline__ double* minres_state(double* sc, int k) { return sc + AD_STATE + AS_N * (k & 1); }
 
 __device__ __forceinline__ void g2_rot(double c, double s, double v[2])
 {
@@ -29,81 +40,91 @@ __device__ __forceinline__ void g2_rot(double c, double s, double v[2])
   v[1] = s * t1 + c * t2;
 }
 
-enum { MR_INIT = 0, MR_ALPHA = 1, MR_GIVENS = 2 };
-
-// the MINRES scalar logic (Minres.h:75-178) in one thread after an ordered sum
-__global__ __launch_bounds__(256) void k_minres_reduce(const double* __restrict__ partial, uint32_t nb, double* sc,
-                                                       int32_t* ai, int mode, double tol, double rel, int it,
-                                                       int max_it, SolveMark mark)
+// the start (Minres.h:89-101) from the partials of z . q: beta_1 = |r0|_P on
+// every thread and whether the solve ends there
+__device__ __forceinline__ bool minres_start(const double* partial, uint32_t nb, double* sc, int32_t* ai, double tol,
+                                             double rel, int max_it, double& beta)
 {
-  __shared__ double smem[4];
-  const int32_t ended = mode != MR_INIT ? ai[AI_DONE] : 0;
-  // the update of this iteration still runs when the convergence flag is
-  // raised by its Givens step
-  if (mode == MR_ALPHA && threadIdx.x == 0) ai[AI_DONE + 2] = ended;
-  if (ended) {
-    if (threadIdx.x == 0) mark_solve(mark, ai[AI_ITERS], 1);
-    return;
-  }
-  const double acc = thread_partials256(partial, nb);
-  const double v = block_sum256(acc, smem);
-  if (threadIdx.x != 0) return;
-  if (mode == MR_INIT) {
-    const double res = sqrt(v);
-    sc[AD_RES] = res;
-    sc[AD_BETA_KP1] = res;
-    const double lt = rel * res < tol ? rel * res : tol;
+  __shared__ double red[5];
+  beta = sqrt(block_total256(partial, nb, red));
+  const double lt = rel * beta < tol ? rel * beta : tol;
+  const bool done = beta < lt || max_it <= 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    double* st = minres_state(sc, 0);
     sc[AD_LTOL] = lt;
-    sc[AD_LT0] = res;
-    sc[AD_LT1] = 0.0;
-    sc[AD_GK_C] = 1.0;
-    sc[AD_GK_S] = 0.0;
-    sc[AD_GKM1_C] = 1.0;
-    sc[AD_GKM1_S] = 0.0;
+    st[AS_BETA] = beta;
+    st[AS_LT0] = beta;
+    st[AS_GK_C] = st[AS_GKM1_C] = 1.0;
+    st[AS_GK_S] = st[AS_GKM1_S] = 0.0;
     ai[AI_ITERS] = 0;
-    ai[AI_DONE] = res < lt || max_it <= 0 ? 1 : 0;
-    ai[AI_DONE + 2] = ai[AI_DONE];
-  } else if (mode == MR_ALPHA) {
-    sc[AD_ALPHA] = v;
-    sc[AD_BETA_K] = sc[AD_BETA_KP1];  // (an iteration's first step over the scalars)
-  } else {
-    const double bb = v > 0.0 ? v : 0.0;
-    const double beta_kp1 = sqrt(bb);
-    sc[AD_BETA_KP1] = beta_kp1;
-    // applyAllPreviousGivensRotationsAndDetermineNewGivens
-    const double gkm2_c = sc[AD_GKM1_C], gkm2_s = sc[AD_GKM1_S];
-    const double gkm1_c = sc[AD_GK_C], gkm1_s = sc[AD_GK_S];
-    double ek[2] = { 0.0, sc[AD_BETA_K] };
-    g2_rot(gkm2_c, gkm2_s, ek);
-    double dk[2] = { ek[1], sc[AD_ALPHA] };
-    g2_rot(gkm1_c, gkm1_s, dk);
-    double tv[2] = { dk[1], beta_kp1 };
-    double c = 1.0, s = 0.0;  // GivensRotation::compute (Givens.h:56-62)
-    const double d = sqrt(tv[0] * tv[0] + tv[1] * tv[1]);
-    if (d) {
-      const double t = 1.0 / d;
-      c = tv[0] * t;
-      s = -tv[1] * t;
-    }
-    g2_rot(c, s, tv);
-    double lt[2] = { sc[AD_LT0], sc[AD_LT1] };
-    g2_rot(c, s, lt);
-    sc[AD_EPS] = ek[0];
-    sc[AD_DELTA] = dk[0];
-    sc[AD_GAMMA] = tv[0];
-    sc[AD_TK] = lt[0];
-    sc[AD_LT0] = lt[1];
-    sc[AD_LT1] = 0.0;
-    sc[AD_GKM1_C] = gkm1_c;
-    sc[AD_GKM1_S] = gkm1_s;
-    sc[AD_GK_C] = c;
-    sc[AD_GK_S] = s;
+    ai[minres_flag(0)] = ai[minres_flag(1)] = done ? 1 : 0;
+  }
+  return done;
+}
+
+// the sum alpha of iteration k on every thread
+__device__ __forceinline__ double minres_alpha(const double* partial, uint32_t nb, double* sc)
+{
+  __shared__ double red[5];
+  const double alpha = block_total256(partial, nb, red);
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc[AD_ALPHA] = alpha;
+  return alpha;
+}
+
+// applyAllPreviousGivensRotationsAndDetermineNewGivens and the termination
+// test of iteration k (Minres.h:131-178); block 0 records the state
+struct MinresStep {
+  double beta, gamma, delta, eps, tk;
+};
+__device__ __forceinline__ MinresStep minres_givens(const double* partial, uint32_t nb, double* sc, int32_t* ai, int k,
+                                                    int max_it, SolveMark mark)
+{
+  __shared__ double red[5];
+  const double v = block_total256(partial, nb, red);
+  const double* st = minres_state(sc, k);
+  MinresStep m;
+  m.beta = sqrt(v > 0.0 ? v : 0.0);
+  double ek[2] = { 0.0, st[AS_BETA] };
+  g2_rot(st[AS_GKM1_C], st[AS_GKM1_S], ek);
+  double dk[2] = { ek[1], sc[AD_ALPHA] };
+  g2_rot(st[AS_GK_C], st[AS_GK_S], dk);
+  double tv[2] = { dk[1], m.beta };
+  double c = 1.0, s = 0.0;  // GivensRotation::compute (Givens.h:56-62)
+  const double d = sqrt(tv[0] * tv[0] + tv[1] * tv[1]);
+  if (d) {
+    const double t = 1.0 / d;
+    c = tv[0] * t;
+    s = -tv[1] * t;
+  }
+  g2_rot(c, s, tv);
+  double lt[2] = { st[AS_LT0], 0.0 };
+  g2_rot(c, s, lt);
+  m.eps = ek[0];
+  m.delta = dk[0];
+  m.gamma = tv[0];
+  m.tk = lt[0];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    double* nx = minres_state(sc, k + 1);
+    nx[AS_BETA] = m.beta;
+    nx[AS_LT0] = lt[1];
+    nx[AS_GKM1_C] = st[AS_GK_C];
+    nx[AS_GKM1_S] = st[AS_GK_S];
+    nx[AS_GK_C] = c;
+    nx[AS_GK_S] = s;
     const double res = lt[1] < 0.0 ? -lt[1] : lt[1];
-    sc[AD_RES] = res;
-    ai[AI_ITERS] = it + 1;
-    const bool done = res < sc[AD_LTOL] || it + 1 >= max_it;
-    if (done) ai[AI_DONE] = 1;
-    mark_solve(mark, it + 1, done);
+    const bool done = res < sc[AD_LTOL] || k + 1 >= max_it;
+    ai[AI_ITERS] = k + 1;
+    if (done) ai[minres_flag(k + 1)] = 1;
+    mark_solve(mark, k + 1, done);
+  }
+  return m;
+}
+// what the update of iteration k does past the end of a solve
+__device__ __forceinline__ void minres_pass(int32_t* ai, int k, SolveMark mark)
+{
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    ai[minres_flag(k + 1)] = 1;
+    mark_solve(mark, ai[AI_ITERS], 1);
   }
 }
 
@@ -121,9 +142,8 @@ __global__ __launch_bounds__(256) void k_imr_init(uint32_t nn, const double* __r
                                                   NodeVec<T> zero1, NodeVec<T> zero2, NodeVec<T> pinv,
                                                   double* __restrict__ partial)
 {
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
   double contrib = 0.0;
-  if (k < nn) {
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
     const double m = gm[k];
     for (int d = 0; d < 3; ++d) {
       const T qv = (T)b(d, k);
@@ -140,18 +160,21 @@ __global__ __launch_bounds__(256) void k_imr_init(uint32_t nn, const double* __r
   block_partial(contrib, partial);
 }
 
-// the start vectors divided by beta_1 (Minres.h:95-98)
+// beta_1 from the start's partials; the start vectors divided by it
+// (Minres.h:95-98)
 template <class T>
 __global__ __launch_bounds__(256) void k_imr_scale(uint32_t nn, const double* __restrict__ gm, NodeVec<T> q,
-                                                   NodeVec<T> z, const double* sc, const int32_t* ai)
+                                                   NodeVec<T> z, const double* __restrict__ partial, double* sc,
+                                                   int32_t* ai, double tol, double rel, int max_it)
 {
-  if (ai[AI_DONE]) return;
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
-  const double b = sc[AD_BETA_KP1];
-  if (k >= nn || gm[k] == 0.0 || !(b > 0.0)) return;
-  for (int d = 0; d < 3; ++d) {
-    q(d, k) /= (T)b;
-    z(d, k) /= (T)b;
+  double b;
+  if (minres_start(partial, gridDim.x, sc, ai, tol, rel, max_it, b) || !(b > 0.0)) return;
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
+    if (gm[k] == 0.0) continue;
+    for (int d = 0; d < 3; ++d) {
+      q(d, k) /= (T)b;
+      z(d, k) /= (T)b;
+    }
   }
 }
 
@@ -160,24 +183,23 @@ __global__ __launch_bounds__(256) void k_imr_scale(uint32_t nn, const double* __
 template <class T>
 __global__ __launch_bounds__(256) void k_imr_lanczos(uint32_t nn, const double* __restrict__ gm, NodeVec<T> q,
                                                      NodeVec<T> qk, NodeVec<T> qkm1, NodeVec<T> z, NodeVec<T> pinv,
-                                                     const double* sc, const int32_t* ai, double* partial)
+                                                     const double* __restrict__ apartial, double* sc,
+                                                     const int32_t* ai, int it, double* partial)
 {
-  if (ai[AI_DONE]) return;
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+  if (ai[minres_flag(it)]) return;
+  const T alpha = (T)minres_alpha(apartial, gridDim.x, sc), beta = (T)minres_state(sc, it)[AS_BETA];
   double contrib = 0.0;
-  if (k < nn) {
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
     const double m = gm[k];
-    if (m != 0.0) {
-      const T alpha = (T)sc[AD_ALPHA], beta = (T)sc[AD_BETA_K];
-      for (int d = 0; d < 3; ++d) {
-        T v = q(d, k);
-        v -= alpha * qk(d, k);
-        v -= beta * qkm1(d, k);
-        q(d, k) = v;
-        const T zv = pinv.p ? v * pinv(d, k) : v / (T)m;
-        z(d, k) = zv;
-        contrib += (double)zv * (double)v;
-      }
+    if (m == 0.0) continue;
+    for (int d = 0; d < 3; ++d) {
+      T v = q(d, k);
+      v -= alpha * qk(d, k);
+      v -= beta * qkm1(d, k);
+      q(d, k) = v;
+      const T zv = pinv.p ? v * pinv(d, k) : v / (T)m;
+      z(d, k) = zv;
+      contrib += (double)zv * (double)v;
     }
   }
   block_partial(contrib, partial);
@@ -188,20 +210,25 @@ __global__ __launch_bounds__(256) void k_imr_lanczos(uint32_t nn, const double* 
 template <class T>
 __global__ __launch_bounds__(256) void k_imr_update(uint32_t nn, const double* __restrict__ gm, NodeVec<T> q,
                                                     NodeVec<T> z, NodeVec<T> mk, NodeVec<T> mkm1, NodeVec<T> mkm2,
-                                                    NodeVec<T> x, const double* sc, const int32_t* ai)
+                                                    NodeVec<T> x, const double* __restrict__ partial, double* sc,
+                                                    int32_t* ai, int it, int max_it, SolveMark mark)
 {
-  if (ai[AI_DONE + 2]) return;  // finished before this iteration's Givens step
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
-  if (k >= nn || gm[k] == 0.0) return;
-  const double bk = sc[AD_BETA_KP1];
-  const T gamma = (T)sc[AD_GAMMA], delta = (T)sc[AD_DELTA], eps = (T)sc[AD_EPS], tk = (T)sc[AD_TK];
-  for (int d = 0; d < 3; ++d) {
-    if (bk > 0.0) {
-      q(d, k) /= (T)bk;
-      z(d, k) /= (T)bk;
+  if (ai[minres_flag(it)]) {
+    minres_pass(ai, it, mark);
+    return;
+  }
+  const MinresStep st = minres_givens(partial, gridDim.x, sc, ai, it, max_it, mark);
+  const T gamma = (T)st.gamma, delta = (T)st.delta, eps = (T)st.eps, tk = (T)st.tk;
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
+    if (gm[k] == 0.0) continue;
+    for (int d = 0; d < 3; ++d) {
+      if (st.beta > 0.0) {
+        q(d, k) /= (T)st.beta;
+        z(d, k) /= (T)st.beta;
+      }
+      const T m = (mk(d, k) - delta * mkm1(d, k) - eps * mkm2(d, k)) / gamma;
+      mk(d, k) = m;
+      x(d, k) += tk * m;
     }
-    const T m = (mk(d, k) - delta * mkm1(d, k) - eps * mkm2(d, k)) / gamma;
-    mk(d, k) = m;
-    x(d, k) += tk * m;
   }
 }
