@@ -936,7 +936,7 @@ __global__ __launch_bounds__(kSumThreads, 4) void k_admm_op64(ParticlesView P, A
   if (ai[AI_DONE]) return;
   __shared__ double tv[3 * kTileNodes];
   __shared__ int32_t nslot[8];
-  __shared__ CellSums cs;
+  __shared__ CellSums<3, true> cs;
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;
   const uint32_t start = group_start[g];
@@ -975,7 +975,7 @@ __global__ __launch_bounds__(kSumThreads, 4) void k_admm_op64(ParticlesView P, A
           add_operator_term(k * om2 * om2, G, Fn, D);
         }
       }
-      cell_sums_put(cs, tid, D, f);
+      cell_sums_put(cs, tid, &D[0][0], f);
     }
     __syncthreads();
     cell_sums_chunk(cs, c0, count, acc);
@@ -1192,7 +1192,7 @@ __global__ __launch_bounds__(kSumThreads, 5) void k_admm_op32(AdmmCache32 C, con
   if (ai[AI_DONE]) return;
   __shared__ float tv[3 * kTileNodes];
   __shared__ int32_t nslot[8];
-  __shared__ CellSums cs;
+  __shared__ CellSums<3, true> cs;
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;
   const uint32_t start = group_start[g];
@@ -1245,7 +1245,7 @@ __global__ __launch_bounds__(kSumThreads, 5) void k_admm_op32(AdmmCache32 C, con
         for (int c = 0; c < 3; ++c) D64[r][c] = (double)(inv_dx * D[r][c]);
         f64[r] = (double)f[r];
       }
-      cell_sums_put(cs, tid, D64, f64);
+      cell_sums_put(cs, tid, &D64[0][0], f64);
     }
     __syncthreads();
     cell_sums_chunk(cs, c0, count, acc);

@@ -18,15 +18,14 @@
 
 enum {
   PF_RHO = 8,      // mr . r of the current iteration
-  PF_SQ = 9,       // s . q
-  PF_ALPHA = 10,
   PF_BETA = 11,    // rho / rho_old for the next direction
   PF_NORM = 12,    // |r|
   PF_REL = 13,     // relative tolerance, cg_relative |r0|
 };
 enum { CI_PF_IT = 2 };
 
-constexpr int kPfFields = 4;  // sum w, sum c w, sum vol w, sum D_p w
+// sum vol w, sum D_p w; in the parabolic form also sum w, sum c w
+constexpr int pf_fields(bool parabolic) { return parabolic ? 4 : 2; }
 
 struct PfParticles {
   double* c;
@@ -53,113 +52,105 @@ __device__ __forceinline__ double det_soa(const double* F, int64_t S, uint32_t i
   return f00 * (f11 * f22 - f21 * f12) - f01 * (f10 * f22 - f20 * f12) + f02 * (f10 * f21 - f20 * f11);
 }
 
-// phaseP2G (:209-257) with the rhs and diagonal sums (:303-325, :405-437):
-// per-wave LDS tiles, staged per group like P2G
-__global__ __launch_bounds__(256) void k_pf_p2g(ParticlesView P, PfParticles pf, PfScalars ps,
-                                                const uint32_t* __restrict__ order,
-                                                const uint32_t* __restrict__ group_start,
-                                                const uint32_t* __restrict__ group_page, double* __restrict__ stage,
-                                                double inv_dx)
+// phaseP2G (:209-257) with the rhs and diagonal sums (:303-325, :405-437), by
+// CellSums: sum vol w, sum D_p w and, in the parabolic form, sum w, sum c w.
+// (3M particles: 162 us with LDS adds, 124 so.)
+template <bool PARA>
+__global__ __launch_bounds__(kSumThreads) void k_pf_p2g(ParticlesView P, PfParticles pf, PfScalars ps,
+                                                        const uint32_t* __restrict__ order,
+                                                        const uint32_t* __restrict__ group_start,
+                                                        const uint32_t* __restrict__ cell_off,
+                                                        double* __restrict__ stage, double inv_dx)
 {
-  constexpr int SS = kPfFields * kTileNodes;
-  __shared__ double tile[4 * SS];
+  constexpr int NF = pf_fields(PARA);
+  __shared__ CellSums<NF, false> cs;
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;
-  for (int k = tid; k < 4 * SS; k += 256) tile[k] = 0.0;
   const uint32_t start = group_start[g];
   const uint32_t n = group_start[g + 1] - start;
-  uint32_t px, py, pz;
-  page_decode(group_page[g], px, py, pz);
-  const int ox = 2 * (int)px, oy = 4 * (int)py, oz = 4 * (int)pz;
+  cell_sums_begin(cs, cell_off + 32 * (size_t)g, n);
   __syncthreads();
-  double* wt = tile + (tid >> 6) * SS;
-  const uint32_t perm = (uint32_t)((tid & 31) * 8 + (tid >> 5));
   const int64_t S = P.stride;
-  const double M = ps.M;
-  for (uint32_t j0 = 0; j0 < n; j0 += 256) {
-    const uint32_t j = j0 + perm;
-    if (j >= n) continue;
-    const uint32_t i = order[start + j];
-    const double xp[3] = { P.x[i], P.x[S + i], P.x[2 * S + i] };
-    const double vol = P.vol[i] * det_soa(P.F, S, i);
-    pf.vol[i] = vol;
-    const double dg = M > 0.0 ? vol * (M * pf.Fp[i] + 1.0 / ps.dt) : vol * pf.Fp[i];
-    const double c = pf.c[i];
-    double w[3][3];
-    int b[3];
+  double acc[NF][3] = {};
+  for (uint32_t c0 = 0; c0 < n; c0 += kSumChunk) {
+    const uint32_t count = n - c0 < (uint32_t)kSumChunk ? n - c0 : (uint32_t)kSumChunk;
+    if ((uint32_t)tid < count) {
+      const uint32_t i = order[start + c0 + tid];
+      double f[3], v[NF];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) b[d] = bspline_w(xp[d] * inv_dx, w[d]);
-    const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
-    if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int bb = 0; bb < 3; ++bb) {
-        const double wab = w[0][a] * w[1][bb];
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-          const double wt_ = wab * w[2][cc];
-          const int t = ((lx + a) * kTileY + (ly + bb)) * kTileZ + (lz + cc);
-          if (M > 0.0) {
-            atomicAdd(&wt[t], wt_);
-            atomicAdd(&wt[kTileNodes + t], c * wt_);
-          }
-          atomicAdd(&wt[2 * kTileNodes + t], vol * wt_);
-          atomicAdd(&wt[3 * kTileNodes + t], dg * wt_);
-        }
+      for (int d = 0; d < 3; ++d) {
+        const double xi = P.x[d * S + i] * inv_dx;
+        f[d] = xi - (double)int_floor(xi - 0.5);
       }
+      const double vol = P.vol[i] * det_soa(P.F, S, i);
+      pf.vol[i] = vol;
+      v[0] = vol;
+      v[1] = PARA ? vol * (ps.M * pf.Fp[i] + 1.0 / ps.dt) : vol * pf.Fp[i];
+      if constexpr (PARA) {
+        v[2] = 1.0;
+        v[3] = pf.c[i];
+      }
+      cell_sums_put(cs, tid, v, f);
+    }
+    __syncthreads();
+    cell_sums_chunk(cs, c0, count, acc);
+    __syncthreads();
   }
+  cell_sums_store(cs, acc, stage + (size_t)g * (NF * kTileNodes));
+}
+
+// block partials of two sums, the second set after the first
+__device__ __forceinline__ void pf_partials(double a, double b, double* partial)
+{
+  __shared__ double smem[4];
+  const double s1 = block_sum256(a, smem);
   __syncthreads();
-  double* out = stage + (size_t)g * SS;
-  for (int k = tid; k < SS; k += 256) out[k] = tile[k] + tile[SS + k] + tile[2 * SS + k] + tile[3 * SS + k];
+  const double s2 = block_sum256(b, smem);
+  if (threadIdx.x == 0) {
+    partial[blockIdx.x] = s1;
+    partial[gridDim.x + blockIdx.x] = s2;
+  }
 }
 
 // node pass: phi, rhs, D, then the CG start (fracture/ConjugateGradient.h:58-65):
 // x = 0, r = rhs, mr = r / D; partials of mr.r (rho) and r.r
+template <bool PARA>
 __global__ __launch_bounds__(256) void k_pf_nodes(uint32_t nn, const int32_t* __restrict__ slot_src,
                                                   const double* __restrict__ stage, const double* __restrict__ gm,
-                                                  PfScalars ps, double* phase, double* rhs, double* diag, double* x,
-                                                  double* r, double* mr, double* partial, uint32_t nb)
+                                                  PfScalars ps, double* phase, double* diag, double* x, double* r,
+                                                  double* mr, double* partial)
 {
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
   double rho = 0.0, rr = 0.0;
-  if (k < nn) {
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
     double ph = 0.0, b = 0.0, D = 0.0, z = 0.0;
     if (gm[k] != 0.0) {
       const uint32_t e = k & 31u;
-      double f[kPfFields];
-      sum_tiles_src<kPfFields>(stage, slot_src + 8 * (size_t)(k >> 5), (int)(e >> 4), (int)((e >> 2) & 3u),
-                               (int)(e & 3u), f);
-      if (ps.M > 0.0) {
-        ph = f[1] / f[0];
-        b = (ps.M + ph / ps.dt) * f[2];
-      } else {
-        b = f[2];
+      double f[pf_fields(PARA)];
+      sum_tiles_src<pf_fields(PARA)>(stage, slot_src + 8 * (size_t)(k >> 5), (int)(e >> 4), (int)((e >> 2) & 3u),
+                                     (int)(e & 3u), f);
+      b = f[0];
+      if constexpr (PARA) {
+        ph = f[3] / f[2];
+        b = (ps.M + ph / ps.dt) * f[0];
       }
-      D = f[3];
+      D = f[1];
       z = b / D;
-      rho = z * b;
-      rr = b * b;
+      rho += z * b;
+      rr += b * b;
     }
     phase[k] = ph;
-    rhs[k] = b;
     diag[k] = D;
     x[k] = 0.0;
     r[k] = b;
     mr[k] = z;
   }
-  __shared__ double smem[4];
-  const double s1 = block_sum256(rho, smem);
-  __syncthreads();
-  const double s2 = block_sum256(rr, smem);
-  if (threadIdx.x == 0) {
-    partial[blockIdx.x] = s1;
-    partial[nb + blockIdx.x] = s2;
-  }
+  pf_partials(rho, rr, partial);
 }
 
 // the gradient term of the operator on the direction s = mr + beta s
 // (:338-403), built on the fly in the LDS tile; one scalar field staged per group
+// (27 LDS adds per particle are cheaper here than CellSums' 9 x 28 operations:
+// 3M 110 us, against 190 so)
 __global__ __launch_bounds__(256) void k_pf_apply(const double* __restrict__ X, int64_t S, PfParticles pf,
                                                   PfScalars ps, const uint32_t* __restrict__ order,
                                                   const uint32_t* __restrict__ group_start,
@@ -206,36 +197,38 @@ __global__ __launch_bounds__(256) void k_pf_apply(const double* __restrict__ X, 
     for (int d = 0; d < 3; ++d) b[d] = bspline_wdw(xp[d] * inv_dx, w[d], dw[d]);
     const int lx = b[0] - ox, ly = b[1] - oy, lz = b[2] - oz;
     if ((unsigned)lx > 1u || (unsigned)ly > 3u || (unsigned)lz > 3u) continue;
+    const int t0 = (lx * kTileY + ly) * kTileZ + lz;
+    // the z sums, then y, then x, as in grad_from_tile
     double gc[3] = { 0.0, 0.0, 0.0 };
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+    for (int a = 0; a < 3; ++a) {
+      double U = 0.0, V = 0.0, W = 0.0;
 #pragma unroll
-      for (int bb = 0; bb < 3; ++bb)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-          double gw[3];
-          wgrad(w, dw, inv_dx, a, bb, cc, gw);
-          const double sv = tv[((lx + a) * kTileY + (ly + bb)) * kTileZ + (lz + cc)];
-          gc[0] += sv * gw[0];
-          gc[1] += sv * gw[1];
-          gc[2] += sv * gw[2];
-        }
+      for (int bb = 0; bb < 3; ++bb) {
+        const double* q = tv + t0 + (a * kTileY + bb) * kTileZ;
+        const double sv = q[0] * w[2][0] + q[1] * w[2][1] + q[2] * w[2][2];
+        const double dv = q[0] * dw[2][0] + q[1] * dw[2][1] + q[2] * dw[2][2];
+        U += sv * w[1][bb];
+        V += sv * dw[1][bb];
+        W += dv * w[1][bb];
+      }
+      gc[0] += dw[0][a] * U;
+      gc[1] += w[0][a] * V;
+      gc[2] += w[0][a] * W;
+    }
     const double l0 = pf.l0[i];
-    const double kap = pf.vol[i] * 4.0 * l0 * l0 * gscale;
+    const double kap = pf.vol[i] * 4.0 * l0 * l0 * gscale * (inv_dx * inv_dx);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) gc[d] *= kap;
-    opaque_weights(w, dw);
+    for (int a = 0; a < 3; ++a) {
+      const double ga = kap * gc[0] * dw[0][a], gb = kap * gc[1] * w[0][a], gz = kap * gc[2] * w[0][a];
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+      for (int bb = 0; bb < 3; ++bb) {
+        const double A = ga * w[1][bb] + gb * dw[1][bb], B = gz * w[1][bb];
 #pragma unroll
-      for (int bb = 0; bb < 3; ++bb)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-          double gw[3];
-          wgrad(w, dw, inv_dx, a, bb, cc, gw);
-          const int t = ((lx + a) * kTileY + (ly + bb)) * kTileZ + (lz + cc);
-          atomicAdd(&wt[t], gc[0] * gw[0] + gc[1] * gw[1] + gc[2] * gw[2]);
-        }
+        for (int cc = 0; cc < 3; ++cc)
+          atomicAdd(&wt[t0 + (a * kTileY + bb) * kTileZ + cc], A * w[2][cc] + B * dw[2][cc]);
+      }
+    }
   }
   __syncthreads();
   double* out = stage + (size_t)g * kTileNodes;
@@ -251,11 +244,10 @@ __global__ __launch_bounds__(256) void k_pf_ap(uint32_t nn, const int32_t* __res
                                                double* partial)
 {
   if (ci[CI_DONE]) return;
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
   const bool first = ci[CI_PF_IT] == 0;
   const double beta = first ? 0.0 : sc[PF_BETA];
   double sq = 0.0;
-  if (k < nn) {
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
     double sv = 0.0, qv = 0.0;
     if (gm[k] != 0.0) {
       const uint32_t e = k & 31u;
@@ -264,7 +256,7 @@ __global__ __launch_bounds__(256) void k_pf_ap(uint32_t nn, const int32_t* __res
                        (int)(e & 3u), f);
       sv = first ? mr[k] : mr[k] + beta * s[k];
       qv = diag[k] * sv + f[0];
-      sq = sv * qv;
+      sq += sv * qv;
     }
     s[k] = sv;
     q[k] = qv;
@@ -272,36 +264,33 @@ __global__ __launch_bounds__(256) void k_pf_ap(uint32_t nn, const int32_t* __res
   block_partial(sq, partial);
 }
 
-// x += alpha s, r -= alpha q, mr = r / D; partials of r.r and mr.r
+// alpha = rho / s.q, s.q from k_pf_ap's partials in every block; x += alpha s,
+// r -= alpha q, mr = r / D; partials of r.r and mr.r
 __global__ __launch_bounds__(256) void k_pf_update(uint32_t nn, const double* __restrict__ gm,
                                                    const double* __restrict__ diag, const double* __restrict__ s,
                                                    const double* __restrict__ q, double* x, double* r, double* mr,
-                                                   const double* sc, const int32_t* ci, double* partial, uint32_t nb)
+                                                   const double* sc, const int32_t* ci,
+                                                   const double* __restrict__ sq_partial, double* partial)
 {
   if (ci[CI_DONE]) return;
-  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
-  const double alpha = sc[PF_ALPHA];
+  __shared__ double red[5];
+  const double sq = block_total256(sq_partial, gridDim.x, red);
+  const double alpha = sq != 0.0 ? sc[PF_RHO] / sq : 1.7976931348623157e308;
   double rr = 0.0, rho = 0.0;
-  if (k < nn && gm[k] != 0.0) {
+  for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < nn; k += gridDim.x * 256u) {
+    if (gm[k] == 0.0) continue;
     x[k] = alpha * s[k] + x[k];
     const double rv = -alpha * q[k] + r[k];
     r[k] = rv;
     const double z = rv / diag[k];
     mr[k] = z;
-    rr = rv * rv;
-    rho = z * rv;
+    rr += rv * rv;
+    rho += z * rv;
   }
-  __shared__ double smem[4];
-  const double s1 = block_sum256(rr, smem);
-  __syncthreads();
-  const double s2 = block_sum256(rho, smem);
-  if (threadIdx.x == 0) {
-    partial[blockIdx.x] = s1;
-    partial[nb + blockIdx.x] = s2;
-  }
+  pf_partials(rr, rho, partial);
 }
 
-enum { PFR_INIT = 0, PFR_ALPHA = 1, PFR_CHECK = 2 };
+enum { PFR_INIT = 0, PFR_CHECK = 1 };
 
 // one-block ordered sums of the partials and the CG scalar logic
 __global__ __launch_bounds__(256) void k_pf_reduce(const double* __restrict__ partial, uint32_t nb, double* sc,
@@ -314,7 +303,7 @@ __global__ __launch_bounds__(256) void k_pf_reduce(const double* __restrict__ pa
     return;
   }
   const double a0 = thread_partials256(partial, nb);
-  const double a1 = mode != PFR_ALPHA ? thread_partials256(partial + nb, nb) : 0.0;
+  const double a1 = thread_partials256(partial + nb, nb);
   const double s0 = block_sum256(a0, smem);
   __syncthreads();
   const double s1 = block_sum256(a1, smem);
@@ -325,9 +314,6 @@ __global__ __launch_bounds__(256) void k_pf_reduce(const double* __restrict__ pa
     sc[PF_REL] = sqrt(s1) * cg_relative;
     ci[CI_DONE] = 0;
     ci[CI_PF_IT] = 0;
-  } else if (mode == PFR_ALPHA) {  // s0 = s.q
-    sc[PF_SQ] = s0;
-    sc[PF_ALPHA] = s0 != 0.0 ? sc[PF_RHO] / s0 : 1.7976931348623157e308;
   } else {  // s0 = r.r, s1 = new mr.r
     const double norm = sqrt(s0);
     sc[PF_NORM] = norm;
@@ -412,7 +398,7 @@ __global__ __launch_bounds__(256) void k_pf_g2p(ParticlesView P, PfParticles pf,
       for (int r = 0; r < 3; ++r) f.a[r][cc] = P.F[(cc * 3 + r) * S + i];
     const double mu = P.mu[i], lam = P.lam[i];
     const double J = det3(f);
-    const double aJ = pow(J, -1.0 / 3.0);
+    const double aJ = J < 0.0 ? __builtin_nan("") : rcbrt(J);  // pow(J, -1/3)
     double tr = 0.0;
 #pragma unroll
     for (int r = 0; r < 3; ++r)

@@ -1591,7 +1591,6 @@ struct zr_engine {
   double* pf_node = nullptr;  // 8 x grid capacity
   size_t pf_node_cap = 0;
   double* pf_partial = nullptr;
-  size_t pf_partial_cap = 0;
   // differentiable form: particle adjoints [38][n] (x 3, v 3, C 9, F 9, mu,
   // lambda, G2P scratch x 3 and F 9), node adjoints [7][grid capacity],
   // device checkpoints of (x, v, C, F) with their times
@@ -2527,26 +2526,24 @@ int do_pf(zr_engine* e, double dt)
     return fail(e, ZR_ERR_STATE, "phase-field solve before the MLS particlesToGrid of the step");
   int rc0 = ensure_scalars(e);
   if (rc0) return rc0;
-  const uint32_t nn = e->S * 32, nb = blocks_for(nn, 256);
+  const uint32_t nn = e->S * 32, nb = std::min(blocks_for(nn, 256), kCgBlocks);
   if (e->pf_node_cap < e->grid_cap) {
     dfree(e->pf_node);
-    ZR_HIP(e, hipMalloc(&e->pf_node, 8 * e->grid_cap * sizeof(double)));
+    e->pf_node_cap = 0;
+    ZR_HIP(e, hipMalloc(&e->pf_node, 7 * e->grid_cap * sizeof(double)));
     e->pf_node_cap = e->grid_cap;
   }
-  if (e->pf_partial_cap < 2 * (size_t)nb) {
-    dfree(e->pf_partial);
-    ZR_HIP(e, hipMalloc(&e->pf_partial, 2 * (size_t)nb * sizeof(double)));
-    e->pf_partial_cap = 2 * (size_t)nb;
-  }
+  if (!e->pf_partial) ZR_HIP(e, hipMalloc(&e->pf_partial, 2 * kCgBlocks * sizeof(double)));
   const size_t C = e->pf_node_cap;
-  double *phase = e->pf_node, *rhs = phase + C, *diag = rhs + C, *x = diag + C, *r = x + C, *mr = r + C,
-         *sv = mr + C, *q = sv + C;
+  double *phase = e->pf_node, *diag = phase + C, *x = diag + C, *r = x + C, *mr = r + C, *sv = mr + C, *q = sv + C;
   const double dx = e->cfg.dx;
   PfScalars ps{ o.parabolic_M, dt, o.cg_tolerance, o.cg_max_iterations };
   PfParticles pf = pf_view(e);
-  k_pf_p2g<<<e->A, 256, 0, s>>>(pview(e), pf, ps, e->order, e->group_start, e->group_page, e->stage, 1.0 / dx);
-  k_pf_nodes<<<nb, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, ps, phase, rhs, diag, x, r, mr, e->pf_partial,
-                                nb);
+  const bool para = ps.M > 0.0;
+  (para ? k_pf_p2g<true> : k_pf_p2g<false>)<<<e->A, kSumThreads, 0, s>>>(pview(e), pf, ps, e->order, e->group_start,
+                                                                         e->cell_off, e->stage, 1.0 / dx);
+  (para ? k_pf_nodes<true> : k_pf_nodes<false>)<<<nb, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, ps, phase, diag,
+                                                                   x, r, mr, e->pf_partial);
   k_pf_reduce<<<1, 256, 0, s>>>(e->pf_partial, nb, e->sc, e->ci, PFR_INIT, o.cg_relative, ps, SolveMark{});
   ZR_LAUNCH_CHECK(e);
   // the fracture CG runs iterations 0..max (it checks it == max after the update)
@@ -2556,9 +2553,8 @@ int do_pf(zr_engine* e, double dt)
   for (int it = 0; it < total && !watch.done; ++it) {
     k_pf_apply<<<e->A, 256, 0, s>>>(e->x, e->n, pf, ps, e->order, e->group_start, e->group_page, e->group_nslot,
                                     e->gm, mr, sv, e->sc, e->ci, e->stage, 1.0 / dx);
-    k_pf_ap<<<nb, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, diag, mr, sv, q, e->sc, e->ci, e->pf_partial);
-    k_pf_reduce<<<1, 256, 0, s>>>(e->pf_partial, nb, e->sc, e->ci, PFR_ALPHA, o.cg_relative, ps, SolveMark{});
-    k_pf_update<<<nb, 256, 0, s>>>(nn, e->gm, diag, sv, q, x, r, mr, e->sc, e->ci, e->pf_partial, nb);
+    k_pf_ap<<<nb, 256, 0, s>>>(nn, e->slot_src, e->stage, e->gm, diag, mr, sv, q, e->sc, e->ci, e->partial2);
+    k_pf_update<<<nb, 256, 0, s>>>(nn, e->gm, diag, sv, q, x, r, mr, e->sc, e->ci, e->partial2, e->pf_partial);
     k_pf_reduce<<<1, 256, 0, s>>>(e->pf_partial, nb, e->sc, e->ci, PFR_CHECK, o.cg_relative, ps, watch.mark(it));
     ZR_LAUNCH_CHECK(e);
     rc0 = watch.issued(it);

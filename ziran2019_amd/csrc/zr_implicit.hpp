@@ -702,14 +702,16 @@ __constant__ HvpTaskSlots kHvpTaskSlots = hvp_task_slots();
 // one for a few particles.  Measured, with LDS adds -> chunks of 256 -> so:
 // k_be_scatter 1M 82 -> 79 -> 74 us, 2.1M 146 -> 123 -> 110; k_admm_op32
 // 2.1M 119 -> 109 -> 108 (with the launches past the end of a solve).
+// The same for NF scalars times w (GRAD false), in the phase field's solve.
 constexpr int kSumThreads = 320, kSumChunk = 304;
 constexpr int kSumStride = kSumChunk + 1;  // of the rows
-union CellSumsData {
-  double row[12 * kSumStride];               // D (row-major), then the fractions
-  double contrib[3][kCells * kAB * 3];
-};
+template <int NF, bool GRAD>
 struct CellSums {
-  CellSumsData u;
+  static constexpr int NV = GRAD ? 3 * NF : NF;  // a particle's values: D row by row, or the scalars
+  union {
+    double row[(NV + 3) * kSumStride];           // the values, then the fractions
+    double contrib[NF][kCells * kAB * 3];
+  } u;
   uint32_t coff[kCells + 1];    // the cells' runs, in the sort's order of cells
   int order[kCells];            // the cells by falling number of particles
 };
@@ -718,7 +720,8 @@ static_assert(kCells * kAB <= kSumThreads && kSumChunk <= kSumThreads && kTileNo
 // cell (bits x, y y, z z from the lowest) in the sort's order of cells
 __device__ __forceinline__ int sum_cell_slot(int e) { return ((e & 1) << 4) | (((e >> 1) & 3) << 2) | (e >> 3); }
 // the caller synchronises before the first chunk
-__device__ __forceinline__ void cell_sums_begin(CellSums& cs, const uint32_t* cell_off, uint32_t n)
+template <class CS>
+__device__ __forceinline__ void cell_sums_begin(CS& cs, const uint32_t* cell_off, uint32_t n)
 {
   const int tid = threadIdx.x;
   if (tid >= 64) return;
@@ -734,19 +737,22 @@ __device__ __forceinline__ void cell_sums_begin(CellSums& cs, const uint32_t* ce
   }
   if (tid < kCells) cs.order[rank] = ((tid >> 4) & 1) | (((tid >> 2) & 3) << 1) | ((tid & 3) << 3);
 }
-__device__ __forceinline__ void cell_sums_put(CellSums& cs, int p, const double D[3][3], const double f[3])
+template <int NF, bool GRAD>
+__device__ __forceinline__ void cell_sums_put(CellSums<NF, GRAD>& cs, int p, const double* v, const double f[3])
 {
+  constexpr int NV = CellSums<NF, GRAD>::NV;
 #pragma unroll
-  for (int r = 0; r < 3; ++r)
+  for (int k = 0; k < NV; ++k) cs.u.row[k * kSumStride + p] = v[k];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) cs.u.row[(3 * r + c) * kSumStride + p] = D[r][c];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) cs.u.row[(9 + d) * kSumStride + p] = f[d];
+  for (int d = 0; d < 3; ++d) cs.u.row[(NV + d) * kSumStride + p] = f[d];
 }
 // this thread's task's sums over the chunk [c0, c0 + count) of the group,
-// added to acc[c][r]; between barriers
-__device__ __forceinline__ void cell_sums_chunk(const CellSums& cs, uint32_t c0, uint32_t count, double acc[3][3])
+// added to acc[field][c]; between barriers
+template <int NF, bool GRAD>
+__device__ __forceinline__ void cell_sums_chunk(const CellSums<NF, GRAD>& cs, uint32_t c0, uint32_t count,
+                                                double acc[NF][3])
 {
+  constexpr int NV = CellSums<NF, GRAD>::NV;
   const int rk = (int)threadIdx.x / kAB, ab = (int)threadIdx.x - rk * kAB;
   if (rk >= kCells) return;
   const int e = cs.order[rk], a = ab / 3, b = ab - 3 * a;
@@ -757,23 +763,34 @@ __device__ __forceinline__ void cell_sums_chunk(const CellSums& cs, uint32_t c0,
   const double sy = 1.5 - 0.5 * b, ky = b == 1 ? -1.0 : 0.5, ey = b == 1 ? 0.75 : 0.0;
   for (uint32_t j = jb; j < je; ++j) {
     const double* q = cs.u.row + j;
-    const double tx = q[9 * kSumStride] - sx, ty = q[10 * kSumStride] - sy, f2 = q[11 * kSumStride];
+    const double tx = q[NV * kSumStride] - sx, ty = q[(NV + 1) * kSumStride] - sy, f2 = q[(NV + 2) * kSumStride];
     const double hx = kx * tx, hy = ky * ty;
     const double wa = fma(hx, tx, ex), wb = fma(hy, ty, ey);
-    const double x0 = (hx + hx) * wb, x1 = wa * (hy + hy), x2 = wa * wb;
-    const double z0 = f2 - 1.5, z1 = f2 - 1.0, z2 = f2 - 0.5;
-    const double wc[3] = { 0.5 * z0 * z0, fma(-z1, z1, 0.75), 0.5 * z2 * z2 }, dc[3] = { z0, -2.0 * z1, z2 };
+    const double z0 = f2 - 1.5, z1 = f2 - 1.0, z2 = f2 - 0.5, x2 = wa * wb;
+    const double wc[3] = { 0.5 * z0 * z0, fma(-z1, z1, 0.75), 0.5 * z2 * z2 };
+    if constexpr (GRAD) {
+      const double dc[3] = { z0, -2.0 * z1, z2 };
+      const double x0 = (hx + hx) * wb, x1 = wa * (hy + hy);
 #pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      const double A = fma(q[(3 * r + 1) * kSumStride], x1, q[3 * r * kSumStride] * x0);
-      const double B = q[(3 * r + 2) * kSumStride] * x2;
+      for (int r = 0; r < NF; ++r) {
+        const double A = fma(q[(3 * r + 1) * kSumStride], x1, q[3 * r * kSumStride] * x0);
+        const double B = q[(3 * r + 2) * kSumStride] * x2;
 #pragma unroll
-      for (int c = 0; c < 3; ++c) acc[c][r] = fma(B, dc[c], fma(A, wc[c], acc[c][r]));
+        for (int c = 0; c < 3; ++c) acc[r][c] = fma(B, dc[c], fma(A, wc[c], acc[r][c]));
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < NF; ++r) {
+        const double A = q[r * kSumStride] * x2;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) acc[r][c] = fma(A, wc[c], acc[r][c]);
+      }
     }
   }
 }
 // after a barrier: the group's sums into its staged tile
-__device__ __forceinline__ void cell_sums_store(CellSums& cs, const double acc[3][3], double* out)
+template <int NF, bool GRAD>
+__device__ __forceinline__ void cell_sums_store(CellSums<NF, GRAD>& cs, const double acc[NF][3], double* out)
 {
   const int t = threadIdx.x;
   const int rk = t / kAB, ab = t - rk * kAB;
@@ -782,21 +799,20 @@ __device__ __forceinline__ void cell_sums_store(CellSums& cs, const double acc[3
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int r = 0; r < 3; ++r) cs.u.contrib[r][(ts >> (10 * c)) & 1023u] = acc[c][r];
+      for (int r = 0; r < NF; ++r) cs.u.contrib[r][(ts >> (10 * c)) & 1023u] = acc[r][c];
   }
   __syncthreads();
   if (t >= kTileNodes) return;
   const int tx = t / (kTileY * kTileZ), ty = (t / kTileZ) % kTileY, tz = t % kTileZ;
   const int k0 = hvp_node_off(tx, ty, tz), nk = hvp_na(tx) * hvp_nb(ty) * hvp_nb(tz);
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-  for (int k = k0; k < k0 + nk; ++k) {
-    a0 += cs.u.contrib[0][k];
-    a1 += cs.u.contrib[1][k];
-    a2 += cs.u.contrib[2][k];
-  }
-  out[t] = a0;
-  out[kTileNodes + t] = a1;
-  out[2 * kTileNodes + t] = a2;
+  double sum[NF];
+#pragma unroll
+  for (int r = 0; r < NF; ++r) sum[r] = 0.0;
+  for (int k = k0; k < k0 + nk; ++k)
+#pragma unroll
+    for (int r = 0; r < NF; ++r) sum[r] += cs.u.contrib[r][k];
+#pragma unroll
+  for (int r = 0; r < NF; ++r) out[r * kTileNodes + t] = sum[r];
 }
 
 // The Newton state of k_be_state<T, false> in three passes, so that the
@@ -942,7 +958,7 @@ __global__ __launch_bounds__(kSumThreads) void k_be_scatter(ParticlesView P, con
                                                     double inv_dx, const double* __restrict__ fb,
                                                     double* __restrict__ stage)
 {
-  __shared__ CellSums cs;
+  __shared__ CellSums<3, true> cs;
   const int tid = threadIdx.x;
   const uint32_t g = blockIdx.x;
   const uint32_t start = group_start[g];
@@ -965,7 +981,7 @@ __global__ __launch_bounds__(kSumThreads) void k_be_scatter(ParticlesView P, con
       for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int r = 0; r < 3; ++r) D[r][c] = inv_dx * fb[(c * 3 + r) * cstride + ks];
-      cell_sums_put(cs, tid, D, f);
+      cell_sums_put(cs, tid, &D[0][0], f);
     }
     __syncthreads();
     cell_sums_chunk(cs, c0, count, acc);
