@@ -11,8 +11,9 @@
 // map's derivative), global dv step (MINRES on M + sum_p rho omega^2 dt^2
 // (Fn^T grad w)(Fn^T grad w)^T, applied matrix-free, with the collision
 // projection and the diagonal preconditioner), dual update y }.  Particle
-// passes use the group's LDS tile of a node vector; scatters use per-wave
-// LDS tiles staged per group and summed per node in a fixed order.
+// passes use the group's LDS tile of a node vector; scatters of gradients sum
+// by cell (CellSums), the others into per-wave LDS tiles; both are staged per
+// group and summed per node in a fixed order.
 
 
 struct AdmmParticles {
@@ -1182,8 +1183,11 @@ __global__ __launch_bounds__(256) void k_admm_cache32(ParticlesView P, AdmmParti
 }
 
 // the global operator's particle term in FP32 (k_admm_op64's sums)
+// (Six waves per SIMD, 80 registers: a block's fifth wave makes one SIMD hold
+// two of it, and at five waves only three blocks find room: 126 us at 2.1M,
+// 114 so.)
 template <bool VISCO>
-__global__ __launch_bounds__(kSumThreads, 5) void k_admm_op32(AdmmCache32 C, const uint32_t* __restrict__ group_start,
+__global__ __launch_bounds__(kSumThreads, 6) void k_admm_op32(AdmmCache32 C, const uint32_t* __restrict__ group_start,
                                                    const uint32_t* __restrict__ cell_off,
                                                    const int32_t* __restrict__ group_nslot,
                                                    const double* __restrict__ gm, const float* __restrict__ xvec,

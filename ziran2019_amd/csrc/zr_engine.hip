@@ -5,13 +5,15 @@
 //   bin      : per particle base node -> SPGrid page code; per-page counts via
 //              atomics on a dense page table; occupancy bitmap
 //   groups   : bitmap popcount scan -> sorted list of particle pages (groups)
-//   scatter  : particles into their group segment, then an in-LDS bitonic sort
-//              of each segment by (cell, index): the reference's sorted keys
+//   scatter  : particles into their group segment, then each segment ordered
+//              in LDS by (cell, index): the reference's sorted keys; large
+//              sets are also moved into that order in memory now and then
 //   pages    : 8 neighbour pages per group, first-touch order by atomicMin on
 //              the touch index -> page slots (the reference's block list)
-//   P2G      : one workgroup per group scatters its particles into per-wave
-//              LDS tiles covering the 4x6x6 stencil footprint of the page,
-//              then writes the tile to a staging buffer (no global atomics)
+//   P2G      : one workgroup per group; a cell's particles are multiplied
+//              with their weights by matrix instructions and the cells added
+//              into per-wave LDS tiles covering the 4x6x6 stencil footprint of
+//              the page, which go to a staging buffer (no global atomics)
 //   grid     : one thread per node of each slot sums the <= 8 overlapping
 //              tiles in a fixed order, normalises, applies gravity/forces and
 //              colliders (+ trial collision)

@@ -10,7 +10,7 @@
 // a kernel into a device buffer of their own, copied to a pinned buffer of
 // their own, and copy that to the caller's pages (uploads the other way
 // round).  A call of one window has the kernel store into the pinned buffer
-// and no thread is made.  2.1M particles (403 MB) down: 32 -> 12 ms.
+// and no thread is made.  2.1M particles (403 MB) down: 40 -> 11 ms.
 //
 // The pinned buffers are the process's (at most 32 MiB, made as needed, freed
 // with the last engine); a transfer holds their lock, so that engines in
