@@ -1262,8 +1262,7 @@ __global__ __launch_bounds__(HvpChunk<T>::threads, HvpChunk<T>::waves) void k_hv
   // (FP64); rows padded by one element so that the rows one particle's tasks
   // read together fall in different banks.  The FP32 tasks form the weights
   // again: 12 LDS values per particle and task instead of 19 and 12 stores
-  // instead of 27, for 17 operations, and four blocks per CU instead of three
-  // (1M 69.2 -> 67.1 us).  In FP64 the operations cost as much (268k 41.4 ->
+  // instead of 27, for 17 operations (1M 69.2 -> 67.1 us).  In FP64 the operations cost as much (268k 41.4 ->
   // 40.8 us, 20k 14.7 -> 15.4).
   constexpr bool kForm = HvpChunk<T>::form_weights;
   __shared__ T pds[kForm ? 12 : 27][CH + 1];
