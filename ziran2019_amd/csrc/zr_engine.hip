@@ -2175,8 +2175,8 @@ int user_order(zr_engine* e)
 // k_move 225 us; k_g2p 282 -> 164 us and k_p2g 238 -> 195, the G2P's writes
 // of 24 rows reaching memory 2.2 times in partial lines before), so they
 // are moved once the steps since the last move have lost that much
-// (kDisorder); a rollout keeps the caller's order, which its records and
-// adjoints are in.  Below kMoveMin the arrays stay in the caches and a
+// (kDisorder); rollouts and adjoint steps keep the caller's order, which their
+// records and adjoints are in.  Below kMoveMin the arrays stay in the caches and a
 // move's launches cost more than they give.
 void note_disorder(zr_engine* e)
 {
@@ -2262,8 +2262,10 @@ int sort_launch(zr_engine* e, SortRun& run)
   return ZR_OK;
 }
 
-// with the sort's counts on the host: what they ask for beyond the launch
-int sort_finish(zr_engine* e, const SortRun& run, zr_step_stats* st)
+// with the sort's counts on the host: what they ask for beyond the launch.
+// move: the particles may go into the sort's order in memory (not where what
+// follows reads arrays that stay in the caller's, the adjoints and records)
+int sort_finish(zr_engine* e, const SortRun& run, zr_step_stats* st, bool move)
 {
   hipStream_t s = e->stream;
   const uint32_t n = (uint32_t)e->n;
@@ -2288,7 +2290,7 @@ int sort_finish(zr_engine* e, const SortRun& run, zr_step_stats* st)
   // a rollout's earlier step asked for a restart: the particles are those
   // after that step (a sort moves none)
   if (e->defer_cfl && (e->hcount[CNT_CFL_RUN] & 1u)) return ZR_CFL_RESTART;
-  if (!e->defer_cfl) {
+  if (move) {
     note_disorder(e);
     if (e->move_next) {
       rc = order_particles(e);
@@ -2313,12 +2315,12 @@ int sort_finish(zr_engine* e, const SortRun& run, zr_step_stats* st)
   return ZR_OK;
 }
 
-int do_sort(zr_engine* e, zr_step_stats* st)
+int do_sort(zr_engine* e, zr_step_stats* st, bool move = true)
 {
   SortRun run;
   int rc = sort_launch(e, run);
   if (!rc) rc = sync_counts(e);
-  return rc ? rc : sort_finish(e, run, st);
+  return rc ? rc : sort_finish(e, run, st, move);
 }
 
 // mls: the MLS P2G with force (explicit) or the APIC one (implicit, ADMM);
@@ -2682,7 +2684,7 @@ int adjoint_kernels(zr_engine* e, double dt, const AdjTables& t)
 
 int do_adjoint_step(zr_engine* e, double dt, bool check)
 {
-  int rc = do_sort(e, nullptr);
+  int rc = do_sort(e, nullptr, false);
   if (rc) return rc;
   rc = do_p2g(e, true);
   if (rc) return rc;
@@ -2808,7 +2810,7 @@ AdjTables record_tables(zr_engine* e, const zr_engine::StepRecord& r)
 // momentum in their own fields), its tables and grid copied into r
 int advance_recorded(zr_engine* e, double dt, zr_engine::StepRecord& r)
 {
-  int rc = do_sort(e, nullptr);
+  int rc = do_sort(e, nullptr, false);
   if (rc) return rc;
   rc = do_p2g(e, true);
   if (rc) return rc;
@@ -4307,7 +4309,7 @@ static int deferred_step(zr_engine* e, double dt, zr_step_stats* st, bool& again
   if (rc) return rc;
   if (!run.one_block) {  // (a_hint was cut to the particle count: not reached)
     rc = sync_counts(e);
-    if (!rc) rc = sort_finish(e, run, st);
+    if (!rc) rc = sort_finish(e, run, st, true);
     again = rc == ZR_OK;
     return rc;
   }
@@ -4327,11 +4329,11 @@ static int deferred_step(zr_engine* e, double dt, zr_step_stats* st, bool& again
   if (!rc) rc = sync_counts(e);
   if (rc) return rc;
   if (e->hcount[CNT_GROUPS] > run.hint || e->hcount[CNT_SLOTS] > run.smax) {
-    rc = sort_finish(e, run, st);
+    rc = sort_finish(e, run, st, true);
     again = rc == ZR_OK;
     return rc;
   }
-  rc = sort_finish(e, run, st);
+  rc = sort_finish(e, run, st, true);
   e->sorted = false;
   if (rc) return rc;
   const uint32_t flags = e->hcount[CNT_CFL];
@@ -4357,7 +4359,7 @@ int zr_advance_one_time_step(zr_engine* e, double dt, zr_step_stats* st)
                                                                         e->pf_opts.delete_threshold);
     ZR_LAUNCH_CHECK(e);
   }
-  int rc = sorted ? ZR_OK : do_sort(e, st);
+  int rc = sorted ? ZR_OK : do_sort(e, st, !e->defer_cfl);  // a rollout keeps the caller's order
   if (rc) return rc;
   rc = do_p2g(e, true, dt);
   if (rc) return rc;
