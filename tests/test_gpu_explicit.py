@@ -208,6 +208,26 @@ def test_domain_error_is_reported_and_recoverable():
     eng.advanceOneTimeStep(1e-4)
 
 
+@pytest.mark.parametrize("refused", [1, 2, 3])
+def test_recovery_after_refused_first_steps(refused):
+    """An engine none of whose steps has succeeded yet forgets every refused
+    one, whichever bank of counters it used."""
+    s = scenes.cube_scene_small(seed=8)
+    bad = dict(s, X=s["X"].copy())
+    bad["X"][3] = (-0.5, 0.5, 0.5)
+    eng, ora = make_pair(s)
+    for _ in range(refused):
+        eng.upload(bad)
+        with pytest.raises(ZrError, match="outside"):
+            eng.advanceOneTimeStep(1e-4)
+    eng.upload(s)
+    for _ in range(2):
+        eng.advanceOneTimeStep(1e-4)
+        ora.step(1e-4)
+    assert rel_err(eng.download()["X"], ora.get_particles()[0]) < 1e-12
+    eng.close()
+
+
 def test_full_size_cube_properties():
     """140,608 particles at dx=1/128: a few steps against the oracle plus
     mass/momentum checks of the rasterised grid."""

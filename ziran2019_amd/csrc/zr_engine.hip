@@ -2234,8 +2234,10 @@ int sort_launch(zr_engine* e, SortRun& run)
     if (rc) return rc;
     hint = e->hcount[CNT_GROUPS];
     if (e->hcount[CNT_DOMAIN]) {
-      // the tables hold clamped entries; A is kept so that the next sort clears them
+      // the tables hold clamped entries; A is kept so that the next sort clears them.
+      // The counters are cleared here: k_scatter, which does it otherwise, has not run
       e->A = hint;
+      ZR_HIP(e, hipMemsetAsync(e->dbase, 0, 2 * kBank * sizeof(uint32_t), s));
       return fail(e, ZR_ERR_DOMAIN, "particle base node outside [0, 2^grid_log2 - 8]");
     }
   }
