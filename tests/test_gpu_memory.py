@@ -1,0 +1,49 @@
+"""Steps whose allocations fail: the call reports it, and the engine works
+again once there is memory."""
+import numpy as np
+import pytest
+
+from ziran2019_amd import scenes
+from ziran2019_amd.engine import MpmEngine, ZrError
+from _device_memory import device_memory_held
+from _helpers import make_pair
+
+pytestmark = pytest.mark.gpu
+
+
+def _spread(n):
+    """n particles, most of them in a page of their own."""
+    rng = np.random.default_rng(5)
+    cube = scenes.cube_scene_small(seed=3, ncells=4)
+    s = {k: np.resize(cube[k], (n,) + cube[k].shape[1:]) for k in ("V", "C", "F", "mass", "vol", "mu", "lam")}
+    return dict(s, X=0.05 + 0.85 * rng.random((n, 3)), dx=1.0 / 256)
+
+
+def _same(a, b):
+    for k in a:
+        assert np.array_equal(a[k], b[k]), k
+
+
+def test_a_sort_that_finds_no_memory_leaves_nothing_behind():
+    """The first sort of many groups allocates the cells' table (38 MB here)
+    after the pages have been counted."""
+    n = 300000
+    s = _spread(n)
+    ref = MpmEngine(dx=s["dx"])
+    ref.upload(s)
+    for _ in range(2):
+        ref.advanceOneTimeStep(1e-5)
+    want = ref.download()
+    ref.close()
+    small = {k: (v[:50000] if isinstance(v, np.ndarray) else v) for k, v in s.items()}
+    eng = MpmEngine(dx=s["dx"])
+    eng.upload(small)
+    eng.advanceOneTimeStep(1e-5)
+    eng.upload(s)
+    with device_memory_held(eng.L, 4 << 20):
+        with pytest.raises(ZrError, match="memory"):
+            eng.advanceOneTimeStep(1e-5)
+    for _ in range(2):
+        eng.advanceOneTimeStep(1e-5)
+    _same(eng.download(), want)
+    eng.close()

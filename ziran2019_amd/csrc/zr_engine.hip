@@ -1659,7 +1659,9 @@ struct zr_engine {
   StepGuard guard;             // of the step being launched (deferred_step)
   uint32_t s_hint = 0;         // slots that a step launched before its counts are known has room for
   bool move_next = false;      // the next sort moves the particles
-  bool tables_clean = true;    // nothing left in the dense page tables by a sort that failed
+  // what the last sort left in the dense page tables: nothing, the entries of
+  // its A groups and S slots, or, where it failed on the way, anything
+  enum { TABLES_CLEAN, TABLES_LISTED, TABLES_UNKNOWN } tables = TABLES_CLEAN;
   // evalMaxParticleSpeed: 7 block maxima per block; the 7 results (pinned)
   double* speed = nullptr;
   double* hspeed = nullptr;
@@ -1768,8 +1770,10 @@ int fail(zr_engine* e, int code, const std::string& msg)
 #define ZR_HIP(e, call)                                                                     \
   do {                                                                                      \
     hipError_t _st = (call);                                                                \
-    if (_st != hipSuccess)                                                                  \
+    if (_st != hipSuccess) {                                                                \
+      (void)hipGetLastError(); /* reported here, not by the next launch's check */          \
       return fail((e), ZR_ERR_HIP, std::string(#call ": ") + hipGetErrorString(_st));       \
+    }                                                                                       \
   } while (0)
 
 #define ZR_LAUNCH_CHECK(e) ZR_HIP(e, hipGetLastError())
@@ -2057,13 +2061,26 @@ int assign_slots(zr_engine* e, uint32_t hint)
 
 int reset_tables(zr_engine* e)
 {
+  if (e->tables == zr_engine::TABLES_UNKNOWN) {  // all of them, and both banks of counters
+    hipStream_t s = e->stream;
+    const size_t dense = e->ndense * sizeof(uint32_t);
+    ZR_HIP(e, hipMemsetAsync(e->page_count, 0, dense, s));
+    ZR_HIP(e, hipMemsetAsync(e->page_group, 0xff, dense, s));
+    ZR_HIP(e, hipMemsetAsync(e->page_touch, 0xff, dense, s));
+    ZR_HIP(e, hipMemsetAsync(e->page_slot, 0xff, dense, s));
+    ZR_HIP(e, hipMemsetAsync(e->page_bits, 0, e->nwords * sizeof(uint32_t), s));
+    ZR_HIP(e, hipMemsetAsync(e->page_sum, 0, e->nsum * sizeof(uint32_t), s));
+    ZR_HIP(e, hipMemsetAsync(e->dbase, 0, 2 * kBank * sizeof(uint32_t), s));
+    e->tables = zr_engine::TABLES_CLEAN;
+    return ZR_OK;
+  }
   const uint32_t rst = e->A > e->S ? e->A : e->S;
   if (rst)
     k_reset_tables<<<blocks_for(rst, 256), 256, 0, e->stream>>>(e->group_page, e->A, e->slot_page, e->S,
                                                                 e->page_count, e->page_group, e->page_bits,
                                                                 e->page_sum, e->page_touch, e->page_slot);
   ZR_LAUNCH_CHECK(e);
-  e->tables_clean = true;
+  e->tables = zr_engine::TABLES_CLEAN;
   return ZR_OK;
 }
 
@@ -2199,12 +2216,12 @@ int sort_launch(zr_engine* e, SortRun& run)
   hipStream_t s = e->stream;
   e->sorted = e->rasterised = e->updated = false;
   int rc = ZR_OK;
-  if (!e->tables_clean) {  // a sort that failed left its entries
+  if (e->tables != zr_engine::TABLES_CLEAN) {  // a sort that failed left its entries
     rc = reset_tables(e);
     if (rc) return rc;
   }
   e->dcount = e->dcount == e->dbase ? e->dbase + kBank : e->dbase;
-  e->tables_clean = false;
+  e->tables = zr_engine::TABLES_UNKNOWN;
   e->A = e->S = 0;
   prof_mark(e, ZR_PROF_SORT);
   k_bin<<<blocks_for(n, 256), 256, 0, s>>>(e->x, e->n, n, 1.0 / e->cfg.dx, (int)e->lim, e->page_count, e->page_bits,
@@ -2236,8 +2253,9 @@ int sort_launch(zr_engine* e, SortRun& run)
     if (e->hcount[CNT_DOMAIN]) {
       // the tables hold clamped entries; A is kept so that the next sort clears them.
       // The counters are cleared here: k_scatter, which does it otherwise, has not run
-      e->A = hint;
       ZR_HIP(e, hipMemsetAsync(e->dbase, 0, 2 * kBank * sizeof(uint32_t), s));
+      e->A = hint;
+      e->tables = zr_engine::TABLES_LISTED;
       return fail(e, ZR_ERR_DOMAIN, "particle base node outside [0, 2^grid_log2 - 8]");
     }
   }
@@ -2275,16 +2293,15 @@ int sort_finish(zr_engine* e, const SortRun& run, zr_step_stats* st, bool move)
   const uint32_t A = e->hcount[CNT_GROUPS];
   const bool exact = A <= run.hint;
   const bool tables = run.one_block && exact && e->hcount[CNT_SLOTS] <= run.smax;  // k_slots went through
-  e->tables_clean = tables;
-  e->A = A;
-  e->S = e->hcount[CNT_SLOTS];
   if (!exact) {
     rc = sort_groups(e, A);
     if (!rc) rc = assign_slots(e, A);
     if (!rc) rc = sync_counts(e);
     if (rc) return rc;
-    e->S = e->hcount[CNT_SLOTS];
   }
+  e->A = A;
+  e->S = e->hcount[CNT_SLOTS];
+  e->tables = tables ? zr_engine::TABLES_CLEAN : zr_engine::TABLES_LISTED;
   if (e->hcount[CNT_DOMAIN])  // (the tables' clamped entries are cleared by the next sort, if not yet)
     return fail(e, ZR_ERR_DOMAIN, "particle base node outside [0, 2^grid_log2 - 8]");
   e->a_hint = A + A / 4 + 64 < n ? A + A / 4 + 64 : n;
@@ -3750,7 +3767,7 @@ int zr_upload_particles(zr_engine* e, const zr_particles* p)
     return fail(e, ZR_ERR_ARG, "all particle attributes are required");
   ZR_HIP(e, hipStreamSynchronize(e->stream));
   // clear what a failed sort of the previous particle set left in the tables
-  if (!e->tables_clean) {
+  if (e->tables != zr_engine::TABLES_CLEAN) {
     int rc = reset_tables(e);
     if (rc) return rc;
     ZR_HIP(e, hipStreamSynchronize(e->stream));
@@ -4315,19 +4332,19 @@ static int deferred_step(zr_engine* e, double dt, zr_step_stats* st, bool& again
     again = rc == ZR_OK;
     return rc;
   }
-  e->A = run.hint;
+  e->A = run.hint;  // the launches' bounds, until sort_finish sets the counts
   e->S = run.smax;
   rc = ensure_grid(e);
-  if (rc) return rc;
   e->guard = StepGuard{ e->dcount, run.hint, run.smax };
   e->sorted = true;
-  rc = do_p2g(e, true, dt);
+  if (!rc) rc = do_p2g(e, true, dt);
   if (!rc) rc = do_grid(e, GRID_COMBINE_UPDATE, dt);
   e->defer_cfl = true;  // the flags are read below
   if (!rc) rc = do_g2p(e, dt, st, true);
   e->defer_cfl = false;
   e->guard = StepGuard{};
   e->sorted = e->rasterised = e->updated = false;
+  e->A = e->S = 0;
   if (!rc) rc = sync_counts(e);
   if (rc) return rc;
   if (e->hcount[CNT_GROUPS] > run.hint || e->hcount[CNT_SLOTS] > run.smax) {
