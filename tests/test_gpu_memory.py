@@ -40,10 +40,39 @@ def test_a_sort_that_finds_no_memory_leaves_nothing_behind():
     eng.upload(small)
     eng.advanceOneTimeStep(1e-5)
     eng.upload(s)
-    with device_memory_held(eng.L, 4 << 20):
+    with device_memory_held(eng.L, 8 << 20):
         with pytest.raises(ZrError, match="memory"):
             eng.advanceOneTimeStep(1e-5)
     for _ in range(2):
         eng.advanceOneTimeStep(1e-5)
+    _same(eng.download(), want)
+    eng.close()
+
+
+def test_a_grid_that_finds_no_memory_is_not_used():
+    """The grid's arrays are freed for larger ones (59 MB the smallest), which
+    are not to be had: the next step does not take the old capacity for
+    granted, nor an upload of as many particles the arrays of one that failed."""
+    cube = scenes.cube_scene_small(seed=3, ncells=8, lo_cell=80, dx=1.0 / 256)
+    eng, _ = make_pair(cube)
+    eng.advanceOneTimeStep(1e-4)
+    first = eng.download()
+    eng.advanceOneTimeStep(1e-4)
+    want = eng.download()
+    eng.upload(_spread(50000))
+    with device_memory_held(eng.L, 16 << 20):
+        with pytest.raises(ZrError, match="memory"):
+            eng.advanceOneTimeStep(1e-6)
+    eng.upload(dict(cube, **first))
+    eng.advanceOneTimeStep(1e-4)
+    _same(eng.download(), want)
+    with device_memory_held(eng.L, 8 << 20):
+        for _ in range(2):
+            with pytest.raises(ZrError, match="memory"):
+                eng.upload(_spread(300000))
+            with pytest.raises(ZrError, match="no particles"):
+                eng.advanceOneTimeStep(1e-4)
+    eng.upload(dict(cube, **first))
+    eng.advanceOneTimeStep(1e-4)
     _same(eng.download(), want)
     eng.close()

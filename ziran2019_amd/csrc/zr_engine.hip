@@ -1790,6 +1790,7 @@ int ensure_scan(zr_engine* e, uint32_t n)
   size_t nt = (n + kScanTile - 1) / kScanTile + 1;
   if (nt <= e->scan_cap) return ZR_OK;
   dfree(e->scan_tmp);
+  e->scan_cap = 0;
   ZR_HIP(e, hipMalloc(&e->scan_tmp, nt * sizeof(uint32_t)));
   e->scan_cap = nt;
   return ZR_OK;
@@ -1999,6 +2000,7 @@ int ensure_grid(zr_engine* e)
   size_t nodes = (size_t)e->S * 32;
   if (nodes > e->grid_cap) {
     dfree(e->gm); dfree(e->gv); dfree(e->gf); dfree(e->gvs);
+    e->grid_cap = 0;
     size_t cap = nodes + nodes / 4 + 1024;
     ZR_HIP(e, hipMalloc(&e->gm, cap * sizeof(double)));
     ZR_HIP(e, hipMalloc(&e->gv, 3 * cap * sizeof(double)));
@@ -2010,6 +2012,7 @@ int ensure_grid(zr_engine* e)
   }
   if ((size_t)e->A > e->stage_cap) {
     dfree(e->stage);
+    e->stage_cap = 0;
     size_t cap = (size_t)e->A + e->A / 4 + 64;
     ZR_HIP(e, hipMalloc(&e->stage, cap * kStageStride * sizeof(double)));
     e->stage_cap = cap;
@@ -2461,13 +2464,13 @@ int do_g2p(zr_engine* e, double dt, zr_step_stats* st, bool mls)
 // device scalars and flags of the Krylov solvers, with pinned host mirrors
 int ensure_scalars(zr_engine* e)
 {
-  if (!e->sc) {
-    ZR_HIP(e, hipMalloc(&e->sc, SC_N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->ci, CI_N * sizeof(int32_t)));
-    ZR_HIP(e, hipMalloc(&e->partial2, kCgBlocks * sizeof(double)));
+  if (!e->sc) ZR_HIP(e, hipMalloc(&e->sc, SC_N * sizeof(double)));
+  if (!e->ci) ZR_HIP(e, hipMalloc(&e->ci, CI_N * sizeof(int32_t)));
+  if (!e->partial2) ZR_HIP(e, hipMalloc(&e->partial2, kCgBlocks * sizeof(double)));
+  if (!e->hvp_bounds) ZR_HIP(e, hipMalloc(&e->hvp_bounds, 18 * sizeof(uint32_t)));
+  if (!e->hvp_ctr) {
     ZR_HIP(e, hipMalloc(&e->hvp_ctr, kHvpCounters * kHvpCounterStride * sizeof(uint32_t)));
     ZR_HIP(e, hipMemset(e->hvp_ctr, 0, kHvpCounters * kHvpCounterStride * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->hvp_bounds, 18 * sizeof(uint32_t)));
   }
   if (!e->hsolve) {
     ZR_HIP(e, hipHostMalloc(&e->hsolve, sizeof(HostScalars), hipHostMallocCoherent));
@@ -2926,6 +2929,7 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
   if (e->admm_n != n || e->admm_visco != visco) {
     const size_t rows = visco ? 41 : 22;
     dfree(e->admm_p);
+    e->admm_n = 0;
     ZR_HIP(e, hipMalloc(&e->admm_p, rows * N * sizeof(double)));
     ZR_HIP(e, hipMemsetAsync(e->admm_p, 0, rows * N * sizeof(double), s));
     e->admm_n = n;
@@ -2935,6 +2939,7 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
   if (e->admm_cap < e->grid_cap) {
     dfree(e->admm_node);
     dfree(e->admm_coll);
+    e->admm_cap = 0;
     ZR_HIP(e, hipMalloc(&e->admm_node, kAdmmNodeRows * e->grid_cap * sizeof(double)));
     ZR_HIP(e, hipMalloc(&e->admm_coll, e->grid_cap * sizeof(int32_t)));
     e->admm_cap = e->grid_cap;
@@ -2942,6 +2947,7 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
   size_t nb = (e->grid_cap + 255) / 256 + 1;
   if (nb > e->partial_cap) {
     dfree(e->partial);
+    e->partial_cap = 0;
     ZR_HIP(e, hipMalloc(&e->partial, nb * sizeof(double)));
     e->partial_cap = nb;
   }
@@ -3077,6 +3083,7 @@ int ensure_implicit(zr_engine* e, int32_t prec)
 {
   if (e->imp_cap < e->grid_cap) {
     double** arrs[] = { &e->ivn, &e->idv, &e->ir, &e->ix, &e->irc, &e->iq, &e->ip, &e->iap };
+    e->imp_cap = 0;
     for (auto a : arrs) {
       dfree(*a);
       ZR_HIP(e, hipMalloc(a, 3 * e->grid_cap * sizeof(double)));
@@ -3085,6 +3092,7 @@ int ensure_implicit(zr_engine* e, int32_t prec)
   }
   if (prec == ZR_FP32_REFINED && e->imp32_cap < e->grid_cap) {
     float** arrs[] = { &e->fx, &e->frc, &e->fq, &e->fp, &e->fap };
+    e->imp32_cap = 0;
     for (auto a : arrs) {
       dfree(*a);
       ZR_HIP(e, hipMalloc(a, 3 * e->grid_cap * sizeof(float)));
@@ -3094,6 +3102,7 @@ int ensure_implicit(zr_engine* e, int32_t prec)
   size_t nb = (e->grid_cap + 255) / 256 + 1;
   if (nb > e->partial_cap) {
     dfree(e->partial);
+    e->partial_cap = 0;
     ZR_HIP(e, hipMalloc(&e->partial, nb * sizeof(double)));
     e->partial_cap = nb;
   }
@@ -3102,16 +3111,19 @@ int ensure_implicit(zr_engine* e, int32_t prec)
   const size_t n = (size_t)(e->n > 0 ? e->n : 1);
   if (e->ccell_n != e->n) {
     dfree(e->ccell);
+    e->ccell_n = 0;
     ZR_HIP(e, hipMalloc(&e->ccell, n * sizeof(uint32_t)));
     e->ccell_n = e->n;
   }
   if (prec == ZR_FP64 && e->c64_n != e->n) {
     dfree(e->c64);
+    e->c64_n = 0;
     ZR_HIP(e, hipMalloc(&e->c64, 26 * n * sizeof(double)));
     e->c64_n = e->n;
   }
   if (prec == ZR_FP32_REFINED && e->c32_n != e->n) {
     dfree(e->c32);
+    e->c32_n = 0;
     ZR_HIP(e, hipMalloc(&e->c32, 26 * n * sizeof(float)));
     e->c32_n = e->n;
   }
@@ -3645,10 +3657,8 @@ double zr_get_time(const zr_engine* e) { return e ? e->time : 0.0; }
 int zr_eval_max_particle_speed(zr_engine* e, double* out)
 {
   if (!e || !out) return ZR_ERR_ARG;
-  if (!e->speed) {
-    ZR_HIP(e, hipHostMalloc(&e->hspeed, kSpeedFields * sizeof(double), hipHostMallocCoherent));
-    ZR_HIP(e, hipMalloc(&e->speed, kSpeedFields * kSpeedBlocks * sizeof(double)));
-  }
+  if (!e->hspeed) ZR_HIP(e, hipHostMalloc(&e->hspeed, kSpeedFields * sizeof(double), hipHostMallocCoherent));
+  if (!e->speed) ZR_HIP(e, hipMalloc(&e->speed, kSpeedFields * kSpeedBlocks * sizeof(double)));
   const uint32_t n = (uint32_t)e->n;
   uint32_t nb = blocks_for((uint64_t)n, 256);
   if (nb > kSpeedBlocks) nb = kSpeedBlocks;
@@ -3757,6 +3767,30 @@ int zr_eval_max_particle_speed_noalloc(const double* x, const double* v, int64_t
   return ZR_OK;
 }
 
+static int alloc_particles(zr_engine* e, size_t N)
+{
+  ZR_HIP(e, hipMalloc(&e->x, 3 * N * sizeof(double)));
+  ZR_HIP(e, hipMalloc(&e->v, 3 * N * sizeof(double)));
+  ZR_HIP(e, hipMalloc(&e->C, 9 * N * sizeof(double)));
+  ZR_HIP(e, hipMalloc(&e->F, 9 * N * sizeof(double)));
+  ZR_HIP(e, hipMalloc(&e->m, N * sizeof(double)));
+  ZR_HIP(e, hipMalloc(&e->vol, N * sizeof(double)));
+  ZR_HIP(e, hipMalloc(&e->mu, N * sizeof(double)));
+  ZR_HIP(e, hipMalloc(&e->lam, N * sizeof(double)));
+  ZR_HIP(e, hipMalloc(&e->p_page, N * sizeof(uint32_t)));
+  ZR_HIP(e, hipMalloc(&e->p_re, N * sizeof(uint32_t)));
+  ZR_HIP(e, hipMalloc(&e->order, N * sizeof(uint32_t)));
+  ZR_HIP(e, hipMalloc(&e->keys, N * sizeof(uint64_t)));
+  ZR_HIP(e, hipMalloc(&e->group_page, N * sizeof(uint32_t)));
+  ZR_HIP(e, hipMalloc(&e->group_count, N * sizeof(uint32_t)));
+  ZR_HIP(e, hipMalloc(&e->group_start, (N + 1) * sizeof(uint32_t)));
+  ZR_HIP(e, hipMalloc(&e->touch_page, 8 * N * sizeof(uint32_t)));
+  ZR_HIP(e, hipMalloc(&e->touch_slot, 8 * N * sizeof(uint32_t)));
+  ZR_HIP(e, hipMalloc(&e->slot_page, 8 * N * sizeof(uint32_t)));
+  ZR_HIP(e, hipMalloc(&e->group_nslot, 8 * N * sizeof(int32_t)));
+  return ZR_OK;
+}
+
 int zr_upload_particles(zr_engine* e, const zr_particles* p)
 {
   if (!e || !p || p->n < 0) return fail(e, ZR_ERR_ARG, "bad particle view");
@@ -3777,30 +3811,16 @@ int zr_upload_particles(zr_engine* e, const zr_particles* p)
   const bool keep = n > 0 && n == e->n && e->x;
   free_particles(e, keep);
   e->sorted = e->rasterised = e->updated = false;
-  e->n = n;
   if (n == 0) return ZR_OK;
   size_t N = (size_t)n;
   if (!keep) {
-    ZR_HIP(e, hipMalloc(&e->x, 3 * N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->v, 3 * N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->C, 9 * N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->F, 9 * N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->m, N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->vol, N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->mu, N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->lam, N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->p_page, N * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->p_re, N * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->order, N * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->keys, N * sizeof(uint64_t)));
-    ZR_HIP(e, hipMalloc(&e->group_page, N * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->group_count, N * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->group_start, (N + 1) * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->touch_page, 8 * N * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->touch_slot, 8 * N * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->slot_page, 8 * N * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->group_nslot, 8 * N * sizeof(int32_t)));
+    const int rc = alloc_particles(e, N);
+    if (rc) {  // none rather than some: an upload of as many would keep them
+      free_particles(e);
+      return rc;
+    }
   }
+  e->n = n;
   const HostArray items[] = { { p->X, e->x, 3 },    { p->V, e->v, 3 },     { p->C, e->C, 9 },   { p->F, e->F, 9 },
                               { p->mass, e->m, 1 }, { p->vol, e->vol, 1 }, { p->mu, e->mu, 1 }, { p->lambda, e->lam, 1 } };
   return transfer_arrays(e, items, 8, false, false);
@@ -3840,13 +3860,11 @@ int zr_set_materials(zr_engine* e, const zr_materials* mt)
   }
   if (plastic && (!mt->plastic_param || !mt->plastic_state))
     return fail(e, ZR_ERR_ARG, "plasticity needs plastic_param and plastic_state");
-  if (!e->mat) {
-    ZR_HIP(e, hipMalloc(&e->mat, N * sizeof(int32_t)));
-    ZR_HIP(e, hipMalloc(&e->pparam, 4 * N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->pstate, N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->gdeg, N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->broken, N * sizeof(int32_t)));
-  }
+  if (!e->pparam) ZR_HIP(e, hipMalloc(&e->pparam, 4 * N * sizeof(double)));
+  if (!e->pstate) ZR_HIP(e, hipMalloc(&e->pstate, N * sizeof(double)));
+  if (!e->gdeg) ZR_HIP(e, hipMalloc(&e->gdeg, N * sizeof(double)));
+  if (!e->broken) ZR_HIP(e, hipMalloc(&e->broken, N * sizeof(int32_t)));
+  if (!e->mat) ZR_HIP(e, hipMalloc(&e->mat, N * sizeof(int32_t)));  // the last: set once all are there
   std::vector<double> pp(4 * N, 0.0), ps(N, 0.0), g(N, 1.0);
   for (size_t i = 0; i < N; ++i) {
     for (int k = 0; k < 4; ++k)
@@ -3883,12 +3901,10 @@ int zr_set_viscoelastic(zr_engine* e, const double* F_neq, const double* mu, con
   const size_t N = (size_t)e->n;
   if (N == 0) return fail(e, ZR_ERR_STATE, "upload the particles before the viscoelastic branch");
   if (int rc_order = user_order(e)) return rc_order;
-  if (!e->fneq) {
-    ZR_HIP(e, hipMalloc(&e->fneq, 9 * N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->vtau_neq, 9 * N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->mu_neq, N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->lam_neq, N * sizeof(double)));
-  }
+  if (!e->fneq) ZR_HIP(e, hipMalloc(&e->fneq, 9 * N * sizeof(double)));
+  if (!e->vtau_neq) ZR_HIP(e, hipMalloc(&e->vtau_neq, 9 * N * sizeof(double)));
+  if (!e->mu_neq) ZR_HIP(e, hipMalloc(&e->mu_neq, N * sizeof(double)));
+  if (!e->lam_neq) ZR_HIP(e, hipMalloc(&e->lam_neq, N * sizeof(double)));
   std::vector<double> f(9 * N);
   for (size_t i = 0; i < N; ++i)
     for (int k = 0; k < 9; ++k) f[k * N + i] = F_neq ? F_neq[9 * i + k] : (k % 4 == 0 ? 1.0 : 0.0);
