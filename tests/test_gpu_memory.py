@@ -76,3 +76,58 @@ def test_a_grid_that_finds_no_memory_is_not_used():
     eng.advanceOneTimeStep(1e-4)
     _same(eng.download(), want)
     eng.close()
+
+
+def _shuffled(n):
+    s = scenes.cube_scene(dx=1.0 / 128, lo_cell=40, ncells=34)
+    p = np.random.default_rng(6).permutation(len(s["mass"]))[:n]
+    return {k: (np.ascontiguousarray(v[p]) if isinstance(v, np.ndarray) else v) for k, v in s.items()}
+
+
+def test_particles_stay_where_their_second_copy_finds_no_memory():
+    """A shuffled set is moved at its second step where there is memory for a
+    second copy (71 MB)."""
+    s = _shuffled(300000)
+    outs = []
+    for left in (None, 8 << 20):
+        eng, _ = make_pair(s, colliders=s["colliders"])
+        eng.advanceOneTimeStep(1e-4)
+        if left is None:
+            for _ in range(3):
+                eng.advanceOneTimeStep(1e-4)
+        else:
+            with device_memory_held(eng.L, left):
+                for _ in range(3):
+                    eng.advanceOneTimeStep(1e-4)
+        outs.append(eng.download())
+        eng.close()
+    _same(*outs)
+
+
+def test_second_copies_are_given_back():
+    """A call that needs memory takes that of the second copies (71 MB, the
+    checkpoint 58 MB); without them the caller's order is restored row by row."""
+    s = _shuffled(300000)
+    ref, _ = make_pair(s, colliders=s["colliders"])
+    eng, _ = make_pair(s, colliders=s["colliders"])
+    for e in (ref, eng):
+        for _ in range(3):
+            e.advanceOneTimeStep(1e-4)
+    want = ref.download()
+    ref.advanceOneTimeStep(1e-4)
+    after = ref.download()
+    ref.sortParticlesAndPolluteGrid()
+    order = ref.dump("order")
+    ref.close()
+    with device_memory_held(eng.L, 8 << 20):
+        eng.checkpoint_save(0)
+        eng.sortParticlesAndPolluteGrid()
+        eng.dump("order")  # in the caller's order from here on
+        _same(eng.download(), want)
+        eng.advanceOneTimeStep(1e-4)
+        _same(eng.download(), after)
+        eng.sortParticlesAndPolluteGrid()
+        assert np.array_equal(eng.dump("order"), order)
+        eng.checkpoint_restore(0)
+        _same(eng.download(), want)
+    eng.close()

@@ -1705,6 +1705,7 @@ struct zr_engine {
   int io_threads = 0;
   hipEvent_t io_ev[kIoThreads] = {};
   bool permuted = false;
+  bool no_moves = false;  // there was no memory for the second copies
   uint32_t* uid = nullptr;
   struct Spare {
     void* p = nullptr;
@@ -1785,13 +1786,45 @@ void dfree(T*& p)
   p = nullptr;
 }
 
+// the memory that no result depends on: the second copies of a move, and the
+// buffers that an upload kept for the next use; whether there was any
+bool give_back(zr_engine* e)
+{
+  bool any = e->adj_spare != nullptr;
+  for (auto& a : e->alt) {
+    any = any || a.p;
+    dfree(a.p);
+    a.bytes = 0;
+  }
+  for (auto& c : e->ckpt_spare) {
+    any = true;
+    dfree(c);
+  }
+  e->ckpt_spare.clear();
+  dfree(e->adj_spare);
+  return any;
+}
+
+// device memory, if need be that of give_back
+template <class T>
+hipError_t dev_malloc(zr_engine* e, T** p, size_t bytes)
+{
+  hipError_t st = hipMalloc(p, bytes);
+  if (st == hipErrorOutOfMemory && give_back(e)) {
+    (void)hipGetLastError();
+    st = hipMalloc(p, bytes);
+  }
+  if (st != hipSuccess) *p = nullptr;
+  return st;
+}
+
 int ensure_scan(zr_engine* e, uint32_t n)
 {
   size_t nt = (n + kScanTile - 1) / kScanTile + 1;
   if (nt <= e->scan_cap) return ZR_OK;
   dfree(e->scan_tmp);
   e->scan_cap = 0;
-  ZR_HIP(e, hipMalloc(&e->scan_tmp, nt * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->scan_tmp, nt * sizeof(uint32_t)));
   e->scan_cap = nt;
   return ZR_OK;
 }
@@ -1896,7 +1929,7 @@ void free_particles(zr_engine* e, bool keep = false)
   }
   e->ckpt.clear();
   e->ckpt_time.clear();
-  e->permuted = false;
+  e->permuted = e->no_moves = false;
   e->disorder = 0.0;
   e->move_next = false;
   e->adj_n = 0;
@@ -2002,19 +2035,19 @@ int ensure_grid(zr_engine* e)
     dfree(e->gm); dfree(e->gv); dfree(e->gf); dfree(e->gvs);
     e->grid_cap = 0;
     size_t cap = nodes + nodes / 4 + 1024;
-    ZR_HIP(e, hipMalloc(&e->gm, cap * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->gv, 3 * cap * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->gf, 3 * cap * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->gvs, 3 * cap * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->gm, cap * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->gv, 3 * cap * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->gf, 3 * cap * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->gvs, 3 * cap * sizeof(double)));
     dfree(e->slot_src);
-    ZR_HIP(e, hipMalloc(&e->slot_src, (cap / 32 + 1) * 8 * sizeof(int32_t)));
+    ZR_HIP(e, dev_malloc(e, &e->slot_src, (cap / 32 + 1) * 8 * sizeof(int32_t)));
     e->grid_cap = cap;
   }
   if ((size_t)e->A > e->stage_cap) {
     dfree(e->stage);
     e->stage_cap = 0;
     size_t cap = (size_t)e->A + e->A / 4 + 64;
-    ZR_HIP(e, hipMalloc(&e->stage, cap * kStageStride * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->stage, cap * kStageStride * sizeof(double)));
     e->stage_cap = cap;
   }
   return ZR_OK;
@@ -2040,7 +2073,7 @@ int sort_groups(zr_engine* e, uint32_t hint)
     dfree(e->cell_off);
     e->cell_cap = 0;
     const size_t cap = (size_t)hint + hint / 4 + 64;
-    ZR_HIP(e, hipMalloc(&e->cell_off, 32 * cap * sizeof(uint32_t)));
+    ZR_HIP(e, dev_malloc(e, &e->cell_off, 32 * cap * sizeof(uint32_t)));
     e->cell_cap = cap;
   }
   k_sort_groups<<<hint, 256, 0, s>>>(e->keys, e->group_start, e->order, e->cell_off, gb, e->dcount, e->group_page,
@@ -2106,26 +2139,40 @@ std::vector<ParticleArray> particle_arrays(zr_engine* e)
            { v(e->uid), -1 } };
 }
 
-int move_particles(zr_engine* e, const uint32_t* from, const uint32_t* to)
+size_t row_bytes(const zr_engine* e, const ParticleArray& a) { return (size_t)e->n * (a.rows > 0 ? 8 : 4); }
+
+// a second copy of every array for move_particles; false, with none left,
+// where there is no memory for them
+bool second_copies(zr_engine* e, const std::vector<ParticleArray>& arrays)
 {
-  const std::vector<ParticleArray> arrays = particle_arrays(e);
   if (e->alt.size() != arrays.size()) e->alt.resize(arrays.size());
+  for (size_t q = 0; q < arrays.size(); ++q) {
+    if (!*arrays[q].p) continue;
+    const size_t bytes = row_bytes(e, arrays[q]) * (size_t)(arrays[q].rows > 0 ? arrays[q].rows : 1);
+    zr_engine::Spare& a = e->alt[q];
+    if (a.bytes == bytes) continue;
+    dfree(a.p);  // an array whose size changed (the ADMM state)
+    a.bytes = 0;
+    if (hipMalloc(&a.p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      a.p = nullptr;
+      give_back(e);
+      return false;
+    }
+    a.bytes = bytes;
+  }
+  return true;
+}
+
+int move_particles(zr_engine* e, const std::vector<ParticleArray>& arrays, const uint32_t* from, const uint32_t* to)
+{
   MoveList L{};
   static_assert(kMoveArrays >= 28, "one entry per array");
-  size_t bytes[kMoveArrays];
   for (size_t q = 0; q < arrays.size(); ++q) {
-    const ParticleArray& a = arrays[q];
-    if (!*a.p) continue;
-    bytes[q] = (size_t)e->n * (a.rows > 0 ? 8 * (size_t)a.rows : 4);
-    if (e->alt[q].bytes != bytes[q]) {  // an array whose size changed (the ADMM state) needs a spare of its own size
-      dfree(e->alt[q].p);
-      e->alt[q].bytes = 0;
-      ZR_HIP(e, hipMalloc(&e->alt[q].p, bytes[q]));
-      e->alt[q].bytes = bytes[q];
-    }
-    L.src[L.count] = *a.p;
+    if (!*arrays[q].p) continue;
+    L.src[L.count] = *arrays[q].p;
     L.dst[L.count] = e->alt[q].p;
-    L.rows[L.count++] = a.rows;
+    L.rows[L.count++] = arrays[q].rows;
   }
   k_move<<<blocks_for((uint64_t)e->n, 256), 256, 0, e->stream>>>(L, (uint32_t)e->n, from, to);
   ZR_LAUNCH_CHECK(e);
@@ -2134,41 +2181,58 @@ int move_particles(zr_engine* e, const uint32_t* from, const uint32_t* to)
   return ZR_OK;
 }
 
+// one row of n values (rows as in ParticleArray) into the caller's order, in
+// the sort's key array (8 bytes per particle, written again before every use)
+int row_to_keys(zr_engine* e, const void* dev, int rows)
+{
+  MoveList L{};
+  L.src[0] = dev;
+  L.dst[0] = e->keys;
+  L.rows[0] = rows > 0 ? 1 : -1;
+  L.count = 1;
+  k_move<<<blocks_for((uint64_t)e->n, 256), 256, 0, e->stream>>>(L, (uint32_t)e->n, nullptr, e->uid);
+  ZR_LAUNCH_CHECK(e);
+  return ZR_OK;
+}
+
 // The particles into the order of the sort that has just run: the transfers
 // of this step and the next then read and write neighbouring places.  A
 // particle's results do not depend on it (the sort's ties go by the caller's
-// index).
+// index), and where there is no memory for the second copies (as much again as
+// the particles' arrays: 236 bytes per particle without options) the particles
+// stay where they are until another set is uploaded.
 int order_particles(zr_engine* e)
 {
   const uint32_t n = (uint32_t)e->n, nb = blocks_for(n, 256);
-  if (!e->uid) ZR_HIP(e, hipMalloc(&e->uid, (size_t)n * sizeof(uint32_t)));
-  int rc = move_particles(e, e->order, nullptr);
+  e->disorder = 0.0;
+  e->move_next = false;
+  if (!e->uid && hipMalloc(&e->uid, (size_t)n * sizeof(uint32_t)) != hipSuccess) {
+    (void)hipGetLastError();
+    e->uid = nullptr;
+  }
+  const std::vector<ParticleArray> arrays = particle_arrays(e);
+  if (!e->uid || !second_copies(e, arrays)) {
+    e->no_moves = true;
+    return ZR_OK;
+  }
+  int rc = move_particles(e, arrays, e->order, nullptr);
   if (rc) return rc;
   k_iota_order<<<nb, 256, 0, e->stream>>>(n, e->order, e->uid, e->permuted ? 0 : 1);
   ZR_LAUNCH_CHECK(e);
   e->permuted = true;
-  e->disorder = 0.0;
-  e->move_next = false;
   return ZR_OK;
 }
 
 // one row of n values (rows as in ParticleArray) to the caller's array in the
-// caller's order, through the sort's key array as scratch (8 bytes per
-// particle, written again before every use)
+// caller's order
 int download_row(zr_engine* e, void* host, const void* dev, int rows)
 {
-  const uint32_t n = (uint32_t)e->n;
   if (e->permuted) {
-    MoveList L{};
-    L.src[0] = dev;
-    L.dst[0] = e->keys;
-    L.rows[0] = rows;
-    L.count = 1;
-    k_move<<<blocks_for(n, 256), 256, 0, e->stream>>>(L, n, nullptr, e->uid);
-    ZR_LAUNCH_CHECK(e);
+    int rc = row_to_keys(e, dev, rows);
+    if (rc) return rc;
     dev = e->keys;
   }
-  ZR_HIP(e, hipMemcpyAsync(host, dev, (size_t)n * (rows > 0 ? 8 : 4), hipMemcpyDeviceToHost, e->stream));
+  ZR_HIP(e, hipMemcpyAsync(host, dev, (size_t)e->n * (rows > 0 ? 8 : 4), hipMemcpyDeviceToHost, e->stream));
   ZR_HIP(e, hipStreamSynchronize(e->stream));
   return ZR_OK;
 }
@@ -2179,8 +2243,23 @@ int user_order(zr_engine* e)
 {
   if (!e->permuted) return ZR_OK;
   const uint32_t n = (uint32_t)e->n;
+  const std::vector<ParticleArray> arrays = particle_arrays(e);
+  const bool copies = second_copies(e, arrays);
   k_user_order<<<blocks_for(n, 256), 256, 0, e->stream>>>(n, e->order, e->uid);
-  int rc = move_particles(e, nullptr, e->uid);
+  int rc = ZR_OK;
+  if (copies)
+    rc = move_particles(e, arrays, nullptr, e->uid);
+  else  // row by row
+    for (const ParticleArray& a : arrays) {
+      if (!*a.p || *a.p == e->uid) continue;  // uid gives the places, and means nothing from here on
+      const size_t bytes = row_bytes(e, a);
+      for (int r = 0; r < (a.rows > 0 ? a.rows : 1); ++r) {
+        char* const row = static_cast<char*>(*a.p) + (size_t)r * bytes;
+        if (!rc) rc = row_to_keys(e, row, a.rows);
+        if (rc) return rc;
+        ZR_HIP(e, hipMemcpyAsync(row, e->keys, bytes, hipMemcpyDeviceToDevice, e->stream));
+      }
+    }
   if (rc) return rc;
   e->permuted = false;
   e->disorder = 0.0;
@@ -2200,7 +2279,7 @@ int user_order(zr_engine* e)
 // move's launches cost more than they give.
 void note_disorder(zr_engine* e)
 {
-  if (e->n < (int64_t)kMoveMin || !e->hcount[CNT_SAMPLED]) return;
+  if (e->no_moves || e->n < (int64_t)kMoveMin || !e->hcount[CNT_SAMPLED]) return;
   e->disorder += (double)e->hcount[CNT_BREAKS] / (double)e->hcount[CNT_SAMPLED];
   e->move_next = e->disorder >= kDisorder;
 }
@@ -2464,12 +2543,12 @@ int do_g2p(zr_engine* e, double dt, zr_step_stats* st, bool mls)
 // device scalars and flags of the Krylov solvers, with pinned host mirrors
 int ensure_scalars(zr_engine* e)
 {
-  if (!e->sc) ZR_HIP(e, hipMalloc(&e->sc, SC_N * sizeof(double)));
-  if (!e->ci) ZR_HIP(e, hipMalloc(&e->ci, CI_N * sizeof(int32_t)));
-  if (!e->partial2) ZR_HIP(e, hipMalloc(&e->partial2, kCgBlocks * sizeof(double)));
-  if (!e->hvp_bounds) ZR_HIP(e, hipMalloc(&e->hvp_bounds, 18 * sizeof(uint32_t)));
+  if (!e->sc) ZR_HIP(e, dev_malloc(e, &e->sc, SC_N * sizeof(double)));
+  if (!e->ci) ZR_HIP(e, dev_malloc(e, &e->ci, CI_N * sizeof(int32_t)));
+  if (!e->partial2) ZR_HIP(e, dev_malloc(e, &e->partial2, kCgBlocks * sizeof(double)));
+  if (!e->hvp_bounds) ZR_HIP(e, dev_malloc(e, &e->hvp_bounds, 18 * sizeof(uint32_t)));
   if (!e->hvp_ctr) {
-    ZR_HIP(e, hipMalloc(&e->hvp_ctr, kHvpCounters * kHvpCounterStride * sizeof(uint32_t)));
+    ZR_HIP(e, dev_malloc(e, &e->hvp_ctr, kHvpCounters * kHvpCounterStride * sizeof(uint32_t)));
     ZR_HIP(e, hipMemset(e->hvp_ctr, 0, kHvpCounters * kHvpCounterStride * sizeof(uint32_t)));
   }
   if (!e->hsolve) {
@@ -2556,10 +2635,10 @@ int do_pf(zr_engine* e, double dt)
   if (e->pf_node_cap < e->grid_cap) {
     dfree(e->pf_node);
     e->pf_node_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->pf_node, 7 * e->grid_cap * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->pf_node, 7 * e->grid_cap * sizeof(double)));
     e->pf_node_cap = e->grid_cap;
   }
-  if (!e->pf_partial) ZR_HIP(e, hipMalloc(&e->pf_partial, 2 * kCgBlocks * sizeof(double)));
+  if (!e->pf_partial) ZR_HIP(e, dev_malloc(e, &e->pf_partial, 2 * kCgBlocks * sizeof(double)));
   const size_t C = e->pf_node_cap;
   double *phase = e->pf_node, *diag = phase + C, *x = diag + C, *r = x + C, *mr = r + C, *sv = mr + C, *q = sv + C;
   const double dx = e->cfg.dx;
@@ -2616,7 +2695,7 @@ int ensure_adjoint(zr_engine* e)
     if (e->adj_spare)
       std::swap(e->adj, e->adj_spare);  // as large: kept by the upload
     else
-      ZR_HIP(e, hipMalloc(&e->adj, kAdjRows * (size_t)e->n * sizeof(double)));
+      ZR_HIP(e, dev_malloc(e, &e->adj, kAdjRows * (size_t)e->n * sizeof(double)));
     ZR_HIP(e, hipMemsetAsync(e->adj, 0, kAdjRows * (size_t)e->n * sizeof(double), e->stream));
     e->adj_n = e->n;
   }
@@ -2675,7 +2754,7 @@ int adjoint_kernels(zr_engine* e, double dt, const AdjTables& t)
   if (e->adj_grid_cap < (size_t)t.stride) {
     dfree(e->adj_grid);
     e->adj_grid_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->adj_grid, kAdjGridFields * (size_t)t.stride * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->adj_grid, kAdjGridFields * (size_t)t.stride * sizeof(double)));
     e->adj_grid_cap = (size_t)t.stride;
   }
   if ((size_t)t.A > e->stage_cap) return fail(e, ZR_ERR_STATE, "adjoint: staging buffer below the step's groups");
@@ -2771,7 +2850,7 @@ int record_step(zr_engine* e, zr_engine::StepRecord& r)
     dfree(r.buf);
     r.cap = 0;
     const size_t cap = L.bytes + L.bytes / 4 + 4096;
-    ZR_HIP(e, hipMalloc(&r.buf, cap));
+    ZR_HIP(e, dev_malloc(e, &r.buf, cap));
     r.cap = cap;
   }
   r.A = e->A;
@@ -2930,7 +3009,7 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
     const size_t rows = visco ? 41 : 22;
     dfree(e->admm_p);
     e->admm_n = 0;
-    ZR_HIP(e, hipMalloc(&e->admm_p, rows * N * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->admm_p, rows * N * sizeof(double)));
     ZR_HIP(e, hipMemsetAsync(e->admm_p, 0, rows * N * sizeof(double), s));
     e->admm_n = n;
     e->admm_visco = visco;
@@ -2940,15 +3019,15 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
     dfree(e->admm_node);
     dfree(e->admm_coll);
     e->admm_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->admm_node, kAdmmNodeRows * e->grid_cap * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->admm_coll, e->grid_cap * sizeof(int32_t)));
+    ZR_HIP(e, dev_malloc(e, &e->admm_node, kAdmmNodeRows * e->grid_cap * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->admm_coll, e->grid_cap * sizeof(int32_t)));
     e->admm_cap = e->grid_cap;
   }
   size_t nb = (e->grid_cap + 255) / 256 + 1;
   if (nb > e->partial_cap) {
     dfree(e->partial);
     e->partial_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->partial, nb * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->partial, nb * sizeof(double)));
     e->partial_cap = nb;
   }
   const int64_t C = (int64_t)e->admm_cap;
@@ -2999,15 +3078,15 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
       dfree(e->admm_c32);
       dfree(e->admm_cell32);
       e->admm_c32_cap = 0;
-      ZR_HIP(e, hipMalloc(&e->admm_c32, rows * N * sizeof(float)));
-      ZR_HIP(e, hipMalloc(&e->admm_cell32, N));
+      ZR_HIP(e, dev_malloc(e, &e->admm_c32, rows * N * sizeof(float)));
+      ZR_HIP(e, dev_malloc(e, &e->admm_cell32, N));
       e->admm_c32_cap = N;
       e->admm_c32_rows = rows;
     }
     if (e->admm_node32_cap < (size_t)C) {
       dfree(e->admm_node32);
       e->admm_node32_cap = 0;
-      ZR_HIP(e, hipMalloc(&e->admm_node32, 21 * (size_t)C * sizeof(float)));
+      ZR_HIP(e, dev_malloc(e, &e->admm_node32, 21 * (size_t)C * sizeof(float)));
       e->admm_node32_cap = (size_t)C;
     }
     float* c = e->admm_c32;
@@ -3031,15 +3110,15 @@ int do_admm(zr_engine* e, double dt, const zr_admm_opts* o, zr_admm_stats* st)
   if (e->be_fb_cap < N) {
     dfree(e->be_fb);
     e->be_fb_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->be_fb, 9 * N * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->be_fb, 9 * N * sizeof(double)));
     e->be_fb_cap = N;
   }
   if (e->admm_before_cap < N) {
     dfree(e->admm_before);
     dfree(e->admm_differs);
     e->admm_before_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->admm_before, 9 * N * sizeof(double)));
-    ZR_HIP(e, hipMalloc(&e->admm_differs, N));
+    ZR_HIP(e, dev_malloc(e, &e->admm_before, 9 * N * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->admm_differs, N));
     e->admm_before_cap = N;
   }
   const AdmmBefore before{ e->admm_before, e->admm_differs };
@@ -3086,7 +3165,7 @@ int ensure_implicit(zr_engine* e, int32_t prec)
     e->imp_cap = 0;
     for (auto a : arrs) {
       dfree(*a);
-      ZR_HIP(e, hipMalloc(a, 3 * e->grid_cap * sizeof(double)));
+      ZR_HIP(e, dev_malloc(e, a, 3 * e->grid_cap * sizeof(double)));
     }
     e->imp_cap = e->grid_cap;
   }
@@ -3095,7 +3174,7 @@ int ensure_implicit(zr_engine* e, int32_t prec)
     e->imp32_cap = 0;
     for (auto a : arrs) {
       dfree(*a);
-      ZR_HIP(e, hipMalloc(a, 3 * e->grid_cap * sizeof(float)));
+      ZR_HIP(e, dev_malloc(e, a, 3 * e->grid_cap * sizeof(float)));
     }
     e->imp32_cap = e->grid_cap;
   }
@@ -3103,7 +3182,7 @@ int ensure_implicit(zr_engine* e, int32_t prec)
   if (nb > e->partial_cap) {
     dfree(e->partial);
     e->partial_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->partial, nb * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->partial, nb * sizeof(double)));
     e->partial_cap = nb;
   }
   int rc = ensure_scalars(e);
@@ -3112,19 +3191,19 @@ int ensure_implicit(zr_engine* e, int32_t prec)
   if (e->ccell_n != e->n) {
     dfree(e->ccell);
     e->ccell_n = 0;
-    ZR_HIP(e, hipMalloc(&e->ccell, n * sizeof(uint32_t)));
+    ZR_HIP(e, dev_malloc(e, &e->ccell, n * sizeof(uint32_t)));
     e->ccell_n = e->n;
   }
   if (prec == ZR_FP64 && e->c64_n != e->n) {
     dfree(e->c64);
     e->c64_n = 0;
-    ZR_HIP(e, hipMalloc(&e->c64, 26 * n * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->c64, 26 * n * sizeof(double)));
     e->c64_n = e->n;
   }
   if (prec == ZR_FP32_REFINED && e->c32_n != e->n) {
     dfree(e->c32);
     e->c32_n = 0;
-    ZR_HIP(e, hipMalloc(&e->c32, 26 * n * sizeof(float)));
+    ZR_HIP(e, dev_malloc(e, &e->c32, 26 * n * sizeof(float)));
     e->c32_n = e->n;
   }
   return ZR_OK;
@@ -3197,7 +3276,7 @@ int be_state_residual(zr_engine* e, bool jac = false)
     if (e->be_fb_cap < N) {
       dfree(e->be_fb);
       e->be_fb_cap = 0;
-      ZR_HIP(e, hipMalloc(&e->be_fb, 9 * N * sizeof(double)));
+      ZR_HIP(e, dev_malloc(e, &e->be_fb, 9 * N * sizeof(double)));
       e->be_fb_cap = N;
     }
     const HvpCache<T> hc = hvp_cache<T>(e);
@@ -3256,14 +3335,14 @@ int ensure_jacobi(zr_engine* e)
   if (e->jac_cap < e->grid_cap) {
     dfree(e->pinv);
     e->jac_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->pinv, 3 * e->grid_cap * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->pinv, 3 * e->grid_cap * sizeof(double)));
     e->jac_cap = e->grid_cap;
   }
   if (e->jstage_cap < (size_t)e->A || !e->jstage) {
     dfree(e->jstage);
     e->jstage_cap = 0;
     const size_t cap = (size_t)e->A + e->A / 4 + 64;
-    ZR_HIP(e, hipMalloc(&e->jstage, cap * kImpStage * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->jstage, cap * kImpStage * sizeof(double)));
     e->jstage_cap = cap;
   }
   return ZR_OK;
@@ -3340,7 +3419,7 @@ int be_minres(zr_engine* e, double rel, const zr_implicit_opts* o, int& iters)
   if (V::extra_cap(e) < e->grid_cap) {
     dfree(V::extra(e));
     V::extra_cap(e) = 0;
-    ZR_HIP(e, hipMalloc(&V::extra(e), 9 * e->grid_cap * sizeof(T)));
+    ZR_HIP(e, dev_malloc(e, &V::extra(e), 9 * e->grid_cap * sizeof(T)));
     V::extra_cap(e) = e->grid_cap;
   }
   T* ex = V::extra(e);
@@ -3434,8 +3513,8 @@ int do_be(zr_engine* e, double dt, const zr_implicit_opts* o, zr_implicit_stats*
       dfree(e->cell_order);
       e->hvp_order_cap = 0;
       const size_t cap = (size_t)e->A + e->A / 4 + 64;
-      ZR_HIP(e, hipMalloc(&e->hvp_order, 2 * cap * sizeof(uint32_t)));
-      ZR_HIP(e, hipMalloc(&e->cell_order, cap * kCells));
+      ZR_HIP(e, dev_malloc(e, &e->hvp_order, 2 * cap * sizeof(uint32_t)));
+      ZR_HIP(e, dev_malloc(e, &e->cell_order, cap * kCells));
       e->hvp_order_cap = cap;
     }
     k_xcd_split<<<1, 1024, 0, e->stream>>>(e->group_start, e->A, n32, n64, e->hvp_bounds, e->hvp_order);
@@ -3453,7 +3532,7 @@ int do_be(zr_engine* e, double dt, const zr_implicit_opts* o, zr_implicit_stats*
   if (e->collided_cap < e->grid_cap) {  // nodes a collider touches, for the Jacobi preconditioner
     dfree(e->collided);
     e->collided_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->collided, e->grid_cap));
+    ZR_HIP(e, dev_malloc(e, &e->collided, e->grid_cap));
     e->collided_cap = e->grid_cap;
   }
   const uint32_t nn = e->S * 32, nb = blocks_for(nn, 256);
@@ -3469,8 +3548,8 @@ int do_be(zr_engine* e, double dt, const zr_implicit_opts* o, zr_implicit_stats*
     dfree(e->act);
     dfree(e->act_scan);
     e->act_cap = 0;
-    ZR_HIP(e, hipMalloc(&e->act, e->grid_cap * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&e->act_scan, e->grid_cap * sizeof(uint32_t)));
+    ZR_HIP(e, dev_malloc(e, &e->act, e->grid_cap * sizeof(uint32_t)));
+    ZR_HIP(e, dev_malloc(e, &e->act_scan, e->grid_cap * sizeof(uint32_t)));
     e->act_cap = e->grid_cap;
   }
   rc = run_scan(e, LdNonzeroMass{ e->gm }, nn, e->act_scan, e->dcount + CNT_TOTAL);
@@ -3658,7 +3737,7 @@ int zr_eval_max_particle_speed(zr_engine* e, double* out)
 {
   if (!e || !out) return ZR_ERR_ARG;
   if (!e->hspeed) ZR_HIP(e, hipHostMalloc(&e->hspeed, kSpeedFields * sizeof(double), hipHostMallocCoherent));
-  if (!e->speed) ZR_HIP(e, hipMalloc(&e->speed, kSpeedFields * kSpeedBlocks * sizeof(double)));
+  if (!e->speed) ZR_HIP(e, dev_malloc(e, &e->speed, kSpeedFields * kSpeedBlocks * sizeof(double)));
   const uint32_t n = (uint32_t)e->n;
   uint32_t nb = blocks_for((uint64_t)n, 256);
   if (nb > kSpeedBlocks) nb = kSpeedBlocks;
@@ -3769,25 +3848,25 @@ int zr_eval_max_particle_speed_noalloc(const double* x, const double* v, int64_t
 
 static int alloc_particles(zr_engine* e, size_t N)
 {
-  ZR_HIP(e, hipMalloc(&e->x, 3 * N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->v, 3 * N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->C, 9 * N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->F, 9 * N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->m, N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->vol, N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->mu, N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->lam, N * sizeof(double)));
-  ZR_HIP(e, hipMalloc(&e->p_page, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->p_re, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->order, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->keys, N * sizeof(uint64_t)));
-  ZR_HIP(e, hipMalloc(&e->group_page, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->group_count, N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->group_start, (N + 1) * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->touch_page, 8 * N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->touch_slot, 8 * N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->slot_page, 8 * N * sizeof(uint32_t)));
-  ZR_HIP(e, hipMalloc(&e->group_nslot, 8 * N * sizeof(int32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->x, 3 * N * sizeof(double)));
+  ZR_HIP(e, dev_malloc(e, &e->v, 3 * N * sizeof(double)));
+  ZR_HIP(e, dev_malloc(e, &e->C, 9 * N * sizeof(double)));
+  ZR_HIP(e, dev_malloc(e, &e->F, 9 * N * sizeof(double)));
+  ZR_HIP(e, dev_malloc(e, &e->m, N * sizeof(double)));
+  ZR_HIP(e, dev_malloc(e, &e->vol, N * sizeof(double)));
+  ZR_HIP(e, dev_malloc(e, &e->mu, N * sizeof(double)));
+  ZR_HIP(e, dev_malloc(e, &e->lam, N * sizeof(double)));
+  ZR_HIP(e, dev_malloc(e, &e->p_page, N * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->p_re, N * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->order, N * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->keys, N * sizeof(uint64_t)));
+  ZR_HIP(e, dev_malloc(e, &e->group_page, N * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->group_count, N * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->group_start, (N + 1) * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->touch_page, 8 * N * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->touch_slot, 8 * N * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->slot_page, 8 * N * sizeof(uint32_t)));
+  ZR_HIP(e, dev_malloc(e, &e->group_nslot, 8 * N * sizeof(int32_t)));
   return ZR_OK;
 }
 
@@ -3860,11 +3939,11 @@ int zr_set_materials(zr_engine* e, const zr_materials* mt)
   }
   if (plastic && (!mt->plastic_param || !mt->plastic_state))
     return fail(e, ZR_ERR_ARG, "plasticity needs plastic_param and plastic_state");
-  if (!e->pparam) ZR_HIP(e, hipMalloc(&e->pparam, 4 * N * sizeof(double)));
-  if (!e->pstate) ZR_HIP(e, hipMalloc(&e->pstate, N * sizeof(double)));
-  if (!e->gdeg) ZR_HIP(e, hipMalloc(&e->gdeg, N * sizeof(double)));
-  if (!e->broken) ZR_HIP(e, hipMalloc(&e->broken, N * sizeof(int32_t)));
-  if (!e->mat) ZR_HIP(e, hipMalloc(&e->mat, N * sizeof(int32_t)));  // the last: set once all are there
+  if (!e->pparam) ZR_HIP(e, dev_malloc(e, &e->pparam, 4 * N * sizeof(double)));
+  if (!e->pstate) ZR_HIP(e, dev_malloc(e, &e->pstate, N * sizeof(double)));
+  if (!e->gdeg) ZR_HIP(e, dev_malloc(e, &e->gdeg, N * sizeof(double)));
+  if (!e->broken) ZR_HIP(e, dev_malloc(e, &e->broken, N * sizeof(int32_t)));
+  if (!e->mat) ZR_HIP(e, dev_malloc(e, &e->mat, N * sizeof(int32_t)));  // the last: set once all are there
   std::vector<double> pp(4 * N, 0.0), ps(N, 0.0), g(N, 1.0);
   for (size_t i = 0; i < N; ++i) {
     for (int k = 0; k < 4; ++k)
@@ -3901,10 +3980,10 @@ int zr_set_viscoelastic(zr_engine* e, const double* F_neq, const double* mu, con
   const size_t N = (size_t)e->n;
   if (N == 0) return fail(e, ZR_ERR_STATE, "upload the particles before the viscoelastic branch");
   if (int rc_order = user_order(e)) return rc_order;
-  if (!e->fneq) ZR_HIP(e, hipMalloc(&e->fneq, 9 * N * sizeof(double)));
-  if (!e->vtau_neq) ZR_HIP(e, hipMalloc(&e->vtau_neq, 9 * N * sizeof(double)));
-  if (!e->mu_neq) ZR_HIP(e, hipMalloc(&e->mu_neq, N * sizeof(double)));
-  if (!e->lam_neq) ZR_HIP(e, hipMalloc(&e->lam_neq, N * sizeof(double)));
+  if (!e->fneq) ZR_HIP(e, dev_malloc(e, &e->fneq, 9 * N * sizeof(double)));
+  if (!e->vtau_neq) ZR_HIP(e, dev_malloc(e, &e->vtau_neq, 9 * N * sizeof(double)));
+  if (!e->mu_neq) ZR_HIP(e, dev_malloc(e, &e->mu_neq, N * sizeof(double)));
+  if (!e->lam_neq) ZR_HIP(e, dev_malloc(e, &e->lam_neq, N * sizeof(double)));
   std::vector<double> f(9 * N);
   for (size_t i = 0; i < N; ++i)
     for (int k = 0; k < 9; ++k) f[k * N + i] = F_neq ? F_neq[9 * i + k] : (k % 4 == 0 ? 1.0 : 0.0);
@@ -3987,11 +4066,11 @@ int zr_set_phase_field(zr_engine* e, const zr_phase_field* pf, const zr_phase_fi
   const double dflt[] = { 1.0, 0.0, 0.0, 0.0, 1.0, HUGE_VAL, 0.001, 0.0 };
   std::vector<double> tmp(N);
   for (int a = 0; a < 8; ++a) {
-    if (!*dst[a]) ZR_HIP(e, hipMalloc(dst[a], N * sizeof(double)));
+    if (!*dst[a]) ZR_HIP(e, dev_malloc(e, dst[a], N * sizeof(double)));
     for (size_t i = 0; i < N; ++i) tmp[i] = src[a] ? src[a][i] : dflt[a];
     ZR_HIP(e, hipMemcpy(*dst[a], tmp.data(), N * sizeof(double), hipMemcpyHostToDevice));
   }
-  if (!e->pf_allow) ZR_HIP(e, hipMalloc(&e->pf_allow, N * sizeof(int32_t)));
+  if (!e->pf_allow) ZR_HIP(e, dev_malloc(e, &e->pf_allow, N * sizeof(int32_t)));
   std::vector<int32_t> al(N, 1);
   if (pf->allow_damage)
     for (size_t i = 0; i < N; ++i) al[i] = pf->allow_damage[i] ? 1 : 0;
@@ -4116,7 +4195,7 @@ int ckpt_save(zr_engine* e, int32_t slot)
     e->ckpt[slot] = e->ckpt_spare.back();
     e->ckpt_spare.pop_back();
   }
-  if (!e->ckpt[slot]) ZR_HIP(e, hipMalloc(&e->ckpt[slot], 24 * (N ? N : 1) * sizeof(double)));
+  if (!e->ckpt[slot]) ZR_HIP(e, dev_malloc(e, &e->ckpt[slot], 24 * (N ? N : 1) * sizeof(double)));
   if (N) {
     k_ckpt_copy<<<blocks_for(N, 256), 256, 0, e->stream>>>(e->x, e->v, e->C, e->F, e->ckpt[slot], (uint32_t)N, 1,
                                                            e->permuted ? e->uid : nullptr);
@@ -4585,7 +4664,7 @@ int zr_debug_dump(zr_engine* e, int32_t what, void* host, size_t bytes)
   ZR_HIP(e, hipStreamSynchronize(s));
   if (what == ZR_DUMP_SORTER || what == ZR_DUMP_BASE_OFFSET) {
     uint64_t* tmp = nullptr;
-    ZR_HIP(e, hipMalloc(&tmp, n * sizeof(uint64_t)));
+    ZR_HIP(e, dev_malloc(e, &tmp, n * sizeof(uint64_t)));
     if (what == ZR_DUMP_SORTER)
       k_dump_sorter<<<blocks_for(n, 256), 256, 0, s>>>(n, e->order, e->p_page, e->p_re, tmp);
     else
@@ -4673,8 +4752,8 @@ int zr_debug_dump(zr_engine* e, int32_t what, void* host, size_t bytes)
   if (what == ZR_DUMP_NODE_IDX) {
     uint32_t* sc = nullptr;
     int64_t* idx = nullptr;
-    ZR_HIP(e, hipMalloc(&sc, (size_t)nn * sizeof(uint32_t)));
-    ZR_HIP(e, hipMalloc(&idx, (size_t)nn * sizeof(int64_t)));
+    ZR_HIP(e, dev_malloc(e, &sc, (size_t)nn * sizeof(uint32_t)));
+    ZR_HIP(e, dev_malloc(e, &idx, (size_t)nn * sizeof(int64_t)));
     int rc = run_scan(e, LdNonzeroMass{ e->gm }, nn, sc, e->dcount + CNT_TOTAL);
     if (rc == ZR_OK) {
       k_node_idx<<<blocks_for(nn, 256), 256, 0, s>>>(nn, e->gm, sc, idx);

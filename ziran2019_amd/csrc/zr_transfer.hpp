@@ -214,7 +214,7 @@ int transfer_arrays(zr_engine* e, const HostArray* items, int count, bool to_hos
   if (e->io_threads < threads) {
     dfree(e->io_dev);
     e->io_threads = 0;
-    ZR_HIP(e, hipMalloc(&e->io_dev, (size_t)threads * kWindow * sizeof(double)));
+    ZR_HIP(e, dev_malloc(e, &e->io_dev, (size_t)threads * kWindow * sizeof(double)));
     e->io_threads = threads;
   }
   for (int t = 0; t < threads; ++t)
