@@ -5,6 +5,7 @@ TimeStepping::nextDt, SimulationBase.h:288-321, TimeStepping.h:45-80) through
 the Python binding and the C++ host against the oracle's frame loop."""
 import os
 import subprocess
+import time
 
 import numpy as np
 import pytest
@@ -181,3 +182,22 @@ def test_rollout_stops_after_the_restart_step():
         assert np.array_equal(got[key], states[3][key]), key
     for e in (a, b, c):
         e.close()
+
+
+def test_a_long_step_leaves_the_processor():
+    """20,000 particles in one page, whose sort takes tens of milliseconds:
+    the host looks for the counts without a pause for 2 ms only."""
+    n = 20000
+    rng = np.random.default_rng(1)
+    s = dict(X=(20.6 + 0.8 * rng.random((n, 3))) / 64, V=np.zeros((n, 3)), C=np.zeros((n, 9)),
+             F=np.tile(np.eye(3).reshape(1, 9), (n, 1)), mass=np.full(n, 1e-3), vol=np.full(n, 1e-6),
+             mu=np.full(n, 1e3), lam=np.full(n, 1e3), dx=1.0 / 64)
+    eng = MpmEngine(dx=s["dx"])
+    eng.upload(s)
+    eng.advanceOneTimeStep(1e-6)
+    wall, cpu = -time.perf_counter(), -time.process_time()
+    for _ in range(3):
+        eng.advanceOneTimeStep(1e-6)
+    wall, cpu = wall + time.perf_counter(), cpu + time.process_time()
+    eng.close()
+    assert wall > 0.03 and cpu < 0.5 * wall, (wall, cpu)
