@@ -1874,22 +1874,22 @@ int prof_mark(zr_engine* e, int k)
 
 // Waits for what a kernel stores in pinned memory.  The host watches for it,
 // which saves some 10 us against a device to host copy and a stream
-// synchronisation, and for 2 ms without a pause (the runtime's own wait does
-// not give the core up either).  A longer wait is long against the 100 us that
+// synchronisation, and for some 2 ms without a pause (in processor cycles; the
+// runtime's own wait does not give the core up either).  A longer wait is long against the 100 us that
 // a sleep may end late; every 32nd asks the stream, so that a failed kernel ends
 // the wait.  A step of one page of 20,000 particles, whose sort takes 69 ms: 4 to 14
 // ms of processor time, against 69 to 82 without the sleeps or with
 // hipStreamSynchronize.
-constexpr auto kSpinTime = std::chrono::milliseconds(2);
+constexpr uint64_t kSpinCycles = 5000000;
 template <class F>
 int wait_pinned(zr_engine* e, F arrived)
 {
-  const auto from = std::chrono::steady_clock::now();
+  const uint64_t from = __builtin_ia32_rdtsc();
   for (uint32_t spins = 1; !arrived(); ++spins) {
     __builtin_ia32_pause();
-    if (spins % 128u != 0u || std::chrono::steady_clock::now() - from < kSpinTime) continue;
+    if (spins % 1024u != 0u || __builtin_ia32_rdtsc() - from < kSpinCycles) continue;
     for (int k = 0; k < 32 && !arrived(); ++k) std::this_thread::sleep_for(std::chrono::microseconds(50));
-    spins = 127u;  // no more looks without a sleep
+    spins = 1023u;  // no more looks without a sleep
     const hipError_t st = arrived() ? hipErrorNotReady : hipStreamQuery(e->stream);
     if (st == hipErrorNotReady)
       (void)hipGetLastError();  // no failure, for the next launch's check
