@@ -2,13 +2,15 @@
 the gradient scatters of the implicit and ADMM steps) where their splits can
 go wrong: cells of one to nine particles (a product takes four at a time),
 cells that a chunk of particles cuts, pages at and past a chunk of 256 and of
-304 particles, one cell with a whole page's particles, and a page past the
-2,048 keys that a block sorts in one piece."""
+304 particles, one cell with a whole page's particles, a page past the 2,048
+keys that a block sorts in one piece, and pages on both sides of the line where
+cells are shared by more threads."""
 import numpy as np
 import pytest
 
 import oracle
-from ziran2019_amd.engine import (ZR_FP32_REFINED, ZR_MODEL_STVK_HENCKY, admm_opts, implicit_opts)
+from ziran2019_amd.engine import (ZR_FP32_REFINED, ZR_MODEL_STVK_HENCKY, admm_opts, implicit_opts,
+                                  phase_field_opts)
 from _helpers import make_pair, perturbed, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -26,6 +28,12 @@ COUNTS = {
     "one cell 700": [0] * 31 + [700],
     "cut cells": [40, 0, 250, 0, 20, 3, 0, 300] + [0] * 23 + [1],
     "2300": [72] * 31 + [68],
+    # past 1,216 particles, the empty cells' threads take parts of the others
+    "one cell 1216": [0] * 9 + [1216] + [0] * 22,
+    "one cell 1217": [0] * 9 + [1217] + [0] * 22,
+    "three cells 2600": [700] + [0] * 20 + [1890] + [0] * 9 + [10],
+    "16 cells 1300": [81, 0] * 15 + [85, 0],
+    "17 cells 1300": [80, 0] * 14 + [80, 50, 50, 80],
 }
 
 
@@ -116,4 +124,28 @@ def test_admm_step(counts, precision):
         assert rel_err(out[k], r) < tol, k
     assert rel_err(st["F"], ref["F"]) < tol
     assert rel_err(st["y"], ref["y"]) < tol * (1 if precision == 0 else 10)
+    eng.close()
+
+
+@pytest.mark.parametrize("counts", list(COUNTS.values())[6:], ids=list(COUNTS)[6:])
+@pytest.mark.parametrize("M", [0.0, 15.0])
+def test_phase_field_solve(counts, M):
+    """The damage solve's sums of two and of four values (the parity tests'
+    bounds; M > 0 makes the system diagonally dominant)."""
+    s = _scene(counts)
+    eng, ora = make_pair(s)
+    kw = dict(l0=0.5 * s["dx"], one_over_sigma_c=np.full(len(s["mass"]), 0.02))
+    eng.set_phase_field(phase_field_opts(parabolic_M=M, cg_tolerance=0.0), **kw)
+    ora.set_phase_field(oracle.pf_opts(parabolic_M=M, cg_tolerance=0.0), **kw)
+    eng.sortParticlesAndPolluteGrid()
+    eng.particlesToGrid()
+    ora.sort_and_pollute()
+    ora.update_stress()
+    ora.p2g()
+    eng.phase_field_solve(1e-4)
+    ora.phase_field_solve(1e-4)
+    pg, po = eng.get_phase_field(), ora.get_phase_field()
+    assert rel_err(pg["c"], po["c"]) < 1e-10
+    assert rel_err(pg["H"], po["H"]) < 1e-12
+    assert rel_err(pg["pf_Fp"], po["pf_Fp"]) < 1e-12
     eng.close()

@@ -703,6 +703,12 @@ __constant__ HvpTaskSlots kHvpTaskSlots = hvp_task_slots();
 // k_be_scatter 1M 82 -> 79 -> 74 us, 2.1M 146 -> 123 -> 110; k_admm_op32
 // 2.1M 119 -> 109 -> 108 (with the launches past the end of a solve).
 // The same for NF scalars times w (GRAD false), in the phase field's solve.
+// Where a crowded group's particles lie in few cells, each cell is shared by as
+// many times nine threads as the empty cells leave, every part'th particle to
+// one, and their sums are added in order (20,000 particles in each of two cells:
+// k_be_scatter 1255 us with nine threads a cell, 758 with LDS adds, 106 so).
+// Groups up to kSumCrowded, 76 particles per cell where the parts begin, have
+// nine threads a cell: there the additions in turn cost what the parts save.
 constexpr int kSumThreads = 320, kSumChunk = 304;
 constexpr int kSumStride = kSumChunk + 1;  // of the rows
 template <int NF, bool GRAD>
@@ -714,7 +720,9 @@ struct CellSums {
   } u;
   uint32_t coff[kCells + 1];    // the cells' runs, in the sort's order of cells
   int order[kCells];            // the cells by falling number of particles
+  int parts;                    // threads that share a task
 };
+constexpr uint32_t kSumCrowded = 4u * kSumChunk;
 static_assert(kCells * kAB <= kSumThreads && kSumChunk <= kSumThreads && kTileNodes <= kSumThreads,
               "a thread per task, particle and node");
 // cell (bits x, y y, z z from the lowest) in the sort's order of cells
@@ -736,6 +744,18 @@ __device__ __forceinline__ void cell_sums_begin(CS& cs, const uint32_t* cell_off
     rank += (ck > cnt || (ck == cnt && k < tid)) ? 1 : 0;
   }
   if (tid < kCells) cs.order[rank] = ((tid >> 4) & 1) | (((tid >> 2) & 3) << 1) | ((tid & 3) << 3);
+  const int used = __popcll(__ballot(cnt > 0));
+  if (tid == 0) cs.parts = n > kSumCrowded ? kCells / used : 1;
+}
+// thread t's task: cell by count, stencil offset (a, b), part
+struct SumTask {
+  int rk, ab, part;
+};
+__device__ __forceinline__ SumTask sum_task(int t, int parts)
+{
+  const int rk = t / kAB;
+  if (parts == 1) return { rk, t - rk * kAB, 0 };
+  return { rk / parts, t - rk * kAB, rk % parts };
 }
 template <int NF, bool GRAD>
 __device__ __forceinline__ void cell_sums_put(CellSums<NF, GRAD>& cs, int p, const double* v, const double f[3])
@@ -753,15 +773,16 @@ __device__ __forceinline__ void cell_sums_chunk(const CellSums<NF, GRAD>& cs, ui
                                                 double acc[NF][3])
 {
   constexpr int NV = CellSums<NF, GRAD>::NV;
-  const int rk = (int)threadIdx.x / kAB, ab = (int)threadIdx.x - rk * kAB;
-  if (rk >= kCells) return;
-  const int e = cs.order[rk], a = ab / 3, b = ab - 3 * a;
+  if (threadIdx.x >= (uint32_t)(kCells * kAB)) return;
+  const int parts = __builtin_amdgcn_readfirstlane(cs.parts);
+  const SumTask t = sum_task((int)threadIdx.x, parts);
+  const int e = cs.order[t.rk], a = t.ab / 3, b = t.ab - 3 * a;
   const uint32_t b0 = cs.coff[sum_cell_slot(e)], b1 = cs.coff[sum_cell_slot(e) + 1];
   const uint32_t jb = b0 > c0 ? b0 - c0 : 0u;
   const uint32_t je = b1 > c0 ? (b1 - c0 < count ? b1 - c0 : count) : 0u;
   const double sx = 1.5 - 0.5 * a, kx = a == 1 ? -1.0 : 0.5, ex = a == 1 ? 0.75 : 0.0;
   const double sy = 1.5 - 0.5 * b, ky = b == 1 ? -1.0 : 0.5, ey = b == 1 ? 0.75 : 0.0;
-  for (uint32_t j = jb; j < je; ++j) {
+  for (uint32_t j = jb + (uint32_t)t.part; j < je; j += (uint32_t)parts) {
     const double* q = cs.u.row + j;
     const double tx = q[NV * kSumStride] - sx, ty = q[(NV + 1) * kSumStride] - sy, f2 = q[(NV + 2) * kSumStride];
     const double hx = kx * tx, hy = ky * ty;
@@ -793,15 +814,26 @@ template <int NF, bool GRAD>
 __device__ __forceinline__ void cell_sums_store(CellSums<NF, GRAD>& cs, const double acc[NF][3], double* out)
 {
   const int t = threadIdx.x;
-  const int rk = t / kAB, ab = t - rk * kAB;
-  if (rk < kCells) {
-    const uint32_t ts = kHvpTaskSlots.v[cs.order[rk] * kAB + ab];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int r = 0; r < NF; ++r) cs.u.contrib[r][(ts >> (10 * c)) & 1023u] = acc[r][c];
+  const int parts = __builtin_amdgcn_readfirstlane(cs.parts);
+  const SumTask st = sum_task(t, parts);
+  const bool has = t < kCells * kAB;
+  const uint32_t ts = has ? kHvpTaskSlots.v[cs.order[st.rk] * kAB + st.ab] : 0u;
+  if (parts > 1) {  // not every cell has a thread
+    for (int k = t; k < NF * kCells * kAB * 3; k += kSumThreads) (&cs.u.contrib[0][0])[k] = 0.0;
+    __syncthreads();
   }
-  __syncthreads();
+  for (int p = 0; p < parts; ++p) {
+    if (has && st.part == p) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int r = 0; r < NF; ++r) {
+          double& to = cs.u.contrib[r][(ts >> (10 * c)) & 1023u];
+          to = p > 0 ? to + acc[r][c] : acc[r][c];
+        }
+    }
+    __syncthreads();
+  }
   if (t >= kTileNodes) return;
   const int tx = t / (kTileY * kTileZ), ty = (t / kTileZ) % kTileY, tz = t % kTileZ;
   const int k0 = hvp_node_off(tx, ty, tz), nk = hvp_na(tx) * hvp_nb(ty) * hvp_nb(tz);
