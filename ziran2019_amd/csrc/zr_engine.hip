@@ -1584,18 +1584,18 @@ struct zr_engine {
   double* g2p_gradv = nullptr;  // set around the APIC G2P whose grad v a step needs
   bool visco = false;
   // phase field: per particle (c, H, l0, 1/sigma_c, pf_Fp, H_max, k, vol, allow)
-  // and per node (phase, rhs, D, x, r, mr, s, q) of the damage solve
+  // and per node (phase, D, x, r, mr, s, q) of the damage solve
   bool pf_on = false;
   zr_phase_field_opts pf_opts{};
   zr_phase_field_stats pf_stats{};
   double *pf_c = nullptr, *pf_H = nullptr, *pf_l0 = nullptr, *pf_osc = nullptr, *pf_Fp = nullptr,
          *pf_Hmax = nullptr, *pf_k = nullptr, *pf_vol = nullptr;
   int32_t* pf_allow = nullptr;
-  double* pf_node = nullptr;  // 8 x grid capacity
+  double* pf_node = nullptr;  // 7 x grid capacity
   size_t pf_node_cap = 0;
   double* pf_partial = nullptr;
-  // differentiable form: particle adjoints [38][n] (x 3, v 3, C 9, F 9, mu,
-  // lambda, G2P scratch x 3 and F 9), node adjoints [7][grid capacity],
+  // differentiable form: particle adjoints [56][n] (x 3, v 3, C 9, F 9, mu,
+  // lambda, G2P scratch x 3 and F 9, V0 tau 9 and its adjoint 9), node adjoints [7][grid capacity],
   // device checkpoints of (x, v, C, F) with their times
   double* adj = nullptr;
   int64_t adj_n = 0;
@@ -1640,7 +1640,6 @@ struct zr_engine {
   uint32_t* slot_page = nullptr;
   int32_t* group_nslot = nullptr;  // [8 * groups]
   int32_t* slot_src = nullptr;     // [8 * slots], capacity grid_cap / 32
-  uint32_t* ticket = nullptr;      // grid-reduction ticket, kept at zero between kernels
   uint32_t *sum_base = nullptr;
 
   uint32_t A = 0, S = 0;  // groups, slots of the current sort
@@ -1659,7 +1658,6 @@ struct zr_engine {
   uint32_t seq = 0;            // publications of the counters so far
   StepGuard guard;             // of the step being launched (deferred_step)
   uint32_t s_hint = 0;         // slots that a step launched before its counts are known has room for
-  bool move_next = false;      // the next sort moves the particles
   // what the last sort left in the dense page tables: nothing, the entries of
   // its A groups and S slots, or, where it failed on the way, anything
   enum { TABLES_CLEAN, TABLES_LISTED, TABLES_UNKNOWN } tables = TABLES_CLEAN;
@@ -1696,15 +1694,15 @@ struct zr_engine {
   // with headroom (0: read the count first)
   uint32_t a_hint = 0;
   uint32_t* cell_off = nullptr;  // [32 * groups] start of each cell's run in its group
+  // host transfers: device windows, one per thread, and their events
+  double* io_dev = nullptr;
+  int io_threads = 0;
+  hipEvent_t io_ev[kIoThreads] = {};
   // The particles' order in memory.  permuted: place k holds the caller's
   // particle uid[k]; otherwise places are the caller's indices.  alt: the
   // second copy of each per-particle array that a move writes to (the two
   // swap); disorder: sum over the steps since the last move of the share of
   // particles not next to their predecessor in the sort's order.
-  // host transfers: device windows, one per thread, and their events
-  double* io_dev = nullptr;
-  int io_threads = 0;
-  hipEvent_t io_ev[kIoThreads] = {};
   bool permuted = false;
   bool no_moves = false;  // there was no memory for the second copies
   uint32_t* uid = nullptr;
@@ -1875,11 +1873,11 @@ int prof_mark(zr_engine* e, int k)
 // Waits for what a kernel stores in pinned memory.  The host watches for it,
 // which saves some 10 us against a device to host copy and a stream
 // synchronisation, and for some 2 ms without a pause (in processor cycles; the
-// runtime's own wait does not give the core up either).  A longer wait is long against the 100 us that
-// a sleep may end late; every 32nd asks the stream, so that a failed kernel ends
-// the wait.  A step of one page of 20,000 particles, whose sort takes 69 ms: 4 to 14
-// ms of processor time, against 69 to 82 without the sleeps or with
-// hipStreamSynchronize.
+// runtime's own wait does not give the core up either).  A longer wait is long
+// against the 100 us that a sleep may end late; every 32nd asks the stream, so
+// that a failed kernel ends the wait.  A step of one page of 20,000 particles,
+// whose sort takes 69 ms: 3 to 17 ms of processor time, against 69 to 82 without
+// the sleeps or with hipStreamSynchronize.
 constexpr uint64_t kSpinCycles = 5000000;
 template <class F>
 int wait_pinned(zr_engine* e, F arrived)
@@ -1943,7 +1941,6 @@ void free_particles(zr_engine* e, bool keep = false)
   e->ckpt_time.clear();
   e->permuted = e->no_moves = false;
   e->disorder = 0.0;
-  e->move_next = false;
   e->adj_n = 0;
   dfree(e->mat); dfree(e->pparam); dfree(e->pstate); dfree(e->gdeg); dfree(e->broken);
   e->has_models = e->has_plastic = false;
@@ -2217,7 +2214,6 @@ int order_particles(zr_engine* e)
 {
   const uint32_t n = (uint32_t)e->n, nb = blocks_for(n, 256);
   e->disorder = 0.0;
-  e->move_next = false;
   if (!e->uid && hipMalloc(&e->uid, (size_t)n * sizeof(uint32_t)) != hipSuccess) {
     (void)hipGetLastError();
     e->uid = nullptr;
@@ -2275,7 +2271,6 @@ int user_order(zr_engine* e)
   if (rc) return rc;
   e->permuted = false;
   e->disorder = 0.0;
-  e->move_next = false;
   // the callers copy from and to these arrays outside the stream
   ZR_HIP(e, hipStreamSynchronize(e->stream));
   return ZR_OK;
@@ -2286,14 +2281,15 @@ int user_order(zr_engine* e)
 // k_move 225 us; k_g2p 282 -> 164 us and k_p2g 238 -> 195, the G2P's writes
 // of 24 rows reaching memory 2.2 times in partial lines before), so they
 // are moved once the steps since the last move have lost that much
-// (kDisorder); rollouts and adjoint steps keep the caller's order, which their
+// (kDisorder), by sort_finish: before the step's transfers or, in a deferred
+// step, after them; rollouts and adjoint steps keep the caller's order, which their
 // records and adjoints are in.  Below kMoveMin the arrays stay in the caches and a
 // move's launches cost more than they give.
-void note_disorder(zr_engine* e)
+bool move_due(zr_engine* e)
 {
-  if (e->no_moves || e->n < (int64_t)kMoveMin || !e->hcount[CNT_SAMPLED]) return;
+  if (e->no_moves || e->n < (int64_t)kMoveMin || !e->hcount[CNT_SAMPLED]) return false;
   e->disorder += (double)e->hcount[CNT_BREAKS] / (double)e->hcount[CNT_SAMPLED];
-  e->move_next = e->disorder >= kDisorder;
+  return e->disorder >= kDisorder;
 }
 
 // a sort that is under way: launched for `hint` groups and, where one block
@@ -2403,12 +2399,9 @@ int sort_finish(zr_engine* e, const SortRun& run, zr_step_stats* st, bool move)
   // a rollout's earlier step asked for a restart: the particles are those
   // after that step (a sort moves none)
   if (e->defer_cfl && (e->hcount[CNT_CFL_RUN] & 1u)) return ZR_CFL_RESTART;
-  if (move) {
-    note_disorder(e);
-    if (e->move_next) {
-      rc = order_particles(e);
-      if (rc) return rc;
-    }
+  if (move && move_due(e)) {
+    rc = order_particles(e);
+    if (rc) return rc;
   }
   rc = ensure_grid(e);
   if (rc) return rc;
@@ -3666,7 +3659,6 @@ int zr_create(const zr_config* cfg, zr_engine** out)
             hipMalloc(&e->page_sumcnt, e->nsum * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&e->sum_base, (e->nsum + 1) * sizeof(uint32_t)) == hipSuccess &&
             hipMalloc(&e->dbase, 3 * kBank * sizeof(uint32_t)) == hipSuccess &&
-            hipMalloc(&e->ticket, sizeof(uint32_t)) == hipSuccess &&
             hipHostMalloc(&e->hcount, CNT_N * sizeof(uint32_t), hipHostMallocCoherent) == hipSuccess;
   ok = ok && hipMemset(e->dbase, 0, 3 * kBank * sizeof(uint32_t)) == hipSuccess;
   if (ok) {
@@ -3681,7 +3673,6 @@ int zr_create(const zr_config* cfg, zr_engine** out)
        hipMemset(e->page_bits, 0, e->nwords * sizeof(uint32_t)) == hipSuccess &&
        hipMemset(e->page_sum, 0, e->nsum * sizeof(uint32_t)) == hipSuccess &&
        hipMemset(e->page_sumcnt, 0, e->nsum * sizeof(uint32_t)) == hipSuccess &&
-       hipMemset(e->ticket, 0, sizeof(uint32_t)) == hipSuccess &&
        hipDeviceSynchronize() == hipSuccess;
   if (!ok) {
     zr_destroy(e);
@@ -3698,7 +3689,7 @@ void zr_destroy(zr_engine* e)
   free_particles(e);
   dfree(e->page_count); dfree(e->page_group); dfree(e->page_touch); dfree(e->page_slot); dfree(e->page_bits);
   dfree(e->page_sum); dfree(e->page_sumcnt); dfree(e->sum_base); dfree(e->stage); dfree(e->gm); dfree(e->gv); dfree(e->gf); dfree(e->gvs);
-  dfree(e->scan_tmp); dfree(e->cell_off); dfree(e->speed); dfree(e->dbase); dfree(e->ticket); dfree(e->slot_src);
+  dfree(e->scan_tmp); dfree(e->cell_off); dfree(e->speed); dfree(e->dbase); dfree(e->slot_src);
   dfree(e->ivn); dfree(e->idv); dfree(e->ir); dfree(e->ix); dfree(e->irc); dfree(e->iq); dfree(e->ip); dfree(e->iap);
   dfree(e->partial); dfree(e->partial2); dfree(e->sc); dfree(e->ci); dfree(e->hvp_ctr); dfree(e->hvp_bounds); dfree(e->hvp_order); dfree(e->cell_order); dfree(e->jstage); dfree(e->pinv); dfree(e->collided); dfree(e->c64); dfree(e->c32); dfree(e->ccell);
   dfree(e->pf_node); dfree(e->pf_partial); dfree(e->adj_grid); dfree(e->admm_node); dfree(e->admm_coll); dfree(e->act); dfree(e->act_scan); dfree(e->be_fb); dfree(e->admm_c32); dfree(e->admm_cell32); dfree(e->admm_node32); dfree(e->admm_before); dfree(e->admm_differs);
@@ -4419,12 +4410,13 @@ int zr_grid_to_particles(zr_engine* e, double dt, zr_step_stats* st)
 // headroom, and stop at the device-side counts (StepGuard).  Counts beyond the
 // launch leave the particles as they were, and the step runs again from its
 // sort's lists with the counts known (`again`).  1,728 particles: 113 -> 71 us
-// a substep (with calculateDt's wait, likewise shortened).  For the sizes whose slots one
-// block assigns; larger steps are long against a wait, and a step that moves
-// the particles or solves for damage needs the counts on the way.
+// a substep (with calculateDt's wait, likewise shortened).  For the sizes whose
+// slots one block assigns; larger steps are long against a wait, and a step that
+// solves for damage needs the counts on the way.  Particles that are due to move
+// do so after the step, in the order of its sort.
 static bool deferred_step_possible(const zr_engine* e)
 {
-  return !e->pf_on && !e->defer_cfl && !e->move_next && e->n > 0 && e->a_hint > 0 && e->a_hint <= kSlotsMax &&
+  return !e->pf_on && !e->defer_cfl && e->n > 0 && e->a_hint > 0 && e->a_hint <= kSlotsMax &&
          e->nsum <= kListMax && e->slot_src && e->s_hint > 0;
 }
 static int deferred_step(zr_engine* e, double dt, zr_step_stats* st, bool& again)

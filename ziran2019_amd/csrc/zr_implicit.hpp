@@ -232,24 +232,6 @@ __device__ __forceinline__ void load_tile3(const int32_t* gslot, const TS* a, co
   __syncthreads();
 }
 
-// tile load from the group's precomputed neighbour slots (8 entries)
-template <class T, class TS>
-__device__ __forceinline__ void load_tile3_slots(const int32_t* gslot, const TS* a, int64_t stride, T* tv,
-                                                 int32_t* nslot)
-{
-  const int tid = threadIdx.x;
-  if (tid < 8) nslot[tid] = gslot[tid];
-  __syncthreads();
-  for (int t = tid; t < kTileNodes; t += blockDim.x) {
-    const int tx = t / (kTileY * kTileZ), ty = (t / kTileZ) % kTileY, tz = t % kTileZ;
-    const int32_t sl = nslot[((tx >> 1) << 2) | ((ty >> 2) << 1) | (tz >> 2)];
-    const int64_t node = (int64_t)sl * 32 + elem_of(tx, ty, tz);
-    for (int d = 0; d < 3; ++d) tv[d * kTileNodes + t] = sl >= 0 ? (T)a[d * stride + node] : (T)0;
-  }
-  __syncthreads();
-}
-
-// CG search direction on the fly: p_new = q + beta p_old for the tile nodes
 // tile node t (< kTileNodes) of a group's 4x6x6 footprint: which of the 8
 // neighbour page slots holds it (4a + 2b + c) and its element in that page
 __device__ __forceinline__ void tile_node_source(int t, int& src, int& elem)
@@ -1672,17 +1654,6 @@ __global__ __launch_bounds__(256) void k_be_residual(uint32_t nn, const uint32_t
     for (int d = 0; d < 3; ++d) r(d, k) = rv[d];
   }
   block_partial(contrib, partial);
-}
-
-// sums nb partials in index order into sc[slot]; skipped once CG is done
-__global__ __launch_bounds__(256) void k_reduce(const double* __restrict__ partial, uint32_t nb, double* sc, int slot,
-                                                const int32_t* ci)
-{
-  __shared__ double smem[4];
-  if (ci && ci[CI_DONE]) return;
-  const double acc = thread_partials256(partial, nb);
-  const double s = block_sum256(acc, smem);
-  if (threadIdx.x == 0) sc[slot] = s;
 }
 
 // JacobiPreconditioner (KrylovSolvers.h:32-57) on the operator's diagonal
