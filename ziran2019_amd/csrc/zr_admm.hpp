@@ -978,11 +978,12 @@ __global__ __launch_bounds__(kSumThreads, 4) void k_admm_op64(ParticlesView P, A
       }
       cell_sums_put(cs, tid, &D[0][0], f);
     }
+    cell_sums_split(cs, n, c0, count);
     __syncthreads();
     cell_sums_chunk(cs, c0, count, acc);
     __syncthreads();
   }
-  cell_sums_store(cs, acc, stage + (size_t)g * (3 * kTileNodes));
+  cell_sums_store(cs, n, acc, stage + (size_t)g * (3 * kTileNodes));
 }
 
 __device__ __forceinline__ void admm_project_node(const AdmmNodes& N, uint32_t k, double r[3])
@@ -1251,11 +1252,12 @@ __global__ __launch_bounds__(kSumThreads, 6) void k_admm_op32(AdmmCache32 C, con
       }
       cell_sums_put(cs, tid, &D64[0][0], f64);
     }
+    cell_sums_split(cs, n, c0, count);
     __syncthreads();
     cell_sums_chunk(cs, c0, count, acc);
     __syncthreads();
   }
-  cell_sums_store(cs, acc, stage + (size_t)g * (3 * kTileNodes));
+  cell_sums_store(cs, n, acc, stage + (size_t)g * (3 * kTileNodes));
 }
 
 

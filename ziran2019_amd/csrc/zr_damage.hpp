@@ -92,11 +92,12 @@ __global__ __launch_bounds__(kSumThreads) void k_pf_p2g(ParticlesView P, PfParti
       }
       cell_sums_put(cs, tid, v, f);
     }
+    cell_sums_split(cs, n, c0, count);
     __syncthreads();
     cell_sums_chunk(cs, c0, count, acc);
     __syncthreads();
   }
-  cell_sums_store(cs, acc, stage + (size_t)g * (NF * kTileNodes));
+  cell_sums_store(cs, n, acc, stage + (size_t)g * (NF * kTileNodes));
 }
 
 // block partials of two sums, the second set after the first

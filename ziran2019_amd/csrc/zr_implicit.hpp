@@ -702,7 +702,8 @@ struct CellSums {
   } u;
   uint32_t coff[kCells + 1];    // the cells' runs, in the sort's order of cells
   int order[kCells];            // the cells by falling number of particles
-  int parts;                    // threads that share a task
+  uint32_t lo[kCells], hi[kCells];  // the particles of each nine threads
+  int parts;                    // of a crowded group: how many of these a cell has
 };
 constexpr uint32_t kSumCrowded = 4u * kSumChunk;
 static_assert(kCells * kAB <= kSumThreads && kSumChunk <= kSumThreads && kTileNodes <= kSumThreads,
@@ -725,19 +726,15 @@ __device__ __forceinline__ void cell_sums_begin(CS& cs, const uint32_t* cell_off
     const int ck = __builtin_amdgcn_readlane(cnt, k);
     rank += (ck > cnt || (ck == cnt && k < tid)) ? 1 : 0;
   }
-  if (tid < kCells) cs.order[rank] = ((tid >> 4) & 1) | (((tid >> 2) & 3) << 1) | ((tid & 3) << 3);
-  const int used = __popcll(__ballot(cnt > 0));
-  if (tid == 0) cs.parts = n > kSumCrowded ? kCells / used : 1;
-}
-// thread t's task: cell by count, stencil offset (a, b), part
-struct SumTask {
-  int rk, ab, part;
-};
-__device__ __forceinline__ SumTask sum_task(int t, int parts)
-{
-  const int rk = t / kAB;
-  if (parts == 1) return { rk, t - rk * kAB, 0 };
-  return { rk / parts, t - rk * kAB, rk % parts };
+  if (tid < kCells) {
+    cs.order[rank] = ((tid >> 4) & 1) | (((tid >> 2) & 3) << 1) | ((tid & 3) << 3);
+    cs.lo[rank] = c;
+    cs.hi[rank] = next;
+  }
+  if (n > kSumCrowded) {
+    const int used = __popcll(__ballot(cnt > 0));
+    if (tid == 0) cs.parts = kCells / used;
+  }
 }
 template <int NF, bool GRAD>
 __device__ __forceinline__ void cell_sums_put(CellSums<NF, GRAD>& cs, int p, const double* v, const double f[3])
@@ -748,6 +745,20 @@ __device__ __forceinline__ void cell_sums_put(CellSums<NF, GRAD>& cs, int p, con
 #pragma unroll
   for (int d = 0; d < 3; ++d) cs.u.row[(NV + d) * kSumStride + p] = f[d];
 }
+// before the chunk [c0, c0 + count) of a group of n particles, before its
+// barrier: a crowded group's cells cut into their parts
+template <class CS>
+__device__ __forceinline__ void cell_sums_split(CS& cs, uint32_t n, uint32_t c0, uint32_t count)
+{
+  if (n <= kSumCrowded || threadIdx.x >= (uint32_t)kCells) return;
+  const uint32_t parts = (uint32_t)cs.parts, part = threadIdx.x % parts;
+  const int slot = sum_cell_slot(cs.order[threadIdx.x / parts]);
+  const uint32_t b0 = cs.coff[slot] > c0 ? cs.coff[slot] : c0;
+  const uint32_t b1 = cs.coff[slot + 1] < c0 + count ? cs.coff[slot + 1] : c0 + count;
+  const uint32_t len = b1 > b0 ? b1 - b0 : 0u;
+  cs.lo[threadIdx.x] = b0 + len * part / parts;
+  cs.hi[threadIdx.x] = b0 + len * (part + 1u) / parts;
+}
 // this thread's task's sums over the chunk [c0, c0 + count) of the group,
 // added to acc[field][c]; between barriers
 template <int NF, bool GRAD>
@@ -755,16 +766,15 @@ __device__ __forceinline__ void cell_sums_chunk(const CellSums<NF, GRAD>& cs, ui
                                                 double acc[NF][3])
 {
   constexpr int NV = CellSums<NF, GRAD>::NV;
-  if (threadIdx.x >= (uint32_t)(kCells * kAB)) return;
-  const int parts = __builtin_amdgcn_readfirstlane(cs.parts);
-  const SumTask t = sum_task((int)threadIdx.x, parts);
-  const int e = cs.order[t.rk], a = t.ab / 3, b = t.ab - 3 * a;
-  const uint32_t b0 = cs.coff[sum_cell_slot(e)], b1 = cs.coff[sum_cell_slot(e) + 1];
+  const int rk = (int)threadIdx.x / kAB, ab = (int)threadIdx.x - rk * kAB;
+  if (rk >= kCells) return;
+  const int a = ab / 3, b = ab - 3 * a;
+  const uint32_t b0 = cs.lo[rk], b1 = cs.hi[rk];
   const uint32_t jb = b0 > c0 ? b0 - c0 : 0u;
   const uint32_t je = b1 > c0 ? (b1 - c0 < count ? b1 - c0 : count) : 0u;
   const double sx = 1.5 - 0.5 * a, kx = a == 1 ? -1.0 : 0.5, ex = a == 1 ? 0.75 : 0.0;
   const double sy = 1.5 - 0.5 * b, ky = b == 1 ? -1.0 : 0.5, ey = b == 1 ? 0.75 : 0.0;
-  for (uint32_t j = jb + (uint32_t)t.part; j < je; j += (uint32_t)parts) {
+  for (uint32_t j = jb; j < je; ++j) {
     const double* q = cs.u.row + j;
     const double tx = q[NV * kSumStride] - sx, ty = q[(NV + 1) * kSumStride] - sy, f2 = q[(NV + 2) * kSumStride];
     const double hx = kx * tx, hy = ky * ty;
@@ -793,29 +803,34 @@ __device__ __forceinline__ void cell_sums_chunk(const CellSums<NF, GRAD>& cs, ui
 }
 // after a barrier: the group's sums into its staged tile
 template <int NF, bool GRAD>
-__device__ __forceinline__ void cell_sums_store(CellSums<NF, GRAD>& cs, const double acc[NF][3], double* out)
+__device__ __forceinline__ void cell_sums_store(CellSums<NF, GRAD>& cs, uint32_t n, const double acc[NF][3],
+                                                double* out)
 {
-  const int t = threadIdx.x;
-  const int parts = __builtin_amdgcn_readfirstlane(cs.parts);
-  const SumTask st = sum_task(t, parts);
-  const bool has = t < kCells * kAB;
-  const uint32_t ts = has ? kHvpTaskSlots.v[cs.order[st.rk] * kAB + st.ab] : 0u;
-  if (parts > 1) {  // not every cell has a thread
-    for (int k = t; k < NF * kCells * kAB * 3; k += kSumThreads) (&cs.u.contrib[0][0])[k] = 0.0;
-    __syncthreads();
-  }
-  for (int p = 0; p < parts; ++p) {
-    if (has && st.part == p) {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // not held from the chunks' loop
+  const int rk = t / kAB, ab = t - rk * kAB;
+  if (n <= kSumCrowded) {
+    if (rk < kCells) {
+      const uint32_t ts = kHvpTaskSlots.v[cs.order[rk] * kAB + ab];
 #pragma unroll
       for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int r = 0; r < NF; ++r) {
-          double& to = cs.u.contrib[r][(ts >> (10 * c)) & 1023u];
-          to = p > 0 ? to + acc[r][c] : acc[r][c];
-        }
+        for (int r = 0; r < NF; ++r) cs.u.contrib[r][(ts >> (10 * c)) & 1023u] = acc[r][c];
     }
-    __syncthreads();
+  } else {  // the parts in order, onto zeros (not every cell has a thread)
+    const int parts = cs.parts;
+    for (int k = t; k < NF * kCells * kAB * 3; k += kSumThreads) (&cs.u.contrib[0][0])[k] = 0.0;
+    const uint32_t ts = rk < kCells ? kHvpTaskSlots.v[cs.order[rk / parts] * kAB + ab] : 0u;
+    for (int p = 0; p < parts; ++p) {
+      __syncthreads();
+      if (rk < kCells && rk % parts == p)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int r = 0; r < NF; ++r) cs.u.contrib[r][(ts >> (10 * c)) & 1023u] += acc[r][c];
+    }
   }
+  __syncthreads();
   if (t >= kTileNodes) return;
   const int tx = t / (kTileY * kTileZ), ty = (t / kTileZ) % kTileY, tz = t % kTileZ;
   const int k0 = hvp_node_off(tx, ty, tz), nk = hvp_na(tx) * hvp_nb(ty) * hvp_nb(tz);
@@ -997,11 +1012,12 @@ __global__ __launch_bounds__(kSumThreads) void k_be_scatter(ParticlesView P, con
         for (int r = 0; r < 3; ++r) D[r][c] = inv_dx * fb[(c * 3 + r) * cstride + ks];
       cell_sums_put(cs, tid, &D[0][0], f);
     }
+    cell_sums_split(cs, n, c0, count);
     __syncthreads();
     cell_sums_chunk(cs, c0, count, acc);
     __syncthreads();
   }
-  cell_sums_store(cs, acc, stage + (size_t)g * kImpStage);
+  cell_sums_store(cs, n, acc, stage + (size_t)g * kImpStage);
 }
 
 // particles per chunk of the operator apply, and the waves per SIMD its LDS
