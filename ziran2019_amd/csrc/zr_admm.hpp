@@ -921,8 +921,8 @@ __global__ __launch_bounds__(256) void k_admm_flocal(ParticlesView P, AdmmPartic
 
 // the global operator's particle term c_p (grad(x) Fn) Fn^T grad w in FP64,
 // c_p = rho omega^2 dt^2; VISCO adds the viscoelastic branch's with FFn.
-// (Four waves per SIMD, with 2 to 6 registers in scratch, so that three blocks
-// fit a CU: 40k 9.7 us, against 13.2 with two.)
+// (Four waves per SIMD, 120 registers, so that three blocks fit a CU: 40k 9.7
+// us, against 13.2 with two.)
 template <bool VISCO>
 __global__ __launch_bounds__(kSumThreads, 4) void k_admm_op64(ParticlesView P, AdmmParticles A, AdmmNodes N,
                                                    const double* __restrict__ xvec,

@@ -685,12 +685,13 @@ __constant__ HvpTaskSlots kHvpTaskSlots = hvp_task_slots();
 // k_be_scatter 1M 82 -> 79 -> 74 us, 2.1M 146 -> 123 -> 110; k_admm_op32
 // 2.1M 119 -> 109 -> 108 (with the launches past the end of a solve).
 // The same for NF scalars times w (GRAD false), in the phase field's solve.
-// Where a crowded group's particles lie in few cells, each cell is shared by as
-// many times nine threads as the empty cells leave, every part'th particle to
-// one, and their sums are added in order (20,000 particles in each of two cells:
-// k_be_scatter 1255 us with nine threads a cell, 758 with LDS adds, 106 so).
-// Groups up to kSumCrowded, 76 particles per cell where the parts begin, have
-// nine threads a cell: there the additions in turn cost what the parts save.
+// Where a crowded group's particles lie in few cells, a cell's run in the chunk
+// is cut into as many parts as the empty cells leave threads for, nine threads
+// to each, and the parts' sums are added in order (20,000 particles in each of
+// two cells: k_be_scatter 1255 us with nine threads a cell, 758 with LDS adds,
+// 106 so).  Groups up to kSumCrowded, 38 particles in each of 32 cells, keep nine
+// threads a cell: body surfaces leave cells empty too, and there the cuts and the
+// additions in turn cost what the parts save.
 constexpr int kSumThreads = 320, kSumChunk = 304;
 constexpr int kSumStride = kSumChunk + 1;  // of the rows
 template <int NF, bool GRAD>
