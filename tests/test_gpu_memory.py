@@ -131,3 +131,16 @@ def test_second_copies_are_given_back():
         eng.checkpoint_restore(0)
         _same(eng.download(), want)
     eng.close()
+
+
+def test_an_engine_that_finds_no_memory_fails_alone():
+    """The page tables of an extent of 2^12 nodes take 34 GB; another engine's
+    next step does not report their failure."""
+    cube = scenes.cube_scene_small(seed=3, ncells=4)
+    eng, _ = make_pair(cube)
+    eng.advanceOneTimeStep(1e-4)
+    with device_memory_held(eng.L, 64 << 20):
+        with pytest.raises(ZrError):
+            MpmEngine(dx=cube["dx"], grid_log2=12)
+        eng.advanceOneTimeStep(1e-4)
+    eng.close()

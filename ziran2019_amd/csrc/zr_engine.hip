@@ -1595,8 +1595,8 @@ struct zr_engine {
   size_t pf_node_cap = 0;
   double* pf_partial = nullptr;
   // differentiable form: particle adjoints [56][n] (x 3, v 3, C 9, F 9, mu,
-  // lambda, G2P scratch x 3 and F 9, V0 tau 9 and its adjoint 9), node adjoints [7][grid capacity],
-  // device checkpoints of (x, v, C, F) with their times
+  // lambda, G2P scratch x 3 and F 9, V0 tau 9 and its adjoint 9), node
+  // adjoints [7][grid capacity], device checkpoints of (x, v, C, F) with their times
   double* adj = nullptr;
   int64_t adj_n = 0;
   double* adj_grid = nullptr;
@@ -2282,9 +2282,9 @@ int user_order(zr_engine* e)
 // of 24 rows reaching memory 2.2 times in partial lines before), so they
 // are moved once the steps since the last move have lost that much
 // (kDisorder), by sort_finish: before the step's transfers or, in a deferred
-// step, after them; rollouts and adjoint steps keep the caller's order, which their
-// records and adjoints are in.  Below kMoveMin the arrays stay in the caches and a
-// move's launches cost more than they give.
+// step, after them; rollouts and adjoint steps keep the caller's order, which
+// their records and adjoints are in.  Below kMoveMin the arrays stay in the
+// caches and a move's launches cost more than they give.
 bool move_due(zr_engine* e)
 {
   if (e->no_moves || e->n < (int64_t)kMoveMin || !e->hcount[CNT_SAMPLED]) return false;
@@ -3675,6 +3675,7 @@ int zr_create(const zr_config* cfg, zr_engine** out)
        hipMemset(e->page_sumcnt, 0, e->nsum * sizeof(uint32_t)) == hipSuccess &&
        hipDeviceSynchronize() == hipSuccess;
   if (!ok) {
+    (void)hipGetLastError();  // not for another engine's next launch
     zr_destroy(e);
     return ZR_ERR_HIP;
   }
